@@ -54,7 +54,7 @@ KERNELS = {"hist": ("k_l1_hist<{key}, 0, false>", "hist_ms"),
            "l1_scatter": ("k_l1_scatter<{key}, 0, false>", "l1_scatter_ms"),
            "sort": ("k_bucket_hash<{key}>", "sort_ms"),
            "compact": ("k_compact<{key}>", "compact_ms")}
-MS_SCATTER = {1: "k_ms_scatter_p", 2: "k_ms_scatter", 3: "k_ms_scatter_seg"}
+MS_SCATTER = {4: "k_split"}
 
 
 def alg_bytes(N, U, V, M, S, W):

@@ -85,7 +85,7 @@ typedef struct pk_mn_table {
  * the kernel launches of each stage). */
 typedef struct pk_timing {
   float parse_ms;    /* line index + read table */
-  float hist_ms;     /* bucket histogram (parse pass 1) */
+  float hist_ms;     /* bucket histogram (rank shares only) */
   float scatter_ms;  /* bucket scatter (parse pass 2) */
   float sort_ms;     /* per-bucket sort + run-length count */
   float split_ms;    /* oversize-bucket splitting (0 when none) */
@@ -98,14 +98,12 @@ typedef struct pk_timing {
   int32_t n_split;      /* buckets that needed splitting */
   float l1_scatter_ms;  /* first scatter level alone (one kernel, part of scatter_ms) */
   float normalize_ms;   /* input-format normalization (pk_count_format; 0 otherwise) */
-  float ms_hist_ms;     /* further partition levels: their histogram kernels, summed */
+  float ms_hist_ms;     /* 0: no level has a histogram pass */
   float ms_scatter_ms;  /* further partition levels: their scatter kernels, summed */
   int32_t ms_levels;    /* further partition levels of the last count (timed: first 4) */
-  int32_t ms_scatter_form; /* their scatter kernel: 1 persistent blocks, 2 one block
-                              per tile, 3 segments of a histogram folded into
-                              level 1's (the last level's; 0 when none ran) */
-  float ms_level_hist_ms[4];    /* per further level (the first 4): its histogram
-                                   kernel, or with form 3 the scan of the folded counts */
+  int32_t ms_scatter_form; /* their scatter kernel: 4 tiles sorted whole (0 when
+                              none ran) */
+  float ms_level_hist_ms[4];    /* 0: no level has a histogram pass */
   float ms_level_scatter_ms[4]; /* per further level: its scatter kernel */
   int32_t ms_level_form[4];     /* per further level: its scatter form as above */
 } pk_timing;
@@ -121,22 +119,18 @@ void* pk_ctx_stream(pk_ctx* ctx);
 uint64_t pk_ctx_device_bytes(const pk_ctx* ctx);
 /* Launch-shape choices of the counting kernels (results do not depend on
  * them).  Zero fields keep the built-in choice.
- *   l1_chunks      reads per level-1 partition block, in chunks of 512 (1..64;
- *                  built-in: 1..8 by input size)
- *   l1_bits        level-1 radix digit width (1..PK_TUNING_L1_BITS_MAX; built-in 8,
- *                  or, when the bucket count needs three or more partition
- *                  levels, the narrowest width >= 5 that adds no level)
+ *   l1_chunks      rank shares: reads per level-1 partition block, in chunks
+ *                  of 512 (1..64; built-in: 1..8 by input size); other counts
+ *                  take any value and do not use it
+ *   l1_bits        level-1 radix digit width (1..PK_TUNING_L1_BITS_MAX; built-in:
+ *                  the bits of all levels spread evenly, at most 9 per level,
+ *                  or 10 where a single level does; 8 for rank shares)
  *   bucket_factor  instances per final bucket as a multiple of the LDS hash
  *                  table's key capacity, i.e. the inverse hash load target
  *                  (built-in 3.0)
- *   ms_scatter     form of the further partition levels' scatter: 1 =
- *                  persistent blocks (two per CU, consecutive tiles each),
- *                  2 = one block per tile (built-in: persistent once every
- *                  block gets >= 256 tiles)
- *   ms_fold        2 = never count the second partition level inside the
- *                  level-1 histogram (built-in: counted there when two or
- *                  more levels follow level 1 and the first two digits have
- *                  at most 8192 values; 1 = the same) */
+ *   ms_scatter     0..2, no effect (chose between two former scatter kernels)
+ *   ms_fold        0..2, no effect (switched a former histogram fold off)
+ */
 #define PK_TUNING_L1_BITS_MAX 10
 typedef struct pk_tuning {
   int32_t l1_chunks;

@@ -2,26 +2,27 @@
 // macro-node construction behind the C ABI of include/pakhip.h.
 //
 // Pipeline of pk_count (one HIP stream per context, everything resident in HBM):
-//   1. line index     k_nl_count / scan / k_nl_write: positions of every '\n'
-//                     (16 B per thread, block-scan compaction).
+//   1. packing        k_pack reads the FASTA once: two bits per input byte
+//                     (plus one exact low bit), the '\n' bits, and their count
+//                     per block; k_nl_write_rx lists the '\n' positions.
 //   2. read table     k_reads: record r = header line j0+2r, sequence line
 //                     j0+2r+1, with the record rules and the format check of
 //                     the reference's Sliding_window (src/kmer_counting.cpp:
 //                     2890-2945); k-mer offsets by exclusive scan.  The
 //                     builder API's records come from k_bld_flags/k_bld_write.
-//   3. partition      multisplit by the top bits of the k-mer.  Level 1
-//                     (k_l1_hist + k_l1_scatter, <= 10 bits) is fused with the
-//                     parse: each chunk of reads is staged in LDS and every
-//                     read is walked by one thread with the reference's rolling
-//                     3-bit update (kmer_shift, distribute_kmers.h:798-805);
-//                     every k-mer is stored at its block's next slot for its
-//                     digit.  Further levels (k_ms_hist + k_ms_scatter, <= 8
-//                     bits) split each bucket tile by tile, sorted by digit in
-//                     LDS and written as contiguous runs.  This is the on-device
-//                     stand-in for the reference's owner routing +
-//                     MPI_Alltoallv (kmer_counting.cpp:254-352); rank-share
-//                     mode keeps one owner's k-mers (own_step).
-//   4. bucket count   k_bucket_hash: one 256-thread workgroup per bucket counts
+//   3. partition      k_split: tiles of k-mers sorted by a digit of the key's
+//                     top bits, one tile per block, each tile written back
+//                     as one contiguous piece with a table of where its
+//                     digits start.  Level 1 cuts the k-mers out of the packed
+//                     bases (the reference's rolling 3-bit update,
+//                     kmer_shift, distribute_kmers.h:798-805, read off a
+//                     window of bits), further levels gather a bucket's runs
+//                     from the tiles of the level before.  This is the
+//                     on-device stand-in for the reference's owner routing +
+//                     MPI_Alltoallv (kmer_counting.cpp:254-352).  Rank-share
+//                     mode keeps one owner's k-mers (k_l1_hist, k_l1_scatter,
+//                     own_step).
+//   4. bucket count   k_bucket_hash: one 512-thread workgroup per bucket counts
 //                     the bucket's distinct keys in an LDS hash table, then
 //                     counting-sorts them by the next bits and writes the
 //                     ascending (key, count) pairs (the reference's sort + RLE
@@ -205,12 +206,6 @@ __global__ void k_fill_u64(ull* p, ull v, uint64_t n) {
 }
 
 __global__ void k_copy_u64(ull* dst, const ull* src) { *dst = *src; }
-
-// out[i] = off[i + 1] - off[i]
-__global__ void k_diff(const ull* off, uint64_t n, ull* out) {
-  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) out[i] = off[i + 1] - off[i];
-}
 
 // ---------------------------------------------------------------------------
 // Exclusive scan (u32 or u64 in, u64 out, out[n] = total).  SCAN_PER
@@ -437,6 +432,143 @@ __global__ __launch_bounds__(NL_NT) void k_nl_write(const uint8_t* fa, uint64_t 
       nl[o++] = p | (f << NL_FLAG_SHIFT);
     }
     slab_base += (tot >> (16 * j)) & 0xFFFFull;
+  }
+}
+
+// Base encodings of the two counting front ends.
+//   ENC_MAIN:    char_to_el, (c >> 1) & 7 (distribute_kmers.h:784-786): the
+//                3-bit code ORs into the previous base's low bit, and the
+//                word is masked to 2k bits (kmer_shift, :798-805).
+//   ENC_BUILDER: symbol_to_kmer (concurrent_kmer_counter.hpp:2097-2110):
+//                A C T G -> 0 1 2 3, every other byte -> 0; the word is not
+//                masked and keeps the last 4*sizeof(kmer_t) bases.
+constexpr int ENC_MAIN = 0;
+constexpr int ENC_BUILDER = 1;
+
+__device__ __forceinline__ bool base_is_acgt(uint32_t c) { return c == 'A' || c == 'C' || c == 'G' || c == 'T'; }
+
+template <int ENC>
+__device__ __forceinline__ uint32_t base_code(uint32_t c) {
+  if (ENC == ENC_MAIN) return (c >> 1) & 7u;
+  return base_is_acgt(c) ? (c >> 1) & 3u : 0u;
+}
+
+// ---------------------------------------------------------------------------
+// Packed input.  The counting path reads the input's bytes once and works on
+// two bits per byte from then on: bases, headers and line ends alike, so that
+// a k-mer of the read at byte p is the bit window of bytes [p, p + K).
+//
+//   E   one 32-bit word per 16 bytes, the first byte's field in the top two
+//       bits: the two low bits of the byte's base code, the low one ORed with
+//       the third code bit of the next byte (ENC_MAIN, the rolling update's
+//       spill into the older base; without it for ENC_BUILDER).
+//   RX  one word per 16 bytes, byte i at bit i: bits 0-15 the exact low bit
+//       of the code (a window's last base has not seen the next byte: its
+//       low bit comes from here), bits 16-31 the event bytes.  At an event
+//       byte, which is no base, bit i says instead that a '>' follows it.
+//
+// One pass over the bytes at 16 per lane, half a byte written per byte; the
+// line index is then written from RX (a quarter of the input) and the first
+// partition level reads E and RX: 2.25 bytes of traffic per input byte, where
+// the byte-wise line index, its second pass, the level-1 histogram and the
+// level-1 scatter each read the input (4 bytes).
+
+constexpr int PK_PAD = 8;  // E words before the input's first (windows reach four words back)
+
+// four 2-bit fields, one per byte of t, first byte highest
+__device__ __forceinline__ uint32_t pack_crumbs(uint32_t t) { return (t * 0x40100401u) >> 24; }
+// bit 0 of each byte of t, first byte lowest
+__device__ __forceinline__ uint32_t pack_bits(uint32_t t) { return ((t * 0x01020408u) >> 24) & 15u; }
+
+template <int ENC>
+__global__ __launch_bounds__(NL_NT) void k_pack(const uint8_t* fa, uint64_t n, uint8_t e0, uint8_t e1,
+                                                ull* blk_cnt, ull* blk_gt, int gt_all, uint32_t* E, uint32_t* RX) {
+  const uint64_t b0 = (uint64_t)blockIdx.x * NL_PER_BLOCK + (uint64_t)threadIdx.x * 16;
+  const bool want_gt = gt_all || blockIdx.x == 0;
+  const int lane = threadIdx.x & 63;
+  uint32_t ev[NL_SLABS], gm[NL_SLABS];
+  uint4 by[NL_SLABS];
+#pragma unroll
+  for (int j = 0; j < NL_SLABS; j++) by[j] = scan16(fa, n, b0 + j * NL_SLAB, e0, e1, want_gt, ev[j], gm[j]);
+  ull c = 0, gt = ~0ull;
+#pragma unroll
+  for (int j = NL_SLABS - 1; j >= 0; j--) {
+    const uint64_t base = b0 + j * NL_SLAB;
+    // the byte after these 16: the next lane's first (0 past the end)
+    uint32_t nx = __shfl_down(by[j].x, 1, 64) & 0xFFu;
+    if (lane == 63) nx = base + 16 < n ? fa[base + 16] : 0u;
+    if (base < n) {
+      const uint32_t w[5] = {by[j].x, by[j].y, by[j].z, by[j].w, nx};
+      uint32_t e = 0, r = 0;
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        uint32_t t = (w[i] >> 1) & 0x03030303u;
+        if (ENC == ENC_MAIN) {
+          r |= pack_bits(t & 0x01010101u) << (4 * i);
+          const uint32_t b = (w[i] >> 3) & 0x01010101u;  // third code bits
+          t |= (b >> 8) | (((w[i + 1] >> 3) & 1u) << 24);
+        } else {
+          // every byte but A, C, G, T counts as 0
+          uint32_t ok = 0;
+#pragma unroll
+          for (int q = 0; q < 4; q++) ok |= (uint32_t)(base_is_acgt((w[i] >> (8 * q)) & 0xFFu)) << (8 * q);
+          t &= ok * 3u;
+          r |= pack_bits(t & 0x01010101u) << (4 * i);
+        }
+        e |= pack_crumbs(t) << (24 - 8 * i);
+      }
+      if (ev[j]) {
+        // which event bytes a '>' follows
+        uint32_t g = (uint32_t)(nx == '>') << 16;
+#pragma unroll
+        for (int i = 0; i < 4; i++) g |= match4(w[i], '>') << (4 * i);
+        r = (r & ~ev[j]) | ((g >> 1) & ev[j]);
+      }
+      E[PK_PAD + base / 16] = e;
+      RX[base / 16] = r | (ev[j] << 16);
+    }
+    c += __popc(ev[j]);
+    if (gm[j]) gt = base + __ffs(gm[j]) - 1;
+  }
+  c = block_sum<NL_NT>(c);
+  gt = block_min<NL_NT>(gt);
+  if (threadIdx.x == 0) {
+    blk_cnt[blockIdx.x] = c;
+    blk_gt[blockIdx.x] = gt;
+  }
+}
+
+// Positions of the event bytes from RX (k_nl_write's output): block b covers
+// the same NL_PER_BLOCK bytes as k_pack's, a thread 64 consecutive ones.
+__global__ __launch_bounds__(NL_NT) void k_nl_write_rx(const uint32_t* RX, uint64_t n, const ull* blk_off, ull* nl,
+                                                       int follow) {
+  static_assert(NL_PER_BLOCK == (uint64_t)NL_NT * 64, "64 bytes per thread");
+  const uint64_t nw = (n + 15) / 16;
+  const uint64_t w0 = (uint64_t)blockIdx.x * (NL_PER_BLOCK / 16) + (uint64_t)threadIdx.x * 4;
+  uint32_t w[4] = {0, 0, 0, 0};
+  if (w0 + 4 <= nw) {
+    const uint4 q = *reinterpret_cast<const uint4*>(RX + w0);
+    w[0] = q.x;
+    w[1] = q.y;
+    w[2] = q.z;
+    w[3] = q.w;
+  } else {
+#pragma unroll
+    for (int i = 0; i < 4; i++) w[i] = w0 + i < nw ? RX[w0 + i] : 0u;
+  }
+  ull c = 0;
+#pragma unroll
+  for (int i = 0; i < 4; i++) c += __popc(w[i] >> 16);
+  ull tot;
+  ull o = blk_off[blockIdx.x] + block_scan_total<NL_NT>(c, &tot);
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    for (uint32_t m = w[i] >> 16; m; m &= m - 1) {
+      const int b = __ffs(m) - 1;
+      const uint64_t p = (w0 + i) * 16 + b;
+      const ull f = !follow ? 0ull : p + 1 >= n ? 2ull : (ull)((w[i] >> b) & 1u);
+      nl[o++] = p | (f << NL_FLAG_SHIFT);
+    }
   }
 }
 
@@ -745,17 +877,17 @@ __global__ void k_reads(uint64_t n, const ull* nl, uint64_t m, uint64_t p0,
       rstart[r] = s;
       if (len > 0xFFFFFFF0ull) {
         atomicMin(too_long, (ull)r);
-        rlen[r] = 0;
+        if (rlen) rlen[r] = 0;
         kc[r] = 0;
       } else {
-        rlen[r] = (uint32_t)len;
+        if (rlen) rlen[r] = (uint32_t)len;
         kc[r] = len >= (uint64_t)K ? (uint32_t)(len - K + 1) : 0u;
       }
     }
   }
   if (!processed) {
     rstart[r] = 0;
-    rlen[r] = 0;
+    if (rlen) rlen[r] = 0;
     kc[r] = 0;
     atomicMin(first_unproc, (ull)r);
   }
@@ -777,102 +909,31 @@ __device__ __forceinline__ uint64_t load_word8(const uint8_t* fa, uint64_t n, ui
   return w;
 }
 
-// Base encodings of the two counting front ends.
-//   ENC_MAIN:    char_to_el, (c >> 1) & 7 (distribute_kmers.h:784-786): the
-//                3-bit code ORs into the previous base's low bit, and the
-//                word is masked to 2k bits (kmer_shift, :798-805).
-//   ENC_BUILDER: symbol_to_kmer (concurrent_kmer_counter.hpp:2097-2110):
-//                A C T G -> 0 1 2 3, every other byte -> 0; the word is not
-//                masked and keeps the last 4*sizeof(kmer_t) bases.
-constexpr int ENC_MAIN = 0;
-constexpr int ENC_BUILDER = 1;
-
-template <int ENC>
-__device__ __forceinline__ uint32_t base_code(uint32_t c) {
-  if (ENC == ENC_MAIN) return (c >> 1) & 7u;
-  const bool acgt = c == 'A' || c == 'C' || c == 'G' || c == 'T';
-  return acgt ? (c >> 1) & 3u : 0u;
-}
-
 // ---------------------------------------------------------------------------
 // Partition (multisplit) into buckets by the top bits of the key.
-//   level 1  k_l1_hist / k_l1_scatter: fused with the parse of the reads, up
-//            to 10 bits; each key goes straight to its slot
-//   level 2+ k_ms_hist / k_ms_scatter: from the previous level's array, at
-//            most 8 bits so that every tile holds tens of keys per digit:
-//            each tile is sorted by digit in LDS and written as runs
+//   k_split    every level of the main and builder paths and the further
+//              levels of the others: tiles sorted in registers and LDS
+//   k_l1_hist / k_l1_scatter  level 1 of a rank's share, whose owner rule
+//              walks every read in order: each key goes straight to its slot
 
 constexpr int L1_NT = 512;  // level-1 histogram blocks
-constexpr int MS_NT = 512;
-constexpr int MS_P_NT = 512;  // threads of a persistent multisplit block (one tile at a time)
-constexpr int L1_MAX_BITS = PK_TUNING_L1_BITS_MAX;  // level-1 digit width (direct scatter)
-constexpr int L1_DEFAULT_BITS = 8;  // wider digits keep more partial lines open
-constexpr int MS_MAX_BITS = 8;   // further levels (tile split into runs)
+constexpr int L1_MAX_BITS = PK_TUNING_L1_BITS_MAX;  // level-1 digit width
+constexpr int L1_DEFAULT_BITS = 8;  // wider digits keep more partial lines open (k_l1_scatter)
+constexpr int PK_MS_TILES = 4;      // pk_timing's form of a k_split level
 constexpr int MS_TIMED_LEVELS = 4;  // further levels with their own timing events
 static_assert(sizeof(pk_timing::ms_level_form) / sizeof(int32_t) == MS_TIMED_LEVELS, "per-level timing slots");
-constexpr uint64_t L2_FOLD_MAX = 8192;  // (bucket, digit) counters of a folded level-2 histogram
 
-template <class Key>
-struct TileCfg {
-  static constexpr int Q = sizeof(Key) == 8 ? 16 : 8;  // keys per thread per tile
-};
-
-// LDS of a tile split by digit: a histogram and its exclusive scan, a
-// counting-sort scatter of the keys into T1, then coalesced stores: sorted
-// slot p, of digit d (recomputed from the key), goes to out[base[d] -
-// toff[d] + p] (delta[d] = base[d] - toff[d]; base[d] stays in the register
-// of thread d): about 68 KB for 8192 one-word or 4096 two-word keys.
-template <class Key, int NT>
-struct TileLds {
-  Key T1[NT * TileCfg<Key>::Q];
-  uint32_t h[256];
-  uint32_t tcur[256];
-  long long delta[256];
-};
-
-// Level-1 producer.  A block owns rpb consecutive reads and walks them in
-// chunks: a chunk is the longest run of <= NT consecutive reads (NT threads
-// per block) whose bytes fit in the LDS staging buffer; thread t then walks
-// read t of the chunk from LDS with the rolling update (a read too long for
-// the buffer is walked from global memory, alone in its chunk).  Records are in file
-// order, so a chunk's bytes are one contiguous range.  The buffer holds the
-// base code of every byte, not the byte: bits 0-1 of the code in plane A
-// (32 bytes per word) and, on the main path, bit 2 in plane B (32 bytes per
-// word), 3/8 of the raw size.  Its size (sb bytes, in dynamic LDS) is chosen
-// per input so that NT typical records fit.
+// Level-1 producer of a rank's share.  A block owns rpb consecutive reads and
+// walks them in chunks: a chunk is the longest run of <= NT consecutive reads
+// (NT threads per block) whose bytes fit in the LDS staging buffer; thread t
+// then walks read t of the chunk from LDS with the rolling update (a read too
+// long for the buffer is walked from global memory, alone in its chunk).
+// Records are in file order, so a chunk's bytes are one contiguous range.
+// The buffer holds the base code of every byte, not the byte: bits 0-1 of the
+// code in plane A (32 bytes per word) and, on the main path, bit 2 in plane B
+// (32 bytes per word), 3/8 of the raw size.  Its size (sb bytes, in dynamic
+// LDS) is chosen per input so that NT typical records fit.
 constexpr int L1_SB_MIN = 8192, L1_SB_MAX = 98304;  // staged bytes per chunk
-
-// Level-1 scatter blocks: 1024 threads on the main path (two blocks per CU,
-// <= 60 KB of LDS and <= 64 VGPRs each; fewer blocks per CU keep fewer
-// partly written lines open), 512 for the rank-share and builder walks,
-// which need more registers.  With one-word keys a scatter block takes the
-// reads of two histogram blocks (k = 32 bacterial 1.27 -> 1.22 ms; the
-// histogram itself is faster at 512 threads over half as many reads); with
-// two-word keys one (k = 64 bacterial 1.50 -> 1.34 ms against 512 threads).
-template <class Key, int ENC, bool OWN>
-struct L1Scatter {
-  static constexpr bool main = ENC == ENC_MAIN && !OWN;
-  static constexpr int NT = main ? 1024 : 512;
-  static constexpr int SB_MAX = main ? 131072 : L1_SB_MAX;
-  // histogram blocks per scatter block (their output runs per digit are
-  // adjacent in the digit-major scan)
-  static constexpr int GF = main && sizeof(Key) == 8 ? 2 : 1;
-};
-
-// Level-2 histogram folded into the level-1 histogram (large inputs with
-// three or more partition levels): the level-2 "segments" are runs of the
-// level-1 output, segment (a, g) = the keys of level-1 bucket a that the
-// histogram blocks [g * spb, (g + 1) * spb) produced (spb a multiple of the
-// histogram blocks per scatter block, so a segment is whole scatter-block
-// runs, contiguous in the digit-major layout); the level-1 histogram kernel
-// counts them per second digit s into H2[(a, s) * nsb + g], so no pass over
-// the written keys is needed to count them.
-struct L2Fold {
-  int d2;         // second-digit bits (0: no fold)
-  int spb;        // histogram blocks per segment
-  uint64_t nsb;   // segments per level-1 bucket
-  uint32_t* H2;   // (2^(d1+d2)) x nsb counts, zeroed before the launch
-};
 
 struct ChunkLds {
   ull base;  // first staged byte (32-byte aligned)
@@ -1073,53 +1134,6 @@ __device__ __forceinline__ int walk_read(const ChunkLds& C, Stage sg, const uint
   return q;
 }
 
-// The histogram's digit of a main-path k-mer is its top d <= 13 key bits:
-// bases 0..6 of the window (key slot j holds base j's 2-bit code at bits
-// 2(K-1-j) and 2(K-1-j)+1, and the third code bit of base j+1 ORs into the
-// low bit of slot j).  A 15-bit register rolled like the key, ((v << 2) |
-// code) & 0x7FFF, holds slots 0..6 of the window that starts 6 bases back
-// (bit 14, the spill of the bases before, is never read; bit 0 still lacks
-// the next base's third bit, so d stays <= 13), and digit = (v >> (14 - d))
-// & (2^d - 1).  The walk stops at the last window's
-// seventh base: len - K + 7 bases per read instead of len, no K-bit key.
-// For K >= 7 only.
-template <class Emit>
-__device__ __forceinline__ void walk_read_top(const ChunkLds& C, Stage sg, const uint8_t* fa, ull s, uint32_t len,
-                                              int K, Emit&& emit) {
-  if (len < (uint32_t)K) return;
-  const uint32_t end = len - (uint32_t)K + 7;  // bases to read
-  uint32_t v = 0, i = 0;
-  if (C.lds) {
-    // 32 bases at a time from the read's own position (two words shifted
-    // together), so every lane runs the same count but on its last piece
-    // (pieces ending at word boundaries differ per read and diverge)
-    while (i < end) {
-      const ull off = s + i - C.base;
-      const ull w = off >> 5;
-      const uint32_t sh = (uint32_t)(off & 31);
-      const uint32_t cnt = end - i < 32u ? end - i : 32u;
-      ull a = sg.A[w] >> (2 * sh);
-      uint32_t b = sg.B[w] >> sh;
-      if (sh + cnt > 32u) {
-        // the piece runs into the next word, which holds bases of this read
-        a |= sg.A[w + 1] << (64 - 2 * sh);
-        b |= sg.B[w + 1] << (32 - sh);
-      }
-      for (uint32_t q = 0; q < cnt; q++, i++) {
-        v = ((v << 2) | ((uint32_t)a & 3u) | ((b & 1u) << 2)) & 0x7FFFu;
-        a >>= 2;
-        b >>= 1;
-        if (i >= 6) emit(v);
-      }
-    }
-    return;
-  }
-  for (; i < end; i++) {
-    v = ((v << 2) | base_code<ENC_MAIN>(fa[s + i])) & 0x7FFFu;
-    if (i >= 6) emit(v);
-  }
-}
-
 // L-mer frequencies (Sliding_window_l, kmer_counting.cpp:391-438): every
 // L-mer of every record's read line, rolling 3-bit update masked to 2L bits.
 __global__ void k_lmer_freq(const uint8_t* fa, const ull* rstart, const uint32_t* rlen, uint64_t R,
@@ -1136,108 +1150,65 @@ __global__ void k_lmer_freq(const uint8_t* fa, const ull* rstart, const uint32_t
   }
 }
 
-// Level-1 histogram: digit = bits [KB - d1, KB) of each key (KB = key bits:
-// 2K on the main path, the whole word for the builder encoding).  Block b's
-// count of digit d goes to H[d * nblk + b] (digit-major), so an exclusive
-// scan of H gives every block the output base of each of its digit runs.
+// Level-1 histogram of a rank's share: digit = bits [KB - d1, KB) of each
+// owned key.  Block b's count of digit d goes to H[d * nblk + b] (digit-major),
+// so an exclusive scan of H gives every block the output base of each of its
+// digit runs.
 template <class Key, int ENC, bool OWN>
 __global__ __launch_bounds__(L1_NT) void k_l1_hist(const uint8_t* fa, uint64_t n, const ull* rstart,
                                                    const uint32_t* rlen, uint64_t R, int K, int KB,
                                                    Key mask, int d1, int rpb, int sb, OwnCfg cf,
-                                                   uint32_t* H, L2Fold f2) {
+                                                   uint32_t* H) {
   __shared__ ChunkLds C;
-  // dynamic LDS: plane A, plane B, 2^d1 digit counts (then, with f2.d2 > 0,
-  // 2^(d1 + d2) counts of the first two digits)
+  // dynamic LDS: plane A, plane B, 2^d1 digit counts
   extern __shared__ ull l1_dyn[];
   const Stage sg{l1_dyn, reinterpret_cast<uint32_t*>(l1_dyn + sb / 32), sb};
   uint32_t* h = sg.B + sb / 32;
   const int nb = 1 << d1;
-  uint32_t* h2 = h + nb;
-  const int nb2 = f2.d2 ? nb << f2.d2 : 0;
   for (int i = threadIdx.x; i < nb; i += L1_NT) h[i] = 0;
-  for (int i = threadIdx.x; i < nb2; i += L1_NT) h2[i] = 0;
   const uint64_t r0 = (uint64_t)blockIdx.x * rpb;
   const uint64_t r1 = r0 + rpb < R ? r0 + rpb : R;
   const int bpos = KB - d1;
-  // the main path's digits (<= 13 bits: the register's bit 0, the low bit of
-  // slot 6, still lacks the next base's third code bit) come from a 15-bit
-  // window of bases
-  const bool top = ENC == ENC_MAIN && !OWN && K >= 7 && KB == 2 * K && d1 + f2.d2 <= 13;
-  const int tsh = 14 - d1, tsh2 = 14 - d1 - f2.d2;
-  const uint32_t tm = (1u << d1) - 1u, tm2 = (1u << (d1 + f2.d2)) - 1u;
   for (uint64_t c0 = r0; c0 < r1;) {
     stage_chunk<ENC, L1_NT>(C, sg, fa, n, rstart, rlen, c0, r1);
     const int m = C.m;
     if ((int)threadIdx.x < m) {
       const uint64_t r = c0 + threadIdx.x;
-      if (top) {
-        // main path: the digit from the window's first seven bases
-        if (nb2) walk_read_top(C, sg, fa, rstart[r], rlen[r], K, [&](uint32_t v) { atomicAdd(&h2[(v >> tsh2) & tm2], 1u); });
-        else walk_read_top(C, sg, fa, rstart[r], rlen[r], K, [&](uint32_t v) { atomicAdd(&h[(v >> tsh) & tm], 1u); });
-      } else {
-        uint32_t i = 0;
-        Key km = 0;
-        OwnState os{0, 0, 0, 0};
-        walk_read<Key, ENC, OWN>(C, sg, fa, rstart[r], rlen[r], i, km, os, cf, K, mask, 0x7fffffff,
-                                 [&](int, Key x) {
-                                   // one LDS atomic per key: with the fold the
-                                   // level-1 counts are sums of h2's rows
-                                   if (nb2) atomicAdd(&h2[key_digit<Key>(x, bpos - f2.d2, d1 + f2.d2)], 1u);
-                                   else atomicAdd(&h[key_digit<Key>(x, bpos, d1)], 1u);
-                                 });
-      }
+      uint32_t i = 0;
+      Key km = 0;
+      OwnState os{0, 0, 0, 0};
+      walk_read<Key, ENC, OWN>(C, sg, fa, rstart[r], rlen[r], i, km, os, cf, K, mask, 0x7fffffff,
+                               [&](int, Key x) { atomicAdd(&h[key_digit<Key>(x, bpos, d1)], 1u); });
     }
     c0 += m;
     __syncthreads();
   }
-  if (nb2) {
-    // h[a] = sum of h2[a, 0 .. 2^d2): one wave per bucket, lanes over s
-    const int lane = (int)threadIdx.x & 63, per = 1 << f2.d2;
-    for (int a = (int)threadIdx.x >> 6; a < nb; a += L1_NT / 64) {
-      uint32_t v = 0;
-      for (int j = lane; j < per; j += 64) v += h2[(a << f2.d2) + j];
-      for (int o = 32; o; o >>= 1) v += __shfl_xor(v, o);
-      if (lane == 0) h[a] = v;
-    }
-    __syncthreads();
-    // (bucket, sub-digit, segment) counts of the level-2 segments
-    for (int i = threadIdx.x; i < nb2; i += L1_NT)
-      if (h2[i]) atomicAdd(&f2.H2[(ull)i * f2.nsb + blockIdx.x / f2.spb], h2[i]);
-  }
   for (int i = threadIdx.x; i < nb; i += L1_NT) H[(ull)i * gridDim.x + blockIdx.x] = h[i];
 }
 
-// Level-1 scatter fused with the parse: the same chunked walk as k_l1_hist
-// over the same reads per block, in blocks of L1Scatter::NT threads; every key
-// takes the next slot of its digit from the block's LDS counter (atomicAdd's
-// return value) and is stored at once at the block's base for that digit
-// (scanned histogram O, same layout as H).  No tile buffer and no barrier
-// inside the walk: the order of keys inside a bucket is arbitrary, which the
-// bucket count does not depend on.  Each block keeps a partly written line
-// open per digit, so fewer, larger blocks per CU write fewer partial lines.
+// Level-1 scatter of a rank's share: the same chunked walk as k_l1_hist over
+// the same reads per block; every key takes the next slot of its digit from
+// the block's LDS cursor (the return value of one 64-bit atomic) and is
+// stored at once.  The order of keys inside a bucket is arbitrary, which the
+// bucket count does not depend on.
 template <class Key, int ENC, bool OWN>
-__global__ __launch_bounds__((L1Scatter<Key, ENC, OWN>::NT)) void k_l1_scatter(const uint8_t* fa, uint64_t n,
-                                                      const ull* rstart, const uint32_t* rlen,
-                                                      uint64_t R, int K, int KB, Key mask, int d1,
-                                                      int rpb, int sb, OwnCfg cf, const ull* O,
-                                                      uint64_t nblk_h, Key* S1) {
-  constexpr int NT = L1Scatter<Key, ENC, OWN>::NT;
-  constexpr int GF = L1Scatter<Key, ENC, OWN>::GF;
+__global__ __launch_bounds__(L1_NT) void k_l1_scatter(const uint8_t* fa, uint64_t n, const ull* rstart,
+                                                      const uint32_t* rlen, uint64_t R, int K, int KB, Key mask,
+                                                      int d1, int rpb, int sb, OwnCfg cf, const ull* O,
+                                                      uint64_t nblk, Key* S1) {
   __shared__ ChunkLds C;
-  // dynamic LDS: plane A, 2^d1 output cursors, plane B (then 2^d1 words
-  // the cursors no longer need: each k-mer takes its slot from one 64-bit
-  // atomic on its digit's cursor)
+  // dynamic LDS: plane A, 2^d1 output cursors, plane B
   extern __shared__ ull l1_dyn[];
   const int nb = 1 << d1;
   ull* cur = l1_dyn + sb / 32;
   const Stage sg{l1_dyn, reinterpret_cast<uint32_t*>(cur + nb), sb};
-  for (int i = threadIdx.x; i < nb; i += NT) cur[i] = O[(ull)i * nblk_h + (ull)blockIdx.x * GF];
-  const uint64_t r0 = (uint64_t)blockIdx.x * GF * rpb;
-  const uint64_t r1 = r0 + (uint64_t)GF * rpb < R ? r0 + (uint64_t)GF * rpb : R;
+  for (int i = threadIdx.x; i < nb; i += L1_NT) cur[i] = O[(ull)i * nblk + blockIdx.x];
+  const uint64_t r0 = (uint64_t)blockIdx.x * rpb;
+  const uint64_t r1 = r0 + rpb < R ? r0 + rpb : R;
   const int bpos = KB - d1;
   // stage_chunk's barriers order the set-up above before the first walk
   for (uint64_t c0 = r0; c0 < r1;) {
-    stage_chunk<ENC, NT>(C, sg, fa, n, rstart, rlen, c0, r1);
+    stage_chunk<ENC, L1_NT>(C, sg, fa, n, rstart, rlen, c0, r1);
     const int m = C.m;
     if ((int)threadIdx.x < m) {
       const uint64_t r = c0 + threadIdx.x;
@@ -1255,396 +1226,440 @@ __global__ __launch_bounds__((L1Scatter<Key, ENC, OWN>::NT)) void k_l1_scatter(c
   }
 }
 
-// bucket offsets of a level from its scanned digit-major histogram:
-// boff[d] = O[d * stride_of(d)] ... for level 1 stride = nblk.
+// bucket offsets of the share's level 1 from its scanned histogram
 __global__ void k_l1_boff(const ull* O, int nb, uint64_t nblk, ull total, ull* boff) {
   const int d = blockIdx.x * blockDim.x + threadIdx.x;
   if (d < nb) boff[d] = O[(ull)d * nblk];
   if (d == nb) boff[nb] = total;
 }
 
-// tiles of a level: tp[a+1] = tp[a] + ceil(n_a / tile) for a < nb (one block)
-__global__ __launch_bounds__(1024) void k_tile_prefix(const ull* boff, int nb, int tile, ull* tp) {
-  __shared__ ull tmp[1025];
-  ull acc = 0;
-  if (threadIdx.x == 0) tp[0] = 0;
-  for (int base = 0; base < nb; base += 1024) {
-    const int a = base + threadIdx.x;
-    const ull v = a < nb ? (boff[a + 1] - boff[a] + tile - 1) / tile : 0ull;
-    const ull ex = block_excl_scan<1024>(v);
-    if (a < nb) tp[a + 1] = acc + ex + v;
-    tmp[threadIdx.x] = ex + v;
-    __syncthreads();
-    acc += tmp[1023];
-    __syncthreads();
-  }
-}
+// ---------------------------------------------------------------------------
+// Tiled partition.  A level splits every bucket of its input by db more key
+// bits.  A bucket's keys are cut into tiles of tk; a block takes one tile into
+// registers, ranks its keys by digit with LDS atomics, orders them through
+// LDS and writes the tile back as one contiguous piece, at the place in the
+// output array that the tile has in its bucket (tile t of bucket a starts at
+// boff[a] + t * tk), with one table entry per digit: start << 16 | count.
+// A bucket of the next level is then a list of runs, one per tile of its
+// parent, which its reader gathers; no level needs a histogram pass over its
+// input, and all writes are whole lines.
+//
+// What bounds it: memory.  Per level the keys are read and written once (a
+// run of tk / 2^db keys costs up to one extra line), the run table is 12
+// bytes per tile and digit, and no store leaves a partly written line but at
+// a tile's ends.  Two 512-thread blocks per CU (64 KB of tile buffer and at
+// most 128 VGPRs each) overlap one's loads with the other's LDS work.
 
-__device__ __forceinline__ int tile_owner(const ull* tp, int nb, ull blk) {
-  int lo = 0, hi = nb - 1;
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (tp[mid] <= blk) lo = mid; else hi = mid - 1;
-  }
-  return lo;
-}
-
-// Level >= 2: bucket a of the previous level (nb buckets, offsets boff,
-// tiles tp) is split by dbits more bits at dpos.  Tile t of bucket a writes
-// its count of sub-digit s to H[tp[a] << dbits + s * ntiles(a) + t]: in
-// (a, s, t) order, so the exclusive scan of H holds every tile's output base
-// per sub-digit and H's scan at t = 0 is the start of sub-bucket (a, s).
-__device__ __forceinline__ ull ms_index(const ull* tp, int a, int s, ull t, int dbits) {
-  return (tp[a] << dbits) + (ull)s * (tp[a + 1] - tp[a]) + t;
-}
+constexpr int SP_NT = 512;
+constexpr int SP_MAX_BITS = 10;  // digit width of a level
+constexpr int SP_TILE_BYTES = 65536;
 
 template <class Key>
-__global__ __launch_bounds__(MS_NT) void k_ms_hist(const Key* Sin, const ull* boff, const ull* tp, int nb,
-                                                   int dpos, int dbits, uint32_t* H) {
-  constexpr int TQ = MS_NT * TileCfg<Key>::Q;
-  __shared__ uint32_t h[256];
-  const ull blk = blockIdx.x;
-  if (blk >= tp[nb]) return;
-  const int a = tile_owner(tp, nb, blk);
-  const ull t = blk - tp[a];
-  const ull b0 = boff[a] + t * TQ;
-  const ull b1 = b0 + TQ < boff[a + 1] ? b0 + TQ : boff[a + 1];
-  const int ns = 1 << dbits;
-  for (int i = threadIdx.x; i < ns; i += MS_NT) h[i] = 0;
+struct SplitCfg {
+  // keys per thread: 64 VGPRs of keys; tiles of 16384 one-word or 8192
+  // two-word keys go through the tile buffer in two rounds
+  static constexpr int Q = sizeof(Key) == 8 ? 32 : 16;
+  static constexpr int TK_MAX = SP_NT * Q;
+  static constexpr int ROUND = SP_TILE_BYTES / (int)sizeof(Key);
+};
+
+// The buckets of a level's output, as the next reader finds them.
+//   M == nullptr: contiguous, bucket b is [boff[b], boff[b + 1]) of the array.
+//   else: bucket b = a << db | s, of parent bucket a (tiles tp[a] ..
+//   tp[a + 1], keys from boff[a] on), is the runs of digit s in the tiles of
+//   a: entry e = (tp[a] << db) + s * ntiles(a) + t of the run table M (start
+//   in the tile << 16 | count) and of V, the exclusive scan of the counts.  V
+//   gives every key a place in key order of the buckets, the "virtual" index
+//   that buckets and tiles are counted in; run e holds the indexes V[e] ..
+//   V[e + 1] at array positions boff[a] + t * tk + start.
+struct Runs {
+  const uint32_t* M;
+  const ull* V;
+  const ull* tp;
+  const ull* boff;
+  int db;
+  int tk;
+};
+
+// count field of a run-table entry, for the scan
+struct RunCount {
+  uint32_t v;
+  __host__ __device__ operator ull() const { return (ull)(v & 0xFFFFu); }
+};
+
+struct RunBucket {
+  ull v0, n;   // virtual start and key count
+  ull e0, nt;  // first run-table entry and number of entries
+  ull base;    // array position of the parent's first tile
+};
+
+// a value that is the same in every lane, moved to scalar registers
+__device__ __forceinline__ ull uniform(ull x) {
+  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)x);
+  const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(x >> 32));
+  return (ull)hi << 32 | lo;
+}
+
+__device__ __forceinline__ RunBucket uniform(const RunBucket& r) {
+  return RunBucket{uniform(r.v0), uniform(r.n), uniform(r.e0), uniform(r.nt), uniform(r.base)};
+}
+
+// (called with one bucket per lane or per block)
+__device__ __forceinline__ RunBucket run_bucket(const Runs& in, ull b) {
+  RunBucket r;
+  if (!in.M) {
+    r.v0 = in.boff[b];
+    r.n = in.boff[b + 1] - r.v0;
+    r.e0 = r.nt = r.base = 0;
+    return r;
+  }
+  const ull a = b >> in.db, s = b & ((1ull << in.db) - 1);
+  const ull t0 = in.tp[a];
+  r.nt = in.tp[a + 1] - t0;
+  r.e0 = (t0 << in.db) + s * r.nt;
+  r.v0 = in.V[r.e0];
+  r.n = in.V[r.e0 + r.nt] - r.v0;
+  r.base = in.boff[a];
+  return r;
+}
+
+// Number of x[0..n) (ascending) that are <= key, found by the whole block:
+// NT samples per step instead of a chain of log2(n) dependent loads.
+template <int NT>
+__device__ __forceinline__ ull block_upper(const ull* x, ull n, ull key) {
+  ull lo = 0;
+  while (n > (ull)NT) {
+    const ull step = (n + NT - 1) / NT;
+    const ull o = (ull)threadIdx.x * step;
+    const int c = __syncthreads_count(o < n && x[lo + o] <= key);
+    if (c == 0) return lo;
+    // sample c - 1 is <= key, sample c (if any) is not
+    const ull skip = (ull)(c - 1) * step;
+    lo += skip;
+    n = n - skip < step ? n - skip : step;
+  }
+  return lo + (ull)__syncthreads_count((ull)threadIdx.x < n && x[lo + threadIdx.x] <= key);
+}
+
+// Exclusive scan of a u32 over the block through nw[NT / 64 + 1] (LDS); the
+// total in *tot.  The caller passes a barrier before nw is used again.
+template <int NT>
+__device__ __forceinline__ uint32_t block_scan_u32(uint32_t v, uint32_t* nw, uint32_t* tot) {
+  constexpr int NW = NT / 64;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  uint32_t x = v;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const uint32_t y = __shfl_up(x, o, 64);
+    if (lane >= o) x += y;
+  }
+  if (lane == 63) nw[w] = x;
   __syncthreads();
-  for (ull i = b0 + threadIdx.x; i < b1; i += MS_NT) atomicAdd(&h[key_digit<Key>(Sin[i], dpos, dbits)], 1u);
-  __syncthreads();
-  for (int i = threadIdx.x; i < ns; i += MS_NT) H[ms_index(tp, a, i, t, dbits)] = h[i];
+  uint32_t before = 0, all = 0;
+#pragma unroll
+  for (int i = 0; i < NW; i++) {
+    const uint32_t t = nw[i];
+    before += i < w ? t : 0u;
+    all += t;
+  }
+  *tot = all;
+  return before + x - v;
 }
 
-// boff2[a << dbits | s] = O[ms_index(a, s, 0)] for every (a, s); boff2[end] = N
-__global__ void k_ms_boff(const ull* O, const ull* tp, int nb, int dbits, ull total, ull* boff2) {
-  const ull g = (ull)blockIdx.x * blockDim.x + threadIdx.x;
-  const ull n2 = (ull)nb << dbits;
-  if (g < n2) {
-    const int a = (int)(g >> dbits);
-    const int s = (int)(g & ((1u << dbits) - 1));
-    boff2[g] = (tp[a + 1] > tp[a]) ? O[ms_index(tp, a, s, 0, dbits)] : O[tp[a] << dbits];
-  }
-  if (g == n2) boff2[n2] = total;
-}
-
-// Tile geometry: bucket a (advanced from the previous tile's, tiles being
-// visited in order), first key b0 and key count m of tile g.
-__device__ __forceinline__ void ms_tile(const ull* boff, const ull* tp, ull g, int TQ, int& a, ull& t,
-                                        ull& b0, int& m) {
-  while (tp[a + 1] <= g) a++;
-  t = g - tp[a];
-  b0 = boff[a] + t * TQ;
-  const ull e = boff[a + 1];
-  m = (int)((b0 + TQ < e ? b0 + TQ : e) - b0);
-}
-
-template <class Key>
-__global__ __launch_bounds__(MS_NT) void k_ms_scatter(const Key* Sin, const ull* boff, const ull* tp,
-                                                      int nb, int dpos, int dbits, const ull* O,
-                                                      Key* Sout) {
-  constexpr int Q = TileCfg<Key>::Q;
-  constexpr int TQ = MS_NT * TileCfg<Key>::Q;
-  __shared__ TileLds<Key, MS_NT> L;
-  const ull blk = blockIdx.x;
-  if (blk >= tp[nb]) return;
-  const int a = tile_owner(tp, nb, blk);
-  const ull t = blk - tp[a];
-  const ull b0 = boff[a] + t * TQ;
-  const ull b1 = b0 + TQ < boff[a + 1] ? b0 + TQ : boff[a + 1];
-  const int m = (int)(b1 - b0);
-  const int ns = 1 << dbits;
-  // sub-digit tid's output base (ns <= 256 <= MS_NT)
-  const ull bse = (int)threadIdx.x < ns ? O[ms_index(tp, a, threadIdx.x, t, dbits)] : 0ull;
-  if ((int)threadIdx.x < ns) L.h[threadIdx.x] = 0;
-  // keys tid, tid + MS_NT, ... of the tile in registers (coalesced loads)
-  Key kr[Q];
-#pragma unroll
-  for (int j = 0; j < Q; j++) {
-    const int idx = (int)threadIdx.x + j * MS_NT;
-    kr[j] = idx < m ? Sin[b0 + idx] : Key(0);
-  }
-  const int np = m > (int)threadIdx.x ? (m - (int)threadIdx.x - 1) / MS_NT + 1 : 0;
-  __syncthreads();
-  // the histogram's atomic returns each key's rank inside its digit (two
-  // 16-bit ranks per register), so the sort needs no second atomic pass
-  uint32_t rk[(Q + 1) / 2] = {};
-#pragma unroll
-  for (int j = 0; j < Q; j++)
-    if (j < np) rk[j / 2] |= atomicAdd(&L.h[key_digit<Key>(kr[j], dpos, dbits)], 1u) << (16 * (j & 1));
-  __syncthreads();
-  const uint32_t v = (int)threadIdx.x < ns ? L.h[threadIdx.x] : 0u;
-  const ull ex = block_excl_scan<MS_NT>(v);
-  if ((int)threadIdx.x < ns) {
-    L.tcur[threadIdx.x] = (uint32_t)ex;
-    L.delta[threadIdx.x] = (long long)bse - (long long)ex;
-  }
-  __syncthreads();
-#pragma unroll
-  for (int j = 0; j < Q; j++) {
-    if (j < np) {
-      const uint32_t d = key_digit<Key>(kr[j], dpos, dbits);
-      L.T1[L.tcur[d] + ((rk[j / 2] >> (16 * (j & 1))) & 0xFFFFu)] = kr[j];
+// Map of the m places [v0, v0 + m) onto the pieces of a list that cover them:
+// piece idx holds the places V[idx] .. V[idx + 1], its first at source
+// position src(idx).  mw[w].x has bit i set when place 32 w + i starts a
+// piece, mw[w].y counts the pieces that start before word w, and piece r of
+// the map has put(r, source position - place, piece) called once; map_piece
+// gives a place's r.  Pieces without places leave no trace.  The list is read
+// from piece f (which covers v0 or ends before it) and has no piece past
+// `end`.  Returns the number of pieces (put is only called for r < cap).
+template <int NT, class Src, class Put>
+__device__ __forceinline__ int map_pieces(uint2* mw, uint32_t* nw, int cap, const ull* V, ull f, ull end, ull v0,
+                                          int m, Src&& src, Put&& put) {
+  const int nwords = (m + 31) >> 5;
+  const ull v1 = v0 + (ull)m;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  for (int i = threadIdx.x; i < nwords; i += NT) mw[i].x = 0;
+  uint32_t cnt = 0;
+  for (ull c0 = f;; c0 += NT) {
+    const ull idx = c0 + threadIdx.x;
+    const bool in = idx < end;
+    ull vs = 0, ve = 0;
+    if (in) {
+      vs = V[idx];
+      ve = V[idx + 1];
     }
-  }
-  __syncthreads();
-  for (int p = threadIdx.x; p < m; p += MS_NT) {
-    const Key v = L.T1[p];
-    Sout[L.delta[key_digit<Key>(v, dpos, dbits)] + p] = v;
-  }
-}
-
-// Persistent form for long levels: block i takes the tiles
-// [i * per, (i + 1) * per) in order and loads the next tile's keys while it
-// sorts the current one (at most 128 VGPRs: two blocks of 8 waves per CU).
-// Consecutive tiles of a bucket write adjacent runs of each sub-digit, so one
-// CU completes the lines at their joins.  The output base of sub-digit s for
-// tile t + 1 of a bucket is tile t's base plus tile t's count of s (the scan
-// of H in (bucket, digit, tile) order), so bases are read from O only for a
-// block's first tile in each bucket: one line per digit per bucket instead of
-// per tile.
-template <class Key, int NT>
-__global__ __launch_bounds__(NT, NT >= 1024 ? 8 : 4) void k_ms_scatter_p(const Key* Sin, const ull* boff, const ull* tp,
-                                                           int nb, int dpos, int dbits, const ull* O,
-                                                           Key* Sout) {
-  // NT threads share one tile of TQ keys (the level's tile), Q per thread
-  constexpr int TQ = MS_NT * TileCfg<Key>::Q;
-  constexpr int Q = TQ / NT;
-  __shared__ TileLds<Key, MS_NT> L;
-  const ull ntl = tp[nb];
-  const ull per = (ntl + gridDim.x - 1) / gridDim.x;
-  const ull g0 = (ull)blockIdx.x * per;
-  const ull g1 = g0 + per < ntl ? g0 + per : ntl;
-  if (g0 >= g1) return;
-  const int ns = 1 << dbits;
-  const int tid = (int)threadIdx.x;
-  // the current tile's keys (tid, tid + NT, ...) and this thread's
-  // sub-digit base (tid < ns)
-  int a = tile_owner(tp, nb, g0);
-  ull t, b0;
-  int m;
-  ms_tile(boff, tp, g0, TQ, a, t, b0, m);
-  Key kr[Q];
+    const bool part = in && ve > vs && vs < v1 && ve > v0;
+    const ull bal = __ballot(part);
+    if (lane == 0) nw[w] = (uint32_t)__popcll(bal);
+    // the list goes on inside the places when the chunk's last piece ends there
+    const int more = __syncthreads_or(threadIdx.x == NT - 1 && in && ve < v1);
+    uint32_t before = cnt, all = 0;
 #pragma unroll
-  for (int j = 0; j < Q; j++) {
-    const int idx = tid + j * NT;
-    kr[j] = idx < m ? Sin[b0 + idx] : Key(0);
-  }
-  ull bs = tid < ns ? O[ms_index(tp, a, tid, t, dbits)] : 0ull;
-  for (ull g = g0; g < g1; g++) {
-    Key kn[Q] = {};
-    ull bn = 0, tn = 0, b0n = 0;
-    int an = a, mn = 0;
-    if (g + 1 < g1) {
-      ms_tile(boff, tp, g + 1, TQ, an, tn, b0n, mn);
-#pragma unroll
-      for (int j = 0; j < Q; j++) {
-        const int idx = tid + j * NT;
-        kn[j] = idx < mn ? Sin[b0n + idx] : Key(0);
-      }
-      // a new bucket: its first base from the scan
-      if (tid < ns && an != a) bn = O[ms_index(tp, an, tid, tn, dbits)];
+    for (int i = 0; i < NT / 64; i++) {
+      before += i < w ? nw[i] : 0u;
+      all += nw[i];
     }
-    if (tid < ns) L.h[tid] = 0;
-    const int np = m > tid ? (m - tid - 1) / NT + 1 : 0;
-    __syncthreads();
-    // ranks inside each digit from the histogram's atomics (see k_ms_scatter)
-    uint32_t rk[(Q + 1) / 2] = {};
-#pragma unroll
-    for (int j = 0; j < Q; j++)
-      if (j < np) rk[j / 2] |= atomicAdd(&L.h[key_digit<Key>(kr[j], dpos, dbits)], 1u) << (16 * (j & 1));
-    __syncthreads();
-    const uint32_t v = tid < ns ? L.h[tid] : 0u;
-    // the next tile of the same bucket starts its runs where this one's end
-    if (an == a) bn = bs + v;
-    const ull ex = block_excl_scan<NT>(v);
-    if (tid < ns) {
-      L.tcur[tid] = (uint32_t)ex;
-      L.delta[tid] = (long long)bs - (long long)ex;
+    if (part) {
+      const uint32_t r = before + (uint32_t)__popcll(bal & ((1ull << lane) - 1));
+      const uint32_t ls = vs > v0 ? (uint32_t)(vs - v0) : 0u;
+      if (r < (uint32_t)cap) put(r, src(idx) - vs + v0, idx);
+      atomicOr(&mw[ls >> 5].x, 1u << (ls & 31));
     }
-    __syncthreads();
-#pragma unroll
-    for (int j = 0; j < Q; j++) {
-      if (j < np) {
-        const uint32_t d = key_digit<Key>(kr[j], dpos, dbits);
-        L.T1[L.tcur[d] + ((rk[j / 2] >> (16 * (j & 1))) & 0xFFFFu)] = kr[j];
-      }
-    }
-    __syncthreads();
-    for (int p = tid; p < m; p += NT) {
-      const Key v = L.T1[p];
-      Sout[L.delta[key_digit<Key>(v, dpos, dbits)] + p] = v;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int j = 0; j < Q; j++) kr[j] = kn[j];
-    bs = bn;
-    a = an;
-    m = mn;
-  }
-}
-
-// Level 2 over the segments of the folded histogram (L2Fold): segment j =
-// (a, g), a = j / nsb, holds [O1[a * nblk + g * spb], O1[a * nblk +
-// min((g + 1) * spb, nblk)]) of the level-1 array; its run of sub-digit s
-// starts at O2T[(j << dbits) + s] (the scan of H2, transposed so that a
-// segment's bases are one contiguous run).  Block i takes
-// the segments that start in its 1/G share of the keys and sorts them tile by
-// tile (TQ keys) as k_ms_scatter_p does, the next tile's keys loaded ahead;
-// within a segment each tile's runs start where the previous tile's ended.
-__device__ __forceinline__ void seg_bounds(const ull* O1, uint64_t nblk, int spb, uint64_t nsb, ull j, ull& st,
-                                           ull& en) {
-  const ull a = j / nsb, sb = j - a * nsb;
-  const ull lo = sb * (ull)spb;
-  const ull hi = lo + (ull)spb < nblk ? lo + (ull)spb : nblk;
-  st = O1[a * nblk + lo];
-  en = O1[a * nblk + hi];
-}
-
-__device__ __forceinline__ ull seg_first_at(const ull* O1, uint64_t nblk, int spb, uint64_t nsb, ull nseg, ull k) {
-  ull lo = 0, hi = nseg;
-  while (lo < hi) {
-    const ull mid = (lo + hi) >> 1;
-    ull st, en;
-    seg_bounds(O1, nblk, spb, nsb, mid, st, en);
-    if (st < k) lo = mid + 1; else hi = mid;
-  }
-  return lo;
-}
-
-template <class Key, int NT>
-__global__ __launch_bounds__(NT, 4) void k_ms_scatter_seg(const Key* Sin, const ull* O1, uint64_t nblk, int spb,
-                                                          uint64_t nsb, int nb1, ull total, int dpos, int dbits,
-                                                          const ull* O2T, Key* Sout) {
-  constexpr int TQ = MS_NT * TileCfg<Key>::Q;
-  constexpr int Q = TQ / NT;
-  __shared__ TileLds<Key, MS_NT> L;
-  const ull nseg = (ull)nb1 * nsb;
-  const ull k0 = total * (ull)blockIdx.x / gridDim.x;
-  const ull k1 = total * ((ull)blockIdx.x + 1) / gridDim.x;
-  ull j = seg_first_at(O1, nblk, spb, nsb, nseg, k0);
-  const ull j1 = blockIdx.x + 1 == gridDim.x ? nseg : seg_first_at(O1, nblk, spb, nsb, nseg, k1);
-  const int ns = 1 << dbits;
-  const int tid = (int)threadIdx.x;
-  // first non-empty segment
-  ull st = 0, en = 0;
-  while (j < j1) {
-    seg_bounds(O1, nblk, spb, nsb, j, st, en);
-    if (en > st) break;
-    j++;
-  }
-  if (j >= j1) return;
-  auto base_of = [&](ull jj) -> ull { return O2T[(jj << dbits) + (ull)tid]; };
-  ull pos = st;
-  int m = (int)(en - pos < (ull)TQ ? en - pos : (ull)TQ);
-  Key kr[Q];
-#pragma unroll
-  for (int q = 0; q < Q; q++) {
-    const int idx = tid + q * NT;
-    kr[q] = idx < m ? Sin[pos + idx] : Key(0);
-  }
-  ull bs = tid < ns ? base_of(j) : 0ull;
-  for (;;) {
-    // the next tile: further in this segment, or the next non-empty segment
-    ull jn = j, posn = pos + (ull)m, enn = en;
-    bool more = true;
-    if (posn >= en) {
-      jn = j + 1;
-      ull s2 = 0, e2 = 0;
-      while (jn < j1) {
-        seg_bounds(O1, nblk, spb, nsb, jn, s2, e2);
-        if (e2 > s2) break;
-        jn++;
-      }
-      more = jn < j1;
-      posn = s2;
-      enn = e2;
-    }
-    Key kn[Q] = {};
-    ull bn = 0;
-    int mn = 0;
-    if (more) {
-      mn = (int)(enn - posn < (ull)TQ ? enn - posn : (ull)TQ);
-#pragma unroll
-      for (int q = 0; q < Q; q++) {
-        const int idx = tid + q * NT;
-        kn[q] = idx < mn ? Sin[posn + idx] : Key(0);
-      }
-      if (tid < ns && jn != j) bn = base_of(jn);
-    }
-    if (tid < ns) L.h[tid] = 0;
-    const int np = m > tid ? (m - tid - 1) / NT + 1 : 0;
-    __syncthreads();
-    uint32_t rk[(Q + 1) / 2] = {};
-#pragma unroll
-    for (int q = 0; q < Q; q++)
-      if (q < np) rk[q / 2] |= atomicAdd(&L.h[key_digit<Key>(kr[q], dpos, dbits)], 1u) << (16 * (q & 1));
-    __syncthreads();
-    const uint32_t v = tid < ns ? L.h[tid] : 0u;
-    if (more && jn == j) bn = bs + v;
-    const ull ex = block_excl_scan<NT>(v);
-    if (tid < ns) {
-      L.tcur[tid] = (uint32_t)ex;
-      L.delta[tid] = (long long)bs - (long long)ex;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int q = 0; q < Q; q++) {
-      if (q < np) {
-        const uint32_t d = key_digit<Key>(kr[q], dpos, dbits);
-        L.T1[L.tcur[d] + ((rk[q / 2] >> (16 * (q & 1))) & 0xFFFFu)] = kr[q];
-      }
-    }
-    __syncthreads();
-    for (int p = tid; p < m; p += NT) {
-      const Key w = L.T1[p];
-      Sout[L.delta[key_digit<Key>(w, dpos, dbits)] + p] = w;
-    }
+    cnt += all;
     __syncthreads();
     if (!more) break;
-#pragma unroll
-    for (int q = 0; q < Q; q++) kr[q] = kn[q];
-    bs = bn;
-    j = jn;
-    pos = posn;
-    en = enn;
-    m = mn;
+  }
+  // pieces before each word
+  uint32_t carry = 0;
+  for (int b = 0; b < nwords; b += NT) {
+    const int i = b + (int)threadIdx.x;
+    uint32_t tot;
+    const uint32_t ex = block_scan_u32<NT>(i < nwords ? (uint32_t)__popc(mw[i].x) : 0u, nw, &tot);
+    if (i < nwords) mw[i].y = carry + ex;
+    carry += tot;
+    __syncthreads();
+  }
+  return (int)cnt;
+}
+
+__device__ __forceinline__ uint32_t map_piece(const uint2* mw, int i) {
+  const uint2 q = mw[i >> 5];
+  return q.y + (uint32_t)__popc(q.x & (0xFFFFFFFFu >> (31 - (i & 31)))) - 1u;
+}
+
+// The same for places tid, tid + NT, ... of thread tid: the word is mt[j *
+// NT / 32] with mt = mw + tid / 32, and the bits up to the place are the
+// same for all (one LDS address per thread instead of one per place).
+__device__ __forceinline__ uint32_t map_low(int tid) { return 0xFFFFFFFFu >> (31 - (tid & 31)); }
+__device__ __forceinline__ uint32_t map_piece(uint2 q, uint32_t low) { return q.y + (uint32_t)__popc(q.x & low) - 1u; }
+
+// Piece of place v by binary search (a map that did not fit): the last one in
+// [f, end) that starts at or before v.
+__device__ __forceinline__ ull find_piece(const ull* V, ull f, ull end, ull v) {
+  ull lo = f, hi = end;  // V[lo] <= v, hi past the last
+  while (hi - lo > 1) {
+    const ull mid = (lo + hi) >> 1;
+    if (V[mid] <= v) lo = mid; else hi = mid;
+  }
+  return lo;
+}
+
+// Tiles of a level: bucket offsets boff[0..B] of its input and tile prefix
+// tp[0..B] (one block).
+__global__ __launch_bounds__(1024) void k_tiles(Runs in, ull B, int tk, ull total, ull* boff, ull* tp) {
+  __shared__ uint32_t nw[17];
+  ull acc = 0;
+  for (ull base = 0; base < B; base += 1024) {
+    const ull b = base + threadIdx.x;
+    RunBucket r{};
+    if (b < B) r = run_bucket(in, b);
+    uint32_t tot;
+    const uint32_t nt = (uint32_t)((r.n + tk - 1) / tk);
+    const uint32_t ex = block_scan_u32<1024>(nt, nw, &tot);
+    if (b < B) {
+      boff[b] = r.v0;
+      tp[b] = acc + ex;
+    }
+    acc += tot;
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) {
+    boff[B] = total;
+    tp[B] = acc;
   }
 }
 
-// O2T[((a * nsb + g) << db) + s] = O2[((a << db) + s) * nsb + g]: per
-// level-1 bucket a, the (digit, segment) matrix of bases transposed through
-// LDS in 32 x 32 tiles (grid: segment tiles, digit tiles, a).
-__global__ __launch_bounds__(256) void k_seg_transpose(const ull* O2, uint64_t nsb, int db, ull* O2T) {
-  __shared__ ull t[32][33];
-  const uint64_t a = blockIdx.z;
-  const int S = 1 << db;
-  const uint64_t g0 = (uint64_t)blockIdx.x * 32;
-  const int s0 = (int)blockIdx.y * 32;
-  const int tx = (int)threadIdx.x & 31, ty = (int)threadIdx.x >> 5;
-  const ull* src = O2 + ((a << db) * nsb);
-  for (int r = ty; r < 32; r += 8) {
-    const int sd = s0 + r;
-    const uint64_t g = g0 + (uint64_t)tx;
-    if (sd < S && g < nsb) t[r][tx] = src[(uint64_t)sd * nsb + g];
+// One bucket over all windows (level 1's input).
+__global__ void k_tiles_one(ull ntiles, ull total, ull* boff, ull* tp) {
+  if (threadIdx.x || blockIdx.x) return;
+  boff[0] = 0;
+  boff[1] = total;
+  tp[0] = 0;
+  tp[1] = ntiles;
+}
+
+// Source of level 1: window i (of all reads' windows in order) belongs to
+// the last read with kofs[r] <= i and starts at byte rstart[r] + i - kofs[r].
+struct WinSrc {
+  const uint32_t* E;
+  const uint32_t* RX;
+  const ull* kofs;    // R + 1 offsets
+  const ull* rstart;
+  ull R;
+  int K;
+};
+
+enum { SPLIT_RUNS, SPLIT_MAIN, SPLIT_BUILDER };
+
+// Low 32-bit words of the window that ends at byte e, nw of them, low first.
+template <int NWORDS>
+__device__ __forceinline__ void window_words(const uint32_t* E, ull e, uint32_t* out) {
+  const uint32_t* p = E + (PK_PAD + (e >> 4) - NWORDS);
+  const uint32_t sh = 30u - 2u * (uint32_t)(e & 15);
+  uint32_t w[NWORDS + 1];
+#pragma unroll
+  for (int i = 0; i <= NWORDS; i++) w[i] = p[i];
+#pragma unroll
+  for (int i = 0; i < NWORDS; i++)
+    out[i] = __builtin_amdgcn_alignbit(w[NWORDS - 1 - i], w[NWORDS - i], sh);
+}
+
+template <class Key>
+__device__ __forceinline__ Key window_key(const WinSrc& s, ull e) {
+  uint32_t o[sizeof(Key) / 4];
+  window_words<(int)sizeof(Key) / 4>(s.E, e, o);
+  Key k = 0;
+#pragma unroll
+  for (int i = (int)sizeof(Key) / 4 - 1; i >= 0; i--) k = (k << 31 << 1) | (Key)o[i];
+  return k;
+}
+
+template <class Key, int SRC>
+__global__ __launch_bounds__(SP_NT, 4) void k_split(const Key* __restrict__ Sin, WinSrc ws, Runs in, int nb, int tk,
+                                                    Key mask, int dpos, int db, const ull* __restrict__ boff,
+                                                    const ull* __restrict__ tp, uint32_t* __restrict__ M,
+                                                    Key* __restrict__ Sout) {
+  constexpr int Q = SplitCfg<Key>::Q;
+  constexpr int ROUND = SplitCfg<Key>::ROUND;
+  // the tile buffer; before the keys are loaded, the map's piece table
+  __shared__ __align__(16) unsigned char buf[SP_TILE_BYTES];
+  // digit counts, then starts; before, the map's words
+  __shared__ uint32_t h[1 << SP_MAX_BITS];
+  __shared__ uint32_t nw[SP_NT / 64 + 1];
+  static_assert(SplitCfg<Key>::TK_MAX / 32 * sizeof(uint2) <= sizeof(h), "map words fit the digit counts");
+  uint2* mw = reinterpret_cast<uint2*>(h);
+  Key* T = reinterpret_cast<Key*>(buf);
+  const int tid = (int)threadIdx.x;
+  const uint2* mt = mw + (tid >> 5);
+  const uint32_t low = map_low(tid);
+  const ull blk = blockIdx.x;
+  if (blk >= tp[nb]) return;
+  const ull a = nb == 1 ? 0 : uniform(block_upper<SP_NT>(tp, (ull)nb, blk) - 1);
+  const ull t0 = uniform(tp[a]), nt = uniform(tp[a + 1]) - t0, t = blk - t0;
+  const ull v0 = uniform(boff[a]) + t * (ull)tk;
+  const ull left = uniform(boff[a + 1]) - v0;
+  const int m = left < (ull)tk ? (int)left : tk;
+  Key kr[Q];
+  if (SRC == SPLIT_RUNS) {
+    if (!in.M) {
+#pragma unroll
+      for (int j = 0; j < Q; j++) {
+        const int i = tid + j * SP_NT;
+        if (i < m) kr[j] = Sin[v0 + i];
+      }
+    } else {
+      const RunBucket rb = uniform(run_bucket(in, a));
+      const ull f = rb.e0 + (rb.nt > SP_NT ? block_upper<SP_NT>(in.V + rb.e0, rb.nt, v0) - 1 : 0);
+      constexpr int CAP = SP_TILE_BYTES / 8;
+      ull* delta = reinterpret_cast<ull*>(buf);
+      auto src = [&](ull e) { return rb.base + (e - rb.e0) * (ull)in.tk + (in.M[e] >> 16); };
+      const int np = map_pieces<SP_NT>(mw, nw, CAP, in.V, f, rb.e0 + rb.nt, v0, m, src,
+                                       [&](uint32_t r, ull d, ull) { delta[r] = d; });
+#pragma unroll
+      for (int j = 0; j < Q; j++) {
+        const int i = tid + j * SP_NT;
+        if (i < m) {
+          ull p;
+          if (np <= CAP) {
+            p = delta[map_piece(mt[j * (SP_NT / 32)], low)] + (ull)i;
+          } else {
+            const ull e = find_piece(in.V, f, rb.e0 + rb.nt, v0 + i);
+            p = src(e) + (v0 + i - in.V[e]);
+          }
+          kr[j] = Sin[p];
+        }
+      }
+    }
+  } else {
+    // level 1: the reads of these windows
+    const ull f = block_upper<SP_NT>(ws.kofs, ws.R, v0) - 1;
+    constexpr bool BLD = SRC == SPLIT_BUILDER;
+    constexpr int CAP = SP_TILE_BYTES / (BLD ? 12 : 8);
+    ull* delta = reinterpret_cast<ull*>(buf);
+    uint32_t* aux = reinterpret_cast<uint32_t*>(buf + 8 * CAP);  // builder: v0 - kofs (mod 2^32)
+    auto src = [&](ull r) { return ws.rstart[r]; };
+    const int np = map_pieces<SP_NT>(mw, nw, CAP, ws.kofs, f, ws.R, v0, m, src, [&](uint32_t r, ull d, ull idx) {
+      delta[r] = d;
+      if (BLD) aux[r] = (uint32_t)(v0 - ws.kofs[idx]);
+    });
+#pragma unroll
+    for (int j = 0; j < Q; j++) {
+      const int i = tid + j * SP_NT;
+      if (i < m) {
+        ull p;
+        uint32_t wi = 0;  // builder: index of the window in its read
+        if (np <= CAP) {
+          const uint32_t r = map_piece(mt[j * (SP_NT / 32)], low);
+          p = delta[r] + (ull)i;
+          if (BLD) wi = aux[r] + (uint32_t)i;
+        } else {
+          const ull r = find_piece(ws.kofs, f, ws.R, v0 + i);
+          p = ws.rstart[r] + (v0 + i - ws.kofs[r]);
+          if (BLD) wi = (uint32_t)(v0 + i - ws.kofs[r]);
+        }
+        const ull e = p + (ull)(ws.K - 1);  // the window's last byte
+        Key k = window_key<Key>(ws, e);
+        if (BLD) {
+          // the word holds the last 4 * sizeof(kmer_t) bases since the
+          // read's start
+          const uint32_t bases = wi + (uint32_t)ws.K;
+          if (bases < 4u * (uint32_t)sizeof(Key)) k &= (Key(1) << (2 * bases)) - 1;
+        } else {
+          // the last base's low bit, without the next byte's spill
+          k = (k & ~Key(1)) | (Key)((ws.RX[e >> 4] >> (e & 15)) & 1u);
+          k &= mask;
+        }
+        kr[j] = k;
+      }
+    }
   }
   __syncthreads();
-  ull* dst = O2T + ((a * nsb) << db);
-  for (int r = ty; r < 32; r += 8) {
-    const uint64_t g = g0 + (uint64_t)r;
-    const int sd = s0 + tx;
-    if (sd < S && g < nsb) dst[(g << db) + (uint64_t)sd] = t[tx][r];
+  const int ns = 1 << db;
+  for (int i = tid; i < ns; i += SP_NT) h[i] = 0;
+  __syncthreads();
+  // each key's rank inside its digit, two 16-bit ranks per register
+  uint32_t rk[Q / 2] = {};
+#pragma unroll
+  for (int j = 0; j < Q; j++)
+    if (tid + j * SP_NT < m) rk[j / 2] |= atomicAdd(&h[key_digit<Key>(kr[j], dpos, db)], 1u) << (16 * (j & 1));
+  __syncthreads();
+  {
+    static_assert((1 << SP_MAX_BITS) == 2 * SP_NT, "two digits per thread");
+    const int d = 2 * tid;
+    const uint32_t c0 = d < ns ? h[d] : 0u, c1 = d + 1 < ns ? h[d + 1] : 0u;
+    uint32_t tot;
+    const uint32_t ex = block_scan_u32<SP_NT>(c0 + c1, nw, &tot);
+    const ull mo = (t0 << db) + (ull)d * nt + t;
+    if (d < ns) {
+      h[d] = ex;
+      M[mo] = ex << 16 | c0;
+    }
+    if (d + 1 < ns) {
+      h[d + 1] = ex + c0;
+      M[mo + nt] = (ex + c0) << 16 | c1;
+    }
   }
-}
-
-// boff2[(a << db) | s] = the first segment's base, O2T[((a * nsb) << db) + s];
-// boff2[end] = total
-__global__ void k_seg_boff(const ull* O2T, uint64_t nsb, int db, ull n2, ull total, ull* boff2) {
-  const ull g = (ull)blockIdx.x * blockDim.x + threadIdx.x;
-  const ull mask = (1ull << db) - 1;
-  if (g < n2) boff2[g] = O2T[(((g >> db) * nsb) << db) + (g & mask)];
-  if (g == n2) boff2[n2] = total;
+  __syncthreads();
+  // place of every key in the sorted tile
+#pragma unroll
+  for (int j = 0; j < Q; j++)
+    if (tid + j * SP_NT < m) rk[j / 2] += h[key_digit<Key>(kr[j], dpos, db)] << (16 * (j & 1));
+  for (int r0 = 0; r0 < m; r0 += ROUND) {
+#pragma unroll
+    for (int j = 0; j < Q; j++) {
+      if (tid + j * SP_NT < m) {
+        const uint32_t p = ((rk[j / 2] >> (16 * (j & 1))) & 0xFFFFu) - (uint32_t)r0;
+        if (p < (uint32_t)ROUND) T[p] = kr[j];
+      }
+    }
+    __syncthreads();
+    const int c = m - r0 < ROUND ? m - r0 : ROUND;
+    Key* o = Sout + v0 + r0;
+    for (int p = tid; p < c; p += SP_NT) o[p] = T[p];
+    __syncthreads();
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -1656,25 +1671,28 @@ __global__ void k_seg_boff(const ull* O2T, uint64_t nsb, int db, ull n2, ull tot
 // merge + aggregate (kmer_counting.cpp:3057-3086, 254-352, 169-250) for the
 // keys of one bucket.
 
-constexpr int BS_NT = 256;
-constexpr int SUB_MAX_BITS = 9;
+constexpr int BS_NT = 512;
+constexpr int SUB_MAX_BITS = 10;
 constexpr int SUB_BINS = 1 << SUB_MAX_BITS;
 
+// Tables of 512 threads, three blocks (6 waves per SIMD) per CU: half as many
+// buckets as with 256 threads, so half the run-table look-ups, barriers and
+// partition digits per key.
 template <class Key>
 struct HashCfg;
 template <>
 struct HashCfg<uint64_t> {
-  static constexpr int T = 2048;      // table slots
-  static constexpr int LIMIT = 1536;  // distinct keys per task (load 0.75)
-  static constexpr int SUB = 9;       // sub-digit bits of the ordering pass
-  static constexpr int BLOCKS = 6;    // blocks per CU the LDS allows (register cap follows)
+  static constexpr int T = 4096;      // table slots (12 bytes each)
+  static constexpr int LIMIT = 3072;  // distinct keys per task (load 0.75)
+  static constexpr int HB = 16;       // keys per thread and batch
+  static constexpr int WAVES = 6;     // waves per SIMD the LDS allows (register cap follows)
 };
 template <>
 struct HashCfg<u128> {
-  static constexpr int T = 1024;
-  static constexpr int LIMIT = 768;
-  static constexpr int SUB = 8;
-  static constexpr int BLOCKS = 5;
+  static constexpr int T = 2048;  // 20 bytes each
+  static constexpr int LIMIT = 1536;
+  static constexpr int HB = 9;
+  static constexpr int WAVES = 6;
 };
 // tasks with more instances than this are split without trying
 constexpr uint64_t TASK_MAX_INSTANCES = 1u << 18;
@@ -1707,6 +1725,13 @@ struct HashTable<uint64_t> {
   // when a long chain finds the table already reported full (*stop)
   // (a read before the CAS, as for u128 keys, was slower here: a new key
   // then waits on two LDS round trips)
+  // one 32-bit product: the kernel is bound by issue, and a 64-bit one is
+  // three quarter-rate instructions
+  __device__ __forceinline__ static uint32_t home(uint64_t k) {
+    const uint32_t lo = (uint32_t)k, hi = (uint32_t)(k >> 32);
+    static_assert((T & (T - 1)) == 0, "a power of two");
+    return ((lo ^ __builtin_amdgcn_alignbit(hi, hi, 13)) * 0x9E3779B1u) >> (32 - __builtin_ctz(T));
+  }
   __device__ __forceinline__ bool try_slot(uint32_t slot, uint64_t k) {
     const ull prev = atomicCAS(&hk[slot], empty, (ull)k);
     if (prev == empty || prev == (ull)k) {
@@ -1716,7 +1741,7 @@ struct HashTable<uint64_t> {
     return false;
   }
   __device__ __forceinline__ bool insert(uint64_t k, const volatile int* stop) {
-    uint32_t slot = (uint32_t)((k * 0x9E3779B97F4A7C15ull) >> 40) & (T - 1);
+    uint32_t slot = home(k);
     for (int probe = 0; probe < STOP_AFTER; probe++) {
       if (try_slot(slot, k)) return true;
       slot = (slot + 1) & (T - 1);
@@ -1732,39 +1757,39 @@ struct HashTable<uint64_t> {
   __device__ __forceinline__ uint64_t key(int i) const { return hk[i]; }
 };
 
-// u128 keys: claim by 64-bit fingerprint, full key stored beside it and
-// verified after all inserts (a fingerprint collision sends the task to the
-// split path, which separates the two keys).
+// u128 keys: claim by a 64-bit fingerprint that gives the low word back when
+// the high word is known; the high word is stored beside it (20 bytes per
+// slot with the count) and checked after the inserts (a fingerprint collision
+// sends the task to the split path, which separates the two keys).
 template <>
 struct HashTable<u128> {
   static constexpr int T = HashCfg<u128>::T;
   static constexpr ull EMPTY = ~0ull;
   ull* hf;
-  u128* hkf;
+  ull* hh;
   uint32_t* hc;
-  ull empty;
-  // the high word through one odd multiply (a bijection) folded into the
-  // low word, then one multiply-xorshift round for the top bits the home
-  // slot takes: two 64-bit products instead of the four of two full mixes
-  // (the table is bound by instruction issue).  Distinct keys of a task
-  // collide with probability ~2^-64 per pair; a collision only sends the
-  // task to the split path.
-  __device__ __forceinline__ static ull fp(u128 k) {
-    ull f = (ull)k ^ ((ull)(k >> 64) * 0x9e3779b97f4a7c15ull);
-    f ^= f >> 29;
-    f *= 0xbf58476d1ce4e5b9ull;
-    return f ^ (f >> 32);
+  // spread of the high word: two 32 x 32 -> 64 products.  Keys of a task that
+  // differ in a few bases of the high word differ in about half the bits of
+  // the products, which the low words of such keys do not match; other pairs
+  // collide with probability ~2^-64.  A collision only costs time.
+  __device__ __forceinline__ static ull spread(ull hi) {
+    const ull a = (ull)(uint32_t)hi * 0x9e3779b1ull;
+    const ull b = (ull)(uint32_t)(hi >> 32) * 0x85ebca77ull;
+    return a ^ (b << 32 | b >> 32) ^ 0x2545f4914f6cdd1dull;
   }
+  __device__ __forceinline__ static ull fp(u128 k) { return (ull)k ^ spread((ull)(k >> 64)); }
   __device__ __forceinline__ void init(int tid, int nt) {
     for (int i = tid; i < T; i += nt) {
       hf[i] = EMPTY;
       hc[i] = 0;
     }
   }
-  // home slot from the fingerprint's top bits, scaled to T (T need not be a
-  // power of two); probes step to the next slot, wrapping
-  __device__ __forceinline__ uint32_t home(ull f) const { return (uint32_t)(((f >> 32) * (ull)T) >> 32); }
-  __device__ __forceinline__ static uint32_t next(uint32_t slot) { return slot + 1 == (uint32_t)T ? 0u : slot + 1; }
+  // home slot: one more 32-bit product; probes step to the next slot
+  __device__ __forceinline__ static uint32_t home(ull f) {
+    static_assert((T & (T - 1)) == 0, "a power of two");
+    return (((uint32_t)f ^ (uint32_t)(f >> 32)) * 0x9E3779B1u) >> (32 - __builtin_ctz(T));
+  }
+  __device__ __forceinline__ static uint32_t next(uint32_t slot) { return (slot + 1) & (T - 1); }
   // a slot changes only once, from EMPTY to its fingerprint: a plain read
   // finds a repeated key or steps over another one without an atomic, and
   // only an empty slot is claimed by CAS (k = 64 bacterial: 2.73 -> 2.56 ms)
@@ -1772,7 +1797,7 @@ struct HashTable<u128> {
     ull prev = __hip_atomic_load(&hf[slot], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     if (prev == EMPTY) {
       prev = atomicCAS(&hf[slot], EMPTY, f);
-      if (prev == EMPTY) hkf[slot] = k;
+      if (prev == EMPTY) hh[slot] = (ull)(k >> 64);
     }
     if (prev == EMPTY || prev == f) {
       atomicAdd(&hc[slot], 1u);
@@ -1780,31 +1805,14 @@ struct HashTable<u128> {
     }
     return false;
   }
-  // the slot that counts k, or -1 (table full, stopped, or a fingerprint
-  // equal to EMPTY)
-  __device__ __forceinline__ int insert_at(u128 k, const volatile int* stop) {
-    const ull f = fp(k);
-    if (f == EMPTY) return -1;
-    uint32_t slot = home(f);
-    for (int probe = 0; probe < STOP_AFTER; probe++) {
-      if (try_slot(slot, f, k)) return (int)slot;
-      slot = next(slot);
-    }
-    for (int probe = STOP_AFTER; probe < HASH_PROBES; probe++) {
-      if ((probe & 7) == 0 && *stop) return -1;
-      if (try_slot(slot, f, k)) return (int)slot;
-      slot = next(slot);
-    }
-    return -1;
-  }
-  __device__ __forceinline__ bool insert(u128 k, const volatile int* stop) { return insert_at(k, stop) >= 0; }
-  // the first probe of insert_at alone: the home slot if it holds f or is
-  // claimed for it, else -1 (the slot holds another fingerprint)
+  // the first probe: the home slot if it holds f or is claimed for it, else
+  // -1 (the slot holds another fingerprint)
   __device__ __forceinline__ int try_home(u128 k, ull f) {
     const uint32_t slot = home(f);
     return try_slot(slot, f, k) ? (int)slot : -1;
   }
-  // the rest of insert_at, for a key whose home slot holds another fingerprint
+  // the rest, for a key whose home slot holds another fingerprint: the slot
+  // that counts k, or -1 (table full, or reported full by another thread)
   __device__ __forceinline__ int insert_after_home(u128 k, ull f, const volatile int* stop) {
     uint32_t slot = next(home(f));
     for (int probe = 1; probe < STOP_AFTER; probe++) {
@@ -1818,19 +1826,12 @@ struct HashTable<u128> {
     }
     return -1;
   }
-  // after a barrier: does key k sit in its fingerprint's slot?
-  __device__ __forceinline__ bool verify(u128 k) const {
-    const ull f = fp(k);
-    uint32_t slot = home(f);
-    for (int probe = 0; probe < T; probe++) {
-      if (hf[slot] == f) return hkf[slot] == k;
-      if (hf[slot] == EMPTY) return false;
-      slot = next(slot);
-    }
-    return false;
+  // after a barrier: does the slot that counted k hold k?
+  __device__ __forceinline__ bool verify(int slot, u128 k) const { return hh[slot] == (ull)(k >> 64); }
+  __device__ __forceinline__ u128 key(int i) const {
+    const ull hi = hh[i];
+    return (u128)hi << 64 | (u128)(hf[i] ^ spread(hi));
   }
-  __device__ __forceinline__ bool used(int i) const { return hc[i] != 0u; }
-  __device__ __forceinline__ u128 key(int i) const { return hkf[i]; }
 };
 
 template <class Key>
@@ -1850,174 +1851,270 @@ struct HashLds<uint64_t> {
 };
 template <>
 struct HashLds<u128> {
-  ull hf[HashCfg<u128>::T];
-  u128 hkf[HashCfg<u128>::T];
+  alignas(16) ull hf[HashCfg<u128>::T];
+  ull hh[HashCfg<u128>::T];  // with hf: room for T whole keys in the ordering
   uint32_t hc[HashCfg<u128>::T];
   __device__ __forceinline__ HashTable<u128> table(ull) {
     HashTable<u128> t;
     t.hf = hf;
-    t.hkf = hkf;
+    t.hh = hh;
     t.hc = hc;
-    t.empty = 0;
     return t;
   }
-  __device__ __forceinline__ u128* out_keys() { return hkf; }
+  __device__ __forceinline__ u128* out_keys() { return reinterpret_cast<u128*>(hf); }
 };
 
-// Tasks: [tstart[i], tstart[i] + tcount[i]) of S, whose keys share their top
-// `fixed` bits (fixed >= 1).  Writes the task's unique (key, count) pairs in
-// ascending order to R / C at the task's start and tu[i] = their number.  A
-// task with more distinct keys than a table holds is processed in 2^s passes,
-// pass p taking the keys whose next s bits equal p (s = 1, 2, ... up to
-// MAX_PASS_BITS); beyond that, or on a u128 fingerprint collision, tu[i] = -1
-// and the task index goes to ovf_list for the host-driven split.
+// A batch of a task's keys is gathered from its runs through a map (see
+// map_pieces) that lies in the idle sub-bin array: a word pair per 32 places
+// and RUN_CAP 32-bit run offsets from the parent's first tile (a task whose
+// parent has 2^32 keys or more goes to the split path).  A batch with more
+// runs than that is cut down to as many places as there is room.
 constexpr int MAX_PASS_BITS = 4;
+constexpr int RUN_CAP = 512;
+constexpr int HASH_QUEUE = 1024;
 
 template <class Key>
-__global__ __launch_bounds__(BS_NT, HashCfg<Key>::BLOCKS) void k_bucket_hash(const Key* S, Key* R, int32_t* C,
-                                                       const ull* tstart, const ull* tcount,
-                                                       uint64_t ntasks, int K, int fixed,
-                                                       long long* tu, ull* ovf_count, ull* ovf_list) {
+struct HashShared {
+  HashLds<Key> lds;
+  alignas(8) uint32_t hs[SUB_BINS];
+  uint32_t nw[BS_NT / 64 + 1];
+  int over;
+  // u128: keys of the batch queued for their probe chains (place in the batch,
+  // then the slot found, 0xFFFF for none)
+  int qn;
+  uint16_t hq[sizeof(Key) == 16 ? HASH_QUEUE : 1];
+};
+
+// The map of a batch built by the block's first wave alone (the others clear
+// the hash table meanwhile): LDS operations of one wave stay in order, so it
+// needs no barrier of its own.  The places are [b, b + m) of the task, offsets
+// are from the parent's first tile.  Returns false when the runs do not fit;
+// the map then points at the parent's first keys.
+constexpr ull WAVE_MAP_RUNS = 4096;  // entries a wave looks through
+
+__device__ __forceinline__ bool wave_map(uint2* mw, int nwords, uint32_t* off, const Runs& in, const RunBucket& rb,
+                                         uint32_t b, int m) {
+  const int lane = (int)threadIdx.x;
+  const uint32_t nt = (uint32_t)rb.nt;
+  const ull* V = in.V + rb.e0;
+  const uint32_t* M = in.M + rb.e0;
+  for (int w = lane; w < nwords; w += 64) mw[w].x = 0;
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  uint32_t cnt = 0;
+  for (uint32_t c = 0; c < nt; c += 64) {
+    const uint32_t idx = c + lane;
+    uint32_t vs = 0, ve = 0, so = 0;
+    if (idx < nt) {
+      vs = (uint32_t)(V[idx] - rb.v0);
+      ve = (uint32_t)(V[idx + 1] - rb.v0);
+      so = idx * (uint32_t)in.tk + (M[idx] >> 16) - vs;
+    }
+    const bool part = ve > vs && vs < b + (uint32_t)m && ve > b;
+    const ull bal = __ballot(part);
+    const uint32_t r = cnt + (uint32_t)__popcll(bal & ((1ull << lane) - 1));
+    if (part && r < (uint32_t)RUN_CAP) {
+      off[r] = so + b;
+      const uint32_t ls = vs > b ? vs - b : 0u;
+      atomicOr(&mw[ls >> 5].x, 1u << (ls & 31));
+    }
+    cnt += (uint32_t)__popcll(bal);
+  }
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  // pieces before each word: consecutive words per lane
+  const int wpl = (nwords + 63) / 64;
+  uint32_t sum = 0;
+  for (int i = 0; i < wpl; i++) {
+    const int w = lane * wpl + i;
+    if (w < nwords) sum += (uint32_t)__popc(mw[w].x);
+  }
+  uint32_t x = sum;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const uint32_t y = __shfl_up(x, o, 64);
+    if (lane >= o) x += y;
+  }
+  x -= sum;
+  for (int i = 0; i < wpl; i++) {
+    const int w = lane * wpl + i;
+    if (w < nwords) {
+      mw[w].y = x;
+      x += (uint32_t)__popc(mw[w].x);
+    }
+  }
+  if (cnt <= (uint32_t)RUN_CAP) return true;
+  for (int w = lane; w < nwords; w += 64) mw[w] = make_uint2(1u, 0u);
+  if (lane == 0) off[0] = 0;
+  return false;
+}
+
+// Loads the keys at [b, b + m) of the task into kb (thread t: t, t + BS_NT,
+// ...); returns m.  LIGHT (a task of at most TASK_MAX_INSTANCES keys and
+// WAVE_MAP_RUNS runs): the map by the first wave, which sets over to 3 when the
+// runs do not fit (kb then holds other keys of the parent).
+template <class Key, bool RUNS, bool LIGHT, int HB>
+__device__ __forceinline__ int load_batch(HashShared<Key>& L, const Key* Sb, const Runs& in, const RunBucket& rb,
+                                          ull b, Key (&kb)[HB]) {
+  constexpr int BATCH = BS_NT * HB;
+  static_assert(BATCH / 32 * sizeof(uint2) + RUN_CAP * 4 <= sizeof(L.hs), "the run map fits the sub-bins");
+  if constexpr (!RUNS) {
+#pragma unroll
+    for (int j = 0; j < HB; j++) {
+      const uint64_t idx = b + threadIdx.x + (uint64_t)j * BS_NT;
+      kb[j] = idx < rb.n ? Sb[idx] : Key(0);
+    }
+    return rb.n - b < (ull)BATCH ? (int)(rb.n - b) : BATCH;
+  } else {
+    int m = rb.n - b < (ull)BATCH ? (int)(rb.n - b) : BATCH;
+    uint2* mw = reinterpret_cast<uint2*>(L.hs);
+    uint32_t* off = L.hs + BATCH / 32 * 2;
+    if constexpr (LIGHT) {
+      if (threadIdx.x < 64 && !wave_map(mw, (m + 31) >> 5, off, in, rb, (uint32_t)b, m)) L.over = 3;
+      __syncthreads();
+    } else {
+      const ull end = rb.e0 + rb.nt, vb = rb.v0 + b;
+      const ull f = rb.e0 + (rb.nt > BS_NT ? block_upper<BS_NT>(in.V + rb.e0, rb.nt, vb) - 1 : 0);
+      auto src = [&](ull e) { return (e - rb.e0) * (ull)in.tk + (in.M[e] >> 16); };
+      for (;;) {
+        __syncthreads();  // hs may still be read
+        const int np = map_pieces<BS_NT>(mw, L.nw, RUN_CAP, in.V, f, end, vb, m, src,
+                                         [&](uint32_t r, ull d, ull) { off[r] = (uint32_t)d; });
+        if (np <= RUN_CAP) break;
+        m = RUN_CAP;
+      }
+    }
+    const uint2* mt = mw + (threadIdx.x >> 5);
+    const uint32_t low = map_low((int)threadIdx.x);
+#pragma unroll
+    for (int j = 0; j < HB; j++) {
+      const int i = (int)threadIdx.x + j * BS_NT;
+      kb[j] = i < m ? Sb[off[map_piece(mt[j * (BS_NT / 32)], low)] + (uint32_t)i] : Key(0);
+    }
+    return m;
+  }
+}
+
+// Counts one task: keys rb of S, which share their top `fixed` bits (fixed >=
+// 1; top = the first of them).  Writes the task's unique (key, count) pairs
+// in ascending order to R / C at rb.v0 and their number to *out_n, returns 0;
+// 1 when the table is too small for the distinct keys, 2 on a u128
+// fingerprint collision, 3 when a batch has too many runs.  With MULTI a task with too many distinct keys is
+// processed in 2^s passes, pass p taking the keys whose next s bits equal p
+// (s = 1, 2, ... up to MAX_PASS_BITS).
+template <class Key, bool RUNS, bool MULTI>
+__device__ __forceinline__ int count_task(HashShared<Key>& L, const Key* S, Key* R, int32_t* C, const Runs& in,
+                                          const RunBucket& rb, bool top, int K, int fixed, ull* out_n) {
   constexpr int T = HashCfg<Key>::T;
   constexpr int PER = T / BS_NT;  // table slots per thread
-  constexpr int HB = sizeof(Key) == 8 ? 16 : 8;
-  __shared__ HashLds<Key> lds;
-  __shared__ uint32_t hs[SUB_BINS];
-  __shared__ int over;
-  __shared__ int qn;  // u128: keys of the batch queued for their probe chains
-
-  const uint64_t task = blockIdx.x;
-  if (task >= ntasks) return;
-  const uint64_t start = tstart[task];
-  const uint64_t n = tcount[task];
-  if (n == 0) {
-    if (threadIdx.x == 0) tu[task] = 0;
-    return;
-  }
+  constexpr int HB = HashCfg<Key>::HB;
+  uint32_t* hs = L.hs;
+  const ull start = rb.v0, n = rb.n;
   const int rem = 2 * K - fixed;
-  // EMPTY for u64 tables: the task's first key with its top key bit flipped
-  // (all keys of the task share that bit, so this value is not in the task)
-  const Key k0 = S[start];
-  const ull empty = (ull)(k0 ^ (Key(1) << (2 * K - 1)));
-  HashTable<Key> ht = lds.table(empty);
-  const int max_s = rem < MAX_PASS_BITS ? rem : MAX_PASS_BITS;
-  bool done = false;
+  // EMPTY for u64 tables: a key whose top bit differs from the task's (all
+  // keys of the task share that bit, so this value is not in the task)
+  HashTable<Key> ht = L.lds.table((ull)(top ? Key(0) : Key(1) << (2 * K - 1)));
+  const Key* Sb = S + (RUNS ? rb.base : start);
+  const int max_s = !MULTI ? 0 : rem < MAX_PASS_BITS ? rem : MAX_PASS_BITS;
   ull out = 0;
+  int s = 0, fail = 0;
   // a first try with all keys is pointless when there are too many of them
-  int s = 0;
-  while (s < max_s && (n >> s) > (uint64_t)TASK_MAX_INSTANCES) s++;
-  for (; s <= max_s && !done; s++) {
+  if (!MULTI && (n > (ull)TASK_MAX_INSTANCES || rb.nt > WAVE_MAP_RUNS)) return 1;
+  while (MULTI && s < max_s && (n >> s) > (ull)TASK_MAX_INSTANCES) s++;
+  for (; s <= max_s; s++) {
     out = 0;
-    bool failed = false;
-    for (int pass = 0; pass < (1 << s) && !failed; pass++) {
+    fail = 0;
+    for (int pass = 0; pass < (MULTI ? 1 << s : 1) && !fail; pass++) {
+      auto mine = [&](Key k) { return !MULTI || (int)key_digit<Key>(k, rem - s, s) == pass; };
+      if (threadIdx.x == 0) L.over = 0;
       ht.init(threadIdx.x, BS_NT);
-      if (threadIdx.x == 0) over = 0;
-      __syncthreads();
+      // (the first batch's map is built before the barrier that ends the
+      // clearing)
+      if (!RUNS || MULTI) __syncthreads();
       // keys are loaded HB at a time into registers so that the global-load
-      // latency is paid once per batch, not once per insert; a task of one
-      // batch keeps them there for the fingerprint check below
+      // latency is paid once per batch, not once per insert
       Key kb[HB];
-      int ksl[HB];  // u128: the slot each key of the (last) batch landed in
-      int ov = 0;   // u128: over as read after the last batch's final barrier
-      for (uint64_t b = 0; b < n; b += (uint64_t)BS_NT * HB) {
-#pragma unroll
-        for (int j = 0; j < HB; j++) {
-          const uint64_t idx = b + threadIdx.x + (uint64_t)j * BS_NT;
-          kb[j] = idx < n ? S[start + idx] : Key(0);
-        }
+      int ksl[HB];  // u128: the slot each key of the batch landed in
+      bool clash = false;
+      // over as read after the last batch's final barrier (nothing writes it
+      // between that read and the next barrier): all threads leave together
+      int ov = 0, m = 0;
+      for (ull b = 0; b < n && !ov; b += m) {
+        m = load_batch<Key, RUNS, !MULTI, HB>(L, Sb, in, rb, b, kb);
         if constexpr (sizeof(Key) == 16) {
           // A wave runs each probe step as long as its slowest lane needs
           // it, so a batch goes in two phases: every key tries its home slot
           // (one probe, the common case), and the keys whose home slot holds
-          // another fingerprint queue up (in hs, idle until the output
-          // phase) and are then probed by all lanes together, so a long
-          // chain holds up one queue round instead of each of the eight
-          // keys of its lane.  Every thread takes the overflow exit on the
-          // value read after the previous batch's last barrier (nothing
-          // writes over between that read and the next barrier), so all
-          // leave the loop together.
-          if (ov) break;
-          if (threadIdx.x == 0) qn = 0;
+          // another fingerprint queue up and are then probed by all lanes
+          // together, so a long chain holds up one queue round instead of
+          // each of the eight keys of its lane.
+          if (threadIdx.x == 0) L.qn = 0;
           __syncthreads();
           int qp[HB];
 #pragma unroll
           for (int j = 0; j < HB; j++) {
             qp[j] = -1;
-            const uint64_t idx = b + threadIdx.x + (uint64_t)j * BS_NT;
-            if (idx < n && (int)key_digit<Key>(kb[j], rem - s, s) == pass) {
+            const int i = (int)threadIdx.x + j * BS_NT;
+            if (i < m && mine(kb[j])) {
               const ull f = HashTable<u128>::fp(kb[j]);
               ksl[j] = f == HashTable<u128>::EMPTY ? -2 : ht.try_home(kb[j], f);
               if (ksl[j] == -2) {
-                over = 1;
+                L.over = 1;
               } else if (ksl[j] < 0) {
-                const int q = atomicAdd(&qn, 1);
-                if (q < SUB_BINS) {
-                  hs[q] = (uint32_t)(threadIdx.x + j * BS_NT);
+                const int q = atomicAdd(&L.qn, 1);
+                if (q < HASH_QUEUE) {
+                  L.hq[q] = (uint16_t)i;
                   qp[j] = q;
                 } else {
-                  ksl[j] = ht.insert_after_home(kb[j], f, &over);
-                  if (ksl[j] < 0) over = 1;
+                  ksl[j] = ht.insert_after_home(kb[j], f, &L.over);
+                  if (ksl[j] < 0) L.over = 1;
                 }
               }
             }
           }
           __syncthreads();
-          const int nq = qn < SUB_BINS ? qn : SUB_BINS;
+          const int nq = L.qn < HASH_QUEUE ? L.qn : HASH_QUEUE;
           for (int q = threadIdx.x; q < nq; q += BS_NT) {
-            const u128 k = S[start + b + hs[q]];
-            const int sl = ht.insert_after_home(k, HashTable<u128>::fp(k), &over);
-            if (sl < 0) over = 1;
-            hs[q] = (uint32_t)sl;
+            const int i = L.hq[q];
+            ull o = b + (ull)i;
+            if constexpr (RUNS)
+              o = (ull)(hs[BS_NT * HB / 32 * 2 + map_piece(reinterpret_cast<const uint2*>(hs), i)] + (uint32_t)i);
+            const u128 k = Sb[o];
+            const int sl = ht.insert_after_home(k, HashTable<u128>::fp(k), &L.over);
+            if (sl < 0) L.over = 1;
+            L.hq[q] = (uint16_t)sl;
           }
           __syncthreads();
-          ov = over;
+          ov = L.over;
+          // a key counted in a slot that holds another high word shares its
+          // fingerprint with that key (ov == 0: every key has a slot)
+          if (!ov) {
 #pragma unroll
-          for (int j = 0; j < HB; j++)
-            if (qp[j] >= 0) ksl[j] = (int)hs[qp[j]];
+            for (int j = 0; j < HB; j++) {
+              if (qp[j] >= 0) ksl[j] = (int)L.hq[qp[j]];
+              const int i = (int)threadIdx.x + j * BS_NT;
+              if (i < m && mine(kb[j]) && !ht.verify(ksl[j], kb[j])) clash = true;
+            }
+          }
         } else {
-          if (*(volatile int*)&over) break;
 #pragma unroll
           for (int j = 0; j < HB; j++) {
-            const uint64_t idx = b + threadIdx.x + (uint64_t)j * BS_NT;
-            if (idx < n && (int)key_digit<Key>(kb[j], rem - s, s) == pass && !ht.insert(kb[j], &over)) over = 1;
+            const int i = (int)threadIdx.x + j * BS_NT;
+            if (i < m && mine(kb[j]) && !ht.insert(kb[j], &L.over)) L.over = 1;
+          }
+          if (b + m < n) {
+            __syncthreads();
+            ov = L.over;
+            __syncthreads();
           }
         }
       }
       __syncthreads();
       if constexpr (sizeof(Key) == 16) {
-        if (!over) {
-          // a key counted in a slot whose stored key differs shares its
-          // fingerprint with that key: the task goes to the split path.  A
-          // one-batch task checks the slots its inserts returned; a longer
-          // one reloads its keys and finds their slots again.
-          const bool one_batch = n <= (uint64_t)BS_NT * HB;
-          for (uint64_t b = 0; b < n; b += (uint64_t)BS_NT * HB) {
-            if (!one_batch) {
-#pragma unroll
-              for (int j = 0; j < HB; j++) {
-                const uint64_t idx = b + threadIdx.x + (uint64_t)j * BS_NT;
-                kb[j] = idx < n ? S[start + idx] : Key(0);
-              }
-            }
-#pragma unroll
-            for (int j = 0; j < HB; j++) {
-              const uint64_t idx = b + threadIdx.x + (uint64_t)j * BS_NT;
-              if (idx < n && (int)key_digit<Key>(kb[j], rem - s, s) == pass &&
-                  !(one_batch ? ht.key(ksl[j]) == kb[j] : ht.verify(kb[j])))
-                over = 2;
-            }
-          }
-        }
+        if (clash) L.over = 2;
         __syncthreads();
       }
-      if (over) {
-        // too many distinct keys: retry with one more split bit; a
-        // fingerprint collision (over == 2) goes to the host split
-        failed = true;
-        if (over == 2) s = max_s;
-        __syncthreads();
-        break;
-      }
+      fail = L.over;
+      __syncthreads();
+      if (fail) break;
       // order the distinct keys: counting sort by the sub-digit below the
       // pass bits, then rank inside each sub-bin (1-2 keys on average)
       const int r2 = rem - s;
@@ -2032,7 +2129,7 @@ __global__ __launch_bounds__(BS_NT, HashCfg<Key>::BLOCKS) void k_bucket_hash(con
 #pragma unroll
       for (int j = 0; j < PER; j++) {
         const int slot = threadIdx.x * PER + j;
-        rc[j] = lds.hc[slot];
+        rc[j] = L.lds.hc[slot];
         rk[j] = rc[j] ? ht.key(slot) : Key(0);
         ri[j] = rc[j] ? atomicAdd(&hs[key_digit<Key>(rk[j], dpos, dbits)], 1u) : 0u;
       }
@@ -2058,8 +2155,8 @@ __global__ __launch_bounds__(BS_NT, HashCfg<Key>::BLOCKS) void k_bucket_hash(con
         }
       }
       __syncthreads();
-      Key* ok = lds.out_keys();
-      uint32_t* oc = lds.hc;
+      Key* ok = L.lds.out_keys();
+      uint32_t* oc = L.lds.hc;
 #pragma unroll
       for (int j = 0; j < PER; j++) {
         if (rc[j]) {
@@ -2070,11 +2167,12 @@ __global__ __launch_bounds__(BS_NT, HashCfg<Key>::BLOCKS) void k_bucket_hash(con
       }
       __syncthreads();
       const uint32_t nd = (uint32_t)ndk;
+      Key* Ro = R + start + out;
+      int32_t* Co = C + start + out;
       for (uint32_t i = threadIdx.x; i < nd; i += BS_NT) {
         const Key v = ok[i];
         const int d = (int)key_digit<Key>(v, dpos, dbits);
-        // the sub-bin's slots: from its start to the next one's (no end
-        // array, so that six tables fit a CU's LDS)
+        // the sub-bin's slots: from its start to the next one's
         const int a = (int)hs[d];
         const int e = d + 1 < nbins ? (int)hs[d + 1] : (int)nd;
         // the sub-bin's first four slots read at once (most hold one or two
@@ -2085,22 +2183,84 @@ __global__ __launch_bounds__(BS_NT, HashCfg<Key>::BLOCKS) void k_bucket_hash(con
         int rank = (int)(w0 < v) + (int)(a + 1 < e && w1 < v) + (int)(a + 2 < e && w2 < v) +
                    (int)(a + 3 < e && w3 < v);
         for (int j = a + 4; j < e; j++) rank += ok[j] < v;
-        R[start + out + a + rank] = v;
-        C[start + out + a + rank] = (int32_t)oc[i];
+        Ro[a + rank] = v;
+        Co[a + rank] = (int32_t)oc[i];
       }
       out += nd;
       __syncthreads();
     }
-    if (!failed) done = true;
+    // too many distinct keys: once more with one more split bit; splitting
+    // does not help a fingerprint collision
+    if (fail != 1) break;
+  }
+  *out_n = out;
+  return fail;
+}
+
+// One block per bucket of `in`: tu[b] = the bucket's distinct keys, bstart[b]
+// = where they are.  Buckets the table is too small for go to the retry list
+// (a single pass needs fewer registers).
+template <class Key, bool RUNS>
+__global__ __launch_bounds__(BS_NT, HashCfg<Key>::WAVES) void k_bucket_hash(const Key* S, Key* R, int32_t* C,
+                                                                            Runs in, int K, int fixed, long long* tu,
+                                                                            ull* bstart, ull* retry_count,
+                                                                            ull* retry_list) {
+  __shared__ HashShared<Key> L;
+  const ull task = blockIdx.x;
+  const RunBucket rb = uniform(run_bucket(in, task));
+  ull out = 0;
+  int fail = 0;
+  if (rb.n) {
+    fail = 1;
+    // (runs are reached by 32-bit offsets from the parent's first tile)
+    if (!RUNS || in.boff[(task >> in.db) + 1] - rb.base < (1ull << 32))
+      fail = count_task<Key, RUNS, false>(L, S, R, C, in, rb, (bool)((task >> (fixed - 1)) & 1), K, fixed, &out);
   }
   if (threadIdx.x == 0) {
-    if (done) {
-      tu[task] = (long long)out;
-    } else {
-      tu[task] = -1;
-      ovf_list[atomicAdd(ovf_count, 1ull)] = task;
+    bstart[task] = rb.v0;
+    tu[task] = (long long)out;
+    if (fail) retry_list[atomicAdd(retry_count, 1ull)] = task;
+  }
+}
+
+// The buckets of the retry list in several passes; what still fails goes to
+// ovf_list with tu = -1 for the host-driven split.
+template <class Key, bool RUNS>
+__global__ __launch_bounds__(BS_NT) void k_bucket_retry(const Key* S, Key* R, int32_t* C, Runs in, int K, int fixed,
+                                                        long long* tu, const ull* retry_count, const ull* retry_list,
+                                                        ull* ovf_count, ull* ovf_list) {
+  __shared__ HashShared<Key> L;
+  const ull nt = *retry_count;
+  for (ull q = blockIdx.x; q < nt; q += gridDim.x) {
+    const ull task = uniform(retry_list[q]);
+    const RunBucket rb = uniform(run_bucket(in, task));
+    ull out = 0;
+    int fail = 1;
+    if (!RUNS || in.boff[(task >> in.db) + 1] - rb.base < (1ull << 32))
+      fail = count_task<Key, RUNS, true>(L, S, R, C, in, rb, (bool)((task >> (fixed - 1)) & 1), K, fixed, &out);
+    if (threadIdx.x == 0) {
+      tu[task] = fail ? -1 : (long long)out;
+      if (fail) ovf_list[atomicAdd(ovf_count, 1ull)] = task;
     }
   }
+}
+
+// Tasks of the split path: [tstart[i], tstart[i] + tcount[i]) of S.
+template <class Key>
+__global__ __launch_bounds__(BS_NT) void k_task_hash(const Key* S, Key* R, int32_t* C, const ull* tstart,
+                                                     const ull* tcount, int K, int fixed, long long* tu) {
+  __shared__ HashShared<Key> L;
+  const ull task = blockIdx.x;
+  RunBucket rb{};
+  rb.v0 = tstart[task];
+  rb.n = tcount[task];
+  ull out = 0;
+  int fail = 0;
+  if (rb.n) {
+    const bool top = (bool)((uint32_t)(S[rb.v0] >> (2 * K - 1)) & 1u);
+    fail = count_task<Key, false, true>(L, S, R, C, Runs{}, rb, top, K, fixed, &out);
+  }
+  if (threadIdx.x == 0) tu[task] = fail ? -1 : (long long)out;
 }
 
 // All keys of the task are identical (no bits left to split on).
@@ -2177,6 +2337,18 @@ __global__ void k_copy_tasks(Key* S, const Key* T, const ull* tstart, const ull*
   const uint64_t s = tstart[t], n = tcount[t];
   const uint64_t off = blk_off[blockIdx.x];
   for (uint64_t i = off + threadIdx.x; i < n && i < off + PT_PER; i += blockDim.x) S[s + i] = T[s + i];
+}
+
+// The runs of the listed buckets gathered at their virtual places (one block
+// per bucket; oversize buckets only).
+template <class Key>
+__global__ void k_gather_buckets(const Key* S, Runs in, const ull* buckets, Key* out) {
+  const RunBucket rb = run_bucket(in, buckets[blockIdx.x]);
+  for (ull t = 0; t < rb.nt; t++) {
+    const ull e = rb.e0 + t, v = in.V[e], c = in.V[e + 1] - v;
+    const Key* src = S + rb.base + t * (ull)in.tk + (in.M[e] >> 16);
+    for (ull i = threadIdx.x; i < c; i += blockDim.x) out[v + i] = src[i];
+  }
 }
 
 // Dense table from per-leaf results (leaves in key order).
@@ -2895,7 +3067,7 @@ enum BufId {
   B_FASTA, B_BLK, B_BLKOFF, B_NL, B_RSTART, B_RLEN, B_KC, B_KOFS, B_SMALL, B_BCNT, B_BOFF, B_BCUR,
   B_S, B_C, B_TU, B_UOFF, B_TK, B_TC, B_HIST, B_KBS, B_KBOFF, B_KK, B_KC2, B_MNQ, B_MNPLAN,
   B_MNNT, B_MNNG, B_MNNOFF, B_MNFLAG, B_NODES, B_TMP, B_OVF, B_PT0, B_PT1, B_PT2, B_PT3, B_PT4,
-  B_PT5, B_PT6, B_BLKGT, B_S2, B_BCNT2, B_BOFF2, B_BCUR2, B_TP, B_HIST1, B_OFF1, B_HIST2, B_OFF2, B_CUTBH, B_LFREQ, B_WORDER, B_WIRE, B_NORM, B_NORMNL, B_NORMLEN, B_NORMOFF, B_NORMLS, B_NORMLL, B_SEGH, B_SEGO, B_SEGT, B_SCAN0, B_SCAN1 = B_SCAN0 + 8, B_COUNT = B_SCAN0 + 16
+  B_PT5, B_PT6, B_BLKGT, B_S2, B_BCNT2, B_BOFF2, B_BCUR2, B_TP, B_TP2, B_HIST1, B_OFF1, B_HIST2, B_OFF2, B_PACK, B_RETRY, B_CUTBH, B_LFREQ, B_WORDER, B_WIRE, B_NORM, B_NORMNL, B_NORMLEN, B_NORMOFF, B_NORMLS, B_NORMLL, B_SCAN0, B_SCAN1 = B_SCAN0 + 8, B_COUNT = B_SCAN0 + 16
 };
 
 }  // namespace
@@ -2908,9 +3080,10 @@ struct pk_ctx {
   uint64_t held = 0;
   std::string err;
   DevBuf buf[B_COUNT];
-  // 0-19: stage boundaries; 20 + 4 L ..: further partition level L (hist
-  // start/end, scatter start/end) for the first MS_TIMED_LEVELS levels
-  hipEvent_t ev[20 + 4 * 4] = {};
+  // 0-19: stage boundaries; 20 + 2 L, 21 + 2 L: around k_split of further
+  // partition level L for the first MS_TIMED_LEVELS levels
+  hipEvent_t ev[20 + 2 * MS_TIMED_LEVELS] = {};
+  bool have_hist = false;  // the last count ran k_l1_hist
   int ms_levels = 0;  // further partition levels of the last count
   int ms_form[MS_TIMED_LEVELS] = {};  // their scatter forms (timed levels)
   pk_timing timing{};
@@ -2938,6 +3111,11 @@ struct pk_ctx {
   char* arena = nullptr;
   uint64_t arena_cap = 0, arena_used = 0;
   bool arena_fixed[B_COUNT] = {};
+  // the packed input sits at the top end of the arena until level 1 has read
+  // it; arena_lim is where the other buffers must end meanwhile
+  uint64_t arena_lim = 0;
+  bool out_short = false;  // the caller's output arrays were too small
+  bool no_pack = false;  // the packed input does not fit: level 1 walks the bytes
   uint8_t win_lut[256] = {};  // byte -> code of the last pk_builder_count_windows
   // buffers from the device's stream-ordered pool (pk_ctx_set_alloc_mode)
   bool stream_alloc = false;
@@ -2974,12 +3152,14 @@ int need(pk_ctx* c, int id, uint64_t count, T** out) {
     if (c->arena_fixed[id]) {
       // a caller's output array: it must hold count entries (an empty
       // table asks for one entry and writes none)
-      if (count * sizeof(T) > b.cap && !(count == 1 && c->U == 0))
+      if (count * sizeof(T) > b.cap && !(count == 1 && c->U == 0)) {
+        c->out_short = true;
         return c->fail(PK_ENOMEM, "output arrays hold fewer entries than the table (" + std::to_string(count) +
                                       " needed)");
+      }
     } else if (b.cap < bytes) {
       const uint64_t take = (bytes + 255) & ~255ull;
-      if (c->arena_used + take > c->arena_cap)
+      if (c->arena_used + take > c->arena_lim)
         return c->fail(PK_ENOMEM, "input needs more than the " + std::to_string(c->arena_cap >> 20) +
                                       " MiB scratch of pk_count_noalloc");
       b.p = c->arena + c->arena_used;
@@ -3074,10 +3254,11 @@ struct Leaf {
   long long u;
 };
 
-// Recursively split oversize tasks; returns the leaves (in key order) for
+// Recursively split oversize tasks (contiguous ranges of S; T is scratch of
+// S's size); returns the leaves (in key order) for
 // each input task.
 template <class Key>
-int resolve_overflow(pk_ctx* c, Key* S, Key* R, int32_t* C, int K, int fixed_bits,
+int resolve_overflow(pk_ctx* c, Key* S, Key* T, Key* R, int32_t* C, int K, int fixed_bits,
                      const std::vector<ull>& starts, const std::vector<ull>& counts,
                      std::vector<std::vector<Leaf>>& leaves) {
   constexpr int CAP = HashCfg<Key>::LIMIT;
@@ -3119,13 +3300,11 @@ int resolve_overflow(pk_ctx* c, Key* S, Key* R, int32_t* C, int K, int fixed_bit
   const uint64_t nt = starts.size(), nblk = bt.size();
   ull *ts, *tc, *bo_d, *th;
   uint32_t* bt_d;
-  Key* T;
   PK_TRY(need(c, B_PT0, nt, &ts));
   PK_TRY(need(c, B_PT1, nt, &tc));
   PK_TRY(need(c, B_PT3, nblk, &bt_d));
   PK_TRY(need(c, B_PT4, nblk, &bo_d));
   PK_TRY(need(c, B_PT5, nt * 256, &th));
-  PK_TRY(need(c, B_TMP, c->N, &T));
   PK_HIP(c, hipMemcpyAsync(ts, starts.data(), nt * 8, hipMemcpyHostToDevice, c->stream));
   PK_HIP(c, hipMemcpyAsync(tc, counts.data(), nt * 8, hipMemcpyHostToDevice, c->stream));
   PK_HIP(c, hipMemcpyAsync(bt_d, bt.data(), nblk * 4, hipMemcpyHostToDevice, c->stream));
@@ -3161,18 +3340,15 @@ int resolve_overflow(pk_ctx* c, Key* S, Key* R, int32_t* C, int K, int fixed_bit
   // sort the sub-tasks that fit
   const int fixed2 = fixed_bits + pbits;
   const uint64_t ns = sub_start.size();
-  ull *ss, *sc, *ovc, *ovl;
+  ull *ss, *sc;
   long long* su;
   PK_TRY(need(c, B_PT6, ns * 3 + 2, &ss));
   sc = ss + ns;
   su = reinterpret_cast<long long*>(ss + 2 * ns);
-  PK_TRY(need(c, B_OVF, ns + 1, &ovl));
-  PK_TRY(need(c, B_PT2, 1, &ovc));
   PK_HIP(c, hipMemcpyAsync(ss, sub_start.data(), ns * 8, hipMemcpyHostToDevice, c->stream));
   PK_HIP(c, hipMemcpyAsync(sc, sub_count.data(), ns * 8, hipMemcpyHostToDevice, c->stream));
-  PK_TRY(fill_u64(c, ovc, 0, 1));
-  hipLaunchKernelGGL(HIP_KERNEL_NAME(k_bucket_hash<Key>), dim3((unsigned)ns), dim3(BS_NT), 0,
-                     c->stream, S, R, C, ss, sc, ns, K, fixed2, su, ovc, ovl);
+  hipLaunchKernelGGL(HIP_KERNEL_NAME(k_task_hash<Key>), dim3((unsigned)ns), dim3(BS_NT), 0, c->stream, S, R, C, ss,
+                     sc, K, fixed2, su);
   PK_HIP(c, hipGetLastError());
   std::vector<long long> hu(ns);
   PK_TRY(d2h(c, hu.data(), su, ns * 8));
@@ -3187,7 +3363,7 @@ int resolve_overflow(pk_ctx* c, Key* S, Key* R, int32_t* C, int K, int fixed_bit
   std::vector<std::vector<Leaf>> sub_leaves(ns);
   if (!o_start.empty()) {
     std::vector<std::vector<Leaf>> rec;
-    PK_TRY(resolve_overflow<Key>(c, S, R, C, K, fixed2, o_start, o_count, rec));
+    PK_TRY(resolve_overflow<Key>(c, S, T, R, C, K, fixed2, o_start, o_count, rec));
     for (size_t j = 0; j < o_idx.size(); j++) sub_leaves[o_idx[j]] = rec[j];
   }
   for (size_t i = 0; i < ns; i++) {
@@ -3201,8 +3377,15 @@ int resolve_overflow(pk_ctx* c, Key* S, Key* R, int32_t* C, int K, int fixed_bit
 // Index of the event bytes ('\n', or '\n' and '>') of fa: *m events at
 // *ev_out; *p0_out = the position of the first '>' (n when there is none).
 // small[0] is scratch for the pass that looks for it in every block.
+// With pk the input is packed on the way (encoding enc).
+struct Packed {
+  uint32_t* E = nullptr;
+  uint32_t* RX = nullptr;
+};
+
 int event_index(pk_ctx* c, const uint8_t* fa, uint64_t n, uint8_t e0, uint8_t e1, ull* small,
-                ull** ev_out, uint64_t* m_out, uint64_t* p0_out, int ev_buf = B_NL, int follow = 0) {
+                ull** ev_out, uint64_t* m_out, uint64_t* p0_out, int ev_buf = B_NL, int follow = 0,
+                const Packed* pk = nullptr, int enc = ENC_MAIN) {
   hipStream_t st = c->stream;
   const uint64_t nb = (n + NL_PER_BLOCK - 1) / NL_PER_BLOCK;
   ull *blk, *blkoff, *nl, *blkgt;
@@ -3210,7 +3393,14 @@ int event_index(pk_ctx* c, const uint8_t* fa, uint64_t n, uint8_t e0, uint8_t e1
   PK_TRY(need(c, B_BLKGT, nb + 1, &blkgt));
   PK_TRY(need(c, B_BLKOFF, nb + 1, &blkoff));
   if (nb) {
-    hipLaunchKernelGGL(k_nl_count, dim3((unsigned)nb), dim3(NL_NT), 0, st, fa, n, e0, e1, blk, blkgt, 0);
+    if (pk && enc == ENC_MAIN)
+      hipLaunchKernelGGL(HIP_KERNEL_NAME(k_pack<ENC_MAIN>), dim3((unsigned)nb), dim3(NL_NT), 0, st, fa, n, e0, e1,
+                         blk, blkgt, 0, pk->E, pk->RX);
+    else if (pk)
+      hipLaunchKernelGGL(HIP_KERNEL_NAME(k_pack<ENC_BUILDER>), dim3((unsigned)nb), dim3(NL_NT), 0, st, fa, n, e0, e1,
+                         blk, blkgt, 0, pk->E, pk->RX);
+    else
+      hipLaunchKernelGGL(k_nl_count, dim3((unsigned)nb), dim3(NL_NT), 0, st, fa, n, e0, e1, blk, blkgt, 0);
     PK_HIP(c, hipGetLastError());
   }
   PK_TRY(scan_excl<ull>(c, blk, blkoff, nb));
@@ -3232,7 +3422,10 @@ int event_index(pk_ctx* c, const uint8_t* fa, uint64_t n, uint8_t e0, uint8_t e1
   const uint64_t m = hm[0];
   PK_TRY(need(c, ev_buf, m + 1, &nl));
   if (nb) {
-    hipLaunchKernelGGL(k_nl_write, dim3((unsigned)nb), dim3(NL_NT), 0, st, fa, n, e0, e1, blkoff, nl, follow);
+    if (pk)
+      hipLaunchKernelGGL(k_nl_write_rx, dim3((unsigned)nb), dim3(NL_NT), 0, st, pk->RX, n, blkoff, nl, follow);
+    else
+      hipLaunchKernelGGL(k_nl_write, dim3((unsigned)nb), dim3(NL_NT), 0, st, fa, n, e0, e1, blkoff, nl, follow);
     PK_HIP(c, hipGetLastError());
   }
   *ev_out = nl;
@@ -3304,26 +3497,58 @@ int normalize_impl(pk_ctx* c, const uint8_t* in, uint64_t n, int fmt, const uint
   return PK_OK;
 }
 
+// Where the packed input goes (pk stays empty when the scratch of
+// pk_count_noalloc has no room for it).
+int pack_buffers(pk_ctx* c, uint64_t n, Packed* pk) {
+  const uint64_t words = (n + 15) / 16;
+  const uint64_t ew = (PK_PAD + words + 67) & ~63ull, bytes = 4 * (ew + words + 64);
+  uint32_t* p;
+  if (c->arena_mode) {
+    const uint64_t take = (bytes + 255) & ~255ull;
+    if (c->no_pack || c->arena_used + take > c->arena_cap) {
+      c->no_pack = true;
+      return PK_OK;
+    }
+    c->arena_lim = c->arena_cap - take;
+    p = reinterpret_cast<uint32_t*>(c->arena + c->arena_lim);
+  } else {
+    PK_TRY(need(c, B_PACK, bytes / 4, &p));
+  }
+  pk->E = p;
+  pk->RX = p + ew;
+  return PK_OK;
+}
+
+// The read table of a count: start byte, length (rlen: only where a walk needs
+// it), offsets of the reads' windows, and the packed input.
+struct Records {
+  ull* rstart = nullptr;
+  uint32_t* rlen = nullptr;
+  ull* kofs = nullptr;
+  uint64_t R = 0, N = 0;
+  Packed pk;
+};
+
 // Read table of the main path: records of the reference's Sliding_window.
-int records_main(pk_ctx* c, const uint8_t* fa, uint64_t n, int K, ull** rs, uint32_t** rl,
-                 uint64_t* R_out, uint64_t* N_out) {
+int records_main(pk_ctx* c, const uint8_t* fa, uint64_t n, int K, Records* rec, bool want_len) {
   hipStream_t st = c->stream;
   ull* small;
   PK_TRY(need(c, B_SMALL, 16, &small));
   // small[0] = first '>', [1] = first unprocessed, [2] = first format error,
-  // [3] = first over-long read, [4] = overflow count
+  // [3] = first over-long read, [4], [5] = overflow and retry counts
   PK_TRY(fill_u64(c, small, ~0ull, 4));
-  PK_TRY(fill_u64(c, small + 4, 0, 1));
+  PK_TRY(fill_u64(c, small + 4, 0, 2));
   if (n >> NL_FLAG_SHIFT) return c->fail(PK_EINVAL, "input larger than 2^62 bytes");
   ull* nl;
   uint64_t m, p0;
   // entries carry what follows each '\n' (bits 62-63): only k_reads reads them
-  PK_TRY(event_index(c, fa, n, '\n', '\n', small, &nl, &m, &p0, B_NL, 1));
+  if (!want_len) PK_TRY(pack_buffers(c, n, &rec->pk));
+  PK_TRY(event_index(c, fa, n, '\n', '\n', small, &nl, &m, &p0, B_NL, 1, rec->pk.E ? &rec->pk : nullptr));
   const uint64_t ncand = m / 2 + 2;
   ull *rstart, *kofs;
-  uint32_t *rlen, *kc;
+  uint32_t *rlen = nullptr, *kc;
   PK_TRY(need(c, B_RSTART, ncand, &rstart));
-  PK_TRY(need(c, B_RLEN, ncand, &rlen));
+  if (!rec->pk.E) PK_TRY(need(c, B_RLEN, ncand, &rlen));
   PK_TRY(need(c, B_KC, ncand, &kc));
   PK_TRY(need(c, B_KOFS, ncand + 1, &kofs));
   hipLaunchKernelGGL(k_reads, dim3(grid_for(ncand, 256)), dim3(256), 0, st, n, nl, m, p0, K,
@@ -3339,24 +3564,26 @@ int records_main(pk_ctx* c, const uint8_t* fa, uint64_t n, int K, ull** rs, uint
     return c->fail(PK_EFORMAT, "input is not strict single-line FASTA (record " +
                                    std::to_string(hs[1]) + " does not start with '>')");
   if (hs[2] != ~0ull && hs[2] < R) return c->fail(PK_EINVAL, "read longer than 4 GiB");
-  *rs = rstart;
-  *rl = rlen;
-  *R_out = R;
-  *N_out = hs[3];
+  rec->rstart = rstart;
+  rec->rlen = rlen;
+  rec->kofs = kofs;
+  rec->R = R;
+  rec->N = hs[3];
   return PK_OK;
 }
 
 // Read table of the builder API (bld_record).
 int records_builder(pk_ctx* c, const uint8_t* fa, uint64_t n, int klen, uint64_t read_len, BldSyms sy,
-                    ull** rs, uint32_t** rl, uint64_t* R_out, uint64_t* N_out) {
+                    Records* rec) {
   hipStream_t st = c->stream;
   ull* small;
   PK_TRY(need(c, B_SMALL, 16, &small));
   PK_TRY(fill_u64(c, small, ~0ull, 4));
-  PK_TRY(fill_u64(c, small + 4, 0, 1));
+  PK_TRY(fill_u64(c, small + 4, 0, 2));
   ull* ev;
   uint64_t m, p0;
-  PK_TRY(event_index(c, fa, n, sy.delim, sy.skip, small, &ev, &m, &p0));
+  PK_TRY(pack_buffers(c, n, &rec->pk));
+  PK_TRY(event_index(c, fa, n, sy.delim, sy.skip, small, &ev, &m, &p0, B_NL, 0, &rec->pk, ENC_BUILDER));
   ull *rstart, *kofs, *idx;
   uint32_t *rlen, *kc, *flag;
   PK_TRY(need(c, B_RSTART, m + 1, &rstart));
@@ -3381,109 +3608,122 @@ int records_builder(pk_ctx* c, const uint8_t* fa, uint64_t n, int klen, uint64_t
   PK_TRY(scan_excl<uint32_t>(c, kc, kofs, R));
   ull N = 0;
   PK_TRY(d2h(c, &N, kofs + R, 8));
-  *rs = rstart;
-  *rl = rlen;
-  *R_out = R;
-  *N_out = N;
+  rec->rstart = rstart;
+  rec->rlen = rlen;
+  rec->kofs = kofs;
+  rec->R = R;
+  rec->N = N;
   return PK_OK;
 }
 
-// Further partition levels from memory, the per-bucket count and the dense
-// table.  S holds the N keys (KB key bits) split into B buckets by their top
-// `fixed` bits, at offsets boff (the B_BOFF buffer); levels of <= MS_MAX_BITS
-// follow until btot bits are fixed.  S2 is the other instance array, C the
-// per-instance counts; small[4] (the overflow count) starts at zero.  set0 =
-// 1 when boff is in B_BOFF2.
+// Input of a partition level or of the bucket count: B buckets that share
+// their top `fixed` key bits, found through `in`.
+struct Part {
+  Runs in;
+  uint64_t B;
+  int fixed;
+  int set;  // which of the two sets of run-table buffers `in` sits in
+};
+
+// Buffers of a level's tiles and run table, in set 0 or 1 (a level reads the
+// other set): tiles is an upper bound on the level's tile count.
+struct LevelBufs {
+  ull *boff, *tp, *V;
+  uint32_t* M;
+};
+
+int level_buffers(pk_ctx* c, int set, uint64_t B, uint64_t tiles, int db, LevelBufs* l) {
+  PK_TRY(need(c, set ? B_BOFF2 : B_BOFF, B + 1, &l->boff));
+  PK_TRY(need(c, set ? B_TP2 : B_TP, B + 1, &l->tp));
+  PK_TRY(need(c, set ? B_HIST2 : B_HIST1, tiles << db, &l->M));
+  PK_TRY(need(c, set ? B_OFF2 : B_OFF1, (tiles << db) + 1, &l->V));
+  return PK_OK;
+}
+
+// The scan of a level's run table (slots past the level's last tile hold
+// anything: they come after every offset that is read).
+int level_runs(pk_ctx* c, const LevelBufs& l, uint64_t tiles, int db, int tk, Runs* out) {
+  PK_TRY(scan_excl<RunCount>(c, reinterpret_cast<const RunCount*>(l.M), l.V, tiles << db));
+  *out = Runs{l.M, l.V, l.tp, l.boff, db, tk};
+  return PK_OK;
+}
+
+// Bits of the next level when `left` remain: as few levels as possible, the
+// bits spread evenly.  A level reads and writes every key once, so one level
+// less beats longer runs until a run is down to about a line: 9 bits leave 32
+// one-word (16 two-word) keys per run of a full tile.
+constexpr int SP_LEVEL_BITS = 9;
+
+int level_bits(int left) {
+  const int nlev = (left + SP_LEVEL_BITS - 1) / SP_LEVEL_BITS;
+  return (left + nlev - 1) / nlev;
+}
+
+// Further partition levels, the per-bucket count and the dense table.  S
+// holds the N keys (KB key bits) as p says; levels follow until btot bits are
+// fixed.  S2 is the other instance array, C the per-instance counts;
+// small[4] and small[5] (the overflow and retry counts) start at zero.
 template <class Key>
-int count_partitioned(pk_ctx* c, Key* S, Key* S2, int32_t* C, ull* boff, uint64_t B, int fixed, int btot,
-                      int KB, uint64_t N, int set0 = 0) {
+int count_partitioned(pk_ctx* c, Key* S, Key* S2, int32_t* C, Part p, int btot, int KB, uint64_t N) {
   Key* TK;
   int32_t* TC;
   hipStream_t st = c->stream;
-  const pk_tuning& tun = c->tuning;
   ull* small;
   PK_TRY(need(c, B_SMALL, 16, &small));
-  // set: which offset / histogram buffers the input level used (boff sits
-  // in B_BOFF when 0, B_BOFF2 when 1)
-  int set = set0;
   Key* Sin = S;
   Key* Sout = S2;
-  constexpr int TQ = MS_NT * TileCfg<Key>::Q;
-  while (fixed < btot) {
-    // the remaining bits over as few levels of <= MS_MAX_BITS as possible,
-    // evenly
-    const int left = btot - fixed;
-    const int nlev = (left + MS_MAX_BITS - 1) / MS_MAX_BITS;
-    const int db = (left + nlev - 1) / nlev;
-    const uint64_t B2 = B << db;
-    const uint64_t tiles = N / TQ + B + 1;  // upper bound on tp[B]
-    ull *boff2, *tp, *O2;
-    uint32_t* H2;
-    const int o = set ? 0 : 1;  // the other offset array
-    PK_TRY(need(c, o ? B_BOFF2 : B_BOFF, B2 + 1, &boff2));
-    PK_TRY(need(c, B_TP, B + 1, &tp));
-    // alternate histogram buffers per level: the previous level's kernels
-    // may still be reading theirs
-    PK_TRY(need(c, o ? B_HIST2 : B_HIST1, tiles << db, &H2));
-    PK_TRY(need(c, o ? B_OFF2 : B_OFF1, (tiles << db) + 1, &O2));
+  const int tk = SplitCfg<Key>::TK_MAX;
+  while (p.fixed < btot) {
+    const int db = level_bits(btot - p.fixed);
+    const uint64_t tiles = N / tk + p.B + 1;  // upper bound
+    const int set = p.set ^ 1;
+    LevelBufs l;
+    PK_TRY(level_buffers(c, set, p.B, tiles, db, &l));
+    hipLaunchKernelGGL(k_tiles, dim3(1), dim3(1024), 0, st, p.in, (ull)p.B, tk, (ull)N, l.boff, l.tp);
+    PK_HIP(c, hipGetLastError());
     const int lv = c->ms_levels < MS_TIMED_LEVELS ? c->ms_levels : -1;
-    hipLaunchKernelGGL(k_tile_prefix, dim3(1), dim3(1024), 0, st, boff, (int)B, TQ, tp);
+    if (lv >= 0) PK_HIP(c, hipEventRecord(c->ev[20 + 2 * lv], st));
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_split<Key, SPLIT_RUNS>), dim3((unsigned)tiles), dim3(SP_NT), 0, st, Sin,
+                       WinSrc{}, p.in, (int)p.B, tk, ~Key(0), KB - p.fixed - db, db, l.boff, l.tp, l.M, Sout);
     PK_HIP(c, hipGetLastError());
-    if (lv >= 0) PK_HIP(c, hipEventRecord(c->ev[20 + 4 * lv], st));
-    // grid and scan over the upper bound of the level's tiles: blocks past
-    // tp[B] return at once, and the scan of their (unused) histogram slots
-    // only extends past every offset that is read
-    const ull ntiles = tiles;
-    const int dpos = KB - fixed - db;
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_ms_hist<Key>), dim3((unsigned)ntiles), dim3(MS_NT), 0, st, Sin,
-                       boff, tp, (int)B, dpos, db, H2);
-    PK_HIP(c, hipGetLastError());
-    if (lv >= 0) PK_HIP(c, hipEventRecord(c->ev[21 + 4 * lv], st));
-    PK_TRY(scan_excl<uint32_t>(c, H2, O2, ntiles << db));
-    hipLaunchKernelGGL(k_ms_boff, dim3(grid_for(B2 + 1, 256)), dim3(256), 0, st, O2, tp, (int)B, db,
-                       (ull)N, boff2);
-    PK_HIP(c, hipGetLastError());
-    // a long level runs on persistent blocks, two per CU (a tile buffer
-    // takes about 68 KB of LDS), once each gets >= 256 tiles: measured faster
-    // at ~1400 tiles per block (k = 64, 2.9e9 instances), slower at ~60
-    // (k = 32, 2.5e8 instances) than one block per tile
-    const ull pgrid = 2ull * (ull)c->ncu;
-    const bool persistent = tun.ms_scatter ? tun.ms_scatter == 1 : ntiles >= 256 * pgrid;
-    if (lv >= 0) PK_HIP(c, hipEventRecord(c->ev[22 + 4 * lv], st));
-    c->timing.ms_scatter_form = persistent ? 1 : 2;
-    if (lv >= 0) c->ms_form[lv] = persistent ? 1 : 2;
-    if (persistent)
-      hipLaunchKernelGGL(HIP_KERNEL_NAME(k_ms_scatter_p<Key, MS_P_NT>), dim3((unsigned)pgrid), dim3(MS_P_NT), 0, st,
-                         Sin, boff, tp, (int)B, dpos, db, O2, Sout);
-    else
-      hipLaunchKernelGGL(HIP_KERNEL_NAME(k_ms_scatter<Key>), dim3((unsigned)ntiles), dim3(MS_NT), 0, st,
-                         Sin, boff, tp, (int)B, dpos, db, O2, Sout);
-    PK_HIP(c, hipGetLastError());
-    if (lv >= 0) PK_HIP(c, hipEventRecord(c->ev[23 + 4 * lv], st));
+    if (lv >= 0) PK_HIP(c, hipEventRecord(c->ev[21 + 2 * lv], st));
+    if (lv >= 0) c->ms_form[lv] = PK_MS_TILES;
+    c->timing.ms_scatter_form = PK_MS_TILES;
     c->ms_levels++;
+    PK_TRY(level_runs(c, l, tiles, db, tk, &p.in));
+    p.B <<= db;
+    p.fixed += db;
+    p.set = set;
     std::swap(Sin, Sout);
-    boff = boff2;
-    B = B2;
-    fixed += db;
-    set = o;
   }
   S = Sin;
   Key* Res = Sout;  // the other array receives the (key, count) results
-  // bucket sizes of the last level
-  ull* bcnt;
-  PK_TRY(need(c, B_BCNT, B, &bcnt));
-  hipLaunchKernelGGL(k_diff, dim3(grid_for(B, 256)), dim3(256), 0, st, boff, B, bcnt);
-  PK_HIP(c, hipGetLastError());
+  const uint64_t B = p.B;
+  const Runs in = p.in;
   PK_HIP(c, hipEventRecord(c->ev[5], st));
   // 4. per-bucket count
   long long* tu;
-  ull *ovl, *uoff;
+  ull *ovl, *uoff, *bstart, *retry;
+  PK_TRY(need(c, B_BCNT, B, &bstart));
   PK_TRY(need(c, B_TU, B, &tu));
+  PK_TRY(need(c, B_RETRY, B, &retry));
   PK_TRY(need(c, B_OVF, B + 1, &ovl));
   PK_TRY(need(c, B_UOFF, B + 1, &uoff));
   PK_HIP(c, hipEventRecord(c->ev[6], st));
-  hipLaunchKernelGGL(HIP_KERNEL_NAME(k_bucket_hash<Key>), dim3((unsigned)B), dim3(BS_NT), 0, st, S,
-                     Res, C, boff, bcnt, B, KB / 2, btot, tu, small + 4, ovl);
+  const unsigned rgrid = (unsigned)std::min<uint64_t>(B, 4ull * (uint64_t)c->ncu);
+  if (in.M) {
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_bucket_hash<Key, true>), dim3((unsigned)B), dim3(BS_NT), 0, st, S, Res, C,
+                       in, KB / 2, btot, tu, bstart, small + 5, retry);
+    PK_HIP(c, hipGetLastError());
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_bucket_retry<Key, true>), dim3(rgrid), dim3(BS_NT), 0, st, S, Res, C, in,
+                       KB / 2, btot, tu, small + 5, retry, small + 4, ovl);
+  } else {
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_bucket_hash<Key, false>), dim3((unsigned)B), dim3(BS_NT), 0, st, S, Res, C,
+                       in, KB / 2, btot, tu, bstart, small + 5, retry);
+    PK_HIP(c, hipGetLastError());
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_bucket_retry<Key, false>), dim3(rgrid), dim3(BS_NT), 0, st, S, Res, C, in,
+                       KB / 2, btot, tu, small + 5, retry, small + 4, ovl);
+  }
   PK_HIP(c, hipGetLastError());
   PK_HIP(c, hipEventRecord(c->ev[7], st));
   // the scan of the distinct counts goes ahead of the overflow check: with
@@ -3496,26 +3736,42 @@ int count_partitioned(pk_ctx* c, Key* S, Key* S2, int32_t* C, ull* boff, uint64_
   const ull novf = hv[0];
   c->timing.n_split = (int32_t)novf;
   PK_HIP(c, hipEventRecord(c->ev[8], st));
-  const ull* lstart = boff;
+  const ull* lstart = bstart;
   const long long* lu = tu;
   uint64_t nleaves = B;
   if (novf) {
     // leaves = buckets, with each oversize bucket replaced by its split
-    std::vector<ull> hbo(B + 1), hbc(B);
+    std::vector<ull> hbo(B + 1);
     std::vector<long long> htu(B);
-    PK_TRY(d2h(c, hbo.data(), boff, (B + 1) * 8));
-    PK_TRY(d2h(c, hbc.data(), bcnt, B * 8));
+    PK_TRY(d2h(c, hbo.data(), bstart, B * 8));
+    hbo[B] = N;
     PK_TRY(d2h(c, htu.data(), tu, B * 8));
     std::vector<ull> os, oc;
     std::vector<size_t> ob;
     for (uint64_t b = 0; b < B; b++)
       if (htu[b] < 0) {
         os.push_back(hbo[b]);
-        oc.push_back(hbc[b]);
+        oc.push_back(hbo[b + 1] - hbo[b]);
         ob.push_back(b);
       }
+    // the split works in place on contiguous keys: gather the runs of the
+    // oversize buckets at their virtual places in a second array, and use
+    // the first as the split's scratch
+    Key* tmp;
+    PK_TRY(need(c, B_TMP, N, &tmp));
+    if (in.M) {
+      std::vector<ull> oi(ob.begin(), ob.end());
+      ull* od;
+      PK_TRY(need(c, B_PT0, oi.size(), &od));
+      PK_HIP(c, hipMemcpyAsync(od, oi.data(), oi.size() * 8, hipMemcpyHostToDevice, st));
+      hipLaunchKernelGGL(HIP_KERNEL_NAME(k_gather_buckets<Key>), dim3((unsigned)oi.size()), dim3(256), 0, st, S, in,
+                         od, tmp);
+      PK_HIP(c, hipGetLastError());
+      PK_HIP(c, hipStreamSynchronize(st));  // od's buffer is used again below
+      std::swap(S, tmp);
+    }
     std::vector<std::vector<Leaf>> rec;
-    PK_TRY(resolve_overflow<Key>(c, S, Res, C, KB / 2, btot, os, oc, rec));
+    PK_TRY(resolve_overflow<Key>(c, S, tmp, Res, C, KB / 2, btot, os, oc, rec));
     std::vector<ull> ls;
     std::vector<long long> lus;
     size_t j = 0;
@@ -3564,17 +3820,10 @@ int count_partitioned(pk_ctx* c, Key* S, Key* S2, int32_t* C, ull* boff, uint64_
   return PK_OK;
 }
 
-// Count the k-mers of the read table (rstart, rlen)[0..R) (records in file
-// order), N instances.
-// K = window length, KB = key bits (2K on the main path, the whole word for
-// the builder encoding), mask = word mask of the rolling update.
-template <class Key, int ENC, bool OWN = false>
-int count_records(pk_ctx* c, const uint8_t* fa, uint64_t n, const ull* rstart, const uint32_t* rlen,
-                  uint64_t R, uint64_t N, int K, int KB, Key mask, OwnCfg cf = OwnCfg{nullptr, 1, 0, 0}) {
-  constexpr int CAP = HashCfg<Key>::LIMIT;
-  hipStream_t st = c->stream;
-  ull* small;
-  PK_TRY(need(c, B_SMALL, 16, &small));
+// What every count notes about its input; N == 0 ends it with an empty table
+// (*empty).
+template <class Key>
+int begin_count(pk_ctx* c, uint64_t R, uint64_t N, int K, bool* empty) {
   c->R = R;
   c->N = N;
   c->k = K;
@@ -3582,36 +3831,90 @@ int count_records(pk_ctx* c, const uint8_t* fa, uint64_t n, const ull* rstart, c
   c->timing.n_instances = N;
   c->timing.n_reads = R;
   c->ms_levels = 0;
-  PK_HIP(c, hipEventRecord(c->ev[1], st));
-  Key *S, *TK;
-  int32_t *C, *TC;
+  c->have_hist = false;
+  *empty = N == 0;
   if (N == 0) {
+    Key* TK;
+    int32_t* TC;
     c->U = 0;
     PK_TRY(need(c, B_TK, 1, &TK));
     PK_TRY(need(c, B_TC, 1, &TC));
     c->have_table = true;
-    return PK_OK;
   }
-  // 3. partition: level 1 fused with the parse, further levels from memory,
-  // at most 8 bits per level, until a bucket holds ~1.5 hash tables' worth
-  // of instances.  Write bases come from scanned digit-major histograms.
-  // with owner routing, about N / P instances are this rank's
+  return PK_OK;
+}
+
+// Count the windows of the read table's reads (in file order) from the packed
+// input.  K = window length, KB = key bits (2K on the main path, the whole
+// word for the builder encoding), mask = the key's bits.
+template <class Key, int ENC>
+int count_records(pk_ctx* c, const Records& rec, int K, int KB, Key mask) {
+  constexpr int CAP = HashCfg<Key>::LIMIT;
+  hipStream_t st = c->stream;
+  const uint64_t N = rec.N;
+  PK_HIP(c, hipEventRecord(c->ev[1], st));
+  bool empty;
+  PK_TRY(begin_count<Key>(c, rec.R, N, K, &empty));
+  if (empty) return PK_OK;
   const pk_tuning& tun = c->tuning;
   const float bf = tun.bucket_factor > 0.f ? tun.bucket_factor : 3.0f;
-  const int btot = choose_bits(OWN ? (N + cf.P - 1) / cf.P : N, KB / 2, CAP, bf);
+  const int btot = choose_bits(N, KB / 2, CAP, bf);
+  c->timing.bucket_bits = btot;
+  // level 1: tiles of N / 512 windows (so that a small input spreads over the
+  // CUs and a bucket has at most RUN_CAP runs), within 4096 and a full tile;
+  // one level of up to 10 bits while its buckets keep to those runs
+  const uint64_t per = (N + RUN_CAP - 1) / RUN_CAP;
+  const int tk = (int)std::min<uint64_t>(SplitCfg<Key>::TK_MAX,
+                                         std::max<uint64_t>(4096, (per + SP_NT - 1) / SP_NT * SP_NT));
   int d1;
-  if (tun.l1_bits > 0 && tun.l1_bits <= L1_MAX_BITS) {
-    d1 = btot < tun.l1_bits ? btot : tun.l1_bits;
-  } else if (btot > L1_DEFAULT_BITS + MS_MAX_BITS) {
-    // three or more levels anyway: the narrowest level-1 digit (>= 5 bits)
-    // that adds no level, since every level-1 digit keeps a partly written
-    // line open per block (k = 64, 2.9e9 instances, 2^21 buckets: level-1
-    // scatter 33.8 ms at 8 bits, 13.8 ms at 5)
-    const int further = (btot - L1_DEFAULT_BITS + MS_MAX_BITS - 1) / MS_MAX_BITS;
-    d1 = std::max(5, btot - further * MS_MAX_BITS);
-  } else {
-    d1 = btot < L1_DEFAULT_BITS ? btot : L1_DEFAULT_BITS;
-  }
+  if (tun.l1_bits > 0 && tun.l1_bits <= L1_MAX_BITS) d1 = std::min(btot, tun.l1_bits);
+  else if (btot <= SP_MAX_BITS && N <= (uint64_t)RUN_CAP * SplitCfg<Key>::TK_MAX) d1 = btot;
+  else d1 = level_bits(btot);
+  const uint64_t tiles = (N + tk - 1) / tk;
+  Key *S, *S2;
+  int32_t* C;
+  PK_TRY(need(c, B_S, N, &S));
+  LevelBufs l;
+  PK_TRY(level_buffers(c, 0, 1, tiles, d1, &l));
+  hipLaunchKernelGGL(k_tiles_one, dim3(1), dim3(1), 0, st, (ull)tiles, (ull)N, l.boff, l.tp);
+  PK_HIP(c, hipGetLastError());
+  PK_HIP(c, hipEventRecord(c->ev[4], st));
+  constexpr int SRC = ENC == ENC_MAIN ? SPLIT_MAIN : SPLIT_BUILDER;
+  hipLaunchKernelGGL(HIP_KERNEL_NAME(k_split<Key, SRC>), dim3((unsigned)tiles), dim3(SP_NT), 0, st,
+                     (const Key*)nullptr, WinSrc{rec.pk.E, rec.pk.RX, rec.kofs, rec.rstart, rec.R, K}, Runs{}, 1, tk,
+                     mask, KB - d1, d1, l.boff, l.tp, l.M, S);
+  PK_HIP(c, hipGetLastError());
+  PK_HIP(c, hipEventRecord(c->ev[16], st));
+  // the packed input has been read: its scratch is free for what follows
+  // in stream order
+  c->arena_lim = c->arena_cap;
+  PK_TRY(need(c, B_S2, N, &S2));
+  PK_TRY(need(c, B_C, N, &C));
+  Part p{Runs{}, 1ull << d1, d1, 0};
+  PK_TRY(level_runs(c, l, tiles, d1, tk, &p.in));
+  return count_partitioned<Key>(c, S, S2, C, p, btot, KB, N);
+}
+
+// One rank's share: level 1 walks every read in order with the owner rule and
+// scatters the owned keys into contiguous buckets.
+template <class Key>
+int count_share(pk_ctx* c, const uint8_t* fa, uint64_t n, const Records& rec, int K, OwnCfg cf) {
+  constexpr int CAP = HashCfg<Key>::LIMIT;
+  hipStream_t st = c->stream;
+  const uint64_t R = rec.R;
+  uint64_t N = rec.N;
+  const int KB = 2 * K;
+  const Key mask = key_mask<Key>(KB);
+  PK_HIP(c, hipEventRecord(c->ev[1], st));
+  bool empty;
+  PK_TRY(begin_count<Key>(c, R, N, K, &empty));
+  if (empty) return PK_OK;
+  const pk_tuning& tun = c->tuning;
+  const float bf = tun.bucket_factor > 0.f ? tun.bucket_factor : 3.0f;
+  // with owner routing, about N / P instances are this rank's
+  const int btot = choose_bits((N + cf.P - 1) / cf.P, K, CAP, bf);
+  c->timing.bucket_bits = btot;
+  const int d1 = std::min(btot, tun.l1_bits > 0 && tun.l1_bits <= L1_MAX_BITS ? tun.l1_bits : L1_DEFAULT_BITS);
   const uint64_t B1 = 1ull << d1;
   // reads per block: up to 8 chunks of L1_NT, fewer for small inputs so that
   // the grid still spreads over the CUs
@@ -3620,105 +3923,44 @@ int count_records(pk_ctx* c, const uint8_t* fa, uint64_t n, const ull* rstart, c
                                : (int)std::min<uint64_t>(8, std::max<uint64_t>(1, R / (L1_NT * 1024ull))));
   const uint64_t nblk = (R + rpb - 1) / rpb;
   // LDS staging: room for one record per thread of the input's mean size,
-  // + 25 %, for each of the two level-1 kernels
-  auto staging = [&](int nt, int cap) {
-    const double want = (double)nt * ((double)n / (double)R) * 1.25;
-    const int b = (int)std::min<double>(cap, std::max<double>(L1_SB_MIN, want));
-    return (b + 1023) & ~1023;
-  };
-  const int sb = staging(L1_NT, L1_SB_MAX);
-  constexpr int snt = L1Scatter<Key, ENC, OWN>::NT;
-  const int sbs = staging(snt, L1Scatter<Key, ENC, OWN>::SB_MAX);
+  // + 25 %
+  const double want = (double)L1_NT * ((double)n / (double)R) * 1.25;
+  const int sb = ((int)std::min<double>(L1_SB_MAX, std::max<double>(L1_SB_MIN, want)) + 1023) & ~1023;
   ull *boff, *O;
   uint32_t* H;
-  Key* S2;
+  Key *S, *S2;
+  int32_t* C;
   PK_TRY(need(c, B_BOFF, B1 + 1, &boff));
   PK_TRY(need(c, B_HIST1, B1 * nblk, &H));
   PK_TRY(need(c, B_OFF1, B1 * nblk + 1, &O));
   PK_TRY(need(c, B_S, N, &S));
   PK_TRY(need(c, B_S2, N, &S2));
   PK_TRY(need(c, B_C, N, &C));
-  c->timing.bucket_bits = btot;
-  // fold the second level's histogram into this one when two or more levels
-  // follow level 1 and its (bucket, digit) counters fit 32 KB of LDS
-  constexpr int sgf = L1Scatter<Key, ENC, OWN>::GF;
-  L2Fold f2{0, sgf, 0, nullptr};
-  {
-    const int left = btot - d1;
-    const int nlev = (left + MS_MAX_BITS - 1) / MS_MAX_BITS;
-    const int db = nlev > 0 ? (left + nlev - 1) / nlev : 0;
-    if (L1Scatter<Key, ENC, OWN>::main && nlev >= 2 && (B1 << db) <= L2_FOLD_MAX && tun.ms_fold != 2) {
-      f2.d2 = db;
-      // segments of about four level-2 tiles on average (whole scatter
-      // blocks): a segment's last tile is a partial one
-      constexpr uint64_t TQ2 = (uint64_t)MS_NT * TileCfg<Key>::Q;
-      const uint64_t want = (nblk * B1 * 4 * TQ2 + N - 1) / N;
-      const uint64_t g = std::max<uint64_t>(1, (want + sgf - 1) / sgf);
-      f2.spb = (int)std::min<uint64_t>(g * sgf, (nblk + sgf - 1) / sgf * sgf);
-      f2.nsb = (nblk + f2.spb - 1) / f2.spb;
-      const uint64_t nh2 = (B1 << db) * f2.nsb;
-      PK_TRY(need(c, B_SEGH, nh2 + 2, &f2.H2));
-      PK_TRY(fill_u64(c, reinterpret_cast<ull*>(f2.H2), 0, (nh2 + 1) / 2));
-    }
-  }
+  c->have_hist = true;
   PK_HIP(c, hipEventRecord(c->ev[2], st));
-  hipLaunchKernelGGL(HIP_KERNEL_NAME(k_l1_hist<Key, ENC, OWN>), dim3((unsigned)nblk), dim3(L1_NT),
-                     l1_lds_bytes(sb, (int)B1, 4) + (f2.d2 ? ((uint32_t)B1 << f2.d2) * 4u : 0u), st, fa, n, rstart,
-                     rlen, R, K, KB, mask, d1, rpb, sb, cf, H, f2);
+  hipLaunchKernelGGL(HIP_KERNEL_NAME(k_l1_hist<Key, ENC_MAIN, true>), dim3((unsigned)nblk), dim3(L1_NT),
+                     l1_lds_bytes(sb, (int)B1, 4), st, fa, n, rec.rstart, rec.rlen, R, K, KB, mask, d1, rpb, sb, cf, H);
   PK_HIP(c, hipGetLastError());
   PK_HIP(c, hipEventRecord(c->ev[3], st));
   PK_TRY(scan_excl<uint32_t>(c, H, O, B1 * nblk));
-  if (OWN) {
-    // this rank's instances
-    ull no = 0;
-    PK_TRY(d2h(c, &no, O + B1 * nblk, 8));
-    N = no;
-    c->N = N;
-    c->timing.n_instances = N;
-    if (N == 0) {
-      c->U = 0;
-      PK_TRY(need(c, B_TK, 1, &TK));
-      PK_TRY(need(c, B_TC, 1, &TC));
-      c->have_table = true;
-      return PK_OK;
-    }
-  }
+  // this rank's instances
+  ull no = 0;
+  PK_TRY(d2h(c, &no, O + B1 * nblk, 8));
+  N = no;
+  PK_TRY(begin_count<Key>(c, R, N, K, &empty));
+  c->have_hist = true;
+  if (empty) return PK_OK;
   hipLaunchKernelGGL(k_l1_boff, dim3(grid_for(B1 + 1, 256)), dim3(256), 0, st, O, (int)B1, nblk, (ull)N,
                      boff);
   PK_HIP(c, hipGetLastError());
   PK_HIP(c, hipEventRecord(c->ev[4], st));
-  hipLaunchKernelGGL(HIP_KERNEL_NAME(k_l1_scatter<Key, ENC, OWN>), dim3((unsigned)((nblk + sgf - 1) / sgf)),
-                     dim3(snt), l1_lds_bytes(sbs, (int)B1, 12), st, fa, n, rstart, rlen, R, K, KB, mask, d1, rpb,
-                     sbs, cf, O, nblk, S);
+  hipLaunchKernelGGL(HIP_KERNEL_NAME(k_l1_scatter<Key, ENC_MAIN, true>), dim3((unsigned)nblk), dim3(L1_NT),
+                     l1_lds_bytes(sb, (int)B1, 8), st, fa, n, rec.rstart, rec.rlen, R, K, KB, mask, d1, rpb, sb, cf, O,
+                     nblk, S);
   PK_HIP(c, hipGetLastError());
   PK_HIP(c, hipEventRecord(c->ev[16], st));
-  if (!f2.d2) return count_partitioned<Key>(c, S, S2, C, boff, B1, d1, btot, KB, N);
-  // level 2 from the folded counts: scan them in (bucket, digit, segment)
-  // order, then the segment scatter
-  const int db = f2.d2;
-  const uint64_t B2 = B1 << db, nh2 = B2 * f2.nsb;
-  ull *O2, *O2T, *boff2;
-  PK_TRY(need(c, B_SEGO, nh2 + 1, &O2));
-  PK_TRY(need(c, B_SEGT, nh2, &O2T));
-  PK_TRY(need(c, B_BOFF2, B2 + 1, &boff2));
-  PK_HIP(c, hipEventRecord(c->ev[20], st));
-  PK_TRY(scan_excl<uint32_t>(c, f2.H2, O2, nh2));
-  hipLaunchKernelGGL(k_seg_transpose, dim3((unsigned)((f2.nsb + 31) / 32), (unsigned)(((1u << db) + 31) / 32), (unsigned)B1),
-                     dim3(256), 0, st, O2, f2.nsb, db, O2T);
-  PK_HIP(c, hipGetLastError());
-  hipLaunchKernelGGL(k_seg_boff, dim3(grid_for(B2 + 1, 256)), dim3(256), 0, st, O2T, f2.nsb, db, (ull)B2, (ull)N,
-                     boff2);
-  PK_HIP(c, hipGetLastError());
-  PK_HIP(c, hipEventRecord(c->ev[21], st));
-  PK_HIP(c, hipEventRecord(c->ev[22], st));
-  hipLaunchKernelGGL(HIP_KERNEL_NAME(k_ms_scatter_seg<Key, MS_P_NT>), dim3(2u * (unsigned)c->ncu), dim3(MS_P_NT), 0, st,
-                     S, O, nblk, f2.spb, f2.nsb, (int)B1, (ull)N, KB - d1 - db, db, O2T, S2);
-  PK_HIP(c, hipGetLastError());
-  PK_HIP(c, hipEventRecord(c->ev[23], st));
-  c->timing.ms_scatter_form = 3;
-  c->ms_form[0] = 3;
-  c->ms_levels = 1;
-  return count_partitioned<Key>(c, S2, S, C, boff2, B2, d1 + db, btot, KB, N, 1);
+  return count_partitioned<Key>(c, S, S2, C, Part{Runs{nullptr, nullptr, nullptr, boff, 0, 0}, B1, d1, 0}, btot, KB,
+                                N);
 }
 
 // Distinct klen-byte windows of the implicit builder counters: keys from
@@ -3727,24 +3969,11 @@ template <class Key>
 int windows_count_impl(pk_ctx* c, const uint8_t* fa, const ull* rstart, const uint32_t* rlen, const ull* woff,
                        uint64_t R, uint64_t N, int klen, int bits, const uint8_t* lut, int has_nul, int KB) {
   hipStream_t st = c->stream;
-  c->R = R;
-  c->N = N;
-  c->k = klen;
-  c->words = sizeof(Key) / 8;
   c->key_bits = -1;  // byte-rank codes: no macro nodes on this table
-  c->timing.n_instances = N;
-  c->timing.n_reads = R;
-  c->ms_levels = 0;
   PK_HIP(c, hipEventRecord(c->ev[1], st));
-  if (N == 0) {
-    Key* TK;
-    int32_t* TC;
-    c->U = 0;
-    PK_TRY(need(c, B_TK, 1, &TK));
-    PK_TRY(need(c, B_TC, 1, &TC));
-    c->have_table = true;
-    return PK_OK;
-  }
+  bool empty;
+  PK_TRY(begin_count<Key>(c, R, N, klen, &empty));
+  if (empty) return PK_OK;
   Key *S, *S2;
   int32_t* C;
   ull *boff, *small;
@@ -3753,20 +3982,18 @@ int windows_count_impl(pk_ctx* c, const uint8_t* fa, const ull* rstart, const ui
   PK_TRY(need(c, B_C, N, &C));
   PK_TRY(need(c, B_BOFF, 2, &boff));
   PK_TRY(need(c, B_SMALL, 16, &small));
-  PK_TRY(fill_u64(c, small + 4, 0, 1));
+  PK_TRY(fill_u64(c, small + 4, 0, 2));
   PK_TRY(fill_u64(c, boff, 0, 1));
   PK_TRY(fill_u64(c, boff + 1, N, 1));
-  PK_HIP(c, hipEventRecord(c->ev[2], st));
   hipLaunchKernelGGL(HIP_KERNEL_NAME(k_win_keys<Key>), dim3(grid_for(R, 256)), dim3(256), 0, st, fa, rstart, rlen,
                      woff, R, klen, bits, lut, has_nul, S);
   PK_HIP(c, hipGetLastError());
-  PK_HIP(c, hipEventRecord(c->ev[3], st));
   PK_HIP(c, hipEventRecord(c->ev[4], st));
   PK_HIP(c, hipEventRecord(c->ev[16], st));
   const float bf = c->tuning.bucket_factor > 0.f ? c->tuning.bucket_factor : 3.0f;
   const int btot = choose_bits(N, KB / 2, HashCfg<Key>::LIMIT, bf);
   c->timing.bucket_bits = btot;
-  return count_partitioned<Key>(c, S, S2, C, boff, 1, 0, btot, KB, N);
+  return count_partitioned<Key>(c, S, S2, C, Part{Runs{nullptr, nullptr, nullptr, boff, 0, 0}, 1, 0, 0}, btot, KB, N);
 }
 
 template <class Key>
@@ -3776,26 +4003,26 @@ int count_impl(pk_ctx* c, const uint8_t* fa, uint64_t n, int K) {
   c->pend_count = c->pend_split = c->pend_cutoff = c->pend_mn = c->pend_norm = false;
   c->key_bits = 2 * K;
   PK_HIP(c, hipEventRecord(c->ev[0], c->stream));
-  ull* rstart;
-  uint32_t* rlen;
-  uint64_t R, N;
-  PK_TRY(records_main(c, fa, n, K, &rstart, &rlen, &R, &N));
-  return count_records<Key, ENC_MAIN>(c, fa, n, rstart, rlen, R, N, K, 2 * K, key_mask<Key>(2 * K));
+  Records rec;
+  PK_TRY(records_main(c, fa, n, K, &rec, false));
+  // without the packed input (pk_count_noalloc's scratch is short of it) the
+  // walk of a share that owns every k-mer takes its place
+  if (!rec.pk.E) return count_share<Key>(c, fa, n, rec, K, OwnCfg{nullptr, 1, 0, 1});
+  return count_records<Key, ENC_MAIN>(c, rec, K, 2 * K, key_mask<Key>(2 * K));
 }
 
 // L-mer frequencies of the whole input into freq (device, LMER_BINS u64),
 // with the record rule of Sliding_window_l (a record needs L bytes).
 int lmer_frequency_impl(pk_ctx* c, const uint8_t* fa, uint64_t n, ull** freq_out) {
-  ull* rs;
-  uint32_t* rl;
-  uint64_t R, N;
-  PK_TRY(records_main(c, fa, n, LMER_L, &rs, &rl, &R, &N));
+  Records rec;
+  PK_TRY(records_main(c, fa, n, LMER_L, &rec, true));
+  const uint64_t R = rec.R;
   ull* freq;
   PK_TRY(need(c, B_LFREQ, LMER_BINS, &freq));
   PK_TRY(fill_u64(c, freq, 0, LMER_BINS));
   if (R) {
     hipLaunchKernelGGL(k_lmer_freq, dim3((unsigned)std::min<uint64_t>(grid_for(R, 256), 4096)), dim3(256), 0,
-                       c->stream, fa, rs, rl, R, freq);
+                       c->stream, fa, rec.rstart, rec.rlen, R, freq);
     PK_HIP(c, hipGetLastError());
   }
   *freq_out = freq;
@@ -3813,12 +4040,9 @@ int rank_share_impl(pk_ctx* c, const uint8_t* fa, uint64_t n, int K, int P, int 
   PK_HIP(c, hipEventRecord(c->ev[0], c->stream));
   ull* freq;
   PK_TRY(lmer_frequency_impl(c, fa, n, &freq));
-  ull* rstart;
-  uint32_t* rlen;
-  uint64_t R, N;
-  PK_TRY(records_main(c, fa, n, K, &rstart, &rlen, &R, &N));
-  return count_records<Key, ENC_MAIN, true>(c, fa, n, rstart, rlen, R, N, K, 2 * K, key_mask<Key>(2 * K),
-                                            OwnCfg{freq, P, rank, 0});
+  Records rec;
+  PK_TRY(records_main(c, fa, n, K, &rec, true));
+  return count_share<Key>(c, fa, n, rec, K, OwnCfg{freq, P, rank, 0});
 }
 
 // One rank's share when every k-mer belongs to rank retrieve_proc_id(kmer)
@@ -3830,12 +4054,9 @@ int rank_share_key_impl(pk_ctx* c, const uint8_t* fa, uint64_t n, int K, int P, 
   c->pend_count = c->pend_split = c->pend_cutoff = c->pend_mn = c->pend_norm = false;
   c->key_bits = 2 * K;
   PK_HIP(c, hipEventRecord(c->ev[0], c->stream));
-  ull* rstart;
-  uint32_t* rlen;
-  uint64_t R, N;
-  PK_TRY(records_main(c, fa, n, K, &rstart, &rlen, &R, &N));
-  return count_records<Key, ENC_MAIN, true>(c, fa, n, rstart, rlen, R, N, K, 2 * K, key_mask<Key>(2 * K),
-                                            OwnCfg{nullptr, P, rank, 1});
+  Records rec;
+  PK_TRY(records_main(c, fa, n, K, &rec, true));
+  return count_share<Key>(c, fa, n, rec, K, OwnCfg{nullptr, P, rank, 1});
 }
 
 template <class Key>
@@ -3846,12 +4067,9 @@ int builder_count_impl(pk_ctx* c, const uint8_t* fa, uint64_t n, int klen, uint6
   c->pend_count = c->pend_split = c->pend_cutoff = c->pend_mn = c->pend_norm = false;
   c->key_bits = (int)sizeof(Key) * 8;
   PK_HIP(c, hipEventRecord(c->ev[0], c->stream));
-  ull* rstart;
-  uint32_t* rlen;
-  uint64_t R, N;
-  PK_TRY(records_builder(c, fa, n, klen, read_len, sy, &rstart, &rlen, &R, &N));
-  return count_records<Key, ENC_BUILDER>(c, fa, n, rstart, rlen, R, N, klen, (int)sizeof(Key) * 8,
-                                         ~Key(0));
+  Records rec;
+  PK_TRY(records_builder(c, fa, n, klen, read_len, sy, &rec));
+  return count_records<Key, ENC_BUILDER>(c, rec, klen, (int)sizeof(Key) * 8, ~Key(0));
 }
 
 __global__ void k_set_int(int* p, int v) { *p = v; }
@@ -4353,11 +4571,23 @@ int pk_count_noalloc(pk_ctx* c, const char* fasta_dev, uint64_t nbytes, int k, u
   c->arena_fixed[B_TK] = c->arena_fixed[B_TC] = true;
   c->arena = arena;
   c->arena_cap = NOALLOC_SCRATCH;
-  c->arena_used = 0;
   c->arena_mode = true;
-  c->U = 0;
   const uint8_t* fa = reinterpret_cast<const uint8_t*>(fasta_dev);
-  int rc = (k <= 32) ? count_impl<uint64_t>(c, fa, nbytes, k) : count_impl<u128>(c, fa, nbytes, k);
+  int rc = PK_OK;
+  for (int attempt = 0; attempt < 2; attempt++) {
+    c->arena_used = 0;
+    c->arena_lim = c->arena_cap;
+    c->no_pack = attempt == 1;
+    c->out_short = false;
+    c->U = 0;
+    rc = (k <= 32) ? count_impl<uint64_t>(c, fa, nbytes, k) : count_impl<u128>(c, fa, nbytes, k);
+    // the scratch ran out with the packed input in it: once more without
+    if (rc != PK_ENOMEM || c->no_pack || c->out_short) break;
+    for (int i = 0; i < B_COUNT; i++)
+      if (!c->arena_fixed[i]) c->buf[i] = DevBuf{};
+    if (hipStreamSynchronize(c->stream) != hipSuccess) break;
+  }
+  c->no_pack = false;
   c->arena_mode = false;
   for (int i = 0; i < B_COUNT; i++) {
     c->buf[i] = saved[i];
@@ -4761,7 +4991,7 @@ int pk_last_timing(const pk_ctx* cc, pk_timing* out) {
   }
   if (c->pend_count) {
     c->timing.parse_ms = el(0, 1);
-    c->timing.hist_ms = el(2, 3);
+    c->timing.hist_ms = c->have_hist ? el(2, 3) : 0.f;
     c->timing.scatter_ms = el(4, 5);
     c->timing.l1_scatter_ms = el(4, 16);
     c->timing.sort_ms = el(6, 7);
@@ -4771,10 +5001,9 @@ int pk_last_timing(const pk_ctx* cc, pk_timing* out) {
     c->timing.ms_hist_ms = c->timing.ms_scatter_ms = 0.f;
     for (int l = 0; l < MS_TIMED_LEVELS; l++) {
       const bool on = l < nl;
-      c->timing.ms_level_hist_ms[l] = on ? el(20 + 4 * l, 21 + 4 * l) : 0.f;
-      c->timing.ms_level_scatter_ms[l] = on ? el(22 + 4 * l, 23 + 4 * l) : 0.f;
+      c->timing.ms_level_hist_ms[l] = 0.f;  // no level has a histogram pass
+      c->timing.ms_level_scatter_ms[l] = on ? el(20 + 2 * l, 21 + 2 * l) : 0.f;
       c->timing.ms_level_form[l] = on ? c->ms_form[l] : 0;
-      c->timing.ms_hist_ms += c->timing.ms_level_hist_ms[l];
       c->timing.ms_scatter_ms += c->timing.ms_level_scatter_ms[l];
     }
     c->timing.ms_levels = c->ms_levels;
