@@ -4,13 +4,15 @@
 // Pipeline of pk_count (one HIP stream per context, everything resident in HBM):
 //   1. packing        k_pack reads the FASTA once: two bits per input byte
 //                     (plus one exact low bit), the '\n' bits, and their count
-//                     per block; k_nl_write_rx lists the '\n' positions.
-//   2. read table     k_reads: record r = header line j0+2r, sequence line
+//                     per block.
+//   2. windows        k_lines / k_valid: which bytes end a k-mer, from the '\n'
+//                     bits: record r = header line j0+2r, sequence line
 //                     j0+2r+1, with the record rules and the format check of
 //                     the reference's Sliding_window (src/kmer_counting.cpp:
-//                     2890-2945); k-mer offsets by exclusive scan.  The
-//                     builder API's records come from k_bld_flags/k_bld_write.
-//   3. partition      k_split: tiles of k-mers sorted by a digit of the key's
+//                     2890-2945).  Rank shares walk a read table instead
+//                     (k_reads); the builder API's records come from
+//                     k_bld_flags / k_bld_write.
+//   3. partition      k_split_main, k_split: tiles of k-mers sorted by a digit of the key's
 //                     top bits, one tile per block, each tile written back
 //                     as one contiguous piece with a table of where its
 //                     digits start.  Level 1 cuts the k-mers out of the packed
@@ -468,10 +470,10 @@ __device__ __forceinline__ uint32_t base_code(uint32_t c) {
 //       byte, which is no base, bit i says instead that a '>' follows it.
 //
 // One pass over the bytes at 16 per lane, half a byte written per byte; the
-// line index is then written from RX (a quarter of the input) and the first
-// partition level reads E and RX: 2.25 bytes of traffic per input byte, where
-// the byte-wise line index, its second pass, the level-1 histogram and the
-// level-1 scatter each read the input (4 bytes).
+// valid window ends then come from RX (a quarter of the input) and the first
+// partition level reads E, RX and those: 2.5 bytes of traffic per input byte,
+// where the byte-wise line index, its second pass, the level-1 histogram and
+// the level-1 scatter each read the input (4 bytes).
 
 constexpr int PK_PAD = 8;  // E words before the input's first (windows reach four words back)
 
@@ -538,10 +540,9 @@ __global__ __launch_bounds__(NL_NT) void k_pack(const uint8_t* fa, uint64_t n, u
   }
 }
 
-// Positions of the event bytes from RX (k_nl_write's output): block b covers
+// Positions of the event bytes from RX (k_nl_write's, without flags): block b covers
 // the same NL_PER_BLOCK bytes as k_pack's, a thread 64 consecutive ones.
-__global__ __launch_bounds__(NL_NT) void k_nl_write_rx(const uint32_t* RX, uint64_t n, const ull* blk_off, ull* nl,
-                                                       int follow) {
+__global__ __launch_bounds__(NL_NT) void k_nl_write_rx(const uint32_t* RX, uint64_t n, const ull* blk_off, ull* nl) {
   static_assert(NL_PER_BLOCK == (uint64_t)NL_NT * 64, "64 bytes per thread");
   const uint64_t nw = (n + 15) / 16;
   const uint64_t w0 = (uint64_t)blockIdx.x * (NL_PER_BLOCK / 16) + (uint64_t)threadIdx.x * 4;
@@ -566,10 +567,136 @@ __global__ __launch_bounds__(NL_NT) void k_nl_write_rx(const uint32_t* RX, uint6
     for (uint32_t m = w[i] >> 16; m; m &= m - 1) {
       const int b = __ffs(m) - 1;
       const uint64_t p = (w0 + i) * 16 + b;
-      const ull f = !follow ? 0ull : p + 1 >= n ? 2ull : (ull)((w[i] >> b) & 1u);
-      nl[o++] = p | (f << NL_FLAG_SHIFT);
+      nl[o++] = p;
     }
   }
+}
+
+// The main path's records without a list of lines.  With j0 = the '\n's
+// before the first '>' (p0), record r's sequence is the bytes that j0 + 2r + 1
+// '\n's come before, and it is taken when its header's '\n' (number j0 + 2r)
+// lies at least K + 1 bytes before the end of the input (k_reads' rules, from
+// counts instead of positions).  lines: [0] j0, [1] R = records taken, [2]
+// '\n's of the input, [3] p0 (n when there is none).  One block.
+__global__ __launch_bounds__(1024) void k_lines(const uint32_t* RX, uint64_t n, const ull* blk_off, uint64_t nb,
+                                                const ull* gt, int K, ull* lines) {
+  const ull p0 = *gt < n ? *gt : n;
+  const uint64_t nw = (n + 15) / 16;
+  const ull m = blk_off[nb];
+  // '\n's in [a, b) of one block's bytes or less
+  auto count = [&](uint64_t a, uint64_t b) -> ull {
+    ull c = 0;
+    for (uint64_t w = a / 16 + threadIdx.x; w < nw && w * 16 < b; w += 1024) {
+      uint32_t x = RX[w] >> 16;
+      if (w * 16 < a) x &= 0xFFFFu << (a - w * 16);
+      if (w * 16 + 16 > b) x &= (1u << (b - w * 16)) - 1u;
+      c += (ull)__popc(x & 0xFFFFu);
+    }
+    return block_sum<1024>(c);
+  };
+  const uint64_t pb = p0 / NL_PER_BLOCK;
+  const ull j0 = p0 < n ? blk_off[pb] + count(pb * NL_PER_BLOCK, p0) : m;
+  const ull tail = count(n > (uint64_t)K ? n - (uint64_t)K : 0, n);
+  if (threadIdx.x == 0) {
+    const ull c = m - tail;  // '\n's at least K + 1 bytes before the end
+    lines[0] = j0;
+    lines[1] = p0 < n && c > j0 ? (c - j0 + 1) / 2 : 0;
+    lines[2] = m;
+    lines[3] = p0;
+  }
+}
+
+// Valid window ends: bit i of W[w] says that the K bytes up to byte 64 w + i
+// are a k-mer's, i.e. that byte lies in the sequence of a record that is
+// taken and no '\n' is among them.  A thread covers 64 bytes, a block the
+// same bytes as k_pack's; cnt[block] = its valid ends.  first_err = the first
+// record r >= 1 that does not start with '>' (the reference's assert).  All from
+// the '\n' bits: a quarter byte read and an eighth written per input byte.
+__global__ __launch_bounds__(NL_NT) void k_valid(const uint32_t* RX, uint64_t n, const ull* blk_off,
+                                                 const ull* lines, int K, ull* W, uint32_t* cnt, ull* first_err) {
+  const uint64_t nw = (n + 15) / 16;
+  const uint64_t w0 = (uint64_t)blockIdx.x * (NL_PER_BLOCK / 16) + (uint64_t)threadIdx.x * 4;
+  const uint64_t base = w0 * 16;
+  const int lane = threadIdx.x & 63;
+  const ull j0 = lines[0], R = lines[1];
+  ull x = 0, g = 0;  // '\n's; at a '\n': a '>' follows
+  if (w0 + 4 <= nw) {
+    const uint4 q = *reinterpret_cast<const uint4*>(RX + w0);
+    x = (ull)(q.x >> 16) | (ull)(q.y >> 16) << 16 | (ull)(q.z >> 16) << 32 | (ull)(q.w >> 16) << 48;
+    g = (ull)(q.x & 0xFFFFu) | (ull)(q.y & 0xFFFFu) << 16 | (ull)(q.z & 0xFFFFu) << 32 | (ull)(q.w & 0xFFFFu) << 48;
+  } else {
+    for (int i = 0; i < 4 && w0 + i < nw; i++) {
+      x |= (ull)(RX[w0 + i] >> 16) << (16 * i);
+      g |= (ull)(RX[w0 + i] & 0xFFFFu) << (16 * i);
+    }
+  }
+  // the 64 bytes before: the previous lane's
+  ull px = __shfl_up(x, 1, 64);
+  if (lane == 0) {
+    px = 0;
+    if (w0 >= 4) {
+      const uint4 q = *reinterpret_cast<const uint4*>(RX + w0 - 4);
+      px = (ull)(q.x >> 16) | (ull)(q.y >> 16) << 16 | (ull)(q.z >> 16) << 32 | (ull)(q.w >> 16) << 48;
+    }
+  }
+  // a '\n' among the last K bytes, up to and with this one
+  u128 near = (u128)x << 64 | (u128)px;
+  for (int c = 1; c < K;) {
+    const int sh = c < K - c ? c : K - c;
+    near |= near << sh;
+    c += sh;
+  }
+  ull tot;
+  const ull cb = blk_off[blockIdx.x] + block_scan_total<NL_NT>((ull)__popcll(x), &tot);
+  // parity of the '\n's before each byte, relative to j0: odd in sequences
+  ull par = x;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) par ^= par << o;
+  ull seq = par ^ x;
+  if ((cb ^ j0) & 1) seq = ~seq;
+  ull ok = seq & ~(ull)(near >> 64);
+  const ull ce = cb + (ull)__popcll(x);
+  // bytes up to the (j0)-th '\n' are before the first sequence, bytes after
+  // the (j0 + 2R)-th belong to records not taken
+  auto nth = [&](ull k) {  // bit of the k-th '\n' of these bytes
+    ull t = x;
+    for (; k; k--) t &= t - 1;
+    return __ffsll((long long)t) - 1;
+  };
+  const ull last = j0 + 2 * R;
+  if (ce <= j0 || cb > last) {
+    ok = 0;
+  } else {
+    if (cb <= j0) {
+      const int b = nth(j0 - cb);
+      ok &= b == 63 ? 0ull : ~0ull << (b + 1);
+    }
+    if (ce > last) ok &= (1ull << nth(last - cb)) - 1;
+  }
+  if (base >= n) ok = 0;
+  else if (base + 64 > n) ok &= (1ull << (n - base)) - 1;
+  // sequence ends that no '>' follows
+  ull bad = x & seq & ~g;
+  if (base + 64 >= n && n > base) bad &= ~(1ull << (n - 1 - base));
+  for (; bad; bad &= bad - 1) {
+    const int b = __ffsll((long long)bad) - 1;
+    const ull c = cb + (ull)__popcll(x & ((1ull << b) - 1));
+    if (c > j0) {
+      atomicMin(first_err, (c - j0 + 1) / 2);
+      break;
+    }
+  }
+  W[w0 / 4] = ok;
+  const ull sum = block_sum<NL_NT>((ull)__popcll(ok));
+  if (threadIdx.x == 0) cnt[blockIdx.x] = (uint32_t)sum;
+}
+
+// Inputs beyond 4 GiB: flag set when some 2^32 - 16 bytes in a row may hold no
+// '\n' (whole blocks without one), i.e. when a read may be too long.
+__global__ void k_long_lines(const ull* blk_off, uint64_t nb, ull* flag) {
+  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  constexpr uint64_t span = 0xFFFFFFF0ull / NL_PER_BLOCK - 1;
+  if (i + span <= nb && blk_off[i + span] == blk_off[i]) *flag = 1;
 }
 
 // ---------------------------------------------------------------------------
@@ -877,17 +1004,17 @@ __global__ void k_reads(uint64_t n, const ull* nl, uint64_t m, uint64_t p0,
       rstart[r] = s;
       if (len > 0xFFFFFFF0ull) {
         atomicMin(too_long, (ull)r);
-        if (rlen) rlen[r] = 0;
+        rlen[r] = 0;
         kc[r] = 0;
       } else {
-        if (rlen) rlen[r] = (uint32_t)len;
+        rlen[r] = (uint32_t)len;
         kc[r] = len >= (uint64_t)K ? (uint32_t)(len - K + 1) : 0u;
       }
     }
   }
   if (!processed) {
     rstart[r] = 0;
-    if (rlen) rlen[r] = 0;
+    rlen[r] = 0;
     kc[r] = 0;
     atomicMin(first_unproc, (ull)r);
   }
@@ -1271,7 +1398,8 @@ struct SplitCfg {
 //   in the tile << 16 | count) and of V, the exclusive scan of the counts.  V
 //   gives every key a place in key order of the buckets, the "virtual" index
 //   that buckets and tiles are counted in; run e holds the indexes V[e] ..
-//   V[e + 1] at array positions boff[a] + t * tk + start.
+//   V[e + 1] at array positions boff[a] + t * tk + start (with tb, whose
+//   tiles vary in size: tb[t << ts] + start).
 struct Runs {
   const uint32_t* M;
   const ull* V;
@@ -1279,7 +1407,12 @@ struct Runs {
   const ull* boff;
   int db;
   int tk;
+  const ull* tb;  // level 1 of the main path: tile t starts at tb[t << ts]
+  int ts;
 };
+
+// Array position of tile t of a bucket, from the bucket's first (base).
+__device__ __forceinline__ ull tile_place(const Runs& in, ull t) { return in.tb ? in.tb[t << in.ts] : t * (ull)in.tk; }
 
 // count field of a run-table entry, for the scan
 struct RunCount {
@@ -1480,18 +1613,17 @@ __global__ void k_tiles_one(ull ntiles, ull total, ull* boff, ull* tp) {
   tp[1] = ntiles;
 }
 
-// Source of level 1: window i (of all reads' windows in order) belongs to
+// Source of the builder's level 1: window i (of all reads' windows in order) belongs to
 // the last read with kofs[r] <= i and starts at byte rstart[r] + i - kofs[r].
 struct WinSrc {
   const uint32_t* E;
-  const uint32_t* RX;
   const ull* kofs;    // R + 1 offsets
   const ull* rstart;
   ull R;
   int K;
 };
 
-enum { SPLIT_RUNS, SPLIT_MAIN, SPLIT_BUILDER };
+enum { SPLIT_RUNS, SPLIT_BUILDER };
 
 // Low 32-bit words of the window that ends at byte e, nw of them, low first.
 template <int NWORDS>
@@ -1518,7 +1650,7 @@ __device__ __forceinline__ Key window_key(const WinSrc& s, ull e) {
 
 template <class Key, int SRC>
 __global__ __launch_bounds__(SP_NT, 4) void k_split(const Key* __restrict__ Sin, WinSrc ws, Runs in, int nb, int tk,
-                                                    Key mask, int dpos, int db, const ull* __restrict__ boff,
+                                                    int dpos, int db, const ull* __restrict__ boff,
                                                     const ull* __restrict__ tp, uint32_t* __restrict__ M,
                                                     Key* __restrict__ Sout) {
   constexpr int Q = SplitCfg<Key>::Q;
@@ -1554,7 +1686,7 @@ __global__ __launch_bounds__(SP_NT, 4) void k_split(const Key* __restrict__ Sin,
       const ull f = rb.e0 + (rb.nt > SP_NT ? block_upper<SP_NT>(in.V + rb.e0, rb.nt, v0) - 1 : 0);
       constexpr int CAP = SP_TILE_BYTES / 8;
       ull* delta = reinterpret_cast<ull*>(buf);
-      auto src = [&](ull e) { return rb.base + (e - rb.e0) * (ull)in.tk + (in.M[e] >> 16); };
+      auto src = [&](ull e) { return rb.base + tile_place(in, e - rb.e0) + (in.M[e] >> 16); };
       const int np = map_pieces<SP_NT>(mw, nw, CAP, in.V, f, rb.e0 + rb.nt, v0, m, src,
                                        [&](uint32_t r, ull d, ull) { delta[r] = d; });
 #pragma unroll
@@ -1575,42 +1707,34 @@ __global__ __launch_bounds__(SP_NT, 4) void k_split(const Key* __restrict__ Sin,
   } else {
     // level 1: the reads of these windows
     const ull f = block_upper<SP_NT>(ws.kofs, ws.R, v0) - 1;
-    constexpr bool BLD = SRC == SPLIT_BUILDER;
-    constexpr int CAP = SP_TILE_BYTES / (BLD ? 12 : 8);
+    constexpr int CAP = SP_TILE_BYTES / 12;
     ull* delta = reinterpret_cast<ull*>(buf);
-    uint32_t* aux = reinterpret_cast<uint32_t*>(buf + 8 * CAP);  // builder: v0 - kofs (mod 2^32)
+    uint32_t* aux = reinterpret_cast<uint32_t*>(buf + 8 * CAP);  // v0 - kofs (mod 2^32)
     auto src = [&](ull r) { return ws.rstart[r]; };
     const int np = map_pieces<SP_NT>(mw, nw, CAP, ws.kofs, f, ws.R, v0, m, src, [&](uint32_t r, ull d, ull idx) {
       delta[r] = d;
-      if (BLD) aux[r] = (uint32_t)(v0 - ws.kofs[idx]);
+      aux[r] = (uint32_t)(v0 - ws.kofs[idx]);
     });
 #pragma unroll
     for (int j = 0; j < Q; j++) {
       const int i = tid + j * SP_NT;
       if (i < m) {
         ull p;
-        uint32_t wi = 0;  // builder: index of the window in its read
+        uint32_t wi;  // index of the window in its read
         if (np <= CAP) {
           const uint32_t r = map_piece(mt[j * (SP_NT / 32)], low);
           p = delta[r] + (ull)i;
-          if (BLD) wi = aux[r] + (uint32_t)i;
+          wi = aux[r] + (uint32_t)i;
         } else {
           const ull r = find_piece(ws.kofs, f, ws.R, v0 + i);
           p = ws.rstart[r] + (v0 + i - ws.kofs[r]);
-          if (BLD) wi = (uint32_t)(v0 + i - ws.kofs[r]);
+          wi = (uint32_t)(v0 + i - ws.kofs[r]);
         }
-        const ull e = p + (ull)(ws.K - 1);  // the window's last byte
-        Key k = window_key<Key>(ws, e);
-        if (BLD) {
-          // the word holds the last 4 * sizeof(kmer_t) bases since the
-          // read's start
-          const uint32_t bases = wi + (uint32_t)ws.K;
-          if (bases < 4u * (uint32_t)sizeof(Key)) k &= (Key(1) << (2 * bases)) - 1;
-        } else {
-          // the last base's low bit, without the next byte's spill
-          k = (k & ~Key(1)) | (Key)((ws.RX[e >> 4] >> (e & 15)) & 1u);
-          k &= mask;
-        }
+        Key k = window_key<Key>(ws, p + (ull)(ws.K - 1));
+        // the word holds the last 4 * sizeof(kmer_t) bases since the read's
+        // start
+        const uint32_t bases = wi + (uint32_t)ws.K;
+        if (bases < 4u * (uint32_t)sizeof(Key)) k &= (Key(1) << (2 * bases)) - 1;
         kr[j] = k;
       }
     }
@@ -1658,6 +1782,106 @@ __global__ __launch_bounds__(SP_NT, 4) void k_split(const Key* __restrict__ Sin,
     const int c = m - r0 < ROUND ? m - r0 : ROUND;
     Key* o = Sout + v0 + r0;
     for (int p = tid; p < c; p += SP_NT) o[p] = T[p];
+    __syncthreads();
+  }
+}
+
+// Level 1 of the main path: tile t is the bytes [t * 16384 * WPT, ...), its
+// keys the k-mers that end there (bits of W).  A thread holds WPT words of E
+// and the NW words before them in registers, so the k-mer that ends at each of
+// its 16 * WPT bytes is NW funnel shifts by constants: cutting a k-mer costs
+// about as much as copying it, so the keys are cut twice, once to rank them
+// by digit and once more to place them, and need no registers in between.
+// That allows 64 VGPRs, two 1024-thread blocks per CU.  Against tiles gathered
+// by window number (search of the read list, a map of its reads, three loads
+// per k-mer): see the figures at count_records.
+constexpr int SM_NT = 1024;
+
+template <class Key, int WPT>
+__global__ __launch_bounds__(SM_NT, 8) void k_split_main(const uint32_t* __restrict__ E,
+                                                         const uint32_t* __restrict__ RX,
+                                                         const uint16_t* __restrict__ W, const ull* __restrict__ tb,
+                                                         ull nblk, Key mask, int dpos, int db,
+                                                         uint32_t* __restrict__ M, Key* __restrict__ Sout) {
+  constexpr int NW = (int)sizeof(Key) / 4;
+  constexpr int P = 16 * WPT;
+  constexpr int ROUND = SP_TILE_BYTES / (int)sizeof(Key);
+  static_assert(NL_PER_BLOCK == 16ull * SM_NT, "a word of E per thread and index block");
+  static_assert(SM_NT == 1 << SP_MAX_BITS, "a digit per thread");
+  __shared__ Key T[ROUND];
+  __shared__ uint32_t h[1 << SP_MAX_BITS];
+  __shared__ uint32_t nw[SM_NT / 64 + 1];
+  const int tid = (int)threadIdx.x;
+  const ull t = blockIdx.x, nt = gridDim.x;
+  const ull v0 = uniform(tb[t * WPT]);
+  const ull t1 = (t + 1) * WPT < nblk ? (t + 1) * WPT : nblk;
+  const int m = (int)(uniform(tb[t1]) - v0);
+  const ull w = (t * SM_NT + (ull)tid) * WPT;
+  uint32_t val = 0;
+  if (w < nblk * SM_NT) val = W[w];
+  if (WPT == 2 && w + 1 < nblk * SM_NT) val |= (uint32_t)W[w + 1] << 16;
+  uint32_t ew[NW + WPT] = {}, rx = 0;
+  if (val) {
+#pragma unroll
+    for (int i = 0; i < NW + WPT; i++) ew[i] = E[PK_PAD + w - NW + i];
+    rx = RX[w] & 0xFFFFu;
+    if (WPT == 2) rx |= RX[w + 1] << 16;
+  }
+  // the k-mer that ends at byte j of the thread's words
+  auto key = [&](int j) {
+    const int c = NW + (j >> 4);
+    const uint32_t sh = 30u - 2u * (uint32_t)(j & 15);
+    Key k = 0;
+#pragma unroll
+    for (int i = NW - 1; i >= 0; i--) {
+      uint32_t o = __builtin_amdgcn_alignbit(ew[c - 1 - i], ew[c - i], sh);
+      // the last base's low bit, without the next byte's spill
+      if (i == 0) o = (o & ~1u) | ((rx >> j) & 1u);
+      k = (k << 31 << 1) | (Key)o;
+    }
+    return k & mask;
+  };
+  // makes the compiler cut the keys anew instead of keeping them in registers
+  auto forget = [&]() {
+#pragma unroll
+    for (int i = 0; i < NW + WPT; i++) asm volatile("" : "+v"(ew[i]));
+    asm volatile("" : "+v"(val), "+v"(rx));
+  };
+  const int ns = 1 << db;
+  if (tid < ns) h[tid] = 0;
+  __syncthreads();
+  uint32_t rk[P / 2] = {};
+#pragma unroll
+  for (int j = 0; j < P; j++)
+    if ((val >> j) & 1u) rk[j / 2] |= atomicAdd(&h[key_digit<Key>(key(j), dpos, db)], 1u) << (16 * (j & 1));
+  __syncthreads();
+  {
+    const uint32_t c = tid < ns ? h[tid] : 0u;
+    uint32_t tot;
+    const uint32_t ex = block_scan_u32<SM_NT>(c, nw, &tot);
+    if (tid < ns) {
+      h[tid] = ex;
+      M[(ull)tid * nt + t] = ex << 16 | c;
+    }
+  }
+  __syncthreads();
+  // place of every key in the sorted tile
+  forget();
+#pragma unroll
+  for (int j = 0; j < P; j++) {
+    if ((val >> j) & 1u) rk[j / 2] += h[key_digit<Key>(key(j), dpos, db)] << (16 * (j & 1));
+  }
+  for (int r0 = 0; r0 < m; r0 += ROUND) {
+    forget();
+#pragma unroll
+    for (int j = 0; j < P; j++) {
+      const uint32_t p = ((rk[j / 2] >> (16 * (j & 1))) & 0xFFFFu) - (uint32_t)r0;
+      if (((val >> j) & 1u) && p < (uint32_t)ROUND) T[p] = key(j);
+    }
+    __syncthreads();
+    const int c = m - r0 < ROUND ? m - r0 : ROUND;
+    Key* o = Sout + v0 + r0;
+    for (int p = tid; p < c; p += SM_NT) o[p] = T[p];
     __syncthreads();
   }
 }
@@ -1907,7 +2131,7 @@ __device__ __forceinline__ bool wave_map(uint2* mw, int nwords, uint32_t* off, c
     if (idx < nt) {
       vs = (uint32_t)(V[idx] - rb.v0);
       ve = (uint32_t)(V[idx + 1] - rb.v0);
-      so = idx * (uint32_t)in.tk + (M[idx] >> 16) - vs;
+      so = (uint32_t)tile_place(in, idx) + (M[idx] >> 16) - vs;
     }
     const bool part = ve > vs && vs < b + (uint32_t)m && ve > b;
     const ull bal = __ballot(part);
@@ -1973,7 +2197,7 @@ __device__ __forceinline__ int load_batch(HashShared<Key>& L, const Key* Sb, con
     } else {
       const ull end = rb.e0 + rb.nt, vb = rb.v0 + b;
       const ull f = rb.e0 + (rb.nt > BS_NT ? block_upper<BS_NT>(in.V + rb.e0, rb.nt, vb) - 1 : 0);
-      auto src = [&](ull e) { return (e - rb.e0) * (ull)in.tk + (in.M[e] >> 16); };
+      auto src = [&](ull e) { return tile_place(in, e - rb.e0) + (in.M[e] >> 16); };
       for (;;) {
         __syncthreads();  // hs may still be read
         const int np = map_pieces<BS_NT>(mw, L.nw, RUN_CAP, in.V, f, end, vb, m, src,
@@ -2346,7 +2570,7 @@ __global__ void k_gather_buckets(const Key* S, Runs in, const ull* buckets, Key*
   const RunBucket rb = run_bucket(in, buckets[blockIdx.x]);
   for (ull t = 0; t < rb.nt; t++) {
     const ull e = rb.e0 + t, v = in.V[e], c = in.V[e + 1] - v;
-    const Key* src = S + rb.base + t * (ull)in.tk + (in.M[e] >> 16);
+    const Key* src = S + rb.base + tile_place(in, t) + (in.M[e] >> 16);
     for (ull i = threadIdx.x; i < c; i += blockDim.x) out[v + i] = src[i];
   }
 }
@@ -3067,7 +3291,7 @@ enum BufId {
   B_FASTA, B_BLK, B_BLKOFF, B_NL, B_RSTART, B_RLEN, B_KC, B_KOFS, B_SMALL, B_BCNT, B_BOFF, B_BCUR,
   B_S, B_C, B_TU, B_UOFF, B_TK, B_TC, B_HIST, B_KBS, B_KBOFF, B_KK, B_KC2, B_MNQ, B_MNPLAN,
   B_MNNT, B_MNNG, B_MNNOFF, B_MNFLAG, B_NODES, B_TMP, B_OVF, B_PT0, B_PT1, B_PT2, B_PT3, B_PT4,
-  B_PT5, B_PT6, B_BLKGT, B_S2, B_BCNT2, B_BOFF2, B_BCUR2, B_TP, B_TP2, B_HIST1, B_OFF1, B_HIST2, B_OFF2, B_PACK, B_RETRY, B_CUTBH, B_LFREQ, B_WORDER, B_WIRE, B_NORM, B_NORMNL, B_NORMLEN, B_NORMOFF, B_NORMLS, B_NORMLL, B_SCAN0, B_SCAN1 = B_SCAN0 + 8, B_COUNT = B_SCAN0 + 16
+  B_PT5, B_PT6, B_BLKGT, B_S2, B_BCNT2, B_BOFF2, B_BCUR2, B_TP, B_TP2, B_HIST1, B_OFF1, B_HIST2, B_OFF2, B_PACK, B_RETRY, B_WCNT, B_WOFF, B_CUTBH, B_LFREQ, B_WORDER, B_WIRE, B_NORM, B_NORMNL, B_NORMLEN, B_NORMOFF, B_NORMLS, B_NORMLL, B_SCAN0, B_SCAN1 = B_SCAN0 + 8, B_COUNT = B_SCAN0 + 16
 };
 
 }  // namespace
@@ -3377,15 +3601,16 @@ int resolve_overflow(pk_ctx* c, Key* S, Key* T, Key* R, int32_t* C, int K, int f
 // Index of the event bytes ('\n', or '\n' and '>') of fa: *m events at
 // *ev_out; *p0_out = the position of the first '>' (n when there is none).
 // small[0] is scratch for the pass that looks for it in every block.
-// With pk the input is packed on the way (encoding enc).
+// With pk the input is packed on the way (builder encoding).
 struct Packed {
   uint32_t* E = nullptr;
   uint32_t* RX = nullptr;
+  ull* W = nullptr;  // main path: valid window ends
 };
 
 int event_index(pk_ctx* c, const uint8_t* fa, uint64_t n, uint8_t e0, uint8_t e1, ull* small,
                 ull** ev_out, uint64_t* m_out, uint64_t* p0_out, int ev_buf = B_NL, int follow = 0,
-                const Packed* pk = nullptr, int enc = ENC_MAIN) {
+                const Packed* pk = nullptr) {
   hipStream_t st = c->stream;
   const uint64_t nb = (n + NL_PER_BLOCK - 1) / NL_PER_BLOCK;
   ull *blk, *blkoff, *nl, *blkgt;
@@ -3393,10 +3618,7 @@ int event_index(pk_ctx* c, const uint8_t* fa, uint64_t n, uint8_t e0, uint8_t e1
   PK_TRY(need(c, B_BLKGT, nb + 1, &blkgt));
   PK_TRY(need(c, B_BLKOFF, nb + 1, &blkoff));
   if (nb) {
-    if (pk && enc == ENC_MAIN)
-      hipLaunchKernelGGL(HIP_KERNEL_NAME(k_pack<ENC_MAIN>), dim3((unsigned)nb), dim3(NL_NT), 0, st, fa, n, e0, e1,
-                         blk, blkgt, 0, pk->E, pk->RX);
-    else if (pk)
+    if (pk)
       hipLaunchKernelGGL(HIP_KERNEL_NAME(k_pack<ENC_BUILDER>), dim3((unsigned)nb), dim3(NL_NT), 0, st, fa, n, e0, e1,
                          blk, blkgt, 0, pk->E, pk->RX);
     else
@@ -3423,7 +3645,7 @@ int event_index(pk_ctx* c, const uint8_t* fa, uint64_t n, uint8_t e0, uint8_t e1
   PK_TRY(need(c, ev_buf, m + 1, &nl));
   if (nb) {
     if (pk)
-      hipLaunchKernelGGL(k_nl_write_rx, dim3((unsigned)nb), dim3(NL_NT), 0, st, pk->RX, n, blkoff, nl, follow);
+      hipLaunchKernelGGL(k_nl_write_rx, dim3((unsigned)nb), dim3(NL_NT), 0, st, pk->RX, n, blkoff, nl);
     else
       hipLaunchKernelGGL(k_nl_write, dim3((unsigned)nb), dim3(NL_NT), 0, st, fa, n, e0, e1, blkoff, nl, follow);
     PK_HIP(c, hipGetLastError());
@@ -3499,9 +3721,11 @@ int normalize_impl(pk_ctx* c, const uint8_t* in, uint64_t n, int fmt, const uint
 
 // Where the packed input goes (pk stays empty when the scratch of
 // pk_count_noalloc has no room for it).
-int pack_buffers(pk_ctx* c, uint64_t n, Packed* pk) {
-  const uint64_t words = (n + 15) / 16;
-  const uint64_t ew = (PK_PAD + words + 67) & ~63ull, bytes = 4 * (ew + words + 64);
+int pack_buffers(pk_ctx* c, uint64_t n, bool valid, Packed* pk) {
+  const uint64_t words = (n + 15) / 16, nb = (n + NL_PER_BLOCK - 1) / NL_PER_BLOCK;
+  const uint64_t ew = (PK_PAD + words + 67) & ~63ull, rw = (words + 64 + 63) & ~63ull;
+  const uint64_t vw = valid ? nb * (NL_PER_BLOCK / 64) * 2 : 0;  // W in 32-bit words
+  const uint64_t bytes = 4 * (ew + rw + vw);
   uint32_t* p;
   if (c->arena_mode) {
     const uint64_t take = (bytes + 255) & ~255ull;
@@ -3516,6 +3740,7 @@ int pack_buffers(pk_ctx* c, uint64_t n, Packed* pk) {
   }
   pk->E = p;
   pk->RX = p + ew;
+  if (valid) pk->W = reinterpret_cast<ull*>(p + ew + rw);
   return PK_OK;
 }
 
@@ -3525,12 +3750,85 @@ struct Records {
   ull* rstart = nullptr;
   uint32_t* rlen = nullptr;
   ull* kofs = nullptr;
+  const ull* tb = nullptr;  // main path: window ends before each index block
+  uint64_t n = 0;  // input bytes
   uint64_t R = 0, N = 0;
   Packed pk;
 };
 
+int format_error(pk_ctx* c, ull r) {
+  return c->fail(PK_EFORMAT,
+                 "input is not strict single-line FASTA (record " + std::to_string(r) + " does not start with '>')");
+}
+
+int records_main(pk_ctx* c, const uint8_t* fa, uint64_t n, int K, Records* rec);
+
+// The windows of the main path from the packed input: valid ends and their
+// number per index block, no list of lines or reads.
+int windows_main(pk_ctx* c, const uint8_t* fa, uint64_t n, int K, Records* rec) {
+  hipStream_t st = c->stream;
+  ull* small;
+  PK_TRY(need(c, B_SMALL, 16, &small));
+  // small[2] = first format error, [3] = a line may be too long, [4], [5] =
+  // overflow and retry counts, [6] .. [9] = k_lines' facts, [10] = first '>'
+  PK_TRY(fill_u64(c, small + 2, ~0ull, 1));
+  PK_TRY(fill_u64(c, small + 3, 0, 3));
+  const uint64_t nb = (n + NL_PER_BLOCK - 1) / NL_PER_BLOCK;
+  const Packed& pk = rec->pk;
+  ull *blk, *blkoff, *blkgt, *tb;
+  uint32_t* cnt;
+  PK_TRY(need(c, B_BLK, nb, &blk));
+  PK_TRY(need(c, B_BLKGT, nb + 1, &blkgt));
+  PK_TRY(need(c, B_BLKOFF, nb + 1, &blkoff));
+  PK_TRY(need(c, B_WCNT, nb, &cnt));
+  PK_TRY(need(c, B_WOFF, nb + 1, &tb));
+  rec->tb = tb;
+  if (!nb) return PK_OK;
+  hipLaunchKernelGGL(HIP_KERNEL_NAME(k_pack<ENC_MAIN>), dim3((unsigned)nb), dim3(NL_NT), 0, st, fa, n, (uint8_t)'\n',
+                     (uint8_t)'\n', blk, blkgt, 0, pk.E, pk.RX);
+  PK_HIP(c, hipGetLastError());
+  PK_TRY(scan_excl<ull>(c, blk, blkoff, nb));
+  const bool check_long = n > 0xFFFFFFF0ull;
+  if (check_long) {
+    hipLaunchKernelGGL(k_long_lines, dim3(grid_for(nb, 256)), dim3(256), 0, st, blkoff, nb, small + 3);
+    PK_HIP(c, hipGetLastError());
+  }
+  ull hs[8], N = 0;
+  // the first '>' is nearly always in the first block (blkgt[0]); else a
+  // second pass looks for it everywhere
+  const ull* gt = blkgt;
+  for (int pass = 0;; pass++) {
+    hipLaunchKernelGGL(k_lines, dim3(1), dim3(1024), 0, st, pk.RX, n, blkoff, nb, gt, K, small + 6);
+    PK_HIP(c, hipGetLastError());
+    hipLaunchKernelGGL(k_valid, dim3((unsigned)nb), dim3(NL_NT), 0, st, pk.RX, n, blkoff, small + 6, K, pk.W, cnt,
+                       small + 2);
+    PK_HIP(c, hipGetLastError());
+    PK_TRY(scan_excl<uint32_t>(c, cnt, tb, nb));
+    PK_HIP(c, hipMemcpyAsync(hs, small + 2, 64, hipMemcpyDeviceToHost, st));
+    PK_HIP(c, hipMemcpyAsync(&N, tb + nb, 8, hipMemcpyDeviceToHost, st));
+    PK_HIP(c, hipStreamSynchronize(st));
+    if (hs[7] < n || pass || nb == 1) break;
+    hipLaunchKernelGGL(k_nl_count, dim3((unsigned)nb), dim3(NL_NT), 0, st, fa, n, (uint8_t)'\n', (uint8_t)'\n', blk,
+                       blkgt, 1);
+    PK_HIP(c, hipGetLastError());
+    hipLaunchKernelGGL(k_min_reduce, dim3(1), dim3(1024), 0, st, blkgt, nb, small + 10);
+    PK_HIP(c, hipGetLastError());
+    gt = small + 10;
+  }
+  rec->R = hs[5];
+  rec->N = N;
+  if (hs[0] != ~0ull && hs[0] <= rec->R) return format_error(c, hs[0]);
+  if (check_long && hs[1]) {
+    // the read table measures every line
+    Records full;
+    PK_TRY(records_main(c, fa, n, K, &full));
+    PK_TRY(fill_u64(c, small + 4, 0, 2));
+  }
+  return PK_OK;
+}
+
 // Read table of the main path: records of the reference's Sliding_window.
-int records_main(pk_ctx* c, const uint8_t* fa, uint64_t n, int K, Records* rec, bool want_len) {
+int records_main(pk_ctx* c, const uint8_t* fa, uint64_t n, int K, Records* rec) {
   hipStream_t st = c->stream;
   ull* small;
   PK_TRY(need(c, B_SMALL, 16, &small));
@@ -3542,13 +3840,12 @@ int records_main(pk_ctx* c, const uint8_t* fa, uint64_t n, int K, Records* rec, 
   ull* nl;
   uint64_t m, p0;
   // entries carry what follows each '\n' (bits 62-63): only k_reads reads them
-  if (!want_len) PK_TRY(pack_buffers(c, n, &rec->pk));
-  PK_TRY(event_index(c, fa, n, '\n', '\n', small, &nl, &m, &p0, B_NL, 1, rec->pk.E ? &rec->pk : nullptr));
+  PK_TRY(event_index(c, fa, n, '\n', '\n', small, &nl, &m, &p0, B_NL, 1));
   const uint64_t ncand = m / 2 + 2;
   ull *rstart, *kofs;
-  uint32_t *rlen = nullptr, *kc;
+  uint32_t *rlen, *kc;
   PK_TRY(need(c, B_RSTART, ncand, &rstart));
-  if (!rec->pk.E) PK_TRY(need(c, B_RLEN, ncand, &rlen));
+  PK_TRY(need(c, B_RLEN, ncand, &rlen));
   PK_TRY(need(c, B_KC, ncand, &kc));
   PK_TRY(need(c, B_KOFS, ncand + 1, &kofs));
   hipLaunchKernelGGL(k_reads, dim3(grid_for(ncand, 256)), dim3(256), 0, st, n, nl, m, p0, K,
@@ -3560,9 +3857,7 @@ int records_main(pk_ctx* c, const uint8_t* fa, uint64_t n, int K, Records* rec, 
   PK_HIP(c, hipMemcpyAsync(&hs[3], kofs + ncand, 8, hipMemcpyDeviceToHost, st));
   PK_HIP(c, hipStreamSynchronize(st));
   const uint64_t R = std::min<uint64_t>(hs[0], ncand);
-  if (hs[1] != ~0ull && hs[1] <= R)
-    return c->fail(PK_EFORMAT, "input is not strict single-line FASTA (record " +
-                                   std::to_string(hs[1]) + " does not start with '>')");
+  if (hs[1] != ~0ull && hs[1] <= R) return format_error(c, hs[1]);
   if (hs[2] != ~0ull && hs[2] < R) return c->fail(PK_EINVAL, "read longer than 4 GiB");
   rec->rstart = rstart;
   rec->rlen = rlen;
@@ -3582,8 +3877,8 @@ int records_builder(pk_ctx* c, const uint8_t* fa, uint64_t n, int klen, uint64_t
   PK_TRY(fill_u64(c, small + 4, 0, 2));
   ull* ev;
   uint64_t m, p0;
-  PK_TRY(pack_buffers(c, n, &rec->pk));
-  PK_TRY(event_index(c, fa, n, sy.delim, sy.skip, small, &ev, &m, &p0, B_NL, 0, &rec->pk, ENC_BUILDER));
+  PK_TRY(pack_buffers(c, n, false, &rec->pk));
+  PK_TRY(event_index(c, fa, n, sy.delim, sy.skip, small, &ev, &m, &p0, B_NL, 0, &rec->pk));
   ull *rstart, *kofs, *idx;
   uint32_t *rlen, *kc, *flag;
   PK_TRY(need(c, B_RSTART, m + 1, &rstart));
@@ -3644,7 +3939,12 @@ int level_buffers(pk_ctx* c, int set, uint64_t B, uint64_t tiles, int db, LevelB
 // anything: they come after every offset that is read).
 int level_runs(pk_ctx* c, const LevelBufs& l, uint64_t tiles, int db, int tk, Runs* out) {
   PK_TRY(scan_excl<RunCount>(c, reinterpret_cast<const RunCount*>(l.M), l.V, tiles << db));
-  *out = Runs{l.M, l.V, l.tp, l.boff, db, tk};
+  out->M = l.M;
+  out->V = l.V;
+  out->tp = l.tp;
+  out->boff = l.boff;
+  out->db = db;
+  out->tk = tk;
   return PK_OK;
 }
 
@@ -3684,12 +3984,13 @@ int count_partitioned(pk_ctx* c, Key* S, Key* S2, int32_t* C, Part p, int btot, 
     const int lv = c->ms_levels < MS_TIMED_LEVELS ? c->ms_levels : -1;
     if (lv >= 0) PK_HIP(c, hipEventRecord(c->ev[20 + 2 * lv], st));
     hipLaunchKernelGGL(HIP_KERNEL_NAME(k_split<Key, SPLIT_RUNS>), dim3((unsigned)tiles), dim3(SP_NT), 0, st, Sin,
-                       WinSrc{}, p.in, (int)p.B, tk, ~Key(0), KB - p.fixed - db, db, l.boff, l.tp, l.M, Sout);
+                       WinSrc{}, p.in, (int)p.B, tk, KB - p.fixed - db, db, l.boff, l.tp, l.M, Sout);
     PK_HIP(c, hipGetLastError());
     if (lv >= 0) PK_HIP(c, hipEventRecord(c->ev[21 + 2 * lv], st));
     if (lv >= 0) c->ms_form[lv] = PK_MS_TILES;
     c->timing.ms_scatter_form = PK_MS_TILES;
     c->ms_levels++;
+    p.in.tb = nullptr;
     PK_TRY(level_runs(c, l, tiles, db, tk, &p.in));
     p.B <<= db;
     p.fixed += db;
@@ -3860,29 +4161,54 @@ int count_records(pk_ctx* c, const Records& rec, int K, int KB, Key mask) {
   const float bf = tun.bucket_factor > 0.f ? tun.bucket_factor : 3.0f;
   const int btot = choose_bits(N, KB / 2, CAP, bf);
   c->timing.bucket_bits = btot;
-  // level 1: tiles of N / 512 windows (so that a small input spreads over the
-  // CUs and a bucket has at most RUN_CAP runs), within 4096 and a full tile;
-  // one level of up to 10 bits while its buckets keep to those runs
-  const uint64_t per = (N + RUN_CAP - 1) / RUN_CAP;
-  const int tk = (int)std::min<uint64_t>(SplitCfg<Key>::TK_MAX,
-                                         std::max<uint64_t>(4096, (per + SP_NT - 1) / SP_NT * SP_NT));
-  int d1;
-  if (tun.l1_bits > 0 && tun.l1_bits <= L1_MAX_BITS) d1 = std::min(btot, tun.l1_bits);
-  else if (btot <= SP_MAX_BITS && N <= (uint64_t)RUN_CAP * SplitCfg<Key>::TK_MAX) d1 = btot;
-  else d1 = level_bits(btot);
-  const uint64_t tiles = (N + tk - 1) / tk;
   Key *S, *S2;
   int32_t* C;
   PK_TRY(need(c, B_S, N, &S));
   LevelBufs l;
-  PK_TRY(level_buffers(c, 0, 1, tiles, d1, &l));
-  hipLaunchKernelGGL(k_tiles_one, dim3(1), dim3(1), 0, st, (ull)tiles, (ull)N, l.boff, l.tp);
-  PK_HIP(c, hipGetLastError());
-  PK_HIP(c, hipEventRecord(c->ev[4], st));
-  constexpr int SRC = ENC == ENC_MAIN ? SPLIT_MAIN : SPLIT_BUILDER;
-  hipLaunchKernelGGL(HIP_KERNEL_NAME(k_split<Key, SRC>), dim3((unsigned)tiles), dim3(SP_NT), 0, st,
-                     (const Key*)nullptr, WinSrc{rec.pk.E, rec.pk.RX, rec.kofs, rec.rstart, rec.R, K}, Runs{}, 1, tk,
-                     mask, KB - d1, d1, l.boff, l.tp, l.M, S);
+  Part p{Runs{}, 0, 0, 0};
+  uint64_t tiles;
+  int d1, tk = 0;
+  auto level1_bits = [&]() {
+    if (tun.l1_bits > 0 && tun.l1_bits <= L1_MAX_BITS) return std::min(btot, tun.l1_bits);
+    // one level of up to 10 bits while a bucket's runs fit the hash's map
+    if (btot <= SP_MAX_BITS && tiles <= (uint64_t)RUN_CAP) return btot;
+    return level_bits(btot);
+  };
+  if (ENC == ENC_MAIN) {
+    // tiles of 16 or 32 KiB of the input: the larger ones' runs are twice as
+    // long, the smaller ones spread an input over more CUs
+    const uint64_t nblk = (rec.n + NL_PER_BLOCK - 1) / NL_PER_BLOCK;
+    const int wpt = nblk >= 4096 ? 2 : 1;
+    tiles = (nblk + wpt - 1) / wpt;
+    d1 = level1_bits();
+    PK_TRY(level_buffers(c, 0, 1, tiles, d1, &l));
+    hipLaunchKernelGGL(k_tiles_one, dim3(1), dim3(1), 0, st, (ull)tiles, (ull)N, l.boff, l.tp);
+    PK_HIP(c, hipGetLastError());
+    PK_HIP(c, hipEventRecord(c->ev[4], st));
+    const uint16_t* W = reinterpret_cast<const uint16_t*>(rec.pk.W);
+    if (wpt == 2)
+      hipLaunchKernelGGL(HIP_KERNEL_NAME(k_split_main<Key, 2>), dim3((unsigned)tiles), dim3(SM_NT), 0, st, rec.pk.E,
+                         rec.pk.RX, W, rec.tb, (ull)nblk, mask, KB - d1, d1, l.M, S);
+    else
+      hipLaunchKernelGGL(HIP_KERNEL_NAME(k_split_main<Key, 1>), dim3((unsigned)tiles), dim3(SM_NT), 0, st, rec.pk.E,
+                         rec.pk.RX, W, rec.tb, (ull)nblk, mask, KB - d1, d1, l.M, S);
+    p.in.tb = rec.tb;
+    p.in.ts = wpt - 1;
+  } else {
+    // tiles of N / 512 windows (so that a small input spreads over the CUs and
+    // a bucket has at most RUN_CAP runs), within 4096 and a full tile
+    const uint64_t per = (N + RUN_CAP - 1) / RUN_CAP;
+    tk = (int)std::min<uint64_t>(SplitCfg<Key>::TK_MAX, std::max<uint64_t>(4096, (per + SP_NT - 1) / SP_NT * SP_NT));
+    tiles = (N + tk - 1) / tk;
+    d1 = level1_bits();
+    PK_TRY(level_buffers(c, 0, 1, tiles, d1, &l));
+    hipLaunchKernelGGL(k_tiles_one, dim3(1), dim3(1), 0, st, (ull)tiles, (ull)N, l.boff, l.tp);
+    PK_HIP(c, hipGetLastError());
+    PK_HIP(c, hipEventRecord(c->ev[4], st));
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_split<Key, SPLIT_BUILDER>), dim3((unsigned)tiles), dim3(SP_NT), 0, st,
+                       (const Key*)nullptr, WinSrc{rec.pk.E, rec.kofs, rec.rstart, rec.R, K}, Runs{}, 1, tk, KB - d1,
+                       d1, l.boff, l.tp, l.M, S);
+  }
   PK_HIP(c, hipGetLastError());
   PK_HIP(c, hipEventRecord(c->ev[16], st));
   // the packed input has been read: its scratch is free for what follows
@@ -3890,7 +4216,8 @@ int count_records(pk_ctx* c, const Records& rec, int K, int KB, Key mask) {
   c->arena_lim = c->arena_cap;
   PK_TRY(need(c, B_S2, N, &S2));
   PK_TRY(need(c, B_C, N, &C));
-  Part p{Runs{}, 1ull << d1, d1, 0};
+  p.B = 1ull << d1;
+  p.fixed = d1;
   PK_TRY(level_runs(c, l, tiles, d1, tk, &p.in));
   return count_partitioned<Key>(c, S, S2, C, p, btot, KB, N);
 }
@@ -3959,7 +4286,7 @@ int count_share(pk_ctx* c, const uint8_t* fa, uint64_t n, const Records& rec, in
                      nblk, S);
   PK_HIP(c, hipGetLastError());
   PK_HIP(c, hipEventRecord(c->ev[16], st));
-  return count_partitioned<Key>(c, S, S2, C, Part{Runs{nullptr, nullptr, nullptr, boff, 0, 0}, B1, d1, 0}, btot, KB,
+  return count_partitioned<Key>(c, S, S2, C, Part{Runs{nullptr, nullptr, nullptr, boff, 0, 0, nullptr, 0}, B1, d1, 0}, btot, KB,
                                 N);
 }
 
@@ -3993,7 +4320,7 @@ int windows_count_impl(pk_ctx* c, const uint8_t* fa, const ull* rstart, const ui
   const float bf = c->tuning.bucket_factor > 0.f ? c->tuning.bucket_factor : 3.0f;
   const int btot = choose_bits(N, KB / 2, HashCfg<Key>::LIMIT, bf);
   c->timing.bucket_bits = btot;
-  return count_partitioned<Key>(c, S, S2, C, Part{Runs{nullptr, nullptr, nullptr, boff, 0, 0}, 1, 0, 0}, btot, KB, N);
+  return count_partitioned<Key>(c, S, S2, C, Part{Runs{nullptr, nullptr, nullptr, boff, 0, 0, nullptr, 0}, 1, 0, 0}, btot, KB, N);
 }
 
 template <class Key>
@@ -4004,10 +4331,15 @@ int count_impl(pk_ctx* c, const uint8_t* fa, uint64_t n, int K) {
   c->key_bits = 2 * K;
   PK_HIP(c, hipEventRecord(c->ev[0], c->stream));
   Records rec;
-  PK_TRY(records_main(c, fa, n, K, &rec, false));
-  // without the packed input (pk_count_noalloc's scratch is short of it) the
-  // walk of a share that owns every k-mer takes its place
-  if (!rec.pk.E) return count_share<Key>(c, fa, n, rec, K, OwnCfg{nullptr, 1, 0, 1});
+  rec.n = n;
+  PK_TRY(pack_buffers(c, n, true, &rec.pk));
+  if (!rec.pk.E) {
+    // pk_count_noalloc's scratch is short of the packed input: the walk of a
+    // share that owns every k-mer takes its place
+    PK_TRY(records_main(c, fa, n, K, &rec));
+    return count_share<Key>(c, fa, n, rec, K, OwnCfg{nullptr, 1, 0, 1});
+  }
+  PK_TRY(windows_main(c, fa, n, K, &rec));
   return count_records<Key, ENC_MAIN>(c, rec, K, 2 * K, key_mask<Key>(2 * K));
 }
 
@@ -4015,7 +4347,7 @@ int count_impl(pk_ctx* c, const uint8_t* fa, uint64_t n, int K) {
 // with the record rule of Sliding_window_l (a record needs L bytes).
 int lmer_frequency_impl(pk_ctx* c, const uint8_t* fa, uint64_t n, ull** freq_out) {
   Records rec;
-  PK_TRY(records_main(c, fa, n, LMER_L, &rec, true));
+  PK_TRY(records_main(c, fa, n, LMER_L, &rec));
   const uint64_t R = rec.R;
   ull* freq;
   PK_TRY(need(c, B_LFREQ, LMER_BINS, &freq));
@@ -4041,7 +4373,7 @@ int rank_share_impl(pk_ctx* c, const uint8_t* fa, uint64_t n, int K, int P, int 
   ull* freq;
   PK_TRY(lmer_frequency_impl(c, fa, n, &freq));
   Records rec;
-  PK_TRY(records_main(c, fa, n, K, &rec, true));
+  PK_TRY(records_main(c, fa, n, K, &rec));
   return count_share<Key>(c, fa, n, rec, K, OwnCfg{freq, P, rank, 0});
 }
 
@@ -4055,7 +4387,7 @@ int rank_share_key_impl(pk_ctx* c, const uint8_t* fa, uint64_t n, int K, int P, 
   c->key_bits = 2 * K;
   PK_HIP(c, hipEventRecord(c->ev[0], c->stream));
   Records rec;
-  PK_TRY(records_main(c, fa, n, K, &rec, true));
+  PK_TRY(records_main(c, fa, n, K, &rec));
   return count_share<Key>(c, fa, n, rec, K, OwnCfg{nullptr, P, rank, 1});
 }
 

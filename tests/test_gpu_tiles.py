@@ -1,0 +1,119 @@
+"""Tiled partition of the counting path (k_pack, k_valid, k_split_main,
+k_split, the run maps and the retry of the bucket count) at the sizes where
+it can go wrong, bit-exact against the oracle: inputs that end just before,
+at and after a 16-byte word, a 64-byte group, a 16 KiB block and a tile;
+lines, headers and reads across those borders; tiles without a k-mer; buckets
+with far more runs than a map holds, with more distinct keys than a table,
+and with nearly all keys of the input."""
+from __future__ import annotations
+
+import sys
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _p(*a):
+    print(*a, flush=True)
+    sys.stdout.flush()
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    from pakman_plus_amd import api
+    c = api.Context(0)
+    yield c
+    c.close()
+
+
+def _bases(rng, n, alpha=b"ACGT"):
+    return bytes(rng.choice(np.frombuffer(alpha, dtype=np.uint8), n))
+
+
+def _check(ctx, oracle_mod, fa, k):
+    ctx.count(fa, k)
+    keys, counts = ctx.table_host()
+    want_k, want_c = oracle_mod.count(fa, k)
+    assert np.array_equal(keys.reshape(-1), np.asarray(want_k).reshape(-1))
+    assert np.array_equal(counts, want_c)
+
+
+@pytest.mark.parametrize("size", [15, 16, 17, 63, 64, 65, 16383, 16384, 16385, 16384 + 63, 32767, 32768, 32769,
+                                  3 * 16384 - 1, 3 * 16384])
+@pytest.mark.parametrize("newline", [True, False])
+def test_one_read_ends_at_a_border(ctx, oracle_mod, size, newline):
+    """One record whose input is `size` bytes long, with and without the
+    final line end, at the smallest, a middle and the largest k."""
+    rng = np.random.default_rng(size)
+    body = size - 3 - int(newline)
+    fa = b">h\n" + _bases(rng, body, b"ACGTN") + (b"\n" if newline else b"")
+    assert len(fa) == size
+    for k in (8, 31, 32, 33, 64):
+        _p(f"case: border size={size} newline={newline} k={k}")
+        _check(ctx, oracle_mod, fa, k)
+
+
+@pytest.mark.parametrize("shift", [0, 1, 31, 62, 63, 64])
+def test_line_ends_around_a_block_border(ctx, oracle_mod, shift):
+    """A read's start, a header and a short read on either side of byte 16384;
+    then 40 KiB of header (whole tiles without a k-mer) and two reads."""
+    rng = np.random.default_rng(100 + shift)
+    first = b">a\n"
+    fa = first + _bases(rng, 16384 - len(first) - shift) + b"\n>b\n" + _bases(rng, 40) + b"\n>c\n" + _bases(rng, 300)
+    fa += b"\n>" + b"h" * 40960 + b"\n" + _bases(rng, 5000) + b"\n>d\n" + _bases(rng, 64) + b"\n"
+    for k in (9, 32, 64):
+        _p(f"case: block border shift={shift} k={k}")
+        _check(ctx, oracle_mod, fa, k)
+
+
+@pytest.mark.parametrize("k", [16, 32, 50])
+@pytest.mark.parametrize("factor", [0.0, 0.02, 6.0])
+def test_levels_and_retries(ctx, oracle_mod, k, factor):
+    """All k-mers distinct (every table of the built-in size and of six times
+    the load retries in several passes), at one, two and three levels."""
+    rng = np.random.default_rng(7)
+    fa = b"".join(b">r%d\n" % i + _bases(rng, 150) + b"\n" for i in range(6000))
+    try:
+        ctx.set_tuning(bucket_factor=factor)
+        _p(f"case: levels k={k} bucket_factor={factor}")
+        _check(ctx, oracle_mod, fa, k)
+    finally:
+        ctx.set_tuning()
+
+
+@pytest.mark.parametrize("k", [21, 40])
+def test_skewed_parent_with_many_short_runs(ctx, oracle_mod, k):
+    """A-rich reads: one level-1 bucket holds most k-mers, so its rare second
+    digits have a few keys in each of hundreds of tiles (more runs than a
+    bucket's map), its common ones far more keys than a table."""
+    rng = np.random.default_rng(11)
+    reads = np.full((130_000, 100), ord("A"), dtype=np.uint8)
+    hit = rng.random(reads.shape) < 0.02
+    reads[hit] = rng.choice(np.frombuffer(b"CGT", dtype=np.uint8), int(hit.sum()))
+    rows = np.concatenate([np.tile(np.frombuffer(b">r\n", dtype=np.uint8), (reads.shape[0], 1)), reads,
+                           np.full((reads.shape[0], 1), 10, dtype=np.uint8)], axis=1)
+    fa = rows.tobytes()
+    try:
+        ctx.set_tuning(l1_bits=6, bucket_factor=0.3)
+        _p(f"case: skewed parent k={k}")
+        _check(ctx, oracle_mod, fa, k)
+    finally:
+        ctx.set_tuning()
+
+
+@pytest.mark.parametrize("klen,bits", [(11, 64), (32, 64), (40, 128), (64, 128)])
+@pytest.mark.parametrize("reads", [1, 45, 700])
+def test_builder_tiles(ctx, oracle_mod, klen, bits, reads):
+    """Builder counts over one tile and several, with words that reach back
+    to the read's start (klen below the word) and full ones."""
+    rng = np.random.default_rng(klen + reads)
+    fa = b"".join(b">r%d\n" % i + _bases(rng, 120, b"ACGTN") + b"\n" for i in range(reads))
+    _p(f"case: builder tiles klen={klen} bits={bits} reads={reads}")
+    n = ctx.builder_count(fa, klen, read_len=100, kmer_bits=bits)
+    keys, counts = ctx.table_host()
+    want_n, want_k, want_c = oracle_mod.builder_count(fa, klen, 100, bits)
+    assert n == want_n
+    assert np.array_equal(keys.reshape(-1), np.asarray(want_k).reshape(-1))
+    assert np.array_equal(counts, want_c)
