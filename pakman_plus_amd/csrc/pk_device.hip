@@ -1787,28 +1787,31 @@ __global__ __launch_bounds__(SP_NT, 4) void k_split(const Key* __restrict__ Sin,
 }
 
 // Level 1 of the main path: tile t is the bytes [t * 16384 * WPT, ...), its
-// keys the k-mers that end there (bits of W).  A thread holds WPT words of E
-// and the NW words before them in registers, so the k-mer that ends at each of
-// its 16 * WPT bytes is NW funnel shifts by constants: cutting a k-mer costs
-// about as much as copying it, so the keys are cut twice, once to rank them
-// by digit and once more to place them, and need no registers in between.
-// That allows 64 VGPRs, two 1024-thread blocks per CU.  Against tiles gathered
-// by window number (search of the read list, a map of its reads, three loads
-// per k-mer): see the figures at count_records.
+// keys the k-mers that end there (bits of W).  Three passes: a thread ranks
+// the k-mers that end at its own 16 * WPT bytes by digit, cut from WPT words
+// of E and the words before them at constant shifts; it notes each one's end
+// (15 bits, and the exact low bit) at its place in the sorted order; then
+// consecutive threads cut consecutive keys of that order out of the tile's
+// packed bases (in LDS) and store them.  The order takes two bytes per key
+// instead of the key, so one round covers the tile, and bytes that end no
+// k-mer cost only the first two passes.  Bound by VALU: with whole keys
+// exchanged through LDS in rounds it issued 115 lane instructions per one-word
+// key (k_l1 figures at count_records).
 constexpr int SM_NT = 1024;
 
 template <class Key, int WPT>
 __global__ __launch_bounds__(SM_NT, 8) void k_split_main(const uint32_t* __restrict__ E,
                                                          const uint32_t* __restrict__ RX,
                                                          const uint16_t* __restrict__ W, const ull* __restrict__ tb,
-                                                         ull nblk, Key mask, int dpos, int db,
+                                                         ull nblk, ull nwords, Key mask, int dpos, int db,
                                                          uint32_t* __restrict__ M, Key* __restrict__ Sout) {
   constexpr int NW = (int)sizeof(Key) / 4;
   constexpr int P = 16 * WPT;
-  constexpr int ROUND = SP_TILE_BYTES / (int)sizeof(Key);
   static_assert(NL_PER_BLOCK == 16ull * SM_NT, "a word of E per thread and index block");
   static_assert(SM_NT == 1 << SP_MAX_BITS, "a digit per thread");
-  __shared__ Key T[ROUND];
+  static_assert(SM_NT * P <= 32768, "15 bits of place");
+  __shared__ uint16_t order[SM_NT * P];
+  __shared__ uint32_t es[SM_NT * WPT + NW];  // E from NW words before the tile
   __shared__ uint32_t h[1 << SP_MAX_BITS];
   __shared__ uint32_t nw[SM_NT / 64 + 1];
   const int tid = (int)threadIdx.x;
@@ -1816,44 +1819,55 @@ __global__ __launch_bounds__(SM_NT, 8) void k_split_main(const uint32_t* __restr
   const ull v0 = uniform(tb[t * WPT]);
   const ull t1 = (t + 1) * WPT < nblk ? (t + 1) * WPT : nblk;
   const int m = (int)(uniform(tb[t1]) - v0);
-  const ull w = (t * SM_NT + (ull)tid) * WPT;
-  uint32_t val = 0;
+  const ull w0 = t * (SM_NT * WPT);  // the tile's first word
+  const ull w = w0 + (ull)(tid * WPT);
+  uint32_t val = 0, rx = 0;
   if (w < nblk * SM_NT) val = W[w];
   if (WPT == 2 && w + 1 < nblk * SM_NT) val |= (uint32_t)W[w + 1] << 16;
-  uint32_t ew[NW + WPT] = {}, rx = 0;
+  uint32_t ew[NW + WPT] = {};
   if (val) {
 #pragma unroll
     for (int i = 0; i < NW + WPT; i++) ew[i] = E[PK_PAD + w - NW + i];
     rx = RX[w] & 0xFFFFu;
     if (WPT == 2) rx |= RX[w + 1] << 16;
   }
-  // the k-mer that ends at byte j of the thread's words
-  auto key = [&](int j) {
-    const int c = NW + (j >> 4);
-    const uint32_t sh = 30u - 2u * (uint32_t)(j & 15);
-    Key k = 0;
-#pragma unroll
-    for (int i = NW - 1; i >= 0; i--) {
-      uint32_t o = __builtin_amdgcn_alignbit(ew[c - 1 - i], ew[c - i], sh);
-      // the last base's low bit, without the next byte's spill
-      if (i == 0) o = (o & ~1u) | ((rx >> j) & 1u);
-      k = (k << 31 << 1) | (Key)o;
-    }
-    return k & mask;
-  };
-  // makes the compiler cut the keys anew instead of keeping them in registers
-  auto forget = [&]() {
-#pragma unroll
-    for (int i = 0; i < NW + WPT; i++) asm volatile("" : "+v"(ew[i]));
-    asm volatile("" : "+v"(val), "+v"(rx));
-  };
   const int ns = 1 << db;
   if (tid < ns) h[tid] = 0;
+  // the tile's words for the last pass (a k-mer that ends here may start in
+  // words whose own bytes end none)
+  for (int i = tid; i < SM_NT * WPT + NW; i += SM_NT)
+    if (w0 + i < nwords + NW) es[i] = E[PK_PAD + w0 - NW + i];
+  // digit words: dw holds the stream E shifted down by dpos bits, so that the
+  // digit of the k-mer that ends at byte j lies at the constant bit position
+  // of byte j in it
+  uint32_t dw[WPT + 1];
+  {
+    const int q = dpos >> 5, sh = dpos & 31;
+#pragma unroll
+    for (int i = 0; i <= WPT; i++) {
+      // dw[i] = bits of words c - q - 1, c - q for c = NW + WPT - 1 - i
+      const int c = NW + WPT - 1 - i;
+      uint32_t hi = 0, lo = 0;
+#pragma unroll
+      for (int x = 0; x < NW; x++) {
+        if (x == q) {
+          if (c - x >= 0) lo = ew[c - x];
+          if (c - x - 1 >= 0) hi = ew[c - x - 1];
+        }
+      }
+      dw[i] = __builtin_amdgcn_alignbit(hi, lo, (uint32_t)sh);
+    }
+  }
+  const uint32_t dm = (1u << db) - 1u;
+  auto digit = [&](int j) -> uint32_t {
+    const int i = WPT - 1 - (j >> 4);
+    return __builtin_amdgcn_alignbit(dw[i + 1], dw[i], 30u - 2u * (uint32_t)(j & 15)) & dm;
+  };
   __syncthreads();
   uint32_t rk[P / 2] = {};
 #pragma unroll
   for (int j = 0; j < P; j++)
-    if ((val >> j) & 1u) rk[j / 2] |= atomicAdd(&h[key_digit<Key>(key(j), dpos, db)], 1u) << (16 * (j & 1));
+    if ((val >> j) & 1u) rk[j / 2] |= atomicAdd(&h[digit(j)], 1u) << (16 * (j & 1));
   __syncthreads();
   {
     const uint32_t c = tid < ns ? h[tid] : 0u;
@@ -1865,24 +1879,28 @@ __global__ __launch_bounds__(SM_NT, 8) void k_split_main(const uint32_t* __restr
     }
   }
   __syncthreads();
-  // place of every key in the sorted tile
-  forget();
 #pragma unroll
   for (int j = 0; j < P; j++) {
-    if ((val >> j) & 1u) rk[j / 2] += h[key_digit<Key>(key(j), dpos, db)] << (16 * (j & 1));
+    if ((val >> j) & 1u)
+      order[h[digit(j)] + ((rk[j / 2] >> (16 * (j & 1))) & 0xFFFFu)] =
+          (uint16_t)((uint32_t)(tid * P + j) | ((rx >> j) & 1u) << 15);
   }
-  for (int r0 = 0; r0 < m; r0 += ROUND) {
-    forget();
+  __syncthreads();
+  Key* o = Sout + v0;
+  for (int p = tid; p < m; p += SM_NT) {
+    const uint32_t s = order[p];
+    const uint32_t e = s & 0x7FFFu;
+    const uint32_t* x = es + (e >> 4);
+    const uint32_t sh = 30u - 2u * (e & 15u);
+    Key k = 0;
 #pragma unroll
-    for (int j = 0; j < P; j++) {
-      const uint32_t p = ((rk[j / 2] >> (16 * (j & 1))) & 0xFFFFu) - (uint32_t)r0;
-      if (((val >> j) & 1u) && p < (uint32_t)ROUND) T[p] = key(j);
+    for (int i = NW - 1; i >= 0; i--) {
+      uint32_t u = __builtin_amdgcn_alignbit(x[NW - 1 - i], x[NW - i], sh);
+      // the last base's low bit, without the next byte's spill
+      if (i == 0) u = (u & ~1u) | s >> 15;
+      k = (k << 31 << 1) | (Key)u;
     }
-    __syncthreads();
-    const int c = m - r0 < ROUND ? m - r0 : ROUND;
-    Key* o = Sout + v0 + r0;
-    for (int p = tid; p < c; p += SM_NT) o[p] = T[p];
-    __syncthreads();
+    o[p] = k & mask;
   }
 }
 
@@ -4188,10 +4206,10 @@ int count_records(pk_ctx* c, const Records& rec, int K, int KB, Key mask) {
     const uint16_t* W = reinterpret_cast<const uint16_t*>(rec.pk.W);
     if (wpt == 2)
       hipLaunchKernelGGL(HIP_KERNEL_NAME(k_split_main<Key, 2>), dim3((unsigned)tiles), dim3(SM_NT), 0, st, rec.pk.E,
-                         rec.pk.RX, W, rec.tb, (ull)nblk, mask, KB - d1, d1, l.M, S);
+                         rec.pk.RX, W, rec.tb, (ull)nblk, (ull)((rec.n + 15) / 16), mask, KB - d1, d1, l.M, S);
     else
       hipLaunchKernelGGL(HIP_KERNEL_NAME(k_split_main<Key, 1>), dim3((unsigned)tiles), dim3(SM_NT), 0, st, rec.pk.E,
-                         rec.pk.RX, W, rec.tb, (ull)nblk, mask, KB - d1, d1, l.M, S);
+                         rec.pk.RX, W, rec.tb, (ull)nblk, (ull)((rec.n + 15) / 16), mask, KB - d1, d1, l.M, S);
     p.in.tb = rec.tb;
     p.in.ts = wpt - 1;
   } else {
