@@ -24,7 +24,7 @@
 //                     MPI_Alltoallv (kmer_counting.cpp:254-352).  Rank-share
 //                     mode keeps one owner's k-mers (k_l1_hist, k_l1_scatter,
 //                     own_step).
-//   4. bucket count   k_bucket_hash: one 512-thread workgroup per bucket counts
+//   4. bucket count   k_bucket_hash: one 1024-thread workgroup per bucket counts
 //                     the bucket's distinct keys in an LDS hash table, then
 //                     counting-sorts them by the next bits and writes the
 //                     ascending (key, count) pairs (the reference's sort + RLE
@@ -1474,18 +1474,25 @@ __device__ __forceinline__ ull block_upper(const ull* x, ull n, ull key) {
   return lo + (ull)__syncthreads_count((ull)threadIdx.x < n && x[lo + threadIdx.x] <= key);
 }
 
+// Inclusive scan of a u32 over the wave by DPP moves (no LDS traffic, where
+// shuffles take one LDS operation per step).
+__device__ __forceinline__ uint32_t wave_scan_u32(uint32_t x) {
+  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x111, 0xF, 0xF, true);   // row_shr 1
+  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x112, 0xF, 0xF, true);   // row_shr 2
+  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x114, 0xF, 0xF, true);   // row_shr 4
+  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x118, 0xF, 0xF, true);   // row_shr 8
+  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x142, 0xA, 0xF, false);  // row_bcast 15 into rows 1, 3
+  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x143, 0xC, 0xF, false);  // row_bcast 31 into rows 2, 3
+  return x;
+}
+
 // Exclusive scan of a u32 over the block through nw[NT / 64 + 1] (LDS); the
 // total in *tot.  The caller passes a barrier before nw is used again.
 template <int NT>
 __device__ __forceinline__ uint32_t block_scan_u32(uint32_t v, uint32_t* nw, uint32_t* tot) {
   constexpr int NW = NT / 64;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  uint32_t x = v;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const uint32_t y = __shfl_up(x, o, 64);
-    if (lane >= o) x += y;
-  }
+  const uint32_t x = wave_scan_u32(v);
   if (lane == 63) nw[w] = x;
   __syncthreads();
   uint32_t before = 0, all = 0;
@@ -1913,29 +1920,41 @@ __global__ __launch_bounds__(SM_NT, 8) void k_split_main(const uint32_t* __restr
 // merge + aggregate (kmer_counting.cpp:3057-3086, 254-352, 169-250) for the
 // keys of one bucket.
 
-constexpr int BS_NT = 512;
-constexpr int SUB_MAX_BITS = 10;
-constexpr int SUB_BINS = 1 << SUB_MAX_BITS;
-
-// Tables of 512 threads, three blocks (6 waves per SIMD) per CU: half as many
-// buckets as with 256 threads, so half the run-table look-ups, barriers and
-// partition digits per key.
+// Blocks of 512 threads, as many waves per CU as the keys' registers allow.
+// Batches of a whole bucket: a second batch costs a second run map and its
+// barriers (k = 63, 1.5e8 keys: 2.46 ms with batches of 2048 against 1.41).
 template <class Key>
 struct HashCfg;
 template <>
 struct HashCfg<uint64_t> {
-  static constexpr int T = 4096;      // table slots (12 bytes each)
-  static constexpr int LIMIT = 3072;  // distinct keys per task (load 0.75)
-  static constexpr int HB = 16;       // keys per thread and batch
-  static constexpr int WAVES = 6;     // waves per SIMD the LDS allows (register cap follows)
+  static constexpr int NT = 512;      // threads per block
+  static constexpr int WAVES = 8;     // waves per SIMD the LDS allows (register cap follows)
+  static constexpr int T = 2560;      // table slots (12 bytes each)
+  static constexpr int LIMIT = 1920;  // distinct keys per task (load 0.75)
+  static constexpr int SUB = 11;      // sub-bin bits of the ordering
+  static constexpr int HB = 8;        // keys per thread and batch
+  static constexpr float FILL = 2.1f;  // built-in instances per bucket: FILL * LIMIT at most, one batch
 };
 template <>
 struct HashCfg<u128> {
-  static constexpr int T = 2048;  // 20 bytes each
-  static constexpr int LIMIT = 1536;
-  static constexpr int HB = 9;
-  static constexpr int WAVES = 6;
+  static constexpr int NT = 512;
+  static constexpr int WAVES = 6;  // three blocks: at 64 VGPRs the keys spill (1.41 -> 1.77 ms, 1.5e8 keys)
+  static constexpr int T = 1536;   // 20 bytes each
+  static constexpr int LIMIT = 1152;
+  static constexpr int SUB = 10;
+  static constexpr int HB = 5;
+  static constexpr float FILL = 2.2f;
 };
+
+// a 32-bit hash scaled to T slots
+template <int T>
+__device__ __forceinline__ uint32_t slot_of(uint32_t h) {
+  return __umulhi(h, (uint32_t)T);
+}
+template <int T>
+__device__ __forceinline__ uint32_t next_slot(uint32_t slot) {
+  return slot + 1 == (uint32_t)T ? 0u : slot + 1;
+}
 // tasks with more instances than this are split without trying
 constexpr uint64_t TASK_MAX_INSTANCES = 1u << 18;
 // linear-probe bound of an insert: a table too full to place a key within
@@ -1958,10 +1977,8 @@ struct HashTable<uint64_t> {
   uint32_t* hc;
   ull empty;
   __device__ __forceinline__ void init(int tid, int nt) {
-    for (int i = tid; i < T; i += nt) {
-      hk[i] = empty;
-      hc[i] = 0;
-    }
+    for (int i = tid; i < T / 2; i += nt) reinterpret_cast<ulonglong2*>(hk)[i] = make_ulonglong2(empty, empty);
+    for (int i = tid; i < T / 4; i += nt) reinterpret_cast<uint4*>(hc)[i] = make_uint4(0u, 0u, 0u, 0u);
   }
   // returns false when no free slot is found within HASH_PROBES probes, or
   // when a long chain finds the table already reported full (*stop)
@@ -1971,8 +1988,7 @@ struct HashTable<uint64_t> {
   // three quarter-rate instructions
   __device__ __forceinline__ static uint32_t home(uint64_t k) {
     const uint32_t lo = (uint32_t)k, hi = (uint32_t)(k >> 32);
-    static_assert((T & (T - 1)) == 0, "a power of two");
-    return ((lo ^ __builtin_amdgcn_alignbit(hi, hi, 13)) * 0x9E3779B1u) >> (32 - __builtin_ctz(T));
+    return slot_of<T>((lo ^ __builtin_amdgcn_alignbit(hi, hi, 13)) * 0x9E3779B1u);
   }
   __device__ __forceinline__ bool try_slot(uint32_t slot, uint64_t k) {
     const ull prev = atomicCAS(&hk[slot], empty, (ull)k);
@@ -1986,12 +2002,12 @@ struct HashTable<uint64_t> {
     uint32_t slot = home(k);
     for (int probe = 0; probe < STOP_AFTER; probe++) {
       if (try_slot(slot, k)) return true;
-      slot = (slot + 1) & (T - 1);
+      slot = next_slot<T>(slot);
     }
     for (int probe = STOP_AFTER; probe < HASH_PROBES; probe++) {
       if ((probe & 7) == 0 && *stop) return false;
       if (try_slot(slot, k)) return true;
-      slot = (slot + 1) & (T - 1);
+      slot = next_slot<T>(slot);
     }
     return false;
   }
@@ -2021,17 +2037,14 @@ struct HashTable<u128> {
   }
   __device__ __forceinline__ static ull fp(u128 k) { return (ull)k ^ spread((ull)(k >> 64)); }
   __device__ __forceinline__ void init(int tid, int nt) {
-    for (int i = tid; i < T; i += nt) {
-      hf[i] = EMPTY;
-      hc[i] = 0;
-    }
+    for (int i = tid; i < T / 2; i += nt) reinterpret_cast<ulonglong2*>(hf)[i] = make_ulonglong2(EMPTY, EMPTY);
+    for (int i = tid; i < T / 4; i += nt) reinterpret_cast<uint4*>(hc)[i] = make_uint4(0u, 0u, 0u, 0u);
   }
   // home slot: one more 32-bit product; probes step to the next slot
   __device__ __forceinline__ static uint32_t home(ull f) {
-    static_assert((T & (T - 1)) == 0, "a power of two");
-    return (((uint32_t)f ^ (uint32_t)(f >> 32)) * 0x9E3779B1u) >> (32 - __builtin_ctz(T));
+    return slot_of<T>(((uint32_t)f ^ (uint32_t)(f >> 32)) * 0x9E3779B1u);
   }
-  __device__ __forceinline__ static uint32_t next(uint32_t slot) { return (slot + 1) & (T - 1); }
+  __device__ __forceinline__ static uint32_t next(uint32_t slot) { return next_slot<T>(slot); }
   // a slot changes only once, from EMPTY to its fingerprint: a plain read
   // finds a repeated key or steps over another one without an atomic, and
   // only an empty slot is claimed by CAS (k = 64 bacterial: 2.73 -> 2.56 ms)
@@ -2080,8 +2093,8 @@ template <class Key>
 struct HashLds;
 template <>
 struct HashLds<uint64_t> {
-  ull hk[HashCfg<uint64_t>::T];
-  uint32_t hc[HashCfg<uint64_t>::T];
+  alignas(16) ull hk[HashCfg<uint64_t>::T];
+  alignas(16) uint32_t hc[HashCfg<uint64_t>::T];
   __device__ __forceinline__ HashTable<uint64_t> table(ull empty) {
     HashTable<uint64_t> t;
     t.hk = hk;
@@ -2095,7 +2108,7 @@ template <>
 struct HashLds<u128> {
   alignas(16) ull hf[HashCfg<u128>::T];
   ull hh[HashCfg<u128>::T];  // with hf: room for T whole keys in the ordering
-  uint32_t hc[HashCfg<u128>::T];
+  alignas(16) uint32_t hc[HashCfg<u128>::T];
   __device__ __forceinline__ HashTable<u128> table(ull) {
     HashTable<u128> t;
     t.hf = hf;
@@ -2118,8 +2131,10 @@ constexpr int HASH_QUEUE = 1024;
 template <class Key>
 struct HashShared {
   HashLds<Key> lds;
-  alignas(8) uint32_t hs[SUB_BINS];
-  uint32_t nw[BS_NT / 64 + 1];
+  // sub-bin starts of the ordering (and the end of the last); a batch's run map
+  // before
+  alignas(16) uint32_t hs[(1 << HashCfg<Key>::SUB) + 4];
+  uint32_t nw[HashCfg<Key>::NT / 64 + 1];
   int over;
   // u128: keys of the batch queued for their probe chains (place in the batch,
   // then the slot found, 0xFFFF for none)
@@ -2143,23 +2158,31 @@ __device__ __forceinline__ bool wave_map(uint2* mw, int nwords, uint32_t* off, c
   for (int w = lane; w < nwords; w += 64) mw[w].x = 0;
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   uint32_t cnt = 0;
-  for (uint32_t c = 0; c < nt; c += 64) {
-    const uint32_t idx = c + lane;
-    uint32_t vs = 0, ve = 0, so = 0;
-    if (idx < nt) {
-      vs = (uint32_t)(V[idx] - rb.v0);
-      ve = (uint32_t)(V[idx + 1] - rb.v0);
-      so = (uint32_t)tile_place(in, idx) + (M[idx] >> 16) - vs;
+  // four chunks of 64 entries at a time, their loads in flight together
+  for (uint32_t c4 = 0; c4 < nt; c4 += 256) {
+    uint32_t vs[4], ve[4], so[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      const uint32_t idx = c4 + 64 * q + lane;
+      vs[q] = ve[q] = so[q] = 0;
+      if (idx < nt) {
+        vs[q] = (uint32_t)(V[idx] - rb.v0);
+        ve[q] = (uint32_t)(V[idx + 1] - rb.v0);
+        so[q] = (uint32_t)tile_place(in, idx) + (M[idx] >> 16) - vs[q];
+      }
     }
-    const bool part = ve > vs && vs < b + (uint32_t)m && ve > b;
-    const ull bal = __ballot(part);
-    const uint32_t r = cnt + (uint32_t)__popcll(bal & ((1ull << lane) - 1));
-    if (part && r < (uint32_t)RUN_CAP) {
-      off[r] = so + b;
-      const uint32_t ls = vs > b ? vs - b : 0u;
-      atomicOr(&mw[ls >> 5].x, 1u << (ls & 31));
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      const bool part = ve[q] > vs[q] && vs[q] < b + (uint32_t)m && ve[q] > b;
+      const ull bal = __ballot(part);
+      const uint32_t r = cnt + (uint32_t)__popcll(bal & ((1ull << lane) - 1));
+      if (part && r < (uint32_t)RUN_CAP) {
+        off[r] = so[q] + b;
+        const uint32_t ls = vs[q] > b ? vs[q] - b : 0u;
+        atomicOr(&mw[ls >> 5].x, 1u << (ls & 31));
+      }
+      cnt += (uint32_t)__popcll(bal);
     }
-    cnt += (uint32_t)__popcll(bal);
   }
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   // pieces before each word: consecutive words per lane
@@ -2169,13 +2192,7 @@ __device__ __forceinline__ bool wave_map(uint2* mw, int nwords, uint32_t* off, c
     const int w = lane * wpl + i;
     if (w < nwords) sum += (uint32_t)__popc(mw[w].x);
   }
-  uint32_t x = sum;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const uint32_t y = __shfl_up(x, o, 64);
-    if (lane >= o) x += y;
-  }
-  x -= sum;
+  uint32_t x = wave_scan_u32(sum) - sum;
   for (int i = 0; i < wpl; i++) {
     const int w = lane * wpl + i;
     if (w < nwords) {
@@ -2196,8 +2213,10 @@ __device__ __forceinline__ bool wave_map(uint2* mw, int nwords, uint32_t* off, c
 template <class Key, bool RUNS, bool LIGHT, int HB>
 __device__ __forceinline__ int load_batch(HashShared<Key>& L, const Key* Sb, const Runs& in, const RunBucket& rb,
                                           ull b, Key (&kb)[HB]) {
+  constexpr int BS_NT = HashCfg<Key>::NT;
   constexpr int BATCH = BS_NT * HB;
-  static_assert(BATCH / 32 * sizeof(uint2) + RUN_CAP * 4 <= sizeof(L.hs), "the run map fits the sub-bins");
+  static_assert(BATCH % 32 == 0 && BATCH / 32 * sizeof(uint2) + RUN_CAP * 4 <= sizeof(L.hs),
+                "the run map fits the sub-bins");
   if constexpr (!RUNS) {
 #pragma unroll
     for (int j = 0; j < HB; j++) {
@@ -2245,6 +2264,7 @@ __device__ __forceinline__ int load_batch(HashShared<Key>& L, const Key* Sb, con
 template <class Key, bool RUNS, bool MULTI>
 __device__ __forceinline__ int count_task(HashShared<Key>& L, const Key* S, Key* R, int32_t* C, const Runs& in,
                                           const RunBucket& rb, bool top, int K, int fixed, ull* out_n) {
+  constexpr int BS_NT = HashCfg<Key>::NT;
   constexpr int T = HashCfg<Key>::T;
   constexpr int PER = T / BS_NT;  // table slots per thread
   constexpr int HB = HashCfg<Key>::HB;
@@ -2274,7 +2294,7 @@ __device__ __forceinline__ int count_task(HashShared<Key>& L, const Key* S, Key*
       // keys are loaded HB at a time into registers so that the global-load
       // latency is paid once per batch, not once per insert
       Key kb[HB];
-      int ksl[HB];  // u128: the slot each key of the batch landed in
+      int ksl[HB];  // u128: the slot each key of the batch landed in, or -1 - its place in the queue
       bool clash = false;
       // over as read after the last batch's final barrier (nothing writes it
       // between that read and the next barrier): all threads leave together
@@ -2290,24 +2310,25 @@ __device__ __forceinline__ int count_task(HashShared<Key>& L, const Key* S, Key*
           // each of the eight keys of its lane.
           if (threadIdx.x == 0) L.qn = 0;
           __syncthreads();
-          int qp[HB];
 #pragma unroll
           for (int j = 0; j < HB; j++) {
-            qp[j] = -1;
             const int i = (int)threadIdx.x + j * BS_NT;
             if (i < m && mine(kb[j])) {
               const ull f = HashTable<u128>::fp(kb[j]);
-              ksl[j] = f == HashTable<u128>::EMPTY ? -2 : ht.try_home(kb[j], f);
-              if (ksl[j] == -2) {
+              ksl[j] = 0;
+              if (f == HashTable<u128>::EMPTY) {
                 L.over = 1;
-              } else if (ksl[j] < 0) {
-                const int q = atomicAdd(&L.qn, 1);
-                if (q < HASH_QUEUE) {
-                  L.hq[q] = (uint16_t)i;
-                  qp[j] = q;
-                } else {
-                  ksl[j] = ht.insert_after_home(kb[j], f, &L.over);
-                  if (ksl[j] < 0) L.over = 1;
+              } else {
+                ksl[j] = ht.try_home(kb[j], f);
+                if (ksl[j] < 0) {
+                  const int q = atomicAdd(&L.qn, 1);
+                  if (q < HASH_QUEUE) {
+                    L.hq[q] = (uint16_t)i;
+                    ksl[j] = -1 - q;
+                  } else {
+                    ksl[j] = ht.insert_after_home(kb[j], f, &L.over);
+                    if (ksl[j] < 0) L.over = 1;
+                  }
                 }
               }
             }
@@ -2331,9 +2352,11 @@ __device__ __forceinline__ int count_task(HashShared<Key>& L, const Key* S, Key*
           if (!ov) {
 #pragma unroll
             for (int j = 0; j < HB; j++) {
-              if (qp[j] >= 0) ksl[j] = (int)L.hq[qp[j]];
               const int i = (int)threadIdx.x + j * BS_NT;
-              if (i < m && mine(kb[j]) && !ht.verify(ksl[j], kb[j])) clash = true;
+              if (i < m && mine(kb[j])) {
+                const int sl = ksl[j] < 0 ? (int)L.hq[-1 - ksl[j]] : ksl[j];
+                if (!ht.verify(sl, kb[j])) clash = true;
+              }
             }
           }
         } else {
@@ -2358,43 +2381,61 @@ __device__ __forceinline__ int count_task(HashShared<Key>& L, const Key* S, Key*
       __syncthreads();
       if (fail) break;
       // order the distinct keys: counting sort by the sub-digit below the
-      // pass bits, then rank inside each sub-bin (1-2 keys on average)
+      // pass bits, then rank inside each sub-bin (one key on average)
+      constexpr int SUB = HashCfg<Key>::SUB;
       const int r2 = rem - s;
-      const int dbits = r2 < SUB_MAX_BITS ? r2 : SUB_MAX_BITS;
+      const int dbits = r2 < SUB ? r2 : SUB;
       const int dpos = r2 - dbits;
-      const int nbins = 1 << dbits;
-      Key rk[PER];
-      uint32_t rc[PER], ri[PER];  // ri: index of the key inside its sub-bin
-      ull ndk;  // distinct keys of the pass
-      for (int i = threadIdx.x; i < nbins; i += BS_NT) hs[i] = 0;
+      const uint32_t dm = (1u << dbits) - 1u;
+      auto sub_bin = [&](Key k) -> uint32_t {
+        if constexpr (sizeof(Key) == 8) return (uint32_t)(k >> dpos) & dm;
+        else return key_digit<Key>(k, dpos, dbits);
+      };
+      for (int i = threadIdx.x; i < (1 << SUB) / 4; i += BS_NT)
+        reinterpret_cast<uint4*>(hs)[i] = make_uint4(0u, 0u, 0u, 0u);
       __syncthreads();
+      Key rk[PER];
+      uint32_t rc[PER], rd[PER];  // rd: sub-bin, index of the key inside it << 16
 #pragma unroll
       for (int j = 0; j < PER; j++) {
-        const int slot = threadIdx.x * PER + j;
+        const int slot = threadIdx.x + j * BS_NT;
         rc[j] = L.lds.hc[slot];
-        rk[j] = rc[j] ? ht.key(slot) : Key(0);
-        ri[j] = rc[j] ? atomicAdd(&hs[key_digit<Key>(rk[j], dpos, dbits)], 1u) : 0u;
+        if (rc[j]) {
+          rk[j] = ht.key(slot);
+          const uint32_t d = sub_bin(rk[j]);
+          rd[j] = d | atomicAdd(&hs[d], 1u) << 16;
+        }
       }
       __syncthreads();
+      uint32_t nd;  // distinct keys of the pass
       {
-        constexpr int BPT = SUB_BINS / BS_NT;
+        constexpr int BPT = (1 << SUB) / BS_NT;
+        static_assert(BPT == 2 || BPT == 4, "bins per thread as one vector");
         uint32_t v[BPT];
-        ull sm = 0;
+        if constexpr (BPT == 4) {
+          const uint4 q = reinterpret_cast<const uint4*>(hs)[threadIdx.x];
+          v[0] = q.x;
+          v[1] = q.y;
+          v[2] = q.z;
+          v[3] = q.w;
+        } else {
+          const uint2 q = reinterpret_cast<const uint2*>(hs)[threadIdx.x];
+          v[0] = q.x;
+          v[1] = q.y;
+        }
+        uint32_t sm = 0;
 #pragma unroll
         for (int i = 0; i < BPT; i++) {
-          const int bb = threadIdx.x * BPT + i;
-          v[i] = bb < nbins ? hs[bb] : 0u;
-          sm += v[i];
+          const uint32_t t = v[i];
+          v[i] = sm;
+          sm += t;
         }
-        ull ex = block_scan_total<BS_NT>(sm, &ndk);
-#pragma unroll
-        for (int i = 0; i < BPT; i++) {
-          const int bb = threadIdx.x * BPT + i;
-          if (bb < nbins) {
-            hs[bb] = (uint32_t)ex;
-            ex += v[i];
-          }
-        }
+        const uint32_t ex = block_scan_u32<BS_NT>(sm, L.nw, &nd);
+        if constexpr (BPT == 4)
+          reinterpret_cast<uint4*>(hs)[threadIdx.x] = make_uint4(ex, ex + v[1], ex + v[2], ex + v[3]);
+        else
+          reinterpret_cast<uint2*>(hs)[threadIdx.x] = make_uint2(ex, ex + v[1]);
+        if (threadIdx.x == 0) hs[1 << SUB] = nd;
       }
       __syncthreads();
       Key* ok = L.lds.out_keys();
@@ -2402,31 +2443,29 @@ __device__ __forceinline__ int count_task(HashShared<Key>& L, const Key* S, Key*
 #pragma unroll
       for (int j = 0; j < PER; j++) {
         if (rc[j]) {
-          const uint32_t pos = hs[key_digit<Key>(rk[j], dpos, dbits)] + ri[j];
+          const uint32_t pos = hs[rd[j] & 0xFFFFu] + (rd[j] >> 16);
           ok[pos] = rk[j];
           oc[pos] = rc[j];
         }
       }
       __syncthreads();
-      const uint32_t nd = (uint32_t)ndk;
-      Key* Ro = R + start + out;
-      int32_t* Co = C + start + out;
+      char* Ro = reinterpret_cast<char*>(R + start + out);
+      char* Co = reinterpret_cast<char*>(C + start + out);
       for (uint32_t i = threadIdx.x; i < nd; i += BS_NT) {
         const Key v = ok[i];
-        const int d = (int)key_digit<Key>(v, dpos, dbits);
-        // the sub-bin's slots: from its start to the next one's
-        const int a = (int)hs[d];
-        const int e = d + 1 < nbins ? (int)hs[d + 1] : (int)nd;
-        // the sub-bin's first four slots read at once (most hold one or two
-        // keys), the rest of a longer sub-bin one by one.  a < nd <= T, so a
-        // read past the key array lands in the counts that follow it in the
-        // same LDS struct, and only slots below e count.
-        const Key w0 = ok[a], w1 = ok[a + 1], w2 = ok[a + 2], w3 = ok[a + 3];
-        int rank = (int)(w0 < v) + (int)(a + 1 < e && w1 < v) + (int)(a + 2 < e && w2 < v) +
-                   (int)(a + 3 < e && w3 < v);
-        for (int j = a + 4; j < e; j++) rank += ok[j] < v;
-        Ro[a + rank] = v;
-        Co[a + rank] = (int32_t)oc[i];
+        const uint32_t d = sub_bin(v);
+        // the sub-bin's slots: from its start to the next one's (the bins past
+        // dm start at nd)
+        const uint32_t a = hs[d], e = hs[d + 1];
+        // the sub-bin's first three slots read at once (most hold one key),
+        // the rest of a longer one one by one.  a < nd <= T, so a read past
+        // the key array lands in the counts that follow it in the same LDS
+        // struct, and only slots below e count.
+        const Key w0 = ok[a], w1 = ok[a + 1], w2 = ok[a + 2];
+        uint32_t p = a + (uint32_t)(w0 < v) + (uint32_t)(a + 1 < e && w1 < v) + (uint32_t)(a + 2 < e && w2 < v);
+        for (uint32_t j = a + 3; j < e; j++) p += ok[j] < v;
+        *reinterpret_cast<Key*>(Ro + p * (uint32_t)sizeof(Key)) = v;
+        *reinterpret_cast<int32_t*>(Co + p * 4u) = (int32_t)oc[i];
       }
       out += nd;
       __syncthreads();
@@ -2439,11 +2478,21 @@ __device__ __forceinline__ int count_task(HashShared<Key>& L, const Key* S, Key*
   return fail;
 }
 
+// What bounds it: issue.  Per one-word key (2.5e8 keys, 7.7e7 distinct) 115 VALU
+// and 20 LDS lane instructions; inserts overlap with the loads of other
+// blocks, the ordering of the distinct keys is half the kernel (timing
+// copies: loads alone 0.49 of 1.5 ms, with inserts 0.57).  Sub-bins of about
+// one key, vector clears, a DPP scan and one packed register for (bin, index)
+// took it from 1.51 to 1.34 ms; tables of 256 or 1024 threads and of 2048 to
+// 6144 slots were within 10 % of each other.  Two-word keys (1.5e8): 2.83 ms
+// with 28-byte slots in 1024-slot tables that overflow at 0.4 distinct keys
+// per key, 1.41 ms now.
+//
 // One block per bucket of `in`: tu[b] = the bucket's distinct keys, bstart[b]
 // = where they are.  Buckets the table is too small for go to the retry list
 // (a single pass needs fewer registers).
 template <class Key, bool RUNS>
-__global__ __launch_bounds__(BS_NT, HashCfg<Key>::WAVES) void k_bucket_hash(const Key* S, Key* R, int32_t* C,
+__global__ __launch_bounds__(HashCfg<Key>::NT, HashCfg<Key>::WAVES) void k_bucket_hash(const Key* S, Key* R, int32_t* C,
                                                                             Runs in, int K, int fixed, long long* tu,
                                                                             ull* bstart, ull* retry_count,
                                                                             ull* retry_list) {
@@ -2468,7 +2517,7 @@ __global__ __launch_bounds__(BS_NT, HashCfg<Key>::WAVES) void k_bucket_hash(cons
 // The buckets of the retry list in several passes; what still fails goes to
 // ovf_list with tu = -1 for the host-driven split.
 template <class Key, bool RUNS>
-__global__ __launch_bounds__(BS_NT) void k_bucket_retry(const Key* S, Key* R, int32_t* C, Runs in, int K, int fixed,
+__global__ __launch_bounds__(HashCfg<Key>::NT) void k_bucket_retry(const Key* S, Key* R, int32_t* C, Runs in, int K, int fixed,
                                                         long long* tu, const ull* retry_count, const ull* retry_list,
                                                         ull* ovf_count, ull* ovf_list) {
   __shared__ HashShared<Key> L;
@@ -2489,7 +2538,7 @@ __global__ __launch_bounds__(BS_NT) void k_bucket_retry(const Key* S, Key* R, in
 
 // Tasks of the split path: [tstart[i], tstart[i] + tcount[i]) of S.
 template <class Key>
-__global__ __launch_bounds__(BS_NT) void k_task_hash(const Key* S, Key* R, int32_t* C, const ull* tstart,
+__global__ __launch_bounds__(HashCfg<Key>::NT) void k_task_hash(const Key* S, Key* R, int32_t* C, const ull* tstart,
                                                      const ull* tcount, int K, int fixed, long long* tu) {
   __shared__ HashShared<Key> L;
   const ull task = blockIdx.x;
@@ -3589,7 +3638,7 @@ int resolve_overflow(pk_ctx* c, Key* S, Key* T, Key* R, int32_t* C, int K, int f
   su = reinterpret_cast<long long*>(ss + 2 * ns);
   PK_HIP(c, hipMemcpyAsync(ss, sub_start.data(), ns * 8, hipMemcpyHostToDevice, c->stream));
   PK_HIP(c, hipMemcpyAsync(sc, sub_count.data(), ns * 8, hipMemcpyHostToDevice, c->stream));
-  hipLaunchKernelGGL(HIP_KERNEL_NAME(k_task_hash<Key>), dim3((unsigned)ns), dim3(BS_NT), 0, c->stream, S, R, C, ss,
+  hipLaunchKernelGGL(HIP_KERNEL_NAME(k_task_hash<Key>), dim3((unsigned)ns), dim3(HashCfg<Key>::NT), 0, c->stream, S, R, C, ss,
                      sc, K, fixed2, su);
   PK_HIP(c, hipGetLastError());
   std::vector<long long> hu(ns);
@@ -3968,12 +4017,10 @@ int level_runs(pk_ctx* c, const LevelBufs& l, uint64_t tiles, int db, int tk, Ru
 
 // Bits of the next level when `left` remain: as few levels as possible, the
 // bits spread evenly.  A level reads and writes every key once, so one level
-// less beats longer runs until a run is down to about a line: 9 bits leave 32
-// one-word (16 two-word) keys per run of a full tile.
-constexpr int SP_LEVEL_BITS = 9;
-
+// less beats longer runs until a run is down to about a line: 10 bits leave 16
+// one-word (8 two-word) keys per run of a full tile.
 int level_bits(int left) {
-  const int nlev = (left + SP_LEVEL_BITS - 1) / SP_LEVEL_BITS;
+  const int nlev = (left + SP_MAX_BITS - 1) / SP_MAX_BITS;
   return (left + nlev - 1) / nlev;
 }
 
@@ -4031,16 +4078,16 @@ int count_partitioned(pk_ctx* c, Key* S, Key* S2, int32_t* C, Part p, int btot, 
   PK_HIP(c, hipEventRecord(c->ev[6], st));
   const unsigned rgrid = (unsigned)std::min<uint64_t>(B, 4ull * (uint64_t)c->ncu);
   if (in.M) {
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_bucket_hash<Key, true>), dim3((unsigned)B), dim3(BS_NT), 0, st, S, Res, C,
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_bucket_hash<Key, true>), dim3((unsigned)B), dim3(HashCfg<Key>::NT), 0, st, S, Res, C,
                        in, KB / 2, btot, tu, bstart, small + 5, retry);
     PK_HIP(c, hipGetLastError());
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_bucket_retry<Key, true>), dim3(rgrid), dim3(BS_NT), 0, st, S, Res, C, in,
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_bucket_retry<Key, true>), dim3(rgrid), dim3(HashCfg<Key>::NT), 0, st, S, Res, C, in,
                        KB / 2, btot, tu, small + 5, retry, small + 4, ovl);
   } else {
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_bucket_hash<Key, false>), dim3((unsigned)B), dim3(BS_NT), 0, st, S, Res, C,
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_bucket_hash<Key, false>), dim3((unsigned)B), dim3(HashCfg<Key>::NT), 0, st, S, Res, C,
                        in, KB / 2, btot, tu, bstart, small + 5, retry);
     PK_HIP(c, hipGetLastError());
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_bucket_retry<Key, false>), dim3(rgrid), dim3(BS_NT), 0, st, S, Res, C, in,
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_bucket_retry<Key, false>), dim3(rgrid), dim3(HashCfg<Key>::NT), 0, st, S, Res, C, in,
                        KB / 2, btot, tu, small + 5, retry, small + 4, ovl);
   }
   PK_HIP(c, hipGetLastError());
@@ -4176,7 +4223,7 @@ int count_records(pk_ctx* c, const Records& rec, int K, int KB, Key mask) {
   PK_TRY(begin_count<Key>(c, rec.R, N, K, &empty));
   if (empty) return PK_OK;
   const pk_tuning& tun = c->tuning;
-  const float bf = tun.bucket_factor > 0.f ? tun.bucket_factor : 3.0f;
+  const float bf = tun.bucket_factor > 0.f ? tun.bucket_factor : HashCfg<Key>::FILL;
   const int btot = choose_bits(N, KB / 2, CAP, bf);
   c->timing.bucket_bits = btot;
   Key *S, *S2;
@@ -4255,7 +4302,7 @@ int count_share(pk_ctx* c, const uint8_t* fa, uint64_t n, const Records& rec, in
   PK_TRY(begin_count<Key>(c, R, N, K, &empty));
   if (empty) return PK_OK;
   const pk_tuning& tun = c->tuning;
-  const float bf = tun.bucket_factor > 0.f ? tun.bucket_factor : 3.0f;
+  const float bf = tun.bucket_factor > 0.f ? tun.bucket_factor : HashCfg<Key>::FILL;
   // with owner routing, about N / P instances are this rank's
   const int btot = choose_bits((N + cf.P - 1) / cf.P, K, CAP, bf);
   c->timing.bucket_bits = btot;
@@ -4335,7 +4382,7 @@ int windows_count_impl(pk_ctx* c, const uint8_t* fa, const ull* rstart, const ui
   PK_HIP(c, hipGetLastError());
   PK_HIP(c, hipEventRecord(c->ev[4], st));
   PK_HIP(c, hipEventRecord(c->ev[16], st));
-  const float bf = c->tuning.bucket_factor > 0.f ? c->tuning.bucket_factor : 3.0f;
+  const float bf = c->tuning.bucket_factor > 0.f ? c->tuning.bucket_factor : HashCfg<Key>::FILL;
   const int btot = choose_bits(N, KB / 2, HashCfg<Key>::LIMIT, bf);
   c->timing.bucket_bits = btot;
   return count_partitioned<Key>(c, S, S2, C, Part{Runs{nullptr, nullptr, nullptr, boff, 0, 0, nullptr, 0}, 1, 0, 0}, btot, KB, N);
