@@ -37,7 +37,7 @@
 //   stream compaction (kmer_histogram.cpp:84-140).
 // pk_macro_nodes: range-partitioned 5-way merge of the kept table seen as
 //   pred keys (ascending) and, per first base a, succ keys (ascending within
-//   the quarter) -- no sort is needed (mn_construct.cpp:212-477).
+//   the quarter): ranges ranked in LDS, then written (mn_construct.cpp:212-477).
 
 #include <hip/hip_runtime.h>
 
@@ -2824,82 +2824,281 @@ __global__ __launch_bounds__(CUT_NT) void k_kept_write(const Key* TK, const int3
 // Macro nodes (mn_construct.cpp:212-477).
 //
 // The kept table KK[0..V) is ascending.  pred(x) = x >> 2 is non-decreasing
-// over it; within quarter a (first base a, indices [q[a], q[a+1])) succ(x) =
-// x & SUCC_MASK is ascending.  Node keys are the union of these five sorted
-// lists.  Range g covers node keys [s_g, s_{g+1}) with s_g = pred(KK[g*PC]).
+// over it; within quarter a (first base a) succ(x) = x without its first base
+// is ascending.  Node keys are the union of these five sorted lists (list 0:
+// pred, lists 1..4: succ of the quarters), so every kept k-mer is one element
+// of list 0 and one of its quarter's.
+//
+// Ranges of node keys go to blocks: range g starts at the node key of list
+// 0's element g * MN_PC, and k_mn_bounds finds where it starts in each list.
+// k_mn_rank puts a range's elements into sub-bins of its key span (a monotone
+// map, about one node per bin), finds which element of equal ones comes first
+// and ranks the nodes inside each bin; it stores every element's rank and the
+// range's node count.  After the scan of the counts k_mn_write assembles each
+// range's records in LDS at their ranks and stores them densely (4.6 Mbp, k =
+// 32, 9.2e6 nodes, against a five-way merge by binary searches and a copy: 730
+// -> 330 us, 12 + 162 + 152
+// for the three kernels; k_mn_write moves 0.22 + 0.44 GB, 4.3 TB/s, k_mn_rank is
+// bound by its chain of LDS phases).
 
 constexpr int MN_NT = 512;
-// 768 pred entries per range keep a u64 block at 36 KB of LDS, four blocks
-// of 512 threads per CU (1024 / 3072 allowed three: 0.88 -> 0.82 ms for the
-// bacterial nodes)
-constexpr int MN_PC = 768;     // pred entries per range
-constexpr int MN_ECAP = 2304;  // LDS capacity (entries of all five lists)
-
-struct MnPlan {
-  ull lo[5];
-  ull hi[5];
-  ull base;
-  ull e;
-};
+constexpr int MN_PC = 640;     // pred elements per range
+constexpr int MN_PER = 3;      // elements per thread of a sub-range
+constexpr int MN_CAP = MN_NT * MN_PER;
+constexpr int MN_STEP = 256;   // elements per list of a sub-range that was cut down
+constexpr int MN_BIN_BITS = 10;
+constexpr int MN_BINS = 1 << MN_BIN_BITS;
+constexpr int MN_ROUND = 640;  // records assembled at a time
+static_assert(5 * MN_STEP <= MN_CAP, "a cut sub-range fits");
+static_assert(MN_BINS == 2 * MN_NT, "two bins per thread");
 
 template <class Key>
 __device__ __forceinline__ Key mn_pred(Key x) { return x >> 2; }
 
+// node key of element i of list l
 template <class Key>
-__global__ void k_mn_quarters(const Key* KK, uint64_t V, int K, ull* q) {
-  if (threadIdx.x >= 5 || blockIdx.x) return;
-  const int a = threadIdx.x;
-  if (a == 0) { q[0] = 0; return; }
-  if (a == 4) { q[4] = V; return; }
-  const Key lim = Key(a) << (2 * K - 2);
-  uint64_t lo = 0, hi = V;
-  while (lo < hi) {
-    uint64_t mid = (lo + hi) >> 1;
-    if (KK[mid] < lim) lo = mid + 1; else hi = mid;
-  }
-  q[a] = lo;
+__device__ __forceinline__ Key mn_key(const Key* KK, int l, ull i, Key msk) {
+  const Key x = KK[i];
+  return l == 0 ? mn_pred(x) : (x & msk);
 }
 
 template <class Key>
-__device__ __forceinline__ uint64_t lb_pred(const Key* KK, uint64_t lo, uint64_t hi, Key x) {
+__device__ __forceinline__ ull mn_lower(const Key* KK, ull lo, ull hi, Key x) {
   while (lo < hi) {
-    uint64_t mid = (lo + hi) >> 1;
-    if (mn_pred(KK[mid]) < x) lo = mid + 1; else hi = mid;
-  }
-  return lo;
-}
-template <class Key>
-__device__ __forceinline__ uint64_t lb_succ(const Key* KK, uint64_t lo, uint64_t hi, Key x, Key m) {
-  while (lo < hi) {
-    uint64_t mid = (lo + hi) >> 1;
-    if ((KK[mid] & m) < x) lo = mid + 1; else hi = mid;
+    const ull mid = (lo + hi) >> 1;
+    if (KK[mid] < x) lo = mid + 1; else hi = mid;
   }
   return lo;
 }
 
+// bd[l * (G + 1) + g] = where range g starts in list l (as an index of KK);
+// one search per thread.
 template <class Key>
-__global__ void k_mn_plan(const Key* KK, uint64_t V, int K, const ull* q, uint64_t G, MnPlan* plan,
-                          ull* maxe) {
-  const uint64_t g = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (g >= G) return;
+__global__ __launch_bounds__(256) void k_mn_bounds(const Key* KK, ull V, int K, ull G, ull* bd) {
+  const ull t = (ull)blockIdx.x * 256 + threadIdx.x;
+  if (t >= 5 * (G + 1)) return;
+  const int l = (int)(t / (G + 1));
+  const ull g = t - (ull)l * (G + 1);
+  ull r;
+  if (l == 0) {
+    r = g == G ? V : g * MN_PC;
+    if (g > 0 && g < G) {
+      // the first of the (up to four) elements of this node
+      const Key s = mn_pred(KK[r]);
+      while (r > 0 && mn_pred(KK[r - 1]) == s) r--;
+    }
+  } else if (g == G) {
+    r = l == 4 ? V : mn_lower<Key>(KK, 0, V, Key(l) << (2 * K - 2));
+  } else {
+    const Key s = g == 0 ? Key(0) : mn_pred(KK[g * MN_PC]);
+    r = mn_lower<Key>(KK, 0, V, (Key(l - 1) << (2 * K - 2)) | s);
+  }
+  bd[t] = r;
+}
+
+// The sub-ranges of a block's range, in key order: [lo[l], hi[l]) of the five
+// lists, at most MN_CAP elements each; a range that fits is one sub-range.
+struct MnSub {
+  ull lo[5], hi[5], end[5];
+};
+
+// Advances to the next sub-range; false when there is none.  Called by the
+// whole block with the same m; sh: five words of LDS.
+template <class Key>
+__device__ __forceinline__ bool mn_next(const Key* KK, Key msk, MnSub& m, ull* sh) {
+  ull e = 0;
+#pragma unroll
+  for (int l = 0; l < 5; l++) {
+    m.lo[l] = m.hi[l];
+    e += m.end[l] - m.lo[l];
+  }
+  if (e == 0) return false;
+  if (e <= (ull)MN_CAP) {
+#pragma unroll
+    for (int l = 0; l < 5; l++) m.hi[l] = m.end[l];
+    return true;
+  }
+  // too many: up to the smallest of the keys MN_STEP further in the lists that
+  // have more (at most MN_STEP elements of each list lie below it, and at
+  // least MN_STEP - 3 of the list it comes from)
+  Key cut = ~Key(0);
+#pragma unroll
+  for (int l = 0; l < 5; l++) {
+    if (m.end[l] - m.lo[l] > (ull)MN_STEP) {
+      const Key x = mn_key<Key>(KK, l, m.lo[l] + MN_STEP, msk);
+      cut = x < cut ? x : cut;
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int l = 0; l < 5; l++) {
+    if ((int)threadIdx.x == l) {
+      ull a = m.lo[l], b = m.end[l] - a > (ull)MN_STEP ? a + MN_STEP : m.end[l];
+      while (a < b) {
+        const ull mid = (a + b) >> 1;
+        if (mn_key<Key>(KK, l, mid, msk) < cut) a = mid + 1; else b = mid;
+      }
+      sh[l] = a;
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int l = 0; l < 5; l++) m.hi[l] = uniform(sh[l]);
+  return true;
+}
+
+__device__ __forceinline__ MnSub mn_range(const ull* bd, ull G, ull g) {
+  MnSub m;
+#pragma unroll
+  for (int l = 0; l < 5; l++) {
+    m.lo[l] = m.hi[l] = uniform(bd[(ull)l * (G + 1) + g]);
+    m.end[l] = uniform(bd[(ull)l * (G + 1) + g + 1]);
+  }
+  return m;
+}
+
+// Element e of a sub-range: its list and index of KK.
+__device__ __forceinline__ void mn_element(const MnSub& m, uint32_t e, int& l, ull& i) {
+  l = 0;
+  uint32_t o = e, n = (uint32_t)(m.hi[0] - m.lo[0]);
+  ull lo = m.lo[0];
+#pragma unroll
+  for (int q = 1; q < 5; q++) {
+    if (l == q - 1 && o >= n) {
+      o -= n;
+      n = (uint32_t)(m.hi[q] - m.lo[q]);
+      lo = m.lo[q];
+      l = q;
+    }
+  }
+  i = lo + o;
+}
+
+__device__ __forceinline__ uint32_t mn_size(const MnSub& m) {
+  uint32_t e = 0;
+#pragma unroll
+  for (int l = 0; l < 5; l++) e += (uint32_t)(m.hi[l] - m.lo[l]);
+  return e;
+}
+
+template <class Key>
+__device__ __forceinline__ int bit_length(Key x) {
+  if (sizeof(Key) == 16) {
+    const ull hi = (ull)((u128)x >> 64);
+    return hi ? 128 - __clzll((long long)hi) : 64 - __clzll((long long)(ull)x);
+  }
+  return 64 - __clzll((long long)(ull)x);
+}
+
+// Ranks: rkp[i] / rks[i] = place of KK[i]'s pred / succ node among its
+// sub-range's nodes; ng[g] = nodes of range g.
+template <class Key>
+__global__ __launch_bounds__(MN_NT, 8) void k_mn_rank(const Key* KK, int K, const ull* bd, ull G, uint16_t* rkp,
+                                                      uint16_t* rks, ull* ng) {
+  __shared__ Key ok[MN_CAP];          // node keys, by bin
+  __shared__ __align__(8) uint32_t h[MN_BINS + 1];  // elements per bin, then starts
+  __shared__ __align__(8) uint32_t hd[MN_BINS];     // nodes per bin, then starts
+  __shared__ uint8_t lead[MN_CAP];     // first of its equals
+  __shared__ Key ext[10];
+  __shared__ uint32_t nw[MN_NT / 64 + 1];
+  __shared__ ull sh[5];
+  const ull g = blockIdx.x;
   const Key msk = key_mask<Key>(2 * (K - 1));
-  const bool first = g == 0, last = g + 1 == G;
-  const Key s_lo = first ? Key(0) : mn_pred(KK[g * MN_PC]);
-  const Key s_hi = last ? Key(0) : mn_pred(KK[(g + 1) * MN_PC]);
-  MnPlan p;
-  p.lo[0] = first ? 0 : lb_pred(KK, 0, V, s_lo);
-  p.hi[0] = last ? V : lb_pred(KK, 0, V, s_hi);
-  ull base = p.lo[0], e = p.hi[0] - p.lo[0];
-  for (int a = 0; a < 4; a++) {
-    p.lo[a + 1] = first ? q[a] : lb_succ(KK, q[a], q[a + 1], s_lo, msk);
-    p.hi[a + 1] = last ? q[a + 1] : lb_succ(KK, q[a], q[a + 1], s_hi, msk);
-    base += p.lo[a + 1] - q[a];
-    e += p.hi[a + 1] - p.lo[a + 1];
+  const int tid = (int)threadIdx.x;
+  MnSub m = mn_range(bd, G, g);
+  ull nodes = 0;
+  while (mn_next<Key>(KK, msk, m, sh)) {
+    const uint32_t E = mn_size(m);
+    Key x[MN_PER];
+    int l[MN_PER];
+    ull idx[MN_PER];
+#pragma unroll
+    for (int j = 0; j < MN_PER; j++) {
+      const uint32_t e = (uint32_t)(tid + j * MN_NT);
+      l[j] = 0;
+      idx[j] = 0;
+      x[j] = Key(0);
+      if (e < E) {
+        mn_element(m, e, l[j], idx[j]);
+        x[j] = mn_key<Key>(KK, l[j], idx[j], msk);
+      }
+    }
+    // the key span
+#pragma unroll
+    for (int q = 0; q < 5; q++) {
+      if (tid == q) {
+        const bool any = m.hi[q] > m.lo[q];
+        ext[q] = any ? mn_key<Key>(KK, q, m.lo[q], msk) : ~Key(0);
+        ext[5 + q] = any ? mn_key<Key>(KK, q, m.hi[q] - 1, msk) : Key(0);
+      }
+    }
+    reinterpret_cast<uint2*>(h)[tid] = make_uint2(0u, 0u);
+    reinterpret_cast<uint2*>(hd)[tid] = make_uint2(0u, 0u);
+    __syncthreads();
+    Key lo = ext[0], hi = ext[5];
+#pragma unroll
+    for (int q = 1; q < 5; q++) {
+      lo = ext[q] < lo ? ext[q] : lo;
+      hi = ext[5 + q] > hi ? ext[5 + q] : hi;
+    }
+    const int bl = bit_length<Key>(hi - lo);
+    const int shift = bl > MN_BIN_BITS ? bl - MN_BIN_BITS : 0;
+    uint32_t d[MN_PER], pos[MN_PER];
+#pragma unroll
+    for (int j = 0; j < MN_PER; j++) {
+      d[j] = 0;
+      pos[j] = 0;
+      if ((uint32_t)(tid + j * MN_NT) < E) {
+        d[j] = (uint32_t)((x[j] - lo) >> shift);
+        pos[j] = atomicAdd(&h[d[j]], 1u);
+      }
+    }
+    __syncthreads();
+    uint32_t tot;
+    {
+      const uint2 c = reinterpret_cast<const uint2*>(h)[tid];
+      const uint32_t ex = block_scan_u32<MN_NT>(c.x + c.y, nw, &tot);
+      reinterpret_cast<uint2*>(h)[tid] = make_uint2(ex, ex + c.x);
+      if (tid == 0) h[MN_BINS] = E;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < MN_PER; j++) {
+      if ((uint32_t)(tid + j * MN_NT) < E) {
+        pos[j] += h[d[j]];
+        ok[pos[j]] = x[j];
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < MN_PER; j++) {
+      if ((uint32_t)(tid + j * MN_NT) < E) {
+        bool first = true;
+        for (uint32_t q = h[d[j]]; q < pos[j]; q++) first = first && ok[q] != x[j];
+        lead[pos[j]] = first ? 1 : 0;
+        if (first) atomicAdd(&hd[d[j]], 1u);
+      }
+    }
+    __syncthreads();
+    {
+      const uint2 c = reinterpret_cast<const uint2*>(hd)[tid];
+      const uint32_t ex = block_scan_u32<MN_NT>(c.x + c.y, nw, &tot);
+      reinterpret_cast<uint2*>(hd)[tid] = make_uint2(ex, ex + c.x);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < MN_PER; j++) {
+      if ((uint32_t)(tid + j * MN_NT) < E) {
+        uint32_t r = hd[d[j]];
+        const uint32_t e = h[d[j] + 1];
+        for (uint32_t q = h[d[j]]; q < e; q++) r += (uint32_t)(lead[q] && ok[q] < x[j]);
+        (l[j] == 0 ? rkp : rks)[idx[j]] = (uint16_t)r;
+      }
+    }
+    nodes += tot;
+    __syncthreads();
   }
-  p.base = base;
-  p.e = e;
-  plan[g] = p;
-  atomicMax(maxe, e);
+  if (tid == 0) ng[g] = nodes;
 }
 
 // Node record as written to memory (matches pk_mnode).
@@ -2909,297 +3108,74 @@ struct MnRec {
   int32_t suf[4];
 };
 
+static_assert(sizeof(MnRec) == 48, "three 16-byte words");
+
+// Records of range g at out + noff[g], from the elements' ranks.
 template <class Key>
-__device__ __forceinline__ void set_key(MnRec& r, Key k);
-template <>
-__device__ __forceinline__ void set_key<uint64_t>(MnRec& r, uint64_t k) {
-  r.key_lo = k;
-  r.key_hi = 0;
-}
-template <>
-__device__ __forceinline__ void set_key<u128>(MnRec& r, u128 k) {
-  r.key_lo = (ull)k;
-  r.key_hi = (ull)(k >> 64);
-}
-
-// List view: 5 sorted lists of node keys, either staged in LDS (lk) or
-// read from KK through pred/succ.  List 0 = pred keys (may repeat, up to 4
-// equal), lists 1..4 = succ keys of quarter a = l - 1 (no repeats).
-template <class Key, bool GLOBAL>
-struct MnLists {
-  const Key* KK;
-  Key msk;
-  const Key* lk;  // LDS copy (GLOBAL == false)
-  ull off[5];     // list start (index into lk, or into KK)
-  ull len[5];
-  __device__ __forceinline__ Key at(ull off_l, bool pred, ull i) const {
-    if (GLOBAL) {
-      const Key x = KK[off_l + i];
-      return pred ? mn_pred(x) : (x & msk);
-    }
-    return lk[off_l + i];
-  }
-};
-
-template <class Key, bool GLOBAL>
-__device__ __forceinline__ ull mn_lb(const MnLists<Key, GLOBAL>& L, ull o, ull n, bool pred, Key x) {
-  ull lo = 0, hi = n;
-  while (lo < hi) {
-    const ull mid = (lo + hi) >> 1;
-    if (L.at(o, pred, mid) < x) lo = mid + 1; else hi = mid;
-  }
-  return lo;
-}
-template <class Key, bool GLOBAL>
-__device__ __forceinline__ ull mn_ub(const MnLists<Key, GLOBAL>& L, ull o, ull n, bool pred, Key x) {
-  ull lo = 0, hi = n;
-  while (lo < hi) {
-    const ull mid = (lo + hi) >> 1;
-    if (L.at(o, pred, mid) <= x) lo = mid + 1; else hi = mid;
-  }
-  return lo;
-}
-
-// Positions of x in all five lists, walked forward from the previous
-// element's positions (x never decreases along a thread's chunk of one list).
-template <class Key, bool GLOBAL>
-struct MnCursor {
-  ull lb[5], ub[5];
-  __device__ __forceinline__ void seek(const MnLists<Key, GLOBAL>& L, Key x) {
-#pragma unroll
-    for (int o = 0; o < 5; o++) {
-      lb[o] = mn_lb<Key, GLOBAL>(L, L.off[o], L.len[o], o == 0, x);
-      ub[o] = lb[o];
-      while (ub[o] < L.len[o] && L.at(L.off[o], o == 0, ub[o]) <= x) ub[o]++;
-    }
-  }
-  __device__ __forceinline__ void advance(const MnLists<Key, GLOBAL>& L, Key x) {
-#pragma unroll
-    for (int o = 0; o < 5; o++) {
-      while (lb[o] < L.len[o] && L.at(L.off[o], o == 0, lb[o]) < x) lb[o]++;
-      if (ub[o] < lb[o]) ub[o] = lb[o];
-      while (ub[o] < L.len[o] && L.at(L.off[o], o == 0, ub[o]) <= x) ub[o]++;
-    }
-  }
-};
-
-// LDS ranges (GLOBAL == false) use the launch's dynamic LDS: the range's
-// five lists (node keys) | per rank: start bit 31, list << 16 | index |
-// per node: rank of its first element.
-template <class Key>
-constexpr size_t mn_lds_bytes() {
-  return MN_ECAP * (sizeof(Key) + 2 * sizeof(uint32_t));
-}
-
-// One block per range.  GLOBAL == false: ranges with e <= MN_ECAP, lists in
-// LDS.  GLOBAL == true: the remaining ranges, lists and rank flags in global
-// memory (gflags, indexed from plan.base).  Each thread handles a contiguous
-// chunk of the concatenated lists and walks its positions in the other lists
-// (pass 1: rank of every element in the merged order and whether it starts
-// a node); pass 2 numbers the nodes; pass 3 writes the records.
-template <class Key, bool GLOBAL>
-__global__ __launch_bounds__(MN_NT) void k_mn_build(const Key* KK, const int32_t* KC, int K,
-                                                    const MnPlan* plan, uint64_t G, MnRec* NT,
-                                                    ull* ng, uint32_t* gflags) {
-  extern __shared__ __align__(16) unsigned char mn_smem[];
-  Key* lk = reinterpret_cast<Key*>(mn_smem);
-  uint32_t* lflag = reinterpret_cast<uint32_t*>(mn_smem + MN_ECAP * sizeof(Key));
-  uint32_t* lstart = lflag + MN_ECAP;
-  __shared__ ull chunk_base;
-  __shared__ ull s_lo[5];   // list starts in the kept table (block-uniform,
-  __shared__ ull s_cum[6];  // indexed at run time from LDS, not registers)
-  const uint64_t g = blockIdx.x;
-  if (g >= G) return;
-  const MnPlan p = plan[g];
-  const bool big = p.e > (ull)MN_ECAP;
-  if (big != GLOBAL) return;
-  const ull E = p.e;
-  MnLists<Key, GLOBAL> L;
-  L.KK = KK;
-  L.msk = key_mask<Key>(2 * (K - 1));
-  L.lk = lk;
-  ull cum[6];
-  {
-    ull o = 0;
-#pragma unroll
-    for (int l = 0; l < 5; l++) {
-      L.len[l] = p.hi[l] - p.lo[l];
-      L.off[l] = GLOBAL ? p.lo[l] : o;
-      cum[l] = o;
-      o += L.len[l];
-    }
-    cum[5] = o;
-  }
-  if (threadIdx.x == 0) {
-#pragma unroll
-    for (int l = 0; l < 5; l++) {
-      s_lo[l] = p.lo[l];
-      s_cum[l] = cum[l];
-    }
-    s_cum[5] = cum[5];
-  }
-  if (!GLOBAL) {
-#pragma unroll
-    for (int l = 0; l < 5; l++) {
-      for (ull i = threadIdx.x; i < L.len[l]; i += MN_NT) {
-        const Key x = KK[p.lo[l] + i];
-        lk[cum[l] + i] = l == 0 ? mn_pred(x) : (x & L.msk);
-      }
-    }
-  }
-  __syncthreads();
-  uint32_t* flags = GLOBAL ? gflags + p.base : lflag;
-  const ull chunk = (E + MN_NT - 1) / MN_NT;
-  const ull e0 = (ull)threadIdx.x * chunk;
-  const ull e1 = e0 + chunk < E ? e0 + chunk : E;
-  // pass 1: merged rank and node-start flag of every element of the chunk
-#pragma unroll
-  for (int l = 0; l < 5; l++) {
-    const ull a = e0 > cum[l] ? e0 : cum[l];
-    const ull b = e1 < cum[l + 1] ? e1 : cum[l + 1];
-    if (a >= b) continue;
-    MnCursor<Key, GLOBAL> cur;
-    for (ull e = a; e < b; e++) {
-      const ull j = e - cum[l];
-      const Key x = L.at(L.off[l], l == 0, j);
-      if (e == a) cur.seek(L, x); else cur.advance(L, x);
-      ull rank = j;
-      bool start = cur.lb[l] == j;
-#pragma unroll
-      for (int o = 0; o < 5; o++) {
-        if (o < l) {
-          rank += cur.ub[o];
-          if (cur.ub[o] != cur.lb[o]) start = false;
-        } else if (o > l) {
-          rank += cur.lb[o];
-        }
-      }
-      if (GLOBAL) flags[rank] = start ? 1u : 0u;
-      else flags[rank] = (start ? 0x80000000u : 0u) | ((uint32_t)l << 16) | (uint32_t)j;
-    }
-  }
-  __syncthreads();
-  // pass 2: exclusive scan of the start flags in rank order (chunks of
-  // MN_NT*4).  Global ranges keep "node index + 1" per start rank; LDS
-  // ranges keep their per-rank element ids and note each node's first rank.
-  if (threadIdx.x == 0) chunk_base = 0;
-  __syncthreads();
-  for (ull c0 = 0; c0 < E; c0 += (ull)MN_NT * 4) {
-    const ull i0 = c0 + (ull)threadIdx.x * 4;
-    uint32_t v[4];
-    ull sm = 0;
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-      v[i] = i0 + i < E ? (GLOBAL ? flags[i0 + i] : flags[i0 + i] >> 31) : 0u;
-      sm += v[i];
-    }
-    ull ex = block_excl_scan<MN_NT>(sm) + chunk_base;
-    const ull tot = block_sum<MN_NT>(sm);
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-      if (GLOBAL) {
-        if (i0 + i < E) flags[i0 + i] = v[i] ? (uint32_t)(ex + 1) : 0u;
-      } else if (v[i]) {
-        lstart[ex] = (uint32_t)(i0 + i);
-      }
-      ex += v[i];
-    }
+__global__ __launch_bounds__(MN_NT, 8) void k_mn_write(const Key* KK, const int32_t* KC, int K, const ull* bd, ull G,
+                                                       const uint16_t* rkp, const uint16_t* rks, const ull* noff,
+                                                       MnRec* out) {
+  __shared__ ulonglong2 key[MN_ROUND];
+  __shared__ uint4 cnt[MN_ROUND * 2];  // pre[4], suf[4] per record
+  __shared__ uint32_t top;
+  __shared__ ull sh[5];
+  const ull g = blockIdx.x;
+  const Key msk = key_mask<Key>(2 * (K - 1));
+  const int tid = (int)threadIdx.x;
+  MnSub m = mn_range(bd, G, g);
+  ull base = uniform(noff[g]);
+  while (mn_next<Key>(KK, msk, m, sh)) {
+    const uint32_t E = mn_size(m);
+    Key x[MN_PER];
+    int32_t c[MN_PER];
+    uint32_t r[MN_PER], f[MN_PER];
+    if (tid == 0) top = 0;
     __syncthreads();
-    if (threadIdx.x == 0) chunk_base += tot;
+    uint32_t rmax = 0;
+#pragma unroll
+    for (int j = 0; j < MN_PER; j++) {
+      const uint32_t e = (uint32_t)(tid + j * MN_NT);
+      r[j] = 0xFFFFFFFFu;
+      x[j] = Key(0);
+      c[j] = 0;
+      f[j] = 0;
+      if (e < E) {
+        int l;
+        ull i;
+        mn_element(m, e, l, i);
+        const Key k = KK[i];
+        c[j] = KC[i];
+        r[j] = (l == 0 ? rkp : rks)[i];
+        f[j] = l == 0 ? 4u + (uint32_t)(k & Key(3)) : (uint32_t)(l - 1);
+        x[j] = l == 0 ? mn_pred(k) : (k & msk);
+        rmax = r[j] + 1 > rmax ? r[j] + 1 : rmax;
+      }
+    }
+    atomicMax(&top, rmax);
     __syncthreads();
-  }
-  const ull nodes = chunk_base;
-  if (!GLOBAL) {
-    // pass 3 (LDS ranges): one thread per node, in node order, so that
-    // consecutive lanes write consecutive records.  A node's elements are
-    // consecutive in rank order: its first, then the ranks up to the next
-    // start.  Suffix b of the node: pred-list element with last base b;
-    // prefix a: the element of quarter list a + 1.
-    for (ull nd = threadIdx.x; nd < nodes; nd += MN_NT) {
-      const uint32_t r0 = lstart[nd];
-      const uint32_t id0 = lflag[r0];
-      MnRec rec;
-      set_key<Key>(rec, lk[s_cum[(id0 >> 16) & 7u] + (id0 & 0xFFFFu)]);
-      int32_t s0 = 0, s1 = 0, s2 = 0, s3 = 0, q0 = 0, q1 = 0, q2 = 0, q3 = 0;
-      for (ull r = r0; r < E; r++) {
-        const uint32_t id = lflag[r];
-        if (r != r0 && (id >> 31)) break;
-        const uint32_t l = (id >> 16) & 7u;
-        const ull gi = s_lo[l] + (id & 0xFFFFu);
-        const int32_t cnt = KC[gi];
-        if (l == 0) {
-          const uint32_t bse = (uint32_t)(KK[gi] & Key(3));
-          s0 = bse == 0 ? cnt : s0;
-          s1 = bse == 1 ? cnt : s1;
-          s2 = bse == 2 ? cnt : s2;
-          s3 = bse == 3 ? cnt : s3;
-        } else {
-          q0 = l == 1 ? cnt : q0;
-          q1 = l == 2 ? cnt : q1;
-          q2 = l == 3 ? cnt : q2;
-          q3 = l == 4 ? cnt : q3;
+    const uint32_t n = top;
+    for (uint32_t r0 = 0; r0 < n; r0 += MN_ROUND) {
+      for (int i = tid; i < 2 * MN_ROUND; i += MN_NT) cnt[i] = make_uint4(0u, 0u, 0u, 0u);
+      __syncthreads();
+#pragma unroll
+      for (int j = 0; j < MN_PER; j++) {
+        const uint32_t p = r[j] - r0;
+        if (r[j] != 0xFFFFFFFFu && p < (uint32_t)MN_ROUND) {
+          key[p] = make_ulonglong2((ull)x[j], sizeof(Key) == 16 ? (ull)((u128)x[j] >> 64) : 0ull);
+          reinterpret_cast<int32_t*>(cnt)[p * 8 + f[j]] = c[j];
         }
       }
-      rec.suf[0] = s0;
-      rec.suf[1] = s1;
-      rec.suf[2] = s2;
-      rec.suf[3] = s3;
-      rec.pre[0] = q0;
-      rec.pre[1] = q1;
-      rec.pre[2] = q2;
-      rec.pre[3] = q3;
-      NT[p.base + nd] = rec;
-    }
-  } else {
-    // pass 3 (global ranges): every node start assembles its record
-#pragma unroll
-    for (int l = 0; l < 5; l++) {
-      const ull a = e0 > cum[l] ? e0 : cum[l];
-      const ull b = e1 < cum[l + 1] ? e1 : cum[l + 1];
-      if (a >= b) continue;
-      MnCursor<Key, GLOBAL> cur;
-      for (ull e = a; e < b; e++) {
-        const ull j = e - cum[l];
-        const Key x = L.at(L.off[l], l == 0, j);
-        if (e == a) cur.seek(L, x); else cur.advance(L, x);
-        if (cur.lb[l] != j) continue;
-        ull rank = j;
-        bool start = true;
-#pragma unroll
-        for (int o = 0; o < 5; o++) {
-          if (o < l) {
-            rank += cur.ub[o];
-            if (cur.ub[o] != cur.lb[o]) start = false;
-          } else if (o > l) {
-            rank += cur.lb[o];
-          }
-        }
-        if (!start) continue;
-        const uint32_t idx1 = flags[rank];
-        MnRec rec;
-        set_key<Key>(rec, x);
-        int32_t s0 = 0, s1 = 0, s2 = 0, s3 = 0;
-        for (ull i = cur.lb[0]; i < cur.ub[0]; i++) {
-          const ull gi = p.lo[0] + i;
-          const uint32_t bse = (uint32_t)(KK[gi] & Key(3));
-          const int32_t cnt = KC[gi];
-          s0 = bse == 0 ? cnt : s0;
-          s1 = bse == 1 ? cnt : s1;
-          s2 = bse == 2 ? cnt : s2;
-          s3 = bse == 3 ? cnt : s3;
-        }
-        rec.suf[0] = s0;
-        rec.suf[1] = s1;
-        rec.suf[2] = s2;
-        rec.suf[3] = s3;
-#pragma unroll
-        for (int q = 0; q < 4; q++)
-          rec.pre[q] = cur.ub[q + 1] > cur.lb[q + 1] ? KC[p.lo[q + 1] + cur.lb[q + 1]] : 0;
-        NT[p.base + idx1 - 1] = rec;
+      __syncthreads();
+      const uint32_t w3 = 3 * (n - r0 < (uint32_t)MN_ROUND ? n - r0 : (uint32_t)MN_ROUND);
+      uint4* o = reinterpret_cast<uint4*>(out + base + r0);
+      for (uint32_t w = tid; w < w3; w += MN_NT) {
+        const uint32_t q = w / 3, part = w - 3 * q;
+        o[w] = part == 0 ? reinterpret_cast<const uint4*>(key)[q] : cnt[2 * q + part - 1];
       }
+      __syncthreads();
     }
+    base += n;
   }
-  if (threadIdx.x == 0) ng[g] = nodes;
 }
 
 // Initial wiring of one macro node per thread (MacroNode::setup_wiring,
@@ -3310,19 +3286,6 @@ __global__ void k_mn_wire(const MnRec* nodes, uint64_t M, const uint8_t* pre_ord
   out[i] = w;
 }
 
-__global__ void k_mn_compact(const MnRec* NT, const MnPlan* plan, const ull* ng, const ull* noff,
-                             uint64_t G, MnRec* out) {
-  const uint64_t g = blockIdx.x;
-  if (g >= G) return;
-  const ull b = plan[g].base, o = noff[g], c = ng[g];
-  // a record is three 16-byte words (both arrays start 256-byte aligned):
-  // copy the range as words, one per lane
-  static_assert(sizeof(MnRec) == 48, "MnRec is three 16-byte words");
-  const uint4* src = reinterpret_cast<const uint4*>(NT + b);
-  uint4* dst = reinterpret_cast<uint4*>(out + o);
-  for (ull i = threadIdx.x; i < 3 * c; i += blockDim.x) dst[i] = src[i];
-}
-
 // Macro-node share of rank `rank` at P ranks: nodes whose (k-1)-mer key is
 // owned by the rank (retrieve_proc_id(pred / succ), mn_construct.cpp:
 // 234-247; the rank receives every kept k-mer of its nodes,
@@ -3356,7 +3319,7 @@ struct DevBuf {
 
 enum BufId {
   B_FASTA, B_BLK, B_BLKOFF, B_NL, B_RSTART, B_RLEN, B_KC, B_KOFS, B_SMALL, B_BCNT, B_BOFF, B_BCUR,
-  B_S, B_C, B_TU, B_UOFF, B_TK, B_TC, B_HIST, B_KBS, B_KBOFF, B_KK, B_KC2, B_MNQ, B_MNPLAN,
+  B_S, B_C, B_TU, B_UOFF, B_TK, B_TC, B_HIST, B_KBS, B_KBOFF, B_KK, B_KC2, B_MNPLAN,
   B_MNNT, B_MNNG, B_MNNOFF, B_MNFLAG, B_NODES, B_TMP, B_OVF, B_PT0, B_PT1, B_PT2, B_PT3, B_PT4,
   B_PT5, B_PT6, B_BLKGT, B_S2, B_BCNT2, B_BOFF2, B_BCUR2, B_TP, B_TP2, B_HIST1, B_OFF1, B_HIST2, B_OFF2, B_PACK, B_RETRY, B_WCNT, B_WOFF, B_CUTBH, B_LFREQ, B_WORDER, B_WIRE, B_NORM, B_NORMNL, B_NORMLEN, B_NORMOFF, B_NORMLS, B_NORMLL, B_SCAN0, B_SCAN1 = B_SCAN0 + 8, B_COUNT = B_SCAN0 + 16
 };
@@ -4565,35 +4528,25 @@ int mn_impl(pk_ctx* c) {
   const uint64_t V = c->V;
   const int K = c->k;
   const uint64_t G = (V + MN_PC - 1) / MN_PC;
-  ull *q, *small, *ng, *noff;
-  MnPlan* plan;
-  MnRec *NT, *nodes;
-  uint32_t* gflags;
-  PK_TRY(need(c, B_MNQ, 8, &q));
-  PK_TRY(need(c, B_SMALL, 16, &small));
-  PK_TRY(need(c, B_MNPLAN, G, &plan));
-  PK_TRY(need(c, B_MNNT, 2 * V, &NT));
+  ull *bd, *ng, *noff;
+  MnRec* nodes;
+  uint16_t* rk;
+  PK_TRY(need(c, B_MNPLAN, 5 * (G + 1), &bd));
   PK_TRY(need(c, B_MNNG, G, &ng));
   PK_TRY(need(c, B_MNNOFF, G + 1, &noff));
-  PK_TRY(need(c, B_MNFLAG, 2 * V, &gflags));
-  ull* maxe = small + 10;
-  PK_TRY(fill_u64(c, maxe, 0, 1));
-  hipLaunchKernelGGL(HIP_KERNEL_NAME(k_mn_quarters<Key>), dim3(1), dim3(64), 0, st, KK, V, K, q);
+  PK_TRY(need(c, B_MNFLAG, 2 * V, &rk));
+  hipLaunchKernelGGL(HIP_KERNEL_NAME(k_mn_bounds<Key>), dim3(grid_for(5 * (G + 1), 256)), dim3(256), 0, st, KK, (ull)V,
+                     K, (ull)G, bd);
   PK_HIP(c, hipGetLastError());
-  hipLaunchKernelGGL(HIP_KERNEL_NAME(k_mn_plan<Key>), dim3(grid_for(G, 256)), dim3(256), 0, st, KK,
-                     V, K, q, G, plan, maxe);
-  PK_HIP(c, hipGetLastError());
-  hipLaunchKernelGGL(HIP_KERNEL_NAME(k_mn_build<Key, false>), dim3((unsigned)G), dim3(MN_NT),
-                     mn_lds_bytes<Key>(), st, KK, KC, K, plan, G, NT, ng, gflags);
-  PK_HIP(c, hipGetLastError());
-  hipLaunchKernelGGL(HIP_KERNEL_NAME(k_mn_build<Key, true>), dim3((unsigned)G), dim3(MN_NT), 0, st,
-                     KK, KC, K, plan, G, NT, ng, gflags);
+  hipLaunchKernelGGL(HIP_KERNEL_NAME(k_mn_rank<Key>), dim3((unsigned)G), dim3(MN_NT), 0, st, KK, K, bd, (ull)G, rk,
+                     rk + V, ng);
   PK_HIP(c, hipGetLastError());
   PK_TRY(scan_excl<ull>(c, ng, noff, G));
   ull M = 0;
   PK_TRY(d2h(c, &M, noff + G, 8));
   PK_TRY(need(c, B_NODES, M, &nodes));
-  hipLaunchKernelGGL(k_mn_compact, dim3((unsigned)G), dim3(256), 0, st, NT, plan, ng, noff, G, nodes);
+  hipLaunchKernelGGL(HIP_KERNEL_NAME(k_mn_write<Key>), dim3((unsigned)G), dim3(MN_NT), 0, st, KK, KC, K, bd, (ull)G,
+                     rk, rk + V, noff, nodes);
   PK_HIP(c, hipGetLastError());
   PK_HIP(c, hipEventRecord(c->ev[15], st));
   c->pend_mn = true;

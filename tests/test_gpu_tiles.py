@@ -117,3 +117,29 @@ def test_builder_tiles(ctx, oracle_mod, klen, bits, reads):
     assert n == want_n
     assert np.array_equal(keys.reshape(-1), np.asarray(want_k).reshape(-1))
     assert np.array_equal(counts, want_c)
+
+
+@pytest.mark.parametrize("k", [12, 32, 33, 64])
+@pytest.mark.parametrize("n", [1, 639, 640, 641, 20_000])
+def test_macro_node_ranges(ctx, oracle_mod, k, n):
+    """Node ranges of one element, of a full one and one more, and ranges
+    with far more succ than pred elements (k-mers c + A...A + random: their
+    succ keys crowd into a quarter of the pred keys' span), which are cut
+    down, the records against the oracle's."""
+    from pakman_plus_amd import api
+    rng = np.random.default_rng(k * 1000 + n)
+    same = min(10, k - 6)
+    rows = rng.choice(np.frombuffer(b"ACGT", dtype=np.uint8), (n, k))
+    rows[:, 1:1 + same] = ord("A")
+    fa = b"".join(b">r\n" + r.tobytes() + b"\n" for r in rows)
+    _p(f"case: node ranges k={k} n={n}")
+    ctx.count(fa, k)
+    kept = ctx.cutoff_threshold(0)
+    keys, counts = ctx.kept_host()
+    assert kept == keys.shape[0]
+    m = ctx.macro_nodes()
+    got = api.nodes_as_arrays(ctx.nodes_host(), k)
+    want = oracle_mod.macro_nodes(keys, counts, k)
+    assert m == want["keys"].shape[0]
+    for f in ("keys", "pre_cnt", "suf_cnt"):
+        assert np.array_equal(got[f], want[f]), f
