@@ -85,7 +85,8 @@ typedef struct pk_mn_table {
  * the kernel launches of each stage). */
 typedef struct pk_timing {
   float parse_ms;    /* line index + read table */
-  float hist_ms;     /* bucket histogram (rank shares only) */
+  float hist_ms;     /* bucket histogram (pk_count_noalloc short of the
+                      * packed input's scratch only) */
   float scatter_ms;  /* bucket scatter (parse pass 2) */
   float sort_ms;     /* per-bucket sort + run-length count */
   float split_ms;    /* oversize-bucket splitting (0 when none) */
@@ -119,15 +120,16 @@ void* pk_ctx_stream(pk_ctx* ctx);
 uint64_t pk_ctx_device_bytes(const pk_ctx* ctx);
 /* Launch-shape choices of the counting kernels (results do not depend on
  * them).  Zero fields keep the built-in choice.
- *   l1_chunks      rank shares: reads per level-1 partition block, in chunks
- *                  of 512 (1..64; built-in: 1..8 by input size); other counts
- *                  take any value and do not use it
+ *   l1_chunks      pk_count_noalloc short of the packed input's scratch: reads
+ *                  per level-1 partition block, in chunks of 512 (1..64;
+ *                  built-in: 1..8 by input size); other counts take any value
+ *                  and do not use it
  *   l1_bits        level-1 radix digit width (1..PK_TUNING_L1_BITS_MAX; built-in:
- *                  the bits of all levels spread evenly, at most 9 per level,
- *                  or 10 where a single level does; 8 for rank shares)
+ *                  the bits of all levels spread evenly, at most 10 per level;
+ *                  rank shares as few as keep their runs at 32 keys)
  *   bucket_factor  instances per final bucket as a multiple of the LDS hash
  *                  table's key capacity, i.e. the inverse hash load target
- *                  (built-in 3.0)
+ *                  (built-in: at most 2.1 for one-word keys, 2.2 for two)
  *   ms_scatter     0..2, no effect (chose between two former scatter kernels)
  *   ms_fold        0..2, no effect (switched a former histogram fold off)
  */

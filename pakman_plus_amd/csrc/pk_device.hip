@@ -9,9 +9,10 @@
 //                     bits: record r = header line j0+2r, sequence line
 //                     j0+2r+1, with the record rules and the format check of
 //                     the reference's Sliding_window (src/kmer_counting.cpp:
-//                     2890-2945).  Rank shares walk a read table instead
-//                     (k_reads); the builder API's records come from
-//                     k_bld_flags / k_bld_write.
+//                     2890-2945).  A rank share keeps the ends its owner rule
+//                     gives the rank (k_own, k_own_walk, k_own_key); the
+//                     builder API's records come from k_bld_flags /
+//                     k_bld_write.
 //   3. partition      k_split_main, k_split: tiles of k-mers sorted by a digit of the key's
 //                     top bits, one tile per block, each tile written back
 //                     as one contiguous piece with a table of where its
@@ -21,10 +22,8 @@
 //                     window of bits), further levels gather a bucket's runs
 //                     from the tiles of the level before.  This is the
 //                     on-device stand-in for the reference's owner routing +
-//                     MPI_Alltoallv (kmer_counting.cpp:254-352).  Rank-share
-//                     mode keeps one owner's k-mers (k_l1_hist, k_l1_scatter,
-//                     own_step).
-//   4. bucket count   k_bucket_hash: one 1024-thread workgroup per bucket counts
+//                     MPI_Alltoallv (kmer_counting.cpp:254-352).
+//   4. bucket count   k_bucket_hash: one workgroup per bucket counts
 //                     the bucket's distinct keys in an LDS hash table, then
 //                     counting-sorts them by the next bits and writes the
 //                     ascending (key, count) pairs (the reference's sort + RLE
@@ -1040,8 +1039,9 @@ __device__ __forceinline__ uint64_t load_word8(const uint8_t* fa, uint64_t n, ui
 // Partition (multisplit) into buckets by the top bits of the key.
 //   k_split    every level of the main and builder paths and the further
 //              levels of the others: tiles sorted in registers and LDS
-//   k_l1_hist / k_l1_scatter  level 1 of a rank's share, whose owner rule
-//              walks every read in order: each key goes straight to its slot
+//   k_l1_hist / k_l1_scatter  level 1 where the packed input has no room
+//              (pk_count_noalloc's smaller scratches): a walk over the bytes of
+//              every read, each key straight to its slot
 
 constexpr int L1_NT = 512;  // level-1 histogram blocks
 constexpr int L1_MAX_BITS = PK_TUNING_L1_BITS_MAX;  // level-1 digit width
@@ -1050,7 +1050,7 @@ constexpr int PK_MS_TILES = 4;      // pk_timing's form of a k_split level
 constexpr int MS_TIMED_LEVELS = 4;  // further levels with their own timing events
 static_assert(sizeof(pk_timing::ms_level_form) / sizeof(int32_t) == MS_TIMED_LEVELS, "per-level timing slots");
 
-// Level-1 producer of a rank's share.  A block owns rpb consecutive reads and
+// Level-1 producer of the walk.  A block owns rpb consecutive reads and
 // walks them in chunks: a chunk is the longest run of <= NT consecutive reads
 // (NT threads per block) whose bytes fit in the LDS staging buffer; thread t
 // then walks read t of the chunk from LDS with the rolling update (a read too
@@ -1123,104 +1123,13 @@ __device__ __forceinline__ void stage_chunk(ChunkLds& C, Stage sg, const uint8_t
 
 // Walks up to Q more k-mers of the thread's read (state s, i, km): emits
 // through emit(q, key); returns how many.
-// Rank-share routing of the reference's Sliding_window (kmer_counting.cpp:
-// 2950-3050): a k-mer belongs to rank hash31(m) % P (retrieve_proc_id,
-// distribute_kmers.cpp:95-105; hash31, distribute_kmers.h:856-873) of its
-// leftmost minimum-frequency L-mer m (L = 8, frequencies of the whole input).
-// The minimum is tracked as the window slides: a new L-mer replaces it only
-// when strictly rarer, and when it leaves the window every L-mer of the
-// current k-mer is re-read from the packed k-mer (recalculate_min_lmer,
-// kmer_counting.cpp:355-388).  The rolling L-mer uses the 3-bit code like
-// the k-mer; the re-read extracts 2-bit fields of the k-mer.
-constexpr int LMER_L = 8;
-constexpr uint32_t LMER_BINS = 1u << (2 * LMER_L);
-
-struct OwnCfg {
-  const ull* freq;  // LMER_BINS L-mer frequencies (min-L-mer owner)
-  int P, rank;
-  int by_key;       // owner of the whole k-mer instead (the -p counters)
-};
-
-struct OwnState {
-  uint32_t lm, min_lmer;
-  ull min_f;
-  int min_pos;
-};
-
-// retrieve_proc_id of a k-mer word (src/distribute_kmers.cpp:95-120): hash31
-// (includes/distribute_kmers.h:856-873: signed 64-bit a * x + b, arithmetic
-// shift) when kmer_t is 64 bits, uhash31 (:836-854: the same in unsigned
-// 128-bit arithmetic) when it is 128 bits; then (int) % P.  Both wrap as the
-// reference's builds do.
-__device__ __forceinline__ int key_owner(uint64_t x, int P) {
-  const long long v = (long long)(68111ull * x + 105929ull);
-  const long long h = (long long)((ull)(v >> 31) + (ull)v) & 2147483647LL;
-  return (int)h % P;
-}
-__device__ __forceinline__ int key_owner(u128 x, int P) {
-  u128 r = (u128)68111 * x + (u128)105929;
-  r = ((r >> 31) + r) & (u128)2147483647;
-  return (int)(long long)r % P;
-}
-
-__device__ __forceinline__ int lmer_owner(uint32_t lmer, int P) {
-  const long long v = 68111LL * (long long)lmer + 105929LL;  // hasha * x + hashb
-  const long long h = ((v >> 31) + v) & 2147483647LL;
-  return (int)h % P;
-}
-
-// One byte of a read (index idx, 3-bit code el; km already updated).
-// Returns whether the k-mer ending here, if any, is owned.
-template <class Key, bool OWN>
-__device__ __forceinline__ bool own_step(OwnState& o, const OwnCfg& cf, Key km, uint32_t el, uint32_t idx,
-                                         int K) {
-  if (!OWN) return true;
-  // the -p counters own a k-mer by a hash of the whole word
-  // (kmer_counting.cpp:1949-1950)
-  if (cf.by_key) return idx >= (uint32_t)(K - 1) && key_owner(km, cf.P) == cf.rank;
-  o.lm = ((o.lm << 2) | el) & (LMER_BINS - 1);
-  if (idx < (uint32_t)(K - 1)) {
-    if (idx >= (uint32_t)(LMER_L - 1)) {
-      const ull f = cf.freq[o.lm];
-      if (idx == (uint32_t)(LMER_L - 1)) {
-        o.min_lmer = o.lm;
-        o.min_f = f;
-      } else if (f < o.min_f) {
-        o.min_lmer = o.lm;
-        o.min_f = f;
-        o.min_pos = (int)idx - (LMER_L - 1);
-      }
-    }
-    return false;
-  }
-  const ull f = cf.freq[o.lm];
-  if (o.min_pos < 0) {
-    for (int kk = 0; kk <= K - LMER_L; kk++) {
-      const uint32_t lo = (uint32_t)(km >> (2 * (K - kk - LMER_L))) & (LMER_BINS - 1);
-      const ull g = cf.freq[lo];
-      if (kk == 0 || g < o.min_f) {
-        o.min_lmer = lo;
-        o.min_f = g;
-        o.min_pos = kk;
-      }
-    }
-  }
-  if (f < o.min_f) {
-    o.min_lmer = o.lm;
-    o.min_f = f;
-    o.min_pos = K - LMER_L;
-  }
-  o.min_pos--;
-  return lmer_owner(o.min_lmer, cf.P) == cf.rank;
-}
-
 // km rolls unmasked (bits above the key shift out of the word, and the
 // key's own bits are the same either way): the mask is applied to the keys
 // handed out, once per k-mer instead of once per base.
-template <class Key, int ENC, bool OWN, class Emit>
+template <class Key, int ENC, class Emit>
 __device__ __forceinline__ int walk_read(const ChunkLds& C, Stage sg, const uint8_t* fa, ull s, uint32_t len,
                                          uint32_t& i,
-                                         Key& km, OwnState& os, const OwnCfg& cf, int K, Key mask, int Q,
+                                         Key& km, int K, Key mask, int Q,
                                          Emit&& emit) {
   int q = 0;
   if (C.lds) {
@@ -1242,11 +1151,10 @@ __device__ __forceinline__ int walk_read(const ChunkLds& C, Stage sg, const uint
       for (uint32_t t = 0; t < cnt && q < Q; t++) {
         const uint32_t el = ((uint32_t)a & 3u) | ((b & 1u) << 2);
         km = (km << 2) | (Key)el;
-        const bool own = own_step<Key, OWN>(os, cf, OWN ? km & mask : km, el, i, K);
         a >>= 2;
         b >>= 1;
         i++;
-        if (i >= (uint32_t)K && own) emit(q++, km & mask);
+        if (i >= (uint32_t)K) emit(q++, km & mask);
       }
     }
     return q;
@@ -1254,38 +1162,19 @@ __device__ __forceinline__ int walk_read(const ChunkLds& C, Stage sg, const uint
   while (q < Q && i < len) {
     const uint32_t el = base_code<ENC>(fa[s + i]);
     km = (km << 2) | (Key)el;
-    const bool own = own_step<Key, OWN>(os, cf, OWN ? km & mask : km, el, i, K);
     i++;
-    if (i >= (uint32_t)K && own) emit(q++, km & mask);
+    if (i >= (uint32_t)K) emit(q++, km & mask);
   }
   return q;
 }
 
-// L-mer frequencies (Sliding_window_l, kmer_counting.cpp:391-438): every
-// L-mer of every record's read line, rolling 3-bit update masked to 2L bits.
-__global__ void k_lmer_freq(const uint8_t* fa, const ull* rstart, const uint32_t* rlen, uint64_t R,
-                            ull* freq) {
-  for (uint64_t r = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; r < R;
-       r += (uint64_t)gridDim.x * blockDim.x) {
-    const ull s = rstart[r];
-    const uint32_t len = rlen[r];
-    uint32_t lm = 0;
-    for (uint32_t i = 0; i < len; i++) {
-      lm = ((lm << 2) | base_code<ENC_MAIN>(fa[s + i])) & (LMER_BINS - 1);
-      if (i >= (uint32_t)(LMER_L - 1)) atomicAdd(&freq[lm], 1ull);
-    }
-  }
-}
-
-// Level-1 histogram of a rank's share: digit = bits [KB - d1, KB) of each
-// owned key.  Block b's count of digit d goes to H[d * nblk + b] (digit-major),
+// Level-1 histogram of the walk: digit = bits [KB - d1, KB) of each key.  Block b's count of digit d goes to H[d * nblk + b] (digit-major),
 // so an exclusive scan of H gives every block the output base of each of its
 // digit runs.
-template <class Key, int ENC, bool OWN>
+template <class Key, int ENC>
 __global__ __launch_bounds__(L1_NT) void k_l1_hist(const uint8_t* fa, uint64_t n, const ull* rstart,
                                                    const uint32_t* rlen, uint64_t R, int K, int KB,
-                                                   Key mask, int d1, int rpb, int sb, OwnCfg cf,
-                                                   uint32_t* H) {
+                                                   Key mask, int d1, int rpb, int sb, uint32_t* H) {
   __shared__ ChunkLds C;
   // dynamic LDS: plane A, plane B, 2^d1 digit counts
   extern __shared__ ull l1_dyn[];
@@ -1303,8 +1192,7 @@ __global__ __launch_bounds__(L1_NT) void k_l1_hist(const uint8_t* fa, uint64_t n
       const uint64_t r = c0 + threadIdx.x;
       uint32_t i = 0;
       Key km = 0;
-      OwnState os{0, 0, 0, 0};
-      walk_read<Key, ENC, OWN>(C, sg, fa, rstart[r], rlen[r], i, km, os, cf, K, mask, 0x7fffffff,
+      walk_read<Key, ENC>(C, sg, fa, rstart[r], rlen[r], i, km, K, mask, 0x7fffffff,
                                [&](int, Key x) { atomicAdd(&h[key_digit<Key>(x, bpos, d1)], 1u); });
     }
     c0 += m;
@@ -1313,15 +1201,15 @@ __global__ __launch_bounds__(L1_NT) void k_l1_hist(const uint8_t* fa, uint64_t n
   for (int i = threadIdx.x; i < nb; i += L1_NT) H[(ull)i * gridDim.x + blockIdx.x] = h[i];
 }
 
-// Level-1 scatter of a rank's share: the same chunked walk as k_l1_hist over
+// Level-1 scatter of the walk: the same chunked walk as k_l1_hist over
 // the same reads per block; every key takes the next slot of its digit from
 // the block's LDS cursor (the return value of one 64-bit atomic) and is
 // stored at once.  The order of keys inside a bucket is arbitrary, which the
 // bucket count does not depend on.
-template <class Key, int ENC, bool OWN>
+template <class Key, int ENC>
 __global__ __launch_bounds__(L1_NT) void k_l1_scatter(const uint8_t* fa, uint64_t n, const ull* rstart,
                                                       const uint32_t* rlen, uint64_t R, int K, int KB, Key mask,
-                                                      int d1, int rpb, int sb, OwnCfg cf, const ull* O,
+                                                      int d1, int rpb, int sb, const ull* O,
                                                       uint64_t nblk, Key* S1) {
   __shared__ ChunkLds C;
   // dynamic LDS: plane A, 2^d1 output cursors, plane B
@@ -1341,8 +1229,7 @@ __global__ __launch_bounds__(L1_NT) void k_l1_scatter(const uint8_t* fa, uint64_
       const uint64_t r = c0 + threadIdx.x;
       uint32_t i = 0;
       Key km = 0;
-      OwnState os{0, 0, 0, 0};
-      walk_read<Key, ENC, OWN>(C, sg, fa, rstart[r], rlen[r], i, km, os, cf, K, mask, 0x7fffffff,
+      walk_read<Key, ENC>(C, sg, fa, rstart[r], rlen[r], i, km, K, mask, 0x7fffffff,
                                [&](int, Key x) {
                                  const uint32_t d = key_digit<Key>(x, bpos, d1);
                                  S1[atomicAdd(&cur[d], 1ull)] = x;
@@ -1353,7 +1240,7 @@ __global__ __launch_bounds__(L1_NT) void k_l1_scatter(const uint8_t* fa, uint64_
   }
 }
 
-// bucket offsets of the share's level 1 from its scanned histogram
+// bucket offsets of the walk's level 1 from its scanned histogram
 __global__ void k_l1_boff(const ull* O, int nb, uint64_t nblk, ull total, ull* boff) {
   const int d = blockIdx.x * blockDim.x + threadIdx.x;
   if (d < nb) boff[d] = O[(ull)d * nblk];
@@ -1803,7 +1690,7 @@ __global__ __launch_bounds__(SP_NT, 4) void k_split(const Key* __restrict__ Sin,
 // instead of the key, so one round covers the tile, and bytes that end no
 // k-mer cost only the first two passes.  Bound by VALU: with whole keys
 // exchanged through LDS in rounds it issued 115 lane instructions per one-word
-// key (k_l1 figures at count_records).
+// key and took 783 us for 1.27e8 keys, now 474.
 constexpr int SM_NT = 1024;
 
 template <class Key, int WPT>
@@ -1910,6 +1797,456 @@ __global__ __launch_bounds__(SM_NT, 8) void k_split_main(const uint32_t* __restr
     o[p] = k & mask;
   }
 }
+
+// ---------------------------------------------------------------------------
+// Rank-share routing of the reference's Sliding_window (kmer_counting.cpp:
+// 2950-3050): a k-mer belongs to rank hash31(m) % P (retrieve_proc_id,
+// distribute_kmers.cpp:95-105) of its leftmost minimum-frequency L-mer m
+// (L = 8, frequencies of the whole input).  The reference tracks the minimum
+// as the window slides: a new L-mer replaces it only when strictly rarer, and
+// when it leaves the window every L-mer of the current k-mer is re-read from
+// the packed k-mer (recalculate_min_lmer, :355-388).  The rolling L-mer that
+// ends at byte e, A(e), has e's exact code; re-read, B(e), its last low bit
+// also holds the next byte's third code bit.  So, with w = K - L + 1 and an end
+// "dirty" when A != B:
+//   - the first window of a read has the leftmost minimum of A over its w ends;
+//   - a window without a dirty end but its own has the same, whatever came
+//     before (the reference's state is the leftmost minimum over A or B of its
+//     ends): k_own, all windows at once;
+//   - the other windows depend on where the minimum was last re-read: from the
+//     window before a run of them, which k_own gives, k_own_walk follows the
+//     reference window by window.  Reads of A, C, G, T have none.
+// The result is a bitmap of window ends like k_valid's, and the count goes on
+// as on the main path.
+
+constexpr int LMER_L = 8;
+constexpr uint32_t LMER_BINS = 1u << (2 * LMER_L);
+constexpr int LM_NT = 1024;
+// index blocks whose L-mers a block adds before it looks for counters of
+// 2^14 or more: three add less than 2^16 - 2^14 to any
+constexpr int LM_FLUSH = 3;
+
+// retrieve_proc_id before its % P (src/distribute_kmers.cpp:95-120): hash31
+// (includes/distribute_kmers.h:856-873, signed 64-bit) and uhash31 (:836-854,
+// unsigned 128-bit) both come to bits 0-30 plus bits 31-61 of a * x + b, which
+// depend on x's low 64 bits alone.
+__device__ __forceinline__ uint32_t owner_hash(ull x) {
+  const ull v = 68111ull * x + 105929ull;
+  return (uint32_t)((v >> 31) + v) & 2147483647u;
+}
+
+// h % P for h < 2^31 as h - ((h * m) >> s) * P.
+struct OwnerMod {
+  ull m;
+  int s;
+  uint32_t P, rank;
+};
+
+__device__ __forceinline__ bool owner_is(uint32_t h, const OwnerMod& o) {
+  return h - (uint32_t)((ull)h * o.m >> o.s) * o.P == o.rank;
+}
+
+// A(e) for byte i of a word e1 of E (e0: the word before; rx: exact low bits)
+__device__ __forceinline__ uint32_t lmer_at(uint32_t e0, uint32_t e1, uint32_t rx, int i) {
+  const uint32_t b = __builtin_amdgcn_alignbit(e0, e1, 30u - 2u * (uint32_t)i) & 0xFFFFu;
+  return (b & ~1u) | ((rx >> i) & 1u);
+}
+
+// L-mer frequencies (Sliding_window_l, kmer_counting.cpp:391-438): the L-mers
+// that end at the set bits of W (k_valid's at K = L).  A block counts in LDS, 16
+// bits per L-mer, and leaves its table in part; counters that grow past 2^14
+// move to freq.  Bound by LDS atomics, one per
+// L-mer (0.19 GB of reads of 100 bases: 83 us; a global atomic per L-mer took 7.7 ms).
+__global__ __launch_bounds__(LM_NT) void k_lmer_count(const uint32_t* __restrict__ E, const uint32_t* __restrict__ RX,
+                                                      const uint16_t* __restrict__ W, ull nb, uint32_t* part,
+                                                      ull* freq) {
+  static_assert(NL_PER_BLOCK == 16ull * LM_NT, "a word of E per thread and index block");
+  static_assert(LM_FLUSH * NL_PER_BLOCK + (1u << 14) <= 1u << 16, "16-bit counters");
+  __shared__ __align__(16) uint32_t h[LMER_BINS / 2];
+  const int tid = (int)threadIdx.x;
+  uint4* hv = reinterpret_cast<uint4*>(h);
+  for (int i = tid; i < (int)LMER_BINS / 8; i += LM_NT) hv[i] = uint4{0, 0, 0, 0};
+  __syncthreads();
+  int since = 0;
+  // an index block's words, loaded while the one before is counted
+  uint32_t n0 = 0, n1 = 0, nr = 0, nv = 0;
+  auto fetch = [&](ull b) {
+    const ull w = b * LM_NT + tid;
+    nv = b < nb ? W[w] : 0u;
+    if (nv) {
+      n0 = E[PK_PAD + w - 1];
+      n1 = E[PK_PAD + w];
+      nr = RX[w];
+    }
+  };
+  fetch(blockIdx.x);
+  for (ull b = blockIdx.x; b < nb; b += gridDim.x) {
+    if (since == LM_FLUSH) {
+      since = 0;
+      __syncthreads();
+      for (int i = tid; i < (int)LMER_BINS / 8; i += LM_NT) {
+        const uint4 q = hv[i];
+        if ((q.x | q.y | q.z | q.w) & 0xC000C000u) {
+          const uint32_t v[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+          for (int j = 0; j < 4; j++) {
+            uint32_t keep = v[j];
+            if (keep & 0xC000u) {
+              atomicAdd(&freq[8 * i + 2 * j], (ull)(keep & 0xFFFFu));
+              keep &= 0xFFFF0000u;
+            }
+            if (keep & 0xC0000000u) {
+              atomicAdd(&freq[8 * i + 2 * j + 1], (ull)(keep >> 16));
+              keep &= 0xFFFFu;
+            }
+            h[4 * i + j] = keep;
+          }
+        }
+      }
+      __syncthreads();
+    }
+    since++;
+    const uint32_t val = nv, e0 = n0, e1 = n1, rx = nr;
+    fetch(b + gridDim.x);
+    if (val) {
+#pragma unroll
+      for (int i = 0; i < 16; i++) {
+        if ((val >> i) & 1u) {
+          const uint32_t l = lmer_at(e0, e1, rx, i);
+          atomicAdd(&h[l >> 1], 1u << (16u * (l & 1u)));
+        }
+      }
+    }
+  }
+  __syncthreads();
+  uint4* o = reinterpret_cast<uint4*>(part + (ull)blockIdx.x * (LMER_BINS / 2));
+  for (int i = tid; i < (int)LMER_BINS / 8; i += LM_NT) o[i] = hv[i];
+}
+
+// freq += the np tables of k_lmer_count: a block takes 64 words of each, its
+// waves every sixteenth table.
+__global__ __launch_bounds__(1024) void k_lmer_sum(const uint32_t* __restrict__ part, int np, ull* freq) {
+  __shared__ uint32_t lo[16][64], hi[16][64];
+  const int lane = (int)threadIdx.x & 63, wv = (int)threadIdx.x >> 6;
+  const uint32_t i = blockIdx.x * 64u + (uint32_t)lane;
+  uint32_t a = 0, b = 0;  // at most np * 2^16
+  for (int t = wv; t < np; t += 16) {
+    const uint32_t v = part[(ull)t * (LMER_BINS / 2) + i];
+    a += v & 0xFFFFu;
+    b += v >> 16;
+  }
+  lo[wv][lane] = a;
+  hi[wv][lane] = b;
+  __syncthreads();
+  if (wv < 2) {
+    ull s = 0;
+    for (int t = 0; t < 16; t++) s += wv ? hi[t][lane] : lo[t][lane];
+    freq[2 * i + wv] += s;
+  }
+}
+
+// The routing compares frequencies only with each other, so k_own takes their
+// ranks (the number of smaller ones, 16 bits) and holds all of them in LDS.
+// Frequencies below 2^16 - 1 rank by a histogram of their values in one block's
+// LDS, 16 bits a value (65536 equal ones carry into a value that none has);
+// the others, few below 10^8 bases, are listed in big and compared by
+// k_freq_big.  One block takes 47 us for the 65536, all of it latency; with the
+// histogram by global atomics and a scan it was five launches and 60 us.
+// own: bit l = L-mer l's k-mers are this rank's.
+__global__ __launch_bounds__(1024) void k_freq_rank(const ull* __restrict__ freq, OwnerMod om, ull* big, ull* nbig,
+                                                    uint16_t* __restrict__ rank, ull* __restrict__ own) {
+  constexpr int PER = (int)LMER_BINS / 1024, WW = (int)LMER_BINS / 2 / 16;  // words per wave
+  __shared__ __align__(16) uint32_t h[LMER_BINS / 2];
+  __shared__ uint32_t wsum[16];
+  __shared__ uint32_t nb;
+  const int tid = (int)threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  for (int i = tid; i < (int)LMER_BINS / 8; i += 1024) reinterpret_cast<uint4*>(h)[i] = uint4{0, 0, 0, 0};
+  if (tid == 0) nb = 0;
+  __syncthreads();
+  uint32_t z = 0;  // values of 0, small inputs' most frequent one
+#pragma unroll 8
+  for (int r = 0; r < PER; r++) {
+    const ull f = freq[r * 1024 + tid];
+    if (f == 0)
+      z++;
+    else if (f < LMER_BINS - 1)
+      atomicAdd(&h[f >> 1], 1u << (16u * (uint32_t)(f & 1)));
+    else
+      big[atomicAdd(&nb, 1u)] = f;
+  }
+  const uint32_t zeros = (uint32_t)block_sum<1024>((ull)z);
+  __syncthreads();
+  // counts -> the number of smaller values, wave by wave
+  uint32_t s = 0;
+  for (int i = 0; i < WW; i += 64) {
+    const uint32_t v = h[wv * WW + i + lane];
+    s += (v & 0xFFFFu) + (v >> 16);
+  }
+  s = wave_scan_u32(s);
+  if (lane == 63) wsum[wv] = s;
+  __syncthreads();
+  uint32_t carry = zeros;
+  for (int i = 0; i < wv; i++) carry += wsum[i];
+  for (int i = 0; i < WW; i += 64) {
+    const uint32_t v = h[wv * WW + i + lane];
+    const uint32_t t = (v & 0xFFFFu) + (v >> 16);
+    const uint32_t x = wave_scan_u32(t);
+    const uint32_t a = carry + x - t;
+    h[wv * WW + i + lane] = (a & 0xFFFFu) | (a + (v & 0xFFFFu)) << 16;
+    carry += __shfl(x, 63, 64);
+  }
+  __syncthreads();
+#pragma unroll 8
+  for (int r = 0; r < PER; r++) {
+    const uint32_t l = (uint32_t)(r * 1024 + tid);
+    const ull f = freq[l];
+    if (f < LMER_BINS - 1) rank[l] = f ? (uint16_t)(h[f >> 1] >> (16u * (uint32_t)(f & 1))) : (uint16_t)0;
+    const ull b = __ballot(owner_is(owner_hash(l), om));
+    if (lane == 0) own[l / 64] = b;
+  }
+  if (tid == 0) *nbig = nb;
+}
+
+// ranks of the frequencies of 2^16 - 1 and more
+__global__ void k_freq_big(const ull* freq, const ull* big, const ull* nbig, uint16_t* rank) {
+  const uint32_t l = blockIdx.x * blockDim.x + threadIdx.x;
+  const ull m = *nbig;
+  if (m == 0 || freq[l] < LMER_BINS - 1) return;
+  const ull f = freq[l];
+  ull r = LMER_BINS - m;
+  for (ull i = 0; i < m; i++) r += big[i] < f;
+  rank[l] = (uint16_t)r;
+}
+
+constexpr int OWN_NT = 512;
+constexpr int OWN_HALO = 4;  // words before a window end's own that its ends reach
+constexpr int OWN_EX = 9;    // exchanged words per thread
+constexpr int OWN_TAB = (int)LMER_BINS / 2 + (int)LMER_BINS / 32;  // ranks, then owner bits
+constexpr int own_lds = 4 * (OWN_TAB + OWN_NT * OWN_EX);
+
+// Windows [e - w + 1, e] of L-mer ends, w = K - L + 1 in [BS, 2 BS) (BS = 16:
+// up to 57): a thread takes the 16 ends of one word of E, looks their ranks up
+// in LDS and takes minima from both ends of each block of BS of them.  A
+// window's minimum is that of the rest of its first block (from the thread
+// that holds it, through LDS), the whole blocks between and the first part of
+// its last.  One block of 512 threads per CU holds the tables and stays for
+// all its tiles; 4 threads of 512 only feed the next ones.  Bound by VALU, 33
+// instructions per byte of input (0.19 GB of reads of 100 bases, w = 25: 272 us,
+// 0.69 TB/s of input; a thread per read, walking twice, took 3.96 ms; 640
+// threads or tiles of one wave gain nothing).
+//   Wout: W without the ends of other ranks and the undecided ones; D: those.
+template <int BS>
+__global__ __launch_bounds__(OWN_NT) void k_own(const uint32_t* __restrict__ E, const uint32_t* __restrict__ RX,
+                                                const uint16_t* __restrict__ W, ull words, ull nwords, int w,
+                                                const uint4* __restrict__ tab, uint16_t* __restrict__ Wout,
+                                                uint16_t* __restrict__ D) {
+  extern __shared__ __align__(16) uint32_t own_dyn[];
+  const uint16_t* rk = reinterpret_cast<const uint16_t*>(own_dyn);
+  const uint32_t* ob = own_dyn + LMER_BINS / 2;
+  uint32_t* ex = own_dyn + OWN_TAB;
+  const int tid = (int)threadIdx.x;
+  for (int i = tid; i < OWN_TAB / 4; i += OWN_NT) reinterpret_cast<uint4*>(own_dyn)[i] = tab[i];
+  constexpr int OUT = OWN_NT - OWN_HALO;
+  // a tile's words, loaded while the tile before is worked on
+  uint32_t n0 = 0, n1 = 0, nr = 0, nv = 0;
+  auto fetch = [&](ull t0) {
+    const long long x = (long long)t0 + tid - OWN_HALO;
+    if (x >= 0 && (ull)x < nwords) {
+      n0 = E[PK_PAD + x - 1];
+      n1 = E[PK_PAD + x];
+      nr = RX[x];
+    }
+    nv = tid >= OWN_HALO && (ull)x < words ? W[x] : 0u;
+  };
+  fetch((ull)blockIdx.x * OUT);
+  for (ull t0 = (ull)blockIdx.x * OUT; t0 < words; t0 += (ull)gridDim.x * OUT) {
+    __syncthreads();  // the tables; the last tile's reads of ex
+    const long long x = (long long)t0 + tid - OWN_HALO;
+    const uint32_t e0 = n0, e1 = n1, rx = nr, val = nv;
+    fetch(t0 + (ull)gridDim.x * OUT);
+    // rank << 16 | place << 1 | owned, places from 2: the least is the
+    // leftmost minimum (place 0: the window's first block, 1: those between)
+    uint32_t pre[16], suf[16];
+    uint32_t dirty = 0;
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+      const uint32_t b = __builtin_amdgcn_alignbit(e0, e1, 30u - 2u * (uint32_t)i);
+      const uint32_t l = (b & 0xFFFEu) | ((rx >> i) & 1u);
+      dirty = __builtin_amdgcn_alignbit(b ^ l, dirty, 1);
+      pre[i] = (uint32_t)rk[l] << 16 | (((ob[l >> 5] >> (l & 31u)) & 1u) | (uint32_t)((i + 2) << 1));
+      suf[i] = pre[i];
+    }
+    // (no window reaches past a line's end: the ends before one do not count)
+    const uint32_t nl = (rx >> 16 | __shfl_down(rx, 1, 64) & 0x10000u) >> 1;
+    dirty = dirty >> 16 & ~nl;
+#pragma unroll
+    for (int i = 14; i >= 0; i--)
+      if (i % BS != BS - 1) suf[i] = suf[i] < suf[i + 1] ? suf[i] : suf[i + 1];
+#pragma unroll
+    for (int i = 1; i < 16; i++)
+      if (i % BS != 0) pre[i] = pre[i] < pre[i - 1] ? pre[i] : pre[i - 1];
+    uint32_t* mine = ex + tid * OWN_EX;
+    uint32_t om = 0;
+#pragma unroll
+    for (int i = 0; i < 16; i++) om = __builtin_amdgcn_alignbit(suf[i], om, 1);
+    om = om >> 16 | dirty << 16;
+#pragma unroll
+    for (int i = 0; i < 8; i++) mine[i] = __builtin_amdgcn_perm(suf[2 * i + 1], suf[2 * i], 0x07060302u);
+    mine[8] = om;
+    __syncthreads();
+    if (tid < OWN_HALO || (ull)x >= words) continue;
+    uint32_t out = 0, und = 0;
+    if (val) {
+      const uint16_t* exh = reinterpret_cast<const uint16_t*>(ex);
+      // the windows start in place sh + q of the thread `far` before
+      const int far = (w + 14) >> 4, sh = 16 * far - (w - 1);
+      const uint16_t* xf = exh + (tid - far) * (2 * OWN_EX);
+      uint32_t oms = ex[(tid - far) * OWN_EX + 8] & 0xFFFFu;
+      if (far) oms |= ex[(tid - far + 1) * OWN_EX + 8] << 16;
+      oms >>= sh;
+      // first place of the thread o before, as a block between
+      auto head = [&](int o) -> uint32_t {
+        const uint32_t* y = ex + (tid - o) * OWN_EX;
+        return y[0] << 16 | 2u | (y[8] & 1u);
+      };
+      // BS = 16: the whole words between, for starts in the thread `far`
+      // before (mf) and in the next (mn)
+      uint32_t mf = ~0u, mn = ~0u;
+      if (BS == 16) {
+        for (int o = 1; o < far; o++) {
+          const uint32_t c = head(o);
+          mn = mf;
+          // an earlier word wins ties
+          mf = mf >> 16 < c >> 16 ? mf : c;
+        }
+      }
+      uint32_t mp = ~0u;  // BS < 16: the last whole block of the thread before
+      if (BS < 16) {
+        const uint32_t* y = ex + (tid - 1) * OWN_EX;
+        const int i = 16 - BS;
+        mp = ((i & 1) ? y[i / 2] & 0xFFFF0000u : y[i / 2] << 16) | 2u | ((y[8] >> i) & 1u);
+      }
+#pragma unroll
+      for (int q = 0; q < 16; q++) {
+        const int i = sh + q;
+        const uint32_t c = (uint32_t)xf[i + (i < 16 ? 0 : 2 * OWN_EX - 16)] << 16 | ((oms >> q) & 1u);
+        uint32_t m = ~0u;
+        if (BS == 16) {
+          m = i < 16 ? mf : mn;
+        } else if (q - (w - 1) < (q / BS - 1) * BS) {
+          const int b = (q / BS - 1) * BS;
+          m = b < 0 ? mp : ((suf[b < 0 ? 0 : b] & 0xFFFF0001u) | 2u);
+        }
+        uint32_t v = pre[q] < c ? pre[q] : c;
+        v = m < v ? m : v;
+        out = __builtin_amdgcn_alignbit(v, out, 1);
+      }
+      out >>= 16;
+      out &= val;
+      // dirty ends among the w - 1 before a window's last
+      u128 dm = (u128)(om >> 16) << 64;
+      for (int o = 1; o <= OWN_HALO; o++) dm |= (u128)(ex[(tid - o) * OWN_EX + 8] >> 16) << (64 - 16 * o);
+      const bool edge = w == 1;
+      if (dm || edge) {
+        const uint32_t before = x > 0 ? W[x - 1] >> 15 : 0u;
+        const uint32_t first = val & ~(val << 1 | before);
+        u128 near = w > 1 ? dm << 1 : 0;
+        for (int c = 1; c < w - 1;) {
+          const int sh = c < w - 1 - c ? c : w - 1 - c;
+          near |= near << sh;
+          c += sh;
+        }
+        und = (uint32_t)(near >> 64) & 0xFFFFu & val & ~first;
+        out &= ~und;
+        // K = L: the reference's first window has no L-mer yet but 0
+        if (edge) out = (out & ~first) | ((ob[0] & 1u) ? first : 0u);
+      }
+    }
+    Wout[x] = (uint16_t)out;
+    D[x] = (uint16_t)und;
+  }
+}
+
+// The undecided windows (see above): a thread follows the runs that start in
+// its word, one after another.
+__global__ void k_own_walk(const uint32_t* E, const uint32_t* RX, const uint16_t* D, ull words, int w,
+                           const uint16_t* rank, const uint32_t* own, uint32_t* Wout) {
+  const ull x = (ull)blockIdx.x * blockDim.x + threadIdx.x;
+  if (x >= words) return;
+  const uint32_t d = D[x];
+  if (!d) return;
+  const uint32_t before = x ? D[x - 1] >> 15 : 0u;
+  auto lmer = [&](ull e, bool exact) -> uint32_t {
+    const ull i = e >> 4;
+    const uint32_t b =
+        __builtin_amdgcn_alignbit(E[PK_PAD + i - 1], E[PK_PAD + i], 30u - 2u * (uint32_t)(e & 15)) & 0xFFFFu;
+    return exact ? (b & ~1u) | ((RX[i] >> (e & 15)) & 1u) : b;
+  };
+  for (uint32_t st = d & ~(d << 1 | before); st; st &= st - 1) {
+    ull j = x * 16 + (ull)(__ffs(st) - 1);
+    // the window before: leftmost minimum of the rolling L-mers
+    uint32_t ml = 0, mr = ~0u;
+    int mp = 0;
+    for (int i = 0; i < w; i++) {
+      const uint32_t l = lmer(j - (ull)w + (ull)i, true), r = rank[l];
+      if (r < mr) {
+        mr = r;
+        ml = l;
+        mp = i - 1;
+      }
+    }
+    for (; j < words * 16 && (D[j >> 4] >> (j & 15) & 1u); j++) {
+      const uint32_t a = lmer(j, true), r = rank[a];
+      if (mp < 0) {
+        mr = ~0u;
+        for (int i = 0; i < w; i++) {
+          const uint32_t l = i == w - 1 ? a : lmer(j - (ull)(w - 1 - i), false), g = rank[l];
+          if (g < mr) {
+            mr = g;
+            ml = l;
+            mp = i;
+          }
+        }
+      }
+      if (r < mr) {
+        mr = r;
+        ml = a;
+        mp = w - 1;
+      }
+      mp--;
+      if (own[ml >> 5] >> (ml & 31u) & 1u) atomicOr(&Wout[j >> 5], 1u << (j & 31));
+    }
+  }
+}
+
+// The -p counters' rule (kmer_counting.cpp:1949-1950): the owner of a hash of
+// the whole k-mer.
+__global__ void k_own_key(const uint32_t* __restrict__ E, const uint32_t* __restrict__ RX,
+                          const uint16_t* __restrict__ W, ull words, ull mask, OwnerMod om, uint16_t* __restrict__ Wout) {
+  const ull x = (ull)blockIdx.x * blockDim.x + threadIdx.x;
+  if (x >= words) return;
+  const uint32_t val = W[x];
+  uint32_t out = 0;
+  if (val) {
+    const uint32_t e0 = E[PK_PAD + x - 2], e1 = E[PK_PAD + x - 1], e2 = E[PK_PAD + x], rx = RX[x];
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+      const uint32_t lo = __builtin_amdgcn_alignbit(e1, e2, 30u - 2u * (uint32_t)i);
+      const uint32_t hi = __builtin_amdgcn_alignbit(e0, e1, 30u - 2u * (uint32_t)i);
+      const ull key = ((ull)hi << 32 | (lo & ~1u) | ((rx >> i) & 1u)) & mask;
+      out |= (uint32_t)owner_is(owner_hash(key), om) << i;
+    }
+  }
+  Wout[x] = (uint16_t)(out & val);
+}
+
+// window ends per index block
+__global__ __launch_bounds__(256) void k_bits_count(const ull* W, uint32_t* cnt) {
+  static_assert(NL_PER_BLOCK == 64 * 256, "a word per thread");
+  const ull s = block_sum<256>((ull)__popcll(W[(ull)blockIdx.x * 256 + threadIdx.x]));
+  if (threadIdx.x == 0) cnt[blockIdx.x] = (uint32_t)s;
+}
+
 
 // ---------------------------------------------------------------------------
 // Per-bucket count: LDS hash table of the bucket's distinct keys (64-bit CAS,
@@ -3297,7 +3634,7 @@ __global__ void k_node_share_flags(const MnRec* nodes, uint64_t M, int P, int ra
   Key key;
   if (sizeof(Key) == 8) key = (Key)nodes[i].key_lo;
   else key = (Key)(((u128)nodes[i].key_hi << 64) | (u128)nodes[i].key_lo);
-  flag[i] = key_owner(key, P) == rank ? 1u : 0u;
+  flag[i] = (int)(owner_hash((ull)key) % (uint32_t)P) == rank ? 1u : 0u;
 }
 
 __global__ void k_node_share_write(const MnRec* nodes, uint64_t M, const uint32_t* flag, const ull* pos,
@@ -3321,7 +3658,7 @@ enum BufId {
   B_FASTA, B_BLK, B_BLKOFF, B_NL, B_RSTART, B_RLEN, B_KC, B_KOFS, B_SMALL, B_BCNT, B_BOFF, B_BCUR,
   B_S, B_C, B_TU, B_UOFF, B_TK, B_TC, B_HIST, B_KBS, B_KBOFF, B_KK, B_KC2, B_MNPLAN,
   B_MNNT, B_MNNG, B_MNNOFF, B_MNFLAG, B_NODES, B_TMP, B_OVF, B_PT0, B_PT1, B_PT2, B_PT3, B_PT4,
-  B_PT5, B_PT6, B_BLKGT, B_S2, B_BCNT2, B_BOFF2, B_BCUR2, B_TP, B_TP2, B_HIST1, B_OFF1, B_HIST2, B_OFF2, B_PACK, B_RETRY, B_WCNT, B_WOFF, B_CUTBH, B_LFREQ, B_WORDER, B_WIRE, B_NORM, B_NORMNL, B_NORMLEN, B_NORMOFF, B_NORMLS, B_NORMLL, B_SCAN0, B_SCAN1 = B_SCAN0 + 8, B_COUNT = B_SCAN0 + 16
+  B_PT5, B_PT6, B_BLKGT, B_S2, B_BCNT2, B_BOFF2, B_BCUR2, B_TP, B_TP2, B_HIST1, B_OFF1, B_HIST2, B_OFF2, B_PACK, B_RETRY, B_WCNT, B_WOFF, B_CUTBH, B_LFREQ, B_LPART, B_LBIG, B_LRANK, B_OWNW, B_OWNCNT, B_OWNOFF, B_WORDER, B_WIRE, B_NORM, B_NORMNL, B_NORMLEN, B_NORMOFF, B_NORMLS, B_NORMLL, B_SCAN0, B_SCAN1 = B_SCAN0 + 8, B_COUNT = B_SCAN0 + 16
 };
 
 }  // namespace
@@ -3783,6 +4120,7 @@ struct Records {
   const ull* tb = nullptr;  // main path: window ends before each index block
   uint64_t n = 0;  // input bytes
   uint64_t R = 0, N = 0;
+  bool part = false;  // one rank's windows only
   Packed pk;
 };
 
@@ -3794,8 +4132,9 @@ int format_error(pk_ctx* c, ull r) {
 int records_main(pk_ctx* c, const uint8_t* fa, uint64_t n, int K, Records* rec);
 
 // The windows of the main path from the packed input: valid ends and their
-// number per index block, no list of lines or reads.
-int windows_main(pk_ctx* c, const uint8_t* fa, uint64_t n, int K, Records* rec) {
+// number per index block, no list of lines or reads.  packed: the last call on
+// this stream packed the same input.
+int windows_main(pk_ctx* c, const uint8_t* fa, uint64_t n, int K, Records* rec, bool packed = false) {
   hipStream_t st = c->stream;
   ull* small;
   PK_TRY(need(c, B_SMALL, 16, &small));
@@ -3814,10 +4153,12 @@ int windows_main(pk_ctx* c, const uint8_t* fa, uint64_t n, int K, Records* rec) 
   PK_TRY(need(c, B_WOFF, nb + 1, &tb));
   rec->tb = tb;
   if (!nb) return PK_OK;
-  hipLaunchKernelGGL(HIP_KERNEL_NAME(k_pack<ENC_MAIN>), dim3((unsigned)nb), dim3(NL_NT), 0, st, fa, n, (uint8_t)'\n',
-                     (uint8_t)'\n', blk, blkgt, 0, pk.E, pk.RX);
-  PK_HIP(c, hipGetLastError());
-  PK_TRY(scan_excl<ull>(c, blk, blkoff, nb));
+  if (!packed) {
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_pack<ENC_MAIN>), dim3((unsigned)nb), dim3(NL_NT), 0, st, fa, n, (uint8_t)'\n',
+                       (uint8_t)'\n', blk, blkgt, 0, pk.E, pk.RX);
+    PK_HIP(c, hipGetLastError());
+    PK_TRY(scan_excl<ull>(c, blk, blkoff, nb));
+  }
   const bool check_long = n > 0xFFFFFFF0ull;
   if (check_long) {
     hipLaunchKernelGGL(k_long_lines, dim3(grid_for(nb, 256)), dim3(256), 0, st, blkoff, nb, small + 3);
@@ -4200,7 +4541,17 @@ int count_records(pk_ctx* c, const Records& rec, int K, int KB, Key mask) {
     if (tun.l1_bits > 0 && tun.l1_bits <= L1_MAX_BITS) return std::min(btot, tun.l1_bits);
     // one level of up to 10 bits while a bucket's runs fit the hash's map
     if (btot <= SP_MAX_BITS && tiles <= (uint64_t)RUN_CAP) return btot;
-    return level_bits(btot);
+    int b = level_bits(btot);
+    if (rec.part) {
+      // a share's tiles hold few keys (1 in P of their windows): a narrower
+      // first digit keeps its runs at 32 keys or so, two lines and more each,
+      // if the further levels can take the rest
+      const int nlev = (btot + SP_MAX_BITS - 1) / SP_MAX_BITS;
+      int f = 0;
+      while (f < b && (N / tiles) >> (f + 6)) f++;
+      b = std::min(b, std::max({1, f, btot - SP_MAX_BITS * (nlev - 1)}));
+    }
+    return b;
   };
   if (ENC == ENC_MAIN) {
     // tiles of 16 or 32 KiB of the input: the larger ones' runs are twice as
@@ -4250,14 +4601,14 @@ int count_records(pk_ctx* c, const Records& rec, int K, int KB, Key mask) {
   return count_partitioned<Key>(c, S, S2, C, p, btot, KB, N);
 }
 
-// One rank's share: level 1 walks every read in order with the owner rule and
-// scatters the owned keys into contiguous buckets.
+// The count without the packed input: level 1 walks every read and scatters its
+// keys into contiguous buckets.
 template <class Key>
-int count_share(pk_ctx* c, const uint8_t* fa, uint64_t n, const Records& rec, int K, OwnCfg cf) {
+int count_walk(pk_ctx* c, const uint8_t* fa, uint64_t n, const Records& rec, int K) {
   constexpr int CAP = HashCfg<Key>::LIMIT;
   hipStream_t st = c->stream;
   const uint64_t R = rec.R;
-  uint64_t N = rec.N;
+  const uint64_t N = rec.N;
   const int KB = 2 * K;
   const Key mask = key_mask<Key>(KB);
   PK_HIP(c, hipEventRecord(c->ev[1], st));
@@ -4266,8 +4617,7 @@ int count_share(pk_ctx* c, const uint8_t* fa, uint64_t n, const Records& rec, in
   if (empty) return PK_OK;
   const pk_tuning& tun = c->tuning;
   const float bf = tun.bucket_factor > 0.f ? tun.bucket_factor : HashCfg<Key>::FILL;
-  // with owner routing, about N / P instances are this rank's
-  const int btot = choose_bits((N + cf.P - 1) / cf.P, K, CAP, bf);
+  const int btot = choose_bits(N, K, CAP, bf);
   c->timing.bucket_bits = btot;
   const int d1 = std::min(btot, tun.l1_bits > 0 && tun.l1_bits <= L1_MAX_BITS ? tun.l1_bits : L1_DEFAULT_BITS);
   const uint64_t B1 = 1ull << d1;
@@ -4293,24 +4643,17 @@ int count_share(pk_ctx* c, const uint8_t* fa, uint64_t n, const Records& rec, in
   PK_TRY(need(c, B_C, N, &C));
   c->have_hist = true;
   PK_HIP(c, hipEventRecord(c->ev[2], st));
-  hipLaunchKernelGGL(HIP_KERNEL_NAME(k_l1_hist<Key, ENC_MAIN, true>), dim3((unsigned)nblk), dim3(L1_NT),
-                     l1_lds_bytes(sb, (int)B1, 4), st, fa, n, rec.rstart, rec.rlen, R, K, KB, mask, d1, rpb, sb, cf, H);
+  hipLaunchKernelGGL(HIP_KERNEL_NAME(k_l1_hist<Key, ENC_MAIN>), dim3((unsigned)nblk), dim3(L1_NT),
+                     l1_lds_bytes(sb, (int)B1, 4), st, fa, n, rec.rstart, rec.rlen, R, K, KB, mask, d1, rpb, sb, H);
   PK_HIP(c, hipGetLastError());
   PK_HIP(c, hipEventRecord(c->ev[3], st));
   PK_TRY(scan_excl<uint32_t>(c, H, O, B1 * nblk));
-  // this rank's instances
-  ull no = 0;
-  PK_TRY(d2h(c, &no, O + B1 * nblk, 8));
-  N = no;
-  PK_TRY(begin_count<Key>(c, R, N, K, &empty));
-  c->have_hist = true;
-  if (empty) return PK_OK;
   hipLaunchKernelGGL(k_l1_boff, dim3(grid_for(B1 + 1, 256)), dim3(256), 0, st, O, (int)B1, nblk, (ull)N,
                      boff);
   PK_HIP(c, hipGetLastError());
   PK_HIP(c, hipEventRecord(c->ev[4], st));
-  hipLaunchKernelGGL(HIP_KERNEL_NAME(k_l1_scatter<Key, ENC_MAIN, true>), dim3((unsigned)nblk), dim3(L1_NT),
-                     l1_lds_bytes(sb, (int)B1, 8), st, fa, n, rec.rstart, rec.rlen, R, K, KB, mask, d1, rpb, sb, cf, O,
+  hipLaunchKernelGGL(HIP_KERNEL_NAME(k_l1_scatter<Key, ENC_MAIN>), dim3((unsigned)nblk), dim3(L1_NT),
+                     l1_lds_bytes(sb, (int)B1, 8), st, fa, n, rec.rstart, rec.rlen, R, K, KB, mask, d1, rpb, sb, O,
                      nblk, S);
   PK_HIP(c, hipGetLastError());
   PK_HIP(c, hipEventRecord(c->ev[16], st));
@@ -4362,61 +4705,135 @@ int count_impl(pk_ctx* c, const uint8_t* fa, uint64_t n, int K) {
   rec.n = n;
   PK_TRY(pack_buffers(c, n, true, &rec.pk));
   if (!rec.pk.E) {
-    // pk_count_noalloc's scratch is short of the packed input: the walk of a
-    // share that owns every k-mer takes its place
+    // pk_count_noalloc's scratch is short of the packed input
     PK_TRY(records_main(c, fa, n, K, &rec));
-    return count_share<Key>(c, fa, n, rec, K, OwnCfg{nullptr, 1, 0, 1});
+    return count_walk<Key>(c, fa, n, rec, K);
   }
   PK_TRY(windows_main(c, fa, n, K, &rec));
   return count_records<Key, ENC_MAIN>(c, rec, K, 2 * K, key_mask<Key>(2 * K));
 }
 
 // L-mer frequencies of the whole input into freq (device, LMER_BINS u64),
-// with the record rule of Sliding_window_l (a record needs L bytes).
-int lmer_frequency_impl(pk_ctx* c, const uint8_t* fa, uint64_t n, ull** freq_out) {
-  Records rec;
-  PK_TRY(records_main(c, fa, n, LMER_L, &rec));
-  const uint64_t R = rec.R;
+// with the record rule of Sliding_window_l (a record needs L bytes).  Packs the
+// input into rec.
+int lmer_frequency_impl(pk_ctx* c, const uint8_t* fa, uint64_t n, Records* rec, ull** freq_out) {
+  hipStream_t st = c->stream;
+  rec->n = n;
+  PK_TRY(pack_buffers(c, n, true, &rec->pk));
+  PK_TRY(windows_main(c, fa, n, LMER_L, rec));
   ull* freq;
   PK_TRY(need(c, B_LFREQ, LMER_BINS, &freq));
   PK_TRY(fill_u64(c, freq, 0, LMER_BINS));
-  if (R) {
-    hipLaunchKernelGGL(k_lmer_freq, dim3((unsigned)std::min<uint64_t>(grid_for(R, 256), 4096)), dim3(256), 0,
-                       c->stream, fa, rec.rstart, rec.rlen, R, freq);
+  if (rec->N) {
+    const uint64_t nb = (n + NL_PER_BLOCK - 1) / NL_PER_BLOCK;
+    const int np = (int)std::min<uint64_t>(nb, (uint64_t)c->ncu);
+    uint32_t* part;
+    PK_TRY(need(c, B_LPART, (uint64_t)np * (LMER_BINS / 2), &part));
+    hipLaunchKernelGGL(k_lmer_count, dim3((unsigned)np), dim3(LM_NT), 0, st, rec->pk.E, rec->pk.RX,
+                       reinterpret_cast<const uint16_t*>(rec->pk.W), (ull)nb, part, freq);
+    PK_HIP(c, hipGetLastError());
+    hipLaunchKernelGGL(k_lmer_sum, dim3(LMER_BINS / 128), dim3(1024), 0, st, part, np, freq);
     PK_HIP(c, hipGetLastError());
   }
   *freq_out = freq;
   return PK_OK;
 }
 
-// One rank's share of the counted table at P ranks (the table rank `rank`
-// holds after the reference's all-to-all): the k-mers whose owner is rank.
-template <class Key>
-int rank_share_impl(pk_ctx* c, const uint8_t* fa, uint64_t n, int K, int P, int rank) {
-  c->have_table = c->have_kept = c->have_nodes = false;
-  c->timing = pk_timing{};
-  c->pend_count = c->pend_split = c->pend_cutoff = c->pend_mn = c->pend_norm = false;
-  c->key_bits = 2 * K;
-  PK_HIP(c, hipEventRecord(c->ev[0], c->stream));
-  ull* freq;
-  PK_TRY(lmer_frequency_impl(c, fa, n, &freq));
-  Records rec;
-  PK_TRY(records_main(c, fa, n, K, &rec));
-  return count_share<Key>(c, fa, n, rec, K, OwnCfg{freq, P, rank, 0});
+OwnerMod owner_mod(int P, int rank) {
+  int l = 0;
+  while ((1ull << l) < (ull)P) l++;
+  return OwnerMod{(1ull << (31 + l)) / (ull)P + 1, 31 + l, (uint32_t)P, (uint32_t)rank};
 }
 
-// One rank's share when every k-mer belongs to rank retrieve_proc_id(kmer)
-// (the -p counters, kmer_counting.cpp:1825-2091, 2095-2271).
+template <int BS>
+int launch_own(pk_ctx* c, const Records& rec, uint64_t words, int w, const uint4* tab, uint16_t* Wout, uint16_t* D) {
+  PK_HIP(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&k_own<BS>),
+                                hipFuncAttributeMaxDynamicSharedMemorySize, own_lds));
+  const uint64_t tiles = (words + (OWN_NT - OWN_HALO) - 1) / (OWN_NT - OWN_HALO);
+  hipLaunchKernelGGL(HIP_KERNEL_NAME(k_own<BS>), dim3((unsigned)std::min<uint64_t>(tiles, (uint64_t)c->ncu)),
+                     dim3(OWN_NT), own_lds, c->stream, rec.pk.E, rec.pk.RX, reinterpret_cast<const uint16_t*>(rec.pk.W),
+                     (ull)words, (ull)((rec.n + 15) / 16), w, tab, Wout, D);
+  PK_HIP(c, hipGetLastError());
+  return PK_OK;
+}
+
+// Leaves in rec only the window ends of one rank: of the minimum L-mer's owner
+// (freq), or of the whole k-mer's (freq null).
+int own_windows(pk_ctx* c, int K, const ull* freq, int P, int rank, Records* rec) {
+  hipStream_t st = c->stream;
+  const uint64_t nb = (rec->n + NL_PER_BLOCK - 1) / NL_PER_BLOCK, words = nb * (NL_PER_BLOCK / 16);
+  const OwnerMod om = owner_mod(P, rank);
+  uint16_t* wo;
+  PK_TRY(need(c, B_OWNW, 2 * words, &wo));
+  uint32_t* cnt;
+  ull* tb;
+  PK_TRY(need(c, B_OWNCNT, nb, &cnt));
+  PK_TRY(need(c, B_OWNOFF, nb + 1, &tb));
+  if (freq) {
+    uint32_t* tab;
+    ull* big;  // then their number
+    PK_TRY(need(c, B_LBIG, LMER_BINS + 1, &big));
+    PK_TRY(need(c, B_LRANK, OWN_TAB, &tab));
+    uint16_t* rk = reinterpret_cast<uint16_t*>(tab);
+    uint32_t* ob = tab + LMER_BINS / 2;
+    hipLaunchKernelGGL(k_freq_rank, dim3(1), dim3(1024), 0, st, freq, om, big, big + LMER_BINS, rk,
+                       reinterpret_cast<ull*>(ob));
+    PK_HIP(c, hipGetLastError());
+    hipLaunchKernelGGL(k_freq_big, dim3(LMER_BINS / 64), dim3(64), 0, st, freq, big, big + LMER_BINS, rk);
+    PK_HIP(c, hipGetLastError());
+    uint16_t* D = wo + words;
+    const uint4* t4 = reinterpret_cast<const uint4*>(tab);
+    const int w = K - LMER_L + 1;
+    if (w >= 16)
+      PK_TRY(launch_own<16>(c, *rec, words, w, t4, wo, D));
+    else if (w >= 8)
+      PK_TRY(launch_own<8>(c, *rec, words, w, t4, wo, D));
+    else if (w >= 4)
+      PK_TRY(launch_own<4>(c, *rec, words, w, t4, wo, D));
+    else if (w >= 2)
+      PK_TRY(launch_own<2>(c, *rec, words, w, t4, wo, D));
+    else
+      PK_TRY(launch_own<1>(c, *rec, words, w, t4, wo, D));
+    hipLaunchKernelGGL(k_own_walk, dim3(grid_for(words, 256)), dim3(256), 0, st, rec->pk.E, rec->pk.RX, D, (ull)words,
+                       w, rk, ob, reinterpret_cast<uint32_t*>(wo));
+    PK_HIP(c, hipGetLastError());
+  } else {
+    hipLaunchKernelGGL(k_own_key, dim3(grid_for(words, 256)), dim3(256), 0, st, rec->pk.E, rec->pk.RX,
+                       reinterpret_cast<const uint16_t*>(rec->pk.W), (ull)words, key_mask<uint64_t>(2 * K), om, wo);
+    PK_HIP(c, hipGetLastError());
+  }
+  hipLaunchKernelGGL(k_bits_count, dim3((unsigned)nb), dim3(256), 0, st, reinterpret_cast<const ull*>(wo), cnt);
+  PK_HIP(c, hipGetLastError());
+  PK_TRY(scan_excl<uint32_t>(c, cnt, tb, nb));
+  PK_TRY(d2h(c, &rec->N, tb + nb, 8));
+  rec->pk.W = reinterpret_cast<ull*>(wo);
+  rec->tb = tb;
+  rec->part = true;
+  return PK_OK;
+}
+
+// One rank's share of the counted table at P ranks (the table rank `rank`
+// holds after the reference's all-to-all): the k-mers whose owner is rank, by
+// the minimum L-mer or (by_key) retrieve_proc_id(kmer) (the -p counters,
+// kmer_counting.cpp:1825-2091, 2095-2271).
 template <class Key>
-int rank_share_key_impl(pk_ctx* c, const uint8_t* fa, uint64_t n, int K, int P, int rank) {
+int rank_share_impl(pk_ctx* c, const uint8_t* fa, uint64_t n, int K, int P, int rank, bool by_key) {
   c->have_table = c->have_kept = c->have_nodes = false;
   c->timing = pk_timing{};
   c->pend_count = c->pend_split = c->pend_cutoff = c->pend_mn = c->pend_norm = false;
   c->key_bits = 2 * K;
   PK_HIP(c, hipEventRecord(c->ev[0], c->stream));
   Records rec;
-  PK_TRY(records_main(c, fa, n, K, &rec));
-  return count_share<Key>(c, fa, n, rec, K, OwnCfg{nullptr, P, rank, 1});
+  ull* freq = nullptr;
+  if (by_key) {
+    rec.n = n;
+    PK_TRY(pack_buffers(c, n, true, &rec.pk));
+  } else {
+    PK_TRY(lmer_frequency_impl(c, fa, n, &rec, &freq));
+  }
+  PK_TRY(windows_main(c, fa, n, K, &rec, !by_key));
+  if (rec.N) PK_TRY(own_windows(c, K, freq, P, rank, &rec));
+  return count_records<Key, ENC_MAIN>(c, rec, K, 2 * K, key_mask<Key>(2 * K));
 }
 
 template <class Key>
@@ -5043,8 +5460,8 @@ int pk_count_rank_share(pk_ctx* c, const char* fasta, uint64_t nbytes, int k, in
   PK_HIP(c, hipSetDevice(c->device));
   const uint8_t* fa;
   PK_TRY(fasta_to_device(c, fasta, nbytes, fasta_on_device, &fa));
-  int rc = (k <= 32) ? rank_share_impl<uint64_t>(c, fa, nbytes, k, nranks, rank)
-                     : rank_share_impl<u128>(c, fa, nbytes, k, nranks, rank);
+  int rc = (k <= 32) ? rank_share_impl<uint64_t>(c, fa, nbytes, k, nranks, rank, false)
+                     : rank_share_impl<u128>(c, fa, nbytes, k, nranks, rank, false);
   if (rc) return rc;
   out->n = c->U;
   out->words = c->words;
@@ -5065,8 +5482,8 @@ int pk_count_rank_share_by_key(pk_ctx* c, const char* fasta, uint64_t nbytes, in
   PK_HIP(c, hipSetDevice(c->device));
   const uint8_t* fa;
   PK_TRY(fasta_to_device(c, fasta, nbytes, fasta_on_device, &fa));
-  int rc = (k <= 32) ? rank_share_key_impl<uint64_t>(c, fa, nbytes, k, nranks, rank)
-                     : rank_share_key_impl<u128>(c, fa, nbytes, k, nranks, rank);
+  int rc = (k <= 32) ? rank_share_impl<uint64_t>(c, fa, nbytes, k, nranks, rank, true)
+                     : rank_share_impl<u128>(c, fa, nbytes, k, nranks, rank, true);
   if (rc) return rc;
   out->n = c->U;
   out->words = c->words;
@@ -5083,7 +5500,8 @@ int pk_lmer_frequency(pk_ctx* c, const char* fasta, uint64_t nbytes, int fasta_o
   const uint8_t* fa;
   PK_TRY(fasta_to_device(c, fasta, nbytes, fasta_on_device, &fa));
   ull* freq;
-  PK_TRY(lmer_frequency_impl(c, fa, nbytes, &freq));
+  Records rec;
+  PK_TRY(lmer_frequency_impl(c, fa, nbytes, &rec, &freq));
   return d2h(c, freq_host, freq, LMER_BINS * 8);
 }
 

@@ -143,3 +143,60 @@ def test_macro_node_ranges(ctx, oracle_mod, k, n):
     assert m == want["keys"].shape[0]
     for f in ("keys", "pre_cnt", "suf_cnt"):
         assert np.array_equal(got[f], want[f]), f
+
+
+@pytest.mark.parametrize("k", [8, 9, 10, 11, 14, 15, 22, 23, 24, 32, 39, 40, 55, 56, 64])
+def test_share_windows(ctx, k):
+    """The share's window minima for every block size of the kernel and the
+    edges between them, over reads shorter and longer than a tile, with clean
+    stretches, isolated bytes whose third code bit is set, and runs of them;
+    against the window-by-window restatement of the reference."""
+    import rank_util as RU
+    rng = np.random.default_rng(k)
+    reads = []
+    for n, p in ((k, 0.0), (k + 1, 0.3), (20_000, 0.0), (12_000, 0.002), (150, 0.0), (400, 0.05), (400, 1.0),
+                 (k - 1, 0.0), (3_000, 0.2), (70, 0.02), (8_128 * 2, 0.0005)):
+        r = rng.choice(np.frombuffer(b"ACGT", dtype=np.uint8), n)
+        bad = rng.random(n) < p
+        r[bad] = rng.choice(np.frombuffer(b"NnHXYz", dtype=np.uint8), int(bad.sum()))
+        reads.append(r.tobytes())
+    reads.append(b"A" * 500 + b"N" + b"A" * 300)
+    fa = b"".join(b">%d\n%s\n" % (i, r) for i, r in enumerate(reads))
+    _p(f"case: share windows k={k}")
+    freq = RU.lmer_freq(fa)
+    assert np.array_equal(ctx.lmer_frequency(fa), freq)
+    walk = RU.owner_walk(fa, k, 3, freq)
+    for r in range(3):
+        ctx.count_rank_share(fa, k, 3, r)
+        keys, counts = ctx.table_host()
+        assert RU.table_counter(keys, counts) == RU.share_counter(walk, r), r
+
+
+def test_lmer_counts_past_16_bits(ctx):
+    """L-mers of one kind filling a block's 16-bit counters several times over,
+    between others, and frequencies that rank beyond the histogram's range."""
+    rng = np.random.default_rng(5)
+    acgt = np.frombuffer(b"ACGT", dtype=np.uint8)
+    part = [b"A" * 3_000_000, rng.choice(acgt, 500_000).tobytes(), b"C" * 300_000, b"AC" * 100_000]
+    reads = part * 8
+    fa = b"".join(b">r\n" + r + b"\n" for r in reads)
+    _p("case: L-mer counters past 16 bits")
+    want = np.zeros(1 << 16, dtype=np.uint64)
+    for r in part:
+        c = (np.frombuffer(r, dtype=np.uint8) >> 1) & 3
+        v = np.zeros(c.size - 7, dtype=np.int64)
+        for j in range(8):
+            v = (v << 2) | c[j:c.size - 7 + j]
+        want += 8 * np.bincount(v, minlength=1 << 16).astype(np.uint64)
+    assert np.array_equal(ctx.lmer_frequency(fa), want)
+    ctx.count(fa, 31)
+    keys, counts = ctx.table_host()
+    full = dict(zip(keys[:, 0].tolist(), counts.tolist()))
+    got = {}
+    for r in range(2):
+        ctx.count_rank_share(fa, 31, 2, r)
+        keys, counts = ctx.table_host()
+        one = dict(zip(keys[:, 0].tolist(), counts.tolist()))
+        assert not set(one) & set(got)
+        got.update(one)
+    assert got == full
