@@ -206,17 +206,36 @@ __global__ void k_fill_u64(ull* p, ull v, uint64_t n) {
   if (i < n) p[i] = v;
 }
 
-__global__ void k_copy_u64(ull* dst, const ull* src) { *dst = *src; }
+// Results on their way to the host: up to four pieces of 8-byte words, one
+// after another into the context's pinned words (box).
+constexpr int BOX_WORDS = 512;
+struct Post {
+  const ull* src[4];
+  int n[4];
+};
+
+__device__ __forceinline__ void post_words(const Post& p, ull* box) {
+  int i = (int)threadIdx.x;
+#pragma unroll
+  for (int q = 0; q < 4; q++) {
+    if (i >= 0 && i < p.n[q]) box[threadIdx.x] = p.src[q][i];
+    i -= p.n[q];
+  }
+}
+
+__global__ __launch_bounds__(BOX_WORDS) void k_post(Post p, ull* box) { post_words(p, box); }
 
 // ---------------------------------------------------------------------------
 // Exclusive scan (u32 or u64 in, u64 out, out[n] = total).  SCAN_PER
 // elements per 1024-thread block, SCAN_EPT consecutive ones per thread
 // (read and written as 16-byte vectors where aligned, so a thread's loads
-// are in flight together), recursive over block sums.
+// are in flight together).  Up to SCAN_ADD blocks add up the block sums before
+// their own themselves (8 KB at most); more scan them first.
 
 constexpr int SCAN_NT = 1024;
 constexpr int SCAN_EPT = 16;
 constexpr int SCAN_PER = SCAN_NT * SCAN_EPT;
+constexpr uint64_t SCAN_ADD = 1024;
 
 // elements [base, base + SCAN_EPT) of in, zero past n
 template <class T>
@@ -251,17 +270,26 @@ __global__ __launch_bounds__(SCAN_NT) void k_scan_reduce(const T* in, ull* sums,
   if (threadIdx.x == 0) sums[blockIdx.x] = s;
 }
 
+// offs: null (one block), the block sums (sums), or their scan.  box: the total
+// and the pieces of p go there too (the last block's).
 template <class T>
-__global__ __launch_bounds__(SCAN_NT) void k_scan_apply(const T* in, ull* out, const ull* offs,
-                                                        uint64_t n) {
+__global__ __launch_bounds__(SCAN_NT) void k_scan_apply(const T* in, ull* out, const ull* offs, bool sums,
+                                                        uint64_t n, Post p, ull* box) {
   const uint64_t base = (uint64_t)blockIdx.x * SCAN_PER + (uint64_t)threadIdx.x * SCAN_EPT;
   ull v[SCAN_EPT];
   scan_load<T>(in, n, base, v);
   ull s = 0;
 #pragma unroll
   for (int i = 0; i < SCAN_EPT; i++) s += v[i];
+  ull before = 0;
+  if (sums) {
+    for (uint32_t i = threadIdx.x; i < blockIdx.x; i += SCAN_NT) before += offs[i];
+    before = block_sum<SCAN_NT>(before);
+  } else if (offs) {
+    before = offs[blockIdx.x];
+  }
   const ull ex = block_excl_scan<SCAN_NT>(s);
-  ull o = (offs ? offs[blockIdx.x] : 0ull) + ex;
+  ull o = before + ex;
   if (base + SCAN_EPT <= n && (reinterpret_cast<uintptr_t>(out + base) & 15) == 0) {
     ulonglong2* q = reinterpret_cast<ulonglong2*>(out + base);
 #pragma unroll
@@ -279,7 +307,11 @@ __global__ __launch_bounds__(SCAN_NT) void k_scan_apply(const T* in, ull* out, c
     }
   }
   // the thread owning element n-1 writes the total
-  if (n > 0 && base <= n - 1 && n - 1 < base + SCAN_EPT) out[n] = o;
+  if (n > 0 && base <= n - 1 && n - 1 < base + SCAN_EPT) {
+    out[n] = o;
+    if (box) box[0] = o;
+  }
+  if (box && blockIdx.x == gridDim.x - 1) post_words(p, box + 1);
 }
 
 // ---------------------------------------------------------------------------
@@ -483,8 +515,10 @@ __device__ __forceinline__ uint32_t pack_bits(uint32_t t) { return ((t * 0x01020
 
 template <int ENC>
 __global__ __launch_bounds__(NL_NT) void k_pack(const uint8_t* fa, uint64_t n, uint8_t e0, uint8_t e1,
-                                                ull* blk_cnt, ull* blk_gt, int gt_all, uint32_t* E, uint32_t* RX) {
+                                                ull* blk_cnt, ull* blk_gt, int gt_all, uint32_t* E, uint32_t* RX, ull* small) {
   const uint64_t b0 = (uint64_t)blockIdx.x * NL_PER_BLOCK + (uint64_t)threadIdx.x * 16;
+  // the main path's flags (windows_main), before the kernels that set them
+  if (small && blockIdx.x == 0 && threadIdx.x < 4) small[2 + threadIdx.x] = threadIdx.x == 0 ? ~0ull : 0ull;
   const bool want_gt = gt_all || blockIdx.x == 0;
   const int lane = threadIdx.x & 63;
   uint32_t ev[NL_SLABS], gm[NL_SLABS];
@@ -577,8 +611,25 @@ __global__ __launch_bounds__(NL_NT) void k_nl_write_rx(const uint32_t* RX, uint6
 // lies at least K + 1 bytes before the end of the input (k_reads' rules, from
 // counts instead of positions).  lines: [0] j0, [1] R = records taken, [2]
 // '\n's of the input, [3] p0 (n when there is none).  One block.
-__global__ __launch_bounds__(1024) void k_lines(const uint32_t* RX, uint64_t n, const ull* blk_off, uint64_t nb,
-                                                const ull* gt, int K, ull* lines) {
+// blk (with nb <= SCAN_PER): the '\n's per block, scanned into blk_off first.
+__global__ __launch_bounds__(1024) void k_lines(const uint32_t* RX, uint64_t n, const ull* blk, ull* blk_off,
+                                                uint64_t nb, const ull* gt, int K, ull* lines) {
+  static_assert(SCAN_NT == 1024, "the scan's block");
+  if (blk) {
+    const uint64_t base = (uint64_t)threadIdx.x * SCAN_EPT;
+    ull v[SCAN_EPT], s = 0;
+    scan_load<ull>(blk, nb, base, v);
+#pragma unroll
+    for (int i = 0; i < SCAN_EPT; i++) s += v[i];
+    ull o = block_excl_scan<SCAN_NT>(s);
+#pragma unroll
+    for (int i = 0; i < SCAN_EPT; i++) {
+      if (base + i < nb) blk_off[base + i] = o;
+      o += v[i];
+      if (base + i + 1 == nb) blk_off[nb] = o;
+    }
+    __syncthreads();
+  }
   const ull p0 = *gt < n ? *gt : n;
   const uint64_t nw = (n + 15) / 16;
   const ull m = blk_off[nb];
@@ -1698,7 +1749,8 @@ __global__ __launch_bounds__(SM_NT, 8) void k_split_main(const uint32_t* __restr
                                                          const uint32_t* __restrict__ RX,
                                                          const uint16_t* __restrict__ W, const ull* __restrict__ tb,
                                                          ull nblk, ull nwords, Key mask, int dpos, int db,
-                                                         uint32_t* __restrict__ M, Key* __restrict__ Sout) {
+                                                         uint32_t* __restrict__ M, Key* __restrict__ Sout,
+                                                         ull* __restrict__ boff, ull* __restrict__ tp) {
   constexpr int NW = (int)sizeof(Key) / 4;
   constexpr int P = 16 * WPT;
   static_assert(NL_PER_BLOCK == 16ull * SM_NT, "a word of E per thread and index block");
@@ -1711,6 +1763,11 @@ __global__ __launch_bounds__(SM_NT, 8) void k_split_main(const uint32_t* __restr
   const int tid = (int)threadIdx.x;
   const ull t = blockIdx.x, nt = gridDim.x;
   const ull v0 = uniform(tb[t * WPT]);
+  if (t == 0 && tid < 2) {
+    // one parent bucket (k_tiles_one's facts)
+    boff[tid] = tid ? tb[nblk] : 0;
+    tp[tid] = tid ? nt : 0;
+  }
   const ull t1 = (t + 1) * WPT < nblk ? (t + 1) * WPT : nblk;
   const int m = (int)(uniform(tb[t1]) - v0);
   const ull w0 = t * (SM_NT * WPT);  // the tile's first word
@@ -3090,15 +3147,59 @@ __global__ void k_kept_from_hist(const uint32_t* BH, uint64_t nb, uint64_t U, in
 }
 
 // min_bucket = first argmin over hist[1..t-1]; an empty range gives t.
-__global__ void k_min_bucket(const ull* hist, int t, int* mb) {
-  if (threadIdx.x || blockIdx.x) return;
+__device__ __forceinline__ int first_min(const ull* hist, int t) {
   int best = t;
   if (t > 1) {
     best = 1;
     for (int i = 2; i < t; i++)
       if (hist[i] < hist[best]) best = i;
   }
-  *mb = best;
+  return best;
+}
+
+__global__ void k_min_bucket(const ull* hist, int t, int* mb) {
+  if (threadIdx.x || blockIdx.x) return;
+  *mb = first_min(hist, t);
+}
+
+// The four steps from the blocks' histograms to their kept entries' places in
+// one block, for up to CUT_PLAN blocks (a plasmid's cutoff is launches: each of
+// the four is 2 to 3 us of work and as much of gap).  The threshold, the kept
+// number and hn words of the histogram also go to box.
+constexpr uint64_t CUT_PLAN = 1024;
+__global__ __launch_bounds__(1024) void k_cut_plan(const uint32_t* __restrict__ BH, uint64_t nb, uint64_t U, int t,
+                                                   ull* __restrict__ hist, int* __restrict__ mb,
+                                                   ull* __restrict__ boffs, int hn, ull* __restrict__ box) {
+  __shared__ ull h[CUT_SMALL_T];
+  __shared__ int m;
+  const int lane = threadIdx.x & 63;
+  for (int c = (int)threadIdx.x >> 6; c < t; c += 16) {
+    ull s = 0;
+    for (uint64_t b = lane; b < nb; b += 64) s += BH[b * t + c];
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+    if (lane == 0) {
+      h[c] = s;
+      hist[c] = s;
+      if (c < hn) box[2 + c] = s;
+    }
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    m = first_min(h, t);
+    *mb = m;
+    box[1] = (ull)(uint32_t)m;
+  }
+  __syncthreads();
+  const uint64_t b = threadIdx.x;
+  ull kept = 0;
+  if (b < nb) {
+    kept = (b + 1) * CUT_PER <= U ? CUT_PER : U - b * CUT_PER;
+    for (int c = 0; c < m && c < t; c++) kept -= BH[b * t + c];
+  }
+  const ull ex = block_excl_scan<1024>(kept);
+  if (b < nb) boffs[b] = ex;
+  if (b + 1 == nb) boffs[nb] = box[0] = ex + kept;
 }
 
 __global__ __launch_bounds__(CUT_NT) void k_kept_count(const int32_t* TC, uint64_t U, const int* mb,
@@ -3663,23 +3764,6 @@ enum BufId {
 
 }  // namespace
 
-// Results on their way to the host: up to four pieces of 8-byte words, one
-// after another into the context's pinned words.
-constexpr int BOX_WORDS = 512;
-struct Post {
-  const ull* src[4];
-  int n[4];
-};
-
-__global__ __launch_bounds__(BOX_WORDS) void k_post(Post p, ull* box) {
-  int i = (int)threadIdx.x;
-#pragma unroll
-  for (int q = 0; q < 4; q++) {
-    if (i >= 0 && i < p.n[q]) box[threadIdx.x] = p.src[q][i];
-    i -= p.n[q];
-  }
-}
-
 struct pk_ctx {
   int device = 0;
   int ncu = 256;  // compute units of the device
@@ -3691,6 +3775,7 @@ struct pk_ctx {
   // 0-19: stage boundaries; 20 + 2 L, 21 + 2 L: around k_split of further
   // partition level L for the first MS_TIMED_LEVELS levels
   hipEvent_t ev[20 + 2 * MS_TIMED_LEVELS] = {};
+  int ev_parsed = 1;  // the event at which the last count had its windows
   bool have_hist = false;  // the last count ran k_l1_hist
   int ms_levels = 0;  // further partition levels of the last count
   int ms_form[MS_TIMED_LEVELS] = {};  // their scatter forms (timed levels)
@@ -3814,30 +3899,33 @@ int fill_u64(pk_ctx* c, ull* p, ull v, uint64_t n) {
 }
 
 // out[0..n) = exclusive scan of in, out[n] = total.  level selects scratch.
+// With p the total and p's pieces (BOX_WORDS - 1 words at most, made by
+// earlier work) are left in c->box; the caller waits.
 template <class T>
-int scan_excl(pk_ctx* c, const T* in, ull* out, uint64_t n, int level = 0) {
+int scan_excl(pk_ctx* c, const T* in, ull* out, uint64_t n, int level = 0, const Post* p = nullptr) {
+  const Post none{};
+  ull* box = p ? c->box : nullptr;
   if (n == 0) {
-    return fill_u64(c, out, 0, 1);
+    PK_TRY(fill_u64(c, out, 0, 1));
+    if (p) {
+      c->box[0] = 0;
+      hipLaunchKernelGGL(k_post, dim3(1), dim3(BOX_WORDS), 0, c->stream, *p, c->box + 1);
+      PK_HIP(c, hipGetLastError());
+    }
+    return PK_OK;
   }
   if (level >= 8) return c->fail(PK_EINVAL, "scan too deep");
   const uint64_t nb = (n + SCAN_PER - 1) / SCAN_PER;
-  if (nb == 1) {
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_scan_apply<T>), dim3(1), dim3(SCAN_NT), 0, c->stream, in,
-                       out, (const ull*)nullptr, n);
+  ull* sums = nullptr;
+  if (nb > 1) {
+    PK_TRY(need(c, B_SCAN0 + level, nb + 1, &sums));
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_scan_reduce<T>), dim3((unsigned)nb), dim3(SCAN_NT), 0,
+                       c->stream, in, sums, n);
     PK_HIP(c, hipGetLastError());
-    return PK_OK;
+    if (nb > SCAN_ADD) PK_TRY(scan_excl<ull>(c, sums, sums, nb, level + 1));
   }
-  ull* sums;
-  PK_TRY(need(c, B_SCAN0 + level, nb + 1, &sums));
-  hipLaunchKernelGGL(HIP_KERNEL_NAME(k_scan_reduce<T>), dim3((unsigned)nb), dim3(SCAN_NT), 0,
-                     c->stream, in, sums, n);
-  PK_HIP(c, hipGetLastError());
-  PK_TRY(scan_excl<ull>(c, sums, sums, nb, level + 1));
-  hipLaunchKernelGGL(HIP_KERNEL_NAME(k_scan_apply<T>), dim3((unsigned)nb), dim3(SCAN_NT), 0,
-                     c->stream, in, out, (const ull*)sums, n);
-  PK_HIP(c, hipGetLastError());
-  // total = sums[nb]
-  hipLaunchKernelGGL(k_copy_u64, dim3(1), dim3(1), 0, c->stream, out + n, sums + nb);
+  hipLaunchKernelGGL(HIP_KERNEL_NAME(k_scan_apply<T>), dim3((unsigned)nb), dim3(SCAN_NT), 0, c->stream, in, out,
+                     (const ull*)sums, nb > 1 && nb <= SCAN_ADD, n, p ? *p : none, box);
   PK_HIP(c, hipGetLastError());
   return PK_OK;
 }
@@ -3852,6 +3940,14 @@ int fetch(pk_ctx* c, const Post& p) {
   if (n > BOX_WORDS) return c->fail(PK_EINVAL, "too many result words");
   hipLaunchKernelGGL(k_post, dim3(1), dim3((unsigned)((n + 63) / 64 * 64)), 0, c->stream, p, c->box);
   PK_HIP(c, hipGetLastError());
+  PK_HIP(c, hipStreamSynchronize(c->stream));
+  return PK_OK;
+}
+
+// scan_excl, then a wait: the total in c->box[0], p's pieces after it.
+template <class T>
+int scan_fetch(pk_ctx* c, const T* in, ull* out, uint64_t n, const Post& p) {
+  PK_TRY(scan_excl<T>(c, in, out, n, 0, &p));
   PK_HIP(c, hipStreamSynchronize(c->stream));
   return PK_OK;
 }
@@ -4025,7 +4121,7 @@ int event_index(pk_ctx* c, const uint8_t* fa, uint64_t n, uint8_t e0, uint8_t e1
   if (nb) {
     if (pk)
       hipLaunchKernelGGL(HIP_KERNEL_NAME(k_pack<ENC_BUILDER>), dim3((unsigned)nb), dim3(NL_NT), 0, st, fa, n, e0, e1,
-                         blk, blkgt, 0, pk->E, pk->RX);
+                         blk, blkgt, 0, pk->E, pk->RX, (ull*)nullptr);
     else
       hipLaunchKernelGGL(k_nl_count, dim3((unsigned)nb), dim3(NL_NT), 0, st, fa, n, e0, e1, blk, blkgt, 0);
     PK_HIP(c, hipGetLastError());
@@ -4175,9 +4271,11 @@ int windows_main(pk_ctx* c, const uint8_t* fa, uint64_t n, int K, Records* rec, 
   PK_TRY(need(c, B_SMALL, 16, &small));
   // small[2] = first format error, [3] = a line may be too long, [4], [5] =
   // overflow and retry counts, [6] .. [9] = k_lines' facts, [10] = first '>'
-  PK_TRY(fill_u64(c, small + 2, ~0ull, 1));
-  PK_TRY(fill_u64(c, small + 3, 0, 3));
   const uint64_t nb = (n + NL_PER_BLOCK - 1) / NL_PER_BLOCK;
+  if (packed || !nb) {
+    PK_TRY(fill_u64(c, small + 2, ~0ull, 1));
+    PK_TRY(fill_u64(c, small + 3, 0, 3));
+  }
   const Packed& pk = rec->pk;
   ull *blk, *blkoff, *blkgt, *tb;
   uint32_t* cnt;
@@ -4190,9 +4288,9 @@ int windows_main(pk_ctx* c, const uint8_t* fa, uint64_t n, int K, Records* rec, 
   if (!nb) return PK_OK;
   if (!packed) {
     hipLaunchKernelGGL(HIP_KERNEL_NAME(k_pack<ENC_MAIN>), dim3((unsigned)nb), dim3(NL_NT), 0, st, fa, n, (uint8_t)'\n',
-                       (uint8_t)'\n', blk, blkgt, 0, pk.E, pk.RX);
+                       (uint8_t)'\n', blk, blkgt, 0, pk.E, pk.RX, small);
     PK_HIP(c, hipGetLastError());
-    PK_TRY(scan_excl<ull>(c, blk, blkoff, nb));
+    if (nb > SCAN_PER) PK_TRY(scan_excl<ull>(c, blk, blkoff, nb));
   }
   const bool check_long = n > 0xFFFFFFF0ull;
   if (check_long) {
@@ -4204,15 +4302,15 @@ int windows_main(pk_ctx* c, const uint8_t* fa, uint64_t n, int K, Records* rec, 
   // second pass looks for it everywhere
   const ull* gt = blkgt;
   for (int pass = 0;; pass++) {
-    hipLaunchKernelGGL(k_lines, dim3(1), dim3(1024), 0, st, pk.RX, n, blkoff, nb, gt, K, small + 6);
+    hipLaunchKernelGGL(k_lines, dim3(1), dim3(1024), 0, st, pk.RX, n,
+                       (const ull*)(nb <= SCAN_PER && !packed && pass == 0 ? blk : nullptr), blkoff, nb, gt, K, small + 6);
     PK_HIP(c, hipGetLastError());
     hipLaunchKernelGGL(k_valid, dim3((unsigned)nb), dim3(NL_NT), 0, st, pk.RX, n, blkoff, small + 6, K, pk.W, cnt,
                        small + 2);
     PK_HIP(c, hipGetLastError());
-    PK_TRY(scan_excl<uint32_t>(c, cnt, tb, nb));
-    PK_TRY(fetch(c, Post{{small + 2, tb + nb}, {8, 1}}));
-    memcpy(hs, c->box, sizeof(hs));
-    N = c->box[8];
+    PK_TRY(scan_fetch<uint32_t>(c, cnt, tb, nb, Post{{small + 2}, {8}}));
+    N = c->box[0];
+    memcpy(hs, c->box + 1, sizeof(hs));
     if (hs[7] < n || pass || nb == 1) break;
     hipLaunchKernelGGL(k_nl_count, dim3((unsigned)nb), dim3(NL_NT), 0, st, fa, n, (uint8_t)'\n', (uint8_t)'\n', blk,
                        blkgt, 1);
@@ -4413,7 +4511,6 @@ int count_partitioned(pk_ctx* c, Key* S, Key* S2, int32_t* C, Part p, int btot, 
   PK_TRY(need(c, B_RETRY, B, &retry));
   PK_TRY(need(c, B_OVF, B + 1, &ovl));
   PK_TRY(need(c, B_UOFF, B + 1, &uoff));
-  PK_HIP(c, hipEventRecord(c->ev[6], st));
   const unsigned rgrid = (unsigned)std::min<uint64_t>(B, 4ull * (uint64_t)c->ncu);
   if (in.M) {
     hipLaunchKernelGGL(HIP_KERNEL_NAME(k_bucket_hash<Key, true>), dim3((unsigned)B), dim3(HashCfg<Key>::NT), 0, st, S, Res, C,
@@ -4432,12 +4529,11 @@ int count_partitioned(pk_ctx* c, Key* S, Key* S2, int32_t* C, Part p, int btot, 
   PK_HIP(c, hipEventRecord(c->ev[7], st));
   // the scan of the distinct counts goes ahead of the overflow check: with
   // no oversize bucket (the usual case) one synchronisation yields both
-  PK_TRY(scan_excl<long long>(c, tu, uoff, B));
-  PK_TRY(fetch(c, Post{{small + 4, uoff + B}, {1, 1}}));
-  const ull hv[2] = {c->box[0], c->box[1]};
+  PK_TRY(scan_fetch<long long>(c, tu, uoff, B, Post{{small + 4}, {1}}));
+  const ull hv[2] = {c->box[1], c->box[0]};
   const ull novf = hv[0];
   c->timing.n_split = (int32_t)novf;
-  PK_HIP(c, hipEventRecord(c->ev[8], st));
+  if (novf) PK_HIP(c, hipEventRecord(c->ev[8], st));
   const ull* lstart = bstart;
   const long long* lu = tu;
   uint64_t nleaves = B;
@@ -4500,7 +4596,7 @@ int count_partitioned(pk_ctx* c, Key* S, Key* S2, int32_t* C, Part p, int btot, 
     lstart = lsd;
     lu = lud;
   }
-  PK_HIP(c, hipEventRecord(c->ev[9], st));
+  if (novf) PK_HIP(c, hipEventRecord(c->ev[9], st));
   ull U = hv[1];
   if (novf) {
     PK_TRY(scan_excl<long long>(c, lu, uoff, nleaves));
@@ -4553,8 +4649,8 @@ template <class Key, int ENC>
 int count_records(pk_ctx* c, const Records& rec, int K, int KB, Key mask) {
   constexpr int CAP = HashCfg<Key>::LIMIT;
   hipStream_t st = c->stream;
+  c->ev_parsed = 4;
   const uint64_t N = rec.N;
-  PK_HIP(c, hipEventRecord(c->ev[1], st));
   bool empty;
   PK_TRY(begin_count<Key>(c, rec.R, N, K, &empty));
   if (empty) return PK_OK;
@@ -4593,16 +4689,14 @@ int count_records(pk_ctx* c, const Records& rec, int K, int KB, Key mask) {
     tiles = (nblk + wpt - 1) / wpt;
     d1 = level1_bits();
     PK_TRY(level_buffers(c, 0, 1, tiles, d1, &l));
-    hipLaunchKernelGGL(k_tiles_one, dim3(1), dim3(1), 0, st, (ull)tiles, (ull)N, l.boff, l.tp);
-    PK_HIP(c, hipGetLastError());
     PK_HIP(c, hipEventRecord(c->ev[4], st));
     const uint16_t* W = reinterpret_cast<const uint16_t*>(rec.pk.W);
     if (wpt == 2)
       hipLaunchKernelGGL(HIP_KERNEL_NAME(k_split_main<Key, 2>), dim3((unsigned)tiles), dim3(SM_NT), 0, st, rec.pk.E,
-                         rec.pk.RX, W, rec.tb, (ull)nblk, (ull)((rec.n + 15) / 16), mask, KB - d1, d1, l.M, S);
+                         rec.pk.RX, W, rec.tb, (ull)nblk, (ull)((rec.n + 15) / 16), mask, KB - d1, d1, l.M, S, l.boff, l.tp);
     else
       hipLaunchKernelGGL(HIP_KERNEL_NAME(k_split_main<Key, 1>), dim3((unsigned)tiles), dim3(SM_NT), 0, st, rec.pk.E,
-                         rec.pk.RX, W, rec.tb, (ull)nblk, (ull)((rec.n + 15) / 16), mask, KB - d1, d1, l.M, S);
+                         rec.pk.RX, W, rec.tb, (ull)nblk, (ull)((rec.n + 15) / 16), mask, KB - d1, d1, l.M, S, l.boff, l.tp);
     p.in.tb = rec.tb;
     p.in.ts = wpt - 1;
   } else {
@@ -4644,6 +4738,7 @@ int count_walk(pk_ctx* c, const uint8_t* fa, uint64_t n, const Records& rec, int
   const int KB = 2 * K;
   const Key mask = key_mask<Key>(KB);
   PK_HIP(c, hipEventRecord(c->ev[1], st));
+  c->ev_parsed = 1;
   bool empty;
   PK_TRY(begin_count<Key>(c, R, N, K, &empty));
   if (empty) return PK_OK;
@@ -4701,6 +4796,7 @@ int windows_count_impl(pk_ctx* c, const uint8_t* fa, const ull* rstart, const ui
   hipStream_t st = c->stream;
   c->key_bits = -1;  // byte-rank codes: no macro nodes on this table
   PK_HIP(c, hipEventRecord(c->ev[1], st));
+  c->ev_parsed = 1;
   bool empty;
   PK_TRY(begin_count<Key>(c, R, N, klen, &empty));
   if (empty) return PK_OK;
@@ -4836,8 +4932,8 @@ int own_windows(pk_ctx* c, int K, const ull* freq, int P, int rank, Records* rec
   }
   hipLaunchKernelGGL(k_bits_count, dim3((unsigned)nb), dim3(256), 0, st, reinterpret_cast<const ull*>(wo), cnt);
   PK_HIP(c, hipGetLastError());
-  PK_TRY(scan_excl<uint32_t>(c, cnt, tb, nb));
-  PK_TRY(d2h(c, &rec->N, tb + nb, 8));
+  PK_TRY(scan_fetch<uint32_t>(c, cnt, tb, nb, Post{}));
+  rec->N = c->box[0];
   rec->pk.W = reinterpret_cast<ull*>(wo);
   rec->tb = tb;
   rec->part = true;
@@ -4896,8 +4992,11 @@ int cutoff_impl(pk_ctx* c, int t, uint64_t* hist_out, int* mb_out, uint64_t* nk_
   ull* small;
   PK_TRY(need(c, B_HIST, (uint64_t)t + 8, &hist));
   PK_TRY(need(c, B_SMALL, 16, &small));
-  PK_TRY(fill_u64(c, hist, 0, (uint64_t)t));
   const uint64_t nb = (U + CUT_PER - 1) / CUT_PER;
+  const bool want_hist = hist_out && fixed_mb <= 0;
+  const int hn = want_hist && t <= BOX_WORDS - 3 ? t : 0;  // histogram words that fit the box
+  const bool plan = fixed_mb <= 0 && t <= CUT_SMALL_T && nb && nb <= CUT_PLAN;
+  if (!plan) PK_TRY(fill_u64(c, hist, 0, (uint64_t)t));
   int* mbd = reinterpret_cast<int*>(small + 8);
   ull *bs, *boffs;
   PK_TRY(need(c, B_KBS, nb + 1, &bs));
@@ -4915,12 +5014,20 @@ int cutoff_impl(pk_ctx* c, int t, uint64_t* hist_out, int* mb_out, uint64_t* nk_
     if (nb) {
       hipLaunchKernelGGL(k_count_hist_blocks, dim3((unsigned)nb), dim3(CUT_NT), 0, st, TC, U, t, BH);
       PK_HIP(c, hipGetLastError());
+    }
+    if (plan) {
+      hipLaunchKernelGGL(k_cut_plan, dim3(1), dim3(1024), 0, st, BH, nb, U, t, hist, mbd, boffs, hn, c->box);
+      PK_HIP(c, hipGetLastError());
+      PK_HIP(c, hipStreamSynchronize(st));
+    } else if (nb) {
       hipLaunchKernelGGL(k_hist_columns, dim3((unsigned)t), dim3(1024), 0, st, BH, nb, t, hist);
       PK_HIP(c, hipGetLastError());
     }
-    hipLaunchKernelGGL(k_min_bucket, dim3(1), dim3(1), 0, st, hist, t, mbd);
-    PK_HIP(c, hipGetLastError());
-    if (nb) {
+    if (!plan) {
+      hipLaunchKernelGGL(k_min_bucket, dim3(1), dim3(1), 0, st, hist, t, mbd);
+      PK_HIP(c, hipGetLastError());
+    }
+    if (nb && !plan) {
       hipLaunchKernelGGL(k_kept_from_hist, dim3(grid_for(nb, 256)), dim3(256), 0, st, BH, nb, U, t,
                          mbd, bs);
       PK_HIP(c, hipGetLastError());
@@ -4937,15 +5044,12 @@ int cutoff_impl(pk_ctx* c, int t, uint64_t* hist_out, int* mb_out, uint64_t* nk_
       PK_HIP(c, hipGetLastError());
     }
   }
-  PK_TRY(scan_excl<ull>(c, bs, boffs, nb));
-  ull V = 0;
-  int mb = 0;
-  const bool want_hist = hist_out && fixed_mb <= 0;
-  const int hn = want_hist && t <= BOX_WORDS - 2 ? t : 0;  // histogram words that fit the box
-  if (want_hist && !hn) PK_HIP(c, hipMemcpyAsync(hist_out, hist, (size_t)t * 8, hipMemcpyDeviceToHost, st));
-  PK_TRY(fetch(c, Post{{boffs + nb, small + 8, hist}, {1, 1, hn}}));
-  V = c->box[0];
-  mb = (int)(uint32_t)c->box[1];
+  if (!plan) {
+    if (want_hist && !hn) PK_HIP(c, hipMemcpyAsync(hist_out, hist, (size_t)t * 8, hipMemcpyDeviceToHost, st));
+    PK_TRY(scan_fetch<ull>(c, bs, boffs, nb, Post{{small + 8, hist}, {1, hn}}));
+  }
+  const ull V = c->box[0];
+  const int mb = (int)(uint32_t)c->box[1];
   if (hn) memcpy(hist_out, c->box + 2, (size_t)t * 8);
   Key* KK;
   int32_t* KC;
@@ -4992,9 +5096,8 @@ int mn_impl(pk_ctx* c) {
   hipLaunchKernelGGL(HIP_KERNEL_NAME(k_mn_rank<Key>), dim3((unsigned)G), dim3(MN_NT), 0, st, KK, K, bd, (ull)G, rk,
                      rk + V, ng);
   PK_HIP(c, hipGetLastError());
-  PK_TRY(scan_excl<ull>(c, ng, noff, G));
-  ull M = 0;
-  PK_TRY(d2h(c, &M, noff + G, 8));
+  PK_TRY(scan_fetch<ull>(c, ng, noff, G, Post{}));
+  const ull M = c->box[0];
   PK_TRY(need(c, B_NODES, M, &nodes));
   hipLaunchKernelGGL(HIP_KERNEL_NAME(k_mn_write<Key>), dim3((unsigned)G), dim3(MN_NT), 0, st, KK, KC, K, bd, (ull)G,
                      rk, rk + V, noff, nodes);
@@ -5796,11 +5899,11 @@ int pk_last_timing(const pk_ctx* cc, pk_timing* out) {
     PK_HIP(c, hipStreamSynchronize(c->stream));
   }
   if (c->pend_count) {
-    c->timing.parse_ms = el(0, 1);
+    c->timing.parse_ms = el(0, c->ev_parsed);
     c->timing.hist_ms = c->have_hist ? el(2, 3) : 0.f;
     c->timing.scatter_ms = el(4, 5);
     c->timing.l1_scatter_ms = el(4, 16);
-    c->timing.sort_ms = el(6, 7);
+    c->timing.sort_ms = el(5, 7);
     c->timing.split_ms = c->pend_split ? el(8, 9) : 0.f;
     c->timing.compact_ms = el(10, 11);
     const int nl = c->ms_levels < MS_TIMED_LEVELS ? c->ms_levels : MS_TIMED_LEVELS;

@@ -200,3 +200,27 @@ def test_lmer_counts_past_16_bits(ctx):
         assert not set(one) & set(got)
         got.update(one)
     assert got == full
+
+
+@pytest.mark.parametrize("u", [16_384 * 1024, 16_384 * 1024 + 1, 16_383, 16_385, 40])
+@pytest.mark.parametrize("t", [2, 3])
+def test_cutoff_plan(ctx, u, t):
+    """Tables of one block of the cutoff, one entry less and more, and of as
+    many blocks as one launch plans and one more entry: histogram, threshold
+    and kept entries against the table's own counts."""
+    rng = np.random.default_rng(u)
+    k = 31
+    r = rng.choice(np.frombuffer(b"ACGT", dtype=np.uint8), u + k - 1).tobytes()
+    fa = b">a\n" + r + b"\n>b\n" + r[:min(u // 3 + k, 5000)] + b"\n"
+    _p(f"case: cutoff u={u} t={t}")
+    ctx.count(fa, k)
+    keys, counts = ctx.table_host()
+    assert keys.shape[0] == u
+    hist, mb, nk = ctx.cutoff(t)
+    want = np.bincount(counts, minlength=t)[:t].astype(np.uint64)
+    assert np.array_equal(np.asarray(hist)[1:t], want[1:t])
+    wmb = 1 + int(np.argmin(want[1:t]))
+    keep = counts >= wmb
+    assert mb == wmb and nk == int(keep.sum())
+    kk, kc = ctx.kept_host()
+    assert np.array_equal(kk, keys[keep]) and np.array_equal(kc, counts[keep])
