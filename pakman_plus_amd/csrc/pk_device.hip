@@ -11,8 +11,8 @@
 //                     the reference's Sliding_window (src/kmer_counting.cpp:
 //                     2890-2945).  A rank share keeps the ends its owner rule
 //                     gives the rank (k_own, k_own_walk, k_own_key); the
-//                     builder API's records come from k_bld_flags /
-//                     k_bld_write.
+//                     builder API's come from k_bld_bits, or
+//                     as a read table from k_bld_flags / k_bld_write.
 //   3. partition      k_split_main, k_split: tiles of k-mers sorted by a digit of the key's
 //                     top bits, one tile per block, each tile written back
 //                     as one contiguous piece with a table of where its
@@ -913,6 +913,37 @@ __device__ __forceinline__ bool bld_record(const uint8_t* fa, uint64_t n, const 
   *rb = ev[e2] + 1;
   *rl = read_len < n - *rb ? read_len : n - *rb;
   return *rl >= (uint64_t)klen;
+}
+
+// Window ends of the records as k_valid's bitmap (W, cleared before), where a
+// key is its window alone (klen >= the word's bases): a thread per event sets
+// the ends of its record, two words for a read of 100 bytes, and no list of
+// reads is made.  stat[0] = records, stat[1] set when a read runs on into the
+// next event: its windows can then end where another's do, which one bit
+// cannot say, and the read table takes its place (2 Mbp at 60x, klen = 32: the
+// table and level 1 from it 520 us, the ends and k_split_main 240; blocks that
+// loop, because one counter takes an add per block: 184 -> 62 us).
+__global__ __launch_bounds__(256) void k_bld_bits(const uint8_t* fa, uint64_t n, const ull* ev, uint64_t m, int klen,
+                                                  uint64_t read_len, BldSyms sy, ull* W, ull* stat) {
+  ull rec = 0;
+  for (uint64_t e = (uint64_t)blockIdx.x * 256 + threadIdx.x; e < m; e += (uint64_t)gridDim.x * 256) {
+    uint64_t rb, rl;
+    if (!bld_record(fa, n, ev, m, e, klen, read_len, sy, &rb, &rl)) continue;
+    rec++;
+    // the header's delimiter lies right before the read
+    uint64_t e2 = e + 1;
+    while (e2 < m && ev[e2] < rb) e2++;
+    if (e2 < m && ev[e2] < rb + rl) stat[1] = 1;
+    const ull a = rb + (uint64_t)klen - 1, b = rb + rl;  // ends [a, b)
+    for (ull w = a >> 6; w * 64 < b; w++) {
+      ull bits = ~0ull;
+      if (w * 64 < a) bits &= ~0ull << (a & 63);
+      if (w * 64 + 64 > b) bits &= (1ull << (b & 63)) - 1;
+      atomicOr(&W[w], bits);
+    }
+  }
+  rec = block_sum<256>(rec);
+  if (threadIdx.x == 0 && rec) atomicAdd(&stat[0], rec);
 }
 
 __global__ void k_bld_flags(const uint8_t* fa, uint64_t n, const ull* ev, uint64_t m, int klen,
@@ -4371,7 +4402,8 @@ int records_main(pk_ctx* c, const uint8_t* fa, uint64_t n, int K, Records* rec) 
 }
 
 // Read table of the builder API (bld_record).
-int records_builder(pk_ctx* c, const uint8_t* fa, uint64_t n, int klen, uint64_t read_len, BldSyms sy,
+// key_bases: bases of a key.
+int records_builder(pk_ctx* c, const uint8_t* fa, uint64_t n, int klen, uint64_t read_len, BldSyms sy, int key_bases,
                     Records* rec) {
   hipStream_t st = c->stream;
   ull* small;
@@ -4380,8 +4412,31 @@ int records_builder(pk_ctx* c, const uint8_t* fa, uint64_t n, int klen, uint64_t
   PK_TRY(fill_u64(c, small + 4, 0, 2));
   ull* ev;
   uint64_t m, p0;
-  PK_TRY(pack_buffers(c, n, false, &rec->pk));
+  const bool ends = klen >= key_bases;
+  PK_TRY(pack_buffers(c, n, ends, &rec->pk));
   PK_TRY(event_index(c, fa, n, sy.delim, sy.skip, small, &ev, &m, &p0, B_NL, 0, &rec->pk));
+  rec->n = n;
+  if (ends && m) {
+    const uint64_t nb = (n + NL_PER_BLOCK - 1) / NL_PER_BLOCK;
+    uint32_t* cnt;
+    ull* tb;
+    PK_TRY(need(c, B_WCNT, nb, &cnt));
+    PK_TRY(need(c, B_WOFF, nb + 1, &tb));
+    PK_TRY(fill_u64(c, rec->pk.W, 0, nb * (NL_PER_BLOCK / 64)));
+    PK_TRY(fill_u64(c, small + 6, 0, 2));
+    hipLaunchKernelGGL(k_bld_bits, dim3(std::min<unsigned>(grid_for(m, 256), 8u * (unsigned)c->ncu)), dim3(256), 0, st, fa, n, ev, m, klen, read_len, sy,
+                       rec->pk.W, small + 6);
+    PK_HIP(c, hipGetLastError());
+    hipLaunchKernelGGL(k_bits_count, dim3((unsigned)nb), dim3(256), 0, st, (const ull*)rec->pk.W, cnt);
+    PK_HIP(c, hipGetLastError());
+    PK_TRY(scan_fetch<uint32_t>(c, cnt, tb, nb, Post{{small + 6}, {2}}));
+    if (!c->box[2]) {
+      rec->N = c->box[0];
+      rec->R = c->box[1];
+      rec->tb = tb;
+      return PK_OK;
+    }
+  }
   ull *rstart, *kofs, *idx;
   uint32_t *rlen, *kc, *flag;
   PK_TRY(need(c, B_RSTART, m + 1, &rstart));
@@ -4681,7 +4736,7 @@ int count_records(pk_ctx* c, const Records& rec, int K, int KB, Key mask) {
     }
     return b;
   };
-  if (ENC == ENC_MAIN) {
+  if (ENC == ENC_MAIN || rec.tb) {
     // tiles of 16 or 32 KiB of the input: the larger ones' runs are twice as
     // long, the smaller ones spread an input over more CUs
     const uint64_t nblk = (rec.n + NL_PER_BLOCK - 1) / NL_PER_BLOCK;
@@ -4699,7 +4754,7 @@ int count_records(pk_ctx* c, const Records& rec, int K, int KB, Key mask) {
                          rec.pk.RX, W, rec.tb, (ull)nblk, (ull)((rec.n + 15) / 16), mask, KB - d1, d1, l.M, S, l.boff, l.tp);
     p.in.tb = rec.tb;
     p.in.ts = wpt - 1;
-  } else {
+  } else if constexpr (ENC == ENC_BUILDER) {
     // tiles of N / 512 windows (so that a small input spreads over the CUs and
     // a bucket has at most RUN_CAP runs), within 4096 and a full tile
     const uint64_t per = (N + RUN_CAP - 1) / RUN_CAP;
@@ -4973,7 +5028,7 @@ int builder_count_impl(pk_ctx* c, const uint8_t* fa, uint64_t n, int klen, uint6
   c->key_bits = (int)sizeof(Key) * 8;
   PK_HIP(c, hipEventRecord(c->ev[0], c->stream));
   Records rec;
-  PK_TRY(records_builder(c, fa, n, klen, read_len, sy, &rec));
+  PK_TRY(records_builder(c, fa, n, klen, read_len, sy, (int)sizeof(Key) * 4, &rec));
   return count_records<Key, ENC_BUILDER>(c, rec, klen, (int)sizeof(Key) * 8, ~Key(0));
 }
 

@@ -224,3 +224,21 @@ def test_cutoff_plan(ctx, u, t):
     assert mb == wmb and nk == int(keep.sum())
     kk, kc = ctx.kept_host()
     assert np.array_equal(kk, keys[keep]) and np.array_equal(kc, counts[keep])
+
+
+@pytest.mark.parametrize("klen,bits", [(32, 64), (33, 64), (45, 64), (64, 128), (70, 128)])
+@pytest.mark.parametrize("read_len", [70, 100, 120, 121, 122, 300])
+def test_builder_window_ends(ctx, oracle_mod, klen, bits, read_len):
+    """Words shorter than or equal to the window, counted from window ends:
+    reads shorter than the line, equal to it, one and two bytes longer (the
+    '\n', then the next record's '>'), and spanning records, whose windows
+    overlap the next read's and need the read table."""
+    rng = np.random.default_rng(klen + read_len)
+    fa = b"".join(b">r%d\n" % i + _bases(rng, 120, b"ACGTN") + b"\n" for i in range(700))
+    _p(f"case: builder window ends klen={klen} bits={bits} read_len={read_len}")
+    n = ctx.builder_count(fa, klen, read_len=read_len, kmer_bits=bits)
+    keys, counts = ctx.table_host()
+    want_n, want_k, want_c = oracle_mod.builder_count(fa, klen, read_len, bits)
+    assert n == want_n
+    assert np.array_equal(keys.reshape(-1), np.asarray(want_k).reshape(-1))
+    assert np.array_equal(counts, want_c)
