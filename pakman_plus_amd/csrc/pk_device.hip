@@ -365,27 +365,6 @@ __device__ __forceinline__ uint4 scan16(const uint8_t* fa, uint64_t n, uint64_t 
   return make_uint4(w[0], w[1], w[2], w[3]);
 }
 
-// scan16 that also returns the 16 bytes (zero past n).
-__device__ __forceinline__ uint4 scan16_keep(const uint8_t* in, uint64_t n, uint64_t base, uint32_t e0,
-                                             uint32_t& ev) {
-  ev = 0;
-  uint4 v = make_uint4(0, 0, 0, 0);
-  if (base + 16 <= n && ((reinterpret_cast<uintptr_t>(in + base) & 15) == 0)) {
-    v = *reinterpret_cast<const uint4*>(in + base);
-    ev = match4(v.x, e0) | (match4(v.y, e0) << 4) | (match4(v.z, e0) << 8) | (match4(v.w, e0) << 12);
-  } else {
-    uint32_t w[4] = {0, 0, 0, 0};
-    for (int i = 0; i < 16; i++) {
-      if (base + i >= n) break;
-      const uint32_t b = in[base + i];
-      w[i >> 2] |= b << (8 * (i & 3));
-      ev |= (uint32_t)(b == e0) << i;
-    }
-    v = make_uint4(w[0], w[1], w[2], w[3]);
-  }
-  return v;
-}
-
 __device__ __forceinline__ uint8_t byte_of(const uint4& v, int i) {
   const uint32_t w = i < 8 ? (i < 4 ? v.x : v.y) : (i < 12 ? v.z : v.w);
   return (uint8_t)(w >> (8 * (i & 3)));
@@ -749,13 +728,38 @@ __global__ void k_long_lines(const ull* blk_off, uint64_t nb, ull* flag) {
   if (i + span <= nb && blk_off[i + span] == blk_off[i]) *flag = 1;
 }
 
+// a value that is the same in every lane, moved to scalar registers
+__device__ __forceinline__ ull uniform(ull x) {
+  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)x);
+  const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(x >> 32));
+  return (ull)hi << 32 | lo;
+}
+
+// Number of x[0..n) (ascending) that are <= key, found by the whole block:
+// NT samples per step instead of a chain of log2(n) dependent loads.
+template <int NT>
+__device__ __forceinline__ ull block_upper(const ull* x, ull n, ull key) {
+  ull lo = 0;
+  while (n > (ull)NT) {
+    const ull step = (n + NT - 1) / NT;
+    const ull o = (ull)threadIdx.x * step;
+    const int c = __syncthreads_count(o < n && x[lo + o] <= key);
+    if (c == 0) return lo;
+    // sample c - 1 is <= key, sample c (if any) is not
+    const ull skip = (ull)(c - 1) * step;
+    lo += skip;
+    n = n - skip < step ? n - skip : step;
+  }
+  return lo + (ull)__syncthreads_count((ull)threadIdx.x < n && x[lo + threadIdx.x] <= key);
+}
+
 // ---------------------------------------------------------------------------
 // Input formats: multi-line FASTA and four-line FASTQ (either with '\r\n'
 // line ends) rewritten into the strict single-line FASTA the counting path
 // reads.  Line j of the input is [a, b): a = 0 or one past the (j-1)-th
 // '\n', b = the j-th '\n' or the end; a '\r' at b - 1 is dropped.  One
 // thread per line computes the line's output length, a scan places the
-// lines, and a byte-parallel pass (k_fmt_copy) moves the bytes.
+// lines, and a pass over the output (k_fmt_copy) fetches the bytes.
 
 constexpr int FMT_FASTA = 1;
 constexpr int FMT_FASTQ = 2;
@@ -820,72 +824,94 @@ __global__ void k_fmt_lines(const uint8_t* in, uint64_t n, const ull* nl, uint64
   olen[j] = (uint32_t)out;
 }
 
-// The copy, byte-parallel in the layout of k_nl_write: lane t of slab j
-// holds 16 input bytes, and the block scan of the '\n' counts gives the
-// line of its first byte (blk_nl = '\n's before each block).  A content
-// byte of line i goes to ooff[i] + (its offset in the line); the '\n' that
-// ends line i (or the input's last byte, for a last line without one) writes
-// the '\n's the line's output length adds after its content.  Sixteen
-// content bytes of one line (most chunks) take one 16-byte store.
+// The copy, by output: a block writes FC_BYTES of it, a thread 16 bytes at a
+// time, aligned.  A chunk's line is found among the starts of the block's
+// lines, which lie in LDS (FC_LINES of them; a block of more, shorter lines
+// searches the list in memory).  Sixteen bytes are one unaligned load, one for
+// each line they hold, shifted into place.  Bound by memory latency (0.21 GB
+// of FASTQ, 0.11 GB written: 176 us; by input bytes, with a store of 16 bytes
+// at any address, it took 371).
+constexpr int FC_NT = 256;
+constexpr uint32_t FC_BYTES = 16384;
+constexpr uint32_t FC_LINES = 2048;
+
+__device__ __forceinline__ u128 load16(const uint8_t* in, uint64_t n, uint64_t a) {
+  u128 v = 0;
+  if (a + 16 <= n) {
+    __builtin_memcpy(&v, in + a, 16);
+  } else {
+    for (int i = 0; i < 16; i++)
+      if (a + i < n) v |= (u128)in[a + i] << (8 * i);
+  }
+  return v;
+}
+
 template <int FMT>
-__global__ __launch_bounds__(NL_NT) void k_fmt_copy(const uint8_t* __restrict__ in, uint64_t n,
-                                                    const ull* __restrict__ blk_nl,
+__global__ __launch_bounds__(FC_NT) void k_fmt_copy(const uint8_t* __restrict__ in, uint64_t n,
                                                     const ull* __restrict__ lstart,
                                                     const uint32_t* __restrict__ llen,
                                                     const uint32_t* __restrict__ olen,
-                                                    const ull* __restrict__ ooff, uint8_t* __restrict__ out) {
-  const uint64_t b0 = (uint64_t)blockIdx.x * NL_PER_BLOCK + (uint64_t)threadIdx.x * 16;
-  uint32_t ev[NL_SLABS];
-  uint4 raw[NL_SLABS];
-  ull packed = 0;
-#pragma unroll
-  for (int j = 0; j < NL_SLABS; j++) {
-    raw[j] = scan16_keep(in, n, b0 + j * NL_SLAB, '\n', ev[j]);
-    packed |= (ull)__popc(ev[j]) << (16 * j);
+                                                    const ull* __restrict__ ooff, ull L, uint8_t* __restrict__ out) {
+  __shared__ uint32_t rel[FC_LINES];  // starts of the lines after the first, in the block's bytes
+  const ull total = ooff[L];
+  const ull o0 = (ull)blockIdx.x * FC_BYTES;
+  if (o0 >= total) return;
+  const uint32_t m = total - o0 < FC_BYTES ? (uint32_t)(total - o0) : FC_BYTES;
+  // the last line that starts at or before the block's first byte
+  const ull j0 = uniform(block_upper<FC_NT>(ooff, L, o0) - 1);
+  const uint32_t nl = L - j0 - 1 < FC_LINES ? (uint32_t)(L - j0 - 1) : FC_LINES;
+  for (uint32_t i = threadIdx.x; i < nl; i += FC_NT) {
+    const ull d = ooff[j0 + 1 + i] - o0;
+    rel[i] = d < FC_BYTES ? (uint32_t)d : FC_BYTES;
   }
-  ull tot;
-  const ull ex = block_scan_total<NL_NT>(packed, &tot);
-  const ull blk_base = blk_nl[blockIdx.x];
-  // slab: 16 bytes v at pos0 whose '\n's are evj, the first in line `line`
-  auto slab = [&](uint64_t pos0, uint4 v, uint32_t evj, uint64_t line) {
-    if (pos0 >= n) return;
-    const int cnt = n - pos0 < 16 ? (int)(n - pos0) : 16;
-    // the line's fields: start, content length, output length and place
-    ull a = lstart[line], oo = ooff[line];
-    uint32_t len = llen[line], ol = olen[line];
-    if (cnt == 16 && evj == 0 && pos0 + 16 <= a + len && pos0 != n - 16) {
-      // (a byte-aligned 16-byte copy: one unaligned dwordx4 store)
-      if (ol && !(FMT == FMT_FASTQ && (line & 3) == 0 && pos0 == a)) __builtin_memcpy(out + oo + (pos0 - a), &v, 16);
-      return;
-    }
-    for (int i = 0; i < cnt; i++) {
-      const uint64_t pos = pos0 + i;
-      const bool is_nl = (evj >> i) & 1u;
-      if (ol) {
-        if (pos < a + len) {
-          const bool gt = FMT == FMT_FASTQ && (line & 3) == 0 && pos == a;
-          out[oo + (pos - a)] = gt ? (uint8_t)'>' : byte_of(v, i);
-        }
-        if (is_nl || pos == n - 1) {
-          // the end of the line: the '\n's after its content
-          for (uint32_t q = len; q < ol; q++) out[oo + q] = '\n';
-        }
+  __syncthreads();
+  const bool fits = nl < FC_LINES || rel[FC_LINES - 1] >= m;
+  for (uint32_t b = threadIdx.x * 16; b < m; b += FC_NT * 16) {
+    ull j;
+    if (fits) {
+      uint32_t lo = 0, hi = nl;  // lines after the first that start at or before b
+      while (lo < hi) {
+        const uint32_t mid = (lo + hi) >> 1;
+        if (rel[mid] <= b) lo = mid + 1; else hi = mid;
       }
-      if (is_nl && pos + 1 < n) {
-        line++;
-        a = lstart[line];
-        oo = ooff[line];
-        len = llen[line];
-        ol = olen[line];
+      j = j0 + lo;
+    } else {
+      ull lo = j0, hi = L;
+      while (hi - lo > 1) {
+        const ull mid = (lo + hi) >> 1;
+        if (ooff[mid] <= o0 + b) lo = mid; else hi = mid;
+      }
+      j = lo;
+    }
+    const uint32_t cnt = m - b < 16 ? m - b : 16;
+    uint32_t q = (uint32_t)(o0 + b - ooff[j]);  // place in the line's output
+    u128 v = 0;
+    for (uint32_t p = 0; p < cnt;) {
+      const uint32_t len = llen[j], ol = olen[j];
+      if (q < len) {
+        const uint32_t t = len - q < cnt - p ? len - q : cnt - p;
+        u128 x = load16(in, n, lstart[j] + q);
+        if (FMT == FMT_FASTQ && q == 0 && (j & 3) == 0) x = (x & ~(u128)0xFF) | '>';
+        if (t < 16) x &= ((u128)1 << (8 * t)) - 1;
+        v |= x << (8 * p);
+        p += t;
+        q += t;
+      }
+      for (; p < cnt && q < ol; q++, p++) v |= (u128)'\n' << (8 * p);
+      if (p < cnt) {
+        j++;  // (a line without output adds nothing)
+        q = 0;
+        if (j >= L) break;
+        while (j + 1 < L && olen[j] == 0) j++;
       }
     }
-  };
-  static_assert(NL_SLABS == 4, "four slabs");
-  const ull t0 = tot & 0xFFFFull, t1 = (tot >> 16) & 0xFFFFull, t2 = (tot >> 32) & 0xFFFFull;
-  slab(b0, raw[0], ev[0], blk_base + (ex & 0xFFFFull));
-  slab(b0 + NL_SLAB, raw[1], ev[1], blk_base + t0 + ((ex >> 16) & 0xFFFFull));
-  slab(b0 + 2 * NL_SLAB, raw[2], ev[2], blk_base + t0 + t1 + ((ex >> 32) & 0xFFFFull));
-  slab(b0 + 3 * NL_SLAB, raw[3], ev[3], blk_base + t0 + t1 + t2 + ((ex >> 48) & 0xFFFFull));
+    if (cnt == 16) {
+      *reinterpret_cast<uint4*>(out + o0 + b) =
+          make_uint4((uint32_t)v, (uint32_t)(v >> 32), (uint32_t)(v >> 64), (uint32_t)(v >> 96));
+    } else {
+      for (uint32_t i = 0; i < cnt; i++) out[o0 + b + i] = (uint8_t)(v >> (8 * i));
+    }
+  }
 }
 
 // Builder-API records (Concurrent_Kmer_Partial_Counter::
@@ -1395,13 +1421,6 @@ struct RunBucket {
   ull base;    // array position of the parent's first tile
 };
 
-// a value that is the same in every lane, moved to scalar registers
-__device__ __forceinline__ ull uniform(ull x) {
-  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)x);
-  const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(x >> 32));
-  return (ull)hi << 32 | lo;
-}
-
 __device__ __forceinline__ RunBucket uniform(const RunBucket& r) {
   return RunBucket{uniform(r.v0), uniform(r.n), uniform(r.e0), uniform(r.nt), uniform(r.base)};
 }
@@ -1423,24 +1442,6 @@ __device__ __forceinline__ RunBucket run_bucket(const Runs& in, ull b) {
   r.n = in.V[r.e0 + r.nt] - r.v0;
   r.base = in.boff[a];
   return r;
-}
-
-// Number of x[0..n) (ascending) that are <= key, found by the whole block:
-// NT samples per step instead of a chain of log2(n) dependent loads.
-template <int NT>
-__device__ __forceinline__ ull block_upper(const ull* x, ull n, ull key) {
-  ull lo = 0;
-  while (n > (ull)NT) {
-    const ull step = (n + NT - 1) / NT;
-    const ull o = (ull)threadIdx.x * step;
-    const int c = __syncthreads_count(o < n && x[lo + o] <= key);
-    if (c == 0) return lo;
-    // sample c - 1 is <= key, sample c (if any) is not
-    const ull skip = (ull)(c - 1) * step;
-    lo += skip;
-    n = n - skip < step ? n - skip : step;
-  }
-  return lo + (ull)__syncthreads_count((ull)threadIdx.x < n && x[lo + threadIdx.x] <= key);
 }
 
 // Inclusive scan of a u32 over the wave by DPP moves (no LDS traffic, where
@@ -4231,16 +4232,14 @@ int normalize_impl(pk_ctx* c, const uint8_t* in, uint64_t n, int fmt, const uint
     return c->fail(PK_EFORMAT, "FASTQ record line " + std::to_string(hv[1]) +
                                    (hv[1] % 4 == 0 ? " does not start with '@'" : " does not start with '+'"));
   if (hv[2] != ~0ull) return c->fail(PK_EINVAL, "line " + std::to_string(hv[2]) + " longer than 4 GiB");
-  if (L) {
-    // '\n's before each index block: the scan event_index left in B_BLKOFF
-    const ull* blk_nl = reinterpret_cast<const ull*>(c->buf[B_BLKOFF].p);
-    const uint64_t nb = (n + NL_PER_BLOCK - 1) / NL_PER_BLOCK;
+  if (hv[0]) {
+    const unsigned ob = (unsigned)((hv[0] + FC_BYTES - 1) / FC_BYTES);
     if (fmt == FMT_FASTA)
-      hipLaunchKernelGGL(HIP_KERNEL_NAME(k_fmt_copy<FMT_FASTA>), dim3((unsigned)nb), dim3(NL_NT), 0, st, in, n,
-                         blk_nl, lstart, llen, olen, ooff, out);
+      hipLaunchKernelGGL(HIP_KERNEL_NAME(k_fmt_copy<FMT_FASTA>), dim3(ob), dim3(FC_NT), 0, st, in, n, lstart, llen,
+                         olen, ooff, (ull)L, out);
     else
-      hipLaunchKernelGGL(HIP_KERNEL_NAME(k_fmt_copy<FMT_FASTQ>), dim3((unsigned)nb), dim3(NL_NT), 0, st, in, n,
-                         blk_nl, lstart, llen, olen, ooff, out);
+      hipLaunchKernelGGL(HIP_KERNEL_NAME(k_fmt_copy<FMT_FASTQ>), dim3(ob), dim3(FC_NT), 0, st, in, n, lstart, llen,
+                         olen, ooff, (ull)L, out);
     PK_HIP(c, hipGetLastError());
   }
   *out_p = out;

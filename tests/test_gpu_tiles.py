@@ -242,3 +242,26 @@ def test_builder_window_ends(ctx, oracle_mod, klen, bits, read_len):
     assert n == want_n
     assert np.array_equal(keys.reshape(-1), np.asarray(want_k).reshape(-1))
     assert np.array_equal(counts, want_c)
+
+
+@pytest.mark.parametrize("size", [1, 2, 13, 15, 16, 17, 31, 33, 100, 16_383, 16_384, 40_000])
+@pytest.mark.parametrize("end", [b"\n", b"\r\n"])
+def test_rewrite_by_output(ctx, oracle_mod, size, end):
+    """Lines around a chunk, a block and more, and so short that a block holds
+    more of them than its table, with and without a last line end."""
+    rng = np.random.default_rng(size)
+    n = max(3, min(9_000, 200_000 // size))
+    _p(f"case: rewrite size={size} end={end!r}")
+    seqs = [_bases(rng, int(rng.integers(max(size - 2, 0), size + 1)), b"ACGTN") for _ in range(n)]
+    fq = b"".join(b"@%d" % (i % 10) + end + q + end + b"+" + end + b"I" * len(q) + end for i, q in enumerate(seqs))
+    fa = b"".join((b">%d" % i + end if i % 5 == 0 else b"") + q + end for i, q in enumerate(seqs))
+    for cut in (0, len(end)):
+        for fmt, data in (("fastq", fq), ("fasta", fa)):
+            data = data[:len(data) - cut]
+            try:
+                want = oracle_mod.normalize(data, fmt)
+            except ValueError:  # an empty last line without its end is no line
+                with pytest.raises(Exception, match="not a multiple of 4"):
+                    ctx.normalize(data, fmt)
+                continue
+            assert ctx.normalize(data, fmt) == want, (fmt, cut)
