@@ -49,12 +49,11 @@ WORKLOADS = {
 
 # single-launch stages timed by HIP events around their kernel -> (kernel
 # name, timing field); the further partition levels are added per level from
-# the per-level fields (ms_level_*), their scatter kernel by form
-KERNELS = {"hist": ("k_l1_hist<{key}, 0, false>", "hist_ms"),
-           "l1_scatter": ("k_l1_scatter<{key}, 0, false>", "l1_scatter_ms"),
-           "sort": ("k_bucket_hash<{key}>", "sort_ms"),
+# the per-level fields (ms_level_*), their kernel by form
+KERNELS = {"l1_scatter": ("k_split_main<{key}, 2>", "l1_scatter_ms"),
+           "sort": ("k_bucket_hash<{key}, true>", "sort_ms"),
            "compact": ("k_compact<{key}>", "compact_ms")}
-MS_SCATTER = {4: "k_split"}
+MS_SCATTER = {4: "k_split<{key}, 0>"}
 
 
 def alg_bytes(N, U, V, M, S, W):
@@ -76,17 +75,13 @@ def alg_bytes(N, U, V, M, S, W):
 
 def kernel_times(tm, W):
     """[(stage, kernel, ms per step)] of every single-launch kernel the stage
-    timings cover: the four fixed stages, then each further partition level's
-    histogram (a k_ms_hist launch unless the level's counts were folded into
-    level 1's histogram, form 3) and scatter."""
+    timings cover: the fixed stages, then each further partition level."""
     key = "unsigned long" if W == 8 else "unsigned __int128"
     out = [(stage, name.format(key=key), float(tm.get(field, 0.0))) for stage, (name, field) in KERNELS.items()]
     levels = min(int(tm.get("ms_levels", 0)), len(tm.get("ms_level_form", [])))
     for lv in range(levels):
         form = int(tm["ms_level_form"][lv])
-        if form != 3:
-            out.append(("ms_hist", f"k_ms_hist<{key}>", float(tm["ms_level_hist_ms"][lv])))
-        out.append(("ms_scatter", f"{MS_SCATTER[form]}<{key}>", float(tm["ms_level_scatter_ms"][lv])))
+        out.append(("ms_scatter", MS_SCATTER[form].format(key=key), float(tm["ms_level_scatter_ms"][lv])))
     return [x for x in out if x[2] > 0]
 
 

@@ -3,10 +3,9 @@
 For every size bucket (FASTA bytes up to max_bytes) and key width (k = 32:
 one word; k = 64: two) it builds a read set of that size (uniform genome,
 100 or 150 bp reads, 50x, 0.5% errors), times count + cutoff + macro nodes
-on the device for each
-candidate (reads per level-1 block, level-1 digit bits, bucket factor = the
-inverse of the hash-table load target) and keeps the fastest.  The table is
-written as JSON (pakman_plus_amd/tuning.json) and applied by Server.set_tuning
+on the device for each candidate (level-1 digit bits, bucket factor = the
+inverse of the hash-table load target) and keeps the fastest, or the built-in
+choices where none beats them by MARGIN.  The table is written as JSON (pakman_plus_amd/tuning.json) and applied by Server.set_tuning
 or per context with Context.set_tuning.  Results never depend on the tuning.
 
   python -m pakman_plus_amd.tune [--out PATH] [--reps 5]
@@ -25,11 +24,10 @@ DEFAULT_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "tuning.
 # sample's 10 bits).  A bucket where no candidate beats the built-in choices
 # keeps them (zero fields).
 BUCKETS = [1 << 21, 1 << 23, 1 << 25, 1 << 27, 1 << 29, 1 << 31]
-CANDIDATES = ([{"l1_chunks": c, "l1_bits": 8, "bucket_factor": f}
-               for c in (1, 2, 4, 8) for f in (1.5, 2.2, 3.0, 5.0)]
-              + [{"l1_chunks": 0, "l1_bits": b, "bucket_factor": 3.0} for b in (6, 7)]
-              + [{"l1_chunks": 0, "l1_bits": b, "bucket_factor": f} for b in (9, 10)
-                 for f in (1.5, 2.2)])
+CANDIDATES = [{"l1_chunks": 0, "l1_bits": b, "bucket_factor": f}
+              for b in (0, 6, 7, 8, 9, 10) for f in (1.1, 1.6, 2.1)]
+# a candidate has to beat the built-in choices by more than runs differ
+MARGIN = 1.02
 
 
 def _sample(max_bytes: int, prev: int, read_len: int):
@@ -130,7 +128,7 @@ def _tune_k(reps: int, k: int, t: int) -> list[dict]:
             if r:
                 ts.append(time.perf_counter() - t0)
         e["builtin_ms"] = float(np.median(ts)) * 1e3
-        if e["builtin_ms"] < e["ms"]:
+        if e["builtin_ms"] < e["ms"] * MARGIN:
             # no candidate beats the built-in choices: zero fields keep them
             e.update(l1_chunks=0, l1_bits=0, bucket_factor=0.0, ms=e["builtin_ms"], builtin=True)
         entries.append(e)
