@@ -589,10 +589,11 @@ __global__ __launch_bounds__(NL_NT) void k_nl_write_rx(const uint32_t* RX, uint6
 // '\n's come before, and it is taken when its header's '\n' (number j0 + 2r)
 // lies at least K + 1 bytes before the end of the input (k_reads' rules, from
 // counts instead of positions).  lines: [0] j0, [1] R = records taken, [2]
-// '\n's of the input, [3] p0 (n when there is none).  One block.
+// '\n's of the input, [3] p0 (n when there is none).  K2 > 0: *R2 = R of that
+// window length.  One block.
 // blk (with nb <= SCAN_PER): the '\n's per block, scanned into blk_off first.
 __global__ __launch_bounds__(1024) void k_lines(const uint32_t* RX, uint64_t n, const ull* blk, ull* blk_off,
-                                                uint64_t nb, const ull* gt, int K, ull* lines) {
+                                                uint64_t nb, const ull* gt, int K, int K2, ull* lines, ull* R2) {
   static_assert(SCAN_NT == 1024, "the scan's block");
   if (blk) {
     const uint64_t base = (uint64_t)threadIdx.x * SCAN_EPT;
@@ -625,13 +626,20 @@ __global__ __launch_bounds__(1024) void k_lines(const uint32_t* RX, uint64_t n, 
   };
   const uint64_t pb = p0 / NL_PER_BLOCK;
   const ull j0 = p0 < n ? blk_off[pb] + count(pb * NL_PER_BLOCK, p0) : m;
-  const ull tail = count(n > (uint64_t)K ? n - (uint64_t)K : 0, n);
+  auto records = [&](int k) -> ull {
+    const ull c = m - count(n > (uint64_t)k ? n - (uint64_t)k : 0, n);  // '\n's at least k + 1 bytes before the end
+    return p0 < n && c > j0 ? (c - j0 + 1) / 2 : 0;
+  };
+  const ull R = records(K);
   if (threadIdx.x == 0) {
-    const ull c = m - tail;  // '\n's at least K + 1 bytes before the end
     lines[0] = j0;
-    lines[1] = p0 < n && c > j0 ? (c - j0 + 1) / 2 : 0;
+    lines[1] = R;
     lines[2] = m;
     lines[3] = p0;
+  }
+  if (K2 > 0) {
+    const ull r2 = records(K2);
+    if (threadIdx.x == 0) *R2 = r2;
   }
 }
 
@@ -640,9 +648,12 @@ __global__ __launch_bounds__(1024) void k_lines(const uint32_t* RX, uint64_t n, 
 // taken and no '\n' is among them.  A thread covers 64 bytes, a block the
 // same bytes as k_pack's; cnt[block] = its valid ends.  first_err = the first
 // record r >= 1 that does not start with '>' (the reference's assert).  All from
-// the '\n' bits: a quarter byte read and an eighth written per input byte.
+// the '\n' bits: a quarter byte read and an eighth written per input byte.  W2:
+// the same bits for windows of K2 <= K bytes (a share's L-mers: 26 us less than
+// a launch of their own for 0.21 GB).
 __global__ __launch_bounds__(NL_NT) void k_valid(const uint32_t* RX, uint64_t n, const ull* blk_off,
-                                                 const ull* lines, int K, ull* W, uint32_t* cnt, ull* first_err) {
+                                                 const ull* lines, int K, ull* W, uint32_t* cnt, ull* first_err, int K2,
+                                                 const ull* R2, ull* W2) {
   const uint64_t nw = (n + 15) / 16;
   const uint64_t w0 = (uint64_t)blockIdx.x * (NL_PER_BLOCK / 16) + (uint64_t)threadIdx.x * 4;
   const uint64_t base = w0 * 16;
@@ -670,11 +681,17 @@ __global__ __launch_bounds__(NL_NT) void k_valid(const uint32_t* RX, uint64_t n,
   }
   // a '\n' among the last K bytes, up to and with this one
   u128 near = (u128)x << 64 | (u128)px;
-  for (int c = 1; c < K;) {
-    const int sh = c < K - c ? c : K - c;
-    near |= near << sh;
-    c += sh;
-  }
+  int c = 1;
+  auto widen = [&](int k) -> ull {
+    while (c < k) {
+      const int sh = c < k - c ? c : k - c;
+      near |= near << sh;
+      c += sh;
+    }
+    return (ull)(near >> 64);
+  };
+  const ull near2 = W2 ? widen(K2) : 0;
+  const ull near1 = widen(K);
   ull tot;
   const ull cb = blk_off[blockIdx.x] + block_scan_total<NL_NT>((ull)__popcll(x), &tot);
   // parity of the '\n's before each byte, relative to j0: odd in sequences
@@ -683,7 +700,6 @@ __global__ __launch_bounds__(NL_NT) void k_valid(const uint32_t* RX, uint64_t n,
   for (int o = 1; o < 64; o <<= 1) par ^= par << o;
   ull seq = par ^ x;
   if ((cb ^ j0) & 1) seq = ~seq;
-  ull ok = seq & ~(ull)(near >> 64);
   const ull ce = cb + (ull)__popcll(x);
   // bytes up to the (j0)-th '\n' are before the first sequence, bytes after
   // the (j0 + 2R)-th belong to records not taken
@@ -692,18 +708,20 @@ __global__ __launch_bounds__(NL_NT) void k_valid(const uint32_t* RX, uint64_t n,
     for (; k; k--) t &= t - 1;
     return __ffsll((long long)t) - 1;
   };
-  const ull last = j0 + 2 * R;
-  if (ce <= j0 || cb > last) {
-    ok = 0;
-  } else {
+  auto taken = [&](ull ok, ull R) -> ull {
+    const ull last = j0 + 2 * R;
+    if (ce <= j0 || cb > last) return 0;
     if (cb <= j0) {
       const int b = nth(j0 - cb);
       ok &= b == 63 ? 0ull : ~0ull << (b + 1);
     }
     if (ce > last) ok &= (1ull << nth(last - cb)) - 1;
-  }
-  if (base >= n) ok = 0;
-  else if (base + 64 > n) ok &= (1ull << (n - base)) - 1;
+    if (base >= n) return 0;
+    if (base + 64 > n) ok &= (1ull << (n - base)) - 1;
+    return ok;
+  };
+  const ull ok = taken(seq & ~near1, R);
+  if (W2) W2[w0 / 4] = taken(seq & ~near2, *R2);
   // sequence ends that no '>' follows
   ull bad = x & seq & ~g;
   if (base + 64 >= n && n > base) bad &= ~(1ull << (n - 1 - base));
@@ -3791,7 +3809,7 @@ enum BufId {
   B_FASTA, B_BLK, B_BLKOFF, B_NL, B_RSTART, B_RLEN, B_KC, B_KOFS, B_SMALL, B_BCNT, B_BOFF, B_BCUR,
   B_S, B_C, B_TU, B_UOFF, B_TK, B_TC, B_HIST, B_KBS, B_KBOFF, B_KK, B_KC2, B_MNPLAN,
   B_MNNT, B_MNNG, B_MNNOFF, B_MNFLAG, B_NODES, B_TMP, B_OVF, B_PT0, B_PT1, B_PT2, B_PT3, B_PT4,
-  B_PT5, B_PT6, B_BLKGT, B_S2, B_BCNT2, B_BOFF2, B_BCUR2, B_TP, B_TP2, B_HIST1, B_OFF1, B_HIST2, B_OFF2, B_PACK, B_RETRY, B_WCNT, B_WOFF, B_CUTBH, B_LFREQ, B_LPART, B_LBIG, B_LRANK, B_OWNW, B_OWNCNT, B_OWNOFF, B_WORDER, B_WIRE, B_NORM, B_NORMNL, B_NORMLEN, B_NORMOFF, B_NORMLS, B_NORMLL, B_SCAN0, B_SCAN1 = B_SCAN0 + 8, B_COUNT = B_SCAN0 + 16
+  B_PT5, B_PT6, B_BLKGT, B_S2, B_BCNT2, B_BOFF2, B_BCUR2, B_TP, B_TP2, B_HIST1, B_OFF1, B_HIST2, B_OFF2, B_PACK, B_RETRY, B_WCNT, B_WOFF, B_CUTBH, B_LFREQ, B_LPART, B_LBIG, B_LRANK, B_LW, B_OWNW, B_OWNCNT, B_OWNOFF, B_WORDER, B_WIRE, B_NORM, B_NORMNL, B_NORMLEN, B_NORMOFF, B_NORMLS, B_NORMLL, B_SCAN0, B_SCAN1 = B_SCAN0 + 8, B_COUNT = B_SCAN0 + 16
 };
 
 }  // namespace
@@ -4293,16 +4311,17 @@ int format_error(pk_ctx* c, ull r) {
 int records_main(pk_ctx* c, const uint8_t* fa, uint64_t n, int K, Records* rec);
 
 // The windows of the main path from the packed input: valid ends and their
-// number per index block, no list of lines or reads.  packed: the last call on
-// this stream packed the same input.
-int windows_main(pk_ctx* c, const uint8_t* fa, uint64_t n, int K, Records* rec, bool packed = false) {
+// number per index block, no list of lines or reads.  W2: also the window ends
+// of the L-mers.
+int windows_main(pk_ctx* c, const uint8_t* fa, uint64_t n, int K, Records* rec, ull* W2 = nullptr) {
   hipStream_t st = c->stream;
   ull* small;
   PK_TRY(need(c, B_SMALL, 16, &small));
   // small[2] = first format error, [3] = a line may be too long, [4], [5] =
-  // overflow and retry counts, [6] .. [9] = k_lines' facts, [10] = first '>'
+  // overflow and retry counts, [6] .. [9] = k_lines' facts, [10] = first '>',
+  // [11] = records of the L-mers
   const uint64_t nb = (n + NL_PER_BLOCK - 1) / NL_PER_BLOCK;
-  if (packed || !nb) {
+  if (!nb) {
     PK_TRY(fill_u64(c, small + 2, ~0ull, 1));
     PK_TRY(fill_u64(c, small + 3, 0, 3));
   }
@@ -4316,31 +4335,31 @@ int windows_main(pk_ctx* c, const uint8_t* fa, uint64_t n, int K, Records* rec, 
   PK_TRY(need(c, B_WOFF, nb + 1, &tb));
   rec->tb = tb;
   if (!nb) return PK_OK;
-  if (!packed) {
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_pack<ENC_MAIN>), dim3((unsigned)nb), dim3(NL_NT), 0, st, fa, n, (uint8_t)'\n',
-                       (uint8_t)'\n', blk, blkgt, 0, pk.E, pk.RX, small);
-    PK_HIP(c, hipGetLastError());
-    if (nb > SCAN_PER) PK_TRY(scan_excl<ull>(c, blk, blkoff, nb));
-  }
+  hipLaunchKernelGGL(HIP_KERNEL_NAME(k_pack<ENC_MAIN>), dim3((unsigned)nb), dim3(NL_NT), 0, st, fa, n, (uint8_t)'\n',
+                     (uint8_t)'\n', blk, blkgt, 0, pk.E, pk.RX, small);
+  PK_HIP(c, hipGetLastError());
+  if (nb > SCAN_PER) PK_TRY(scan_excl<ull>(c, blk, blkoff, nb));
   const bool check_long = n > 0xFFFFFFF0ull;
   if (check_long) {
     hipLaunchKernelGGL(k_long_lines, dim3(grid_for(nb, 256)), dim3(256), 0, st, blkoff, nb, small + 3);
     PK_HIP(c, hipGetLastError());
   }
-  ull hs[8], N = 0;
+  ull hs[8], N = 0, R2 = 0;
   // the first '>' is nearly always in the first block (blkgt[0]); else a
   // second pass looks for it everywhere
   const ull* gt = blkgt;
   for (int pass = 0;; pass++) {
     hipLaunchKernelGGL(k_lines, dim3(1), dim3(1024), 0, st, pk.RX, n,
-                       (const ull*)(nb <= SCAN_PER && !packed && pass == 0 ? blk : nullptr), blkoff, nb, gt, K, small + 6);
+                       (const ull*)(nb <= SCAN_PER && pass == 0 ? blk : nullptr), blkoff, nb, gt, K, W2 ? LMER_L : 0, small + 6,
+                       small + 11);
     PK_HIP(c, hipGetLastError());
     hipLaunchKernelGGL(k_valid, dim3((unsigned)nb), dim3(NL_NT), 0, st, pk.RX, n, blkoff, small + 6, K, pk.W, cnt,
-                       small + 2);
+                       small + 2, LMER_L, (const ull*)(small + 11), W2);
     PK_HIP(c, hipGetLastError());
-    PK_TRY(scan_fetch<uint32_t>(c, cnt, tb, nb, Post{{small + 2}, {8}}));
+    PK_TRY(scan_fetch<uint32_t>(c, cnt, tb, nb, Post{{small + 2, small + 11}, {8, W2 ? 1 : 0}}));
     N = c->box[0];
     memcpy(hs, c->box + 1, sizeof(hs));
+    R2 = W2 ? c->box[9] : 0;
     if (hs[7] < n || pass || nb == 1) break;
     hipLaunchKernelGGL(k_nl_count, dim3((unsigned)nb), dim3(NL_NT), 0, st, fa, n, (uint8_t)'\n', (uint8_t)'\n', blk,
                        blkgt, 1);
@@ -4351,7 +4370,8 @@ int windows_main(pk_ctx* c, const uint8_t* fa, uint64_t n, int K, Records* rec, 
   }
   rec->R = hs[5];
   rec->N = N;
-  if (hs[0] != ~0ull && hs[0] <= rec->R) return format_error(c, hs[0]);
+  // (the L-mers' records, if asked for, include the windows')
+  if (hs[0] != ~0ull && hs[0] <= std::max<uint64_t>(rec->R, R2)) return format_error(c, hs[0]);
   if (check_long && hs[1]) {
     // the read table measures every line
     Records full;
@@ -4895,24 +4915,20 @@ int count_impl(pk_ctx* c, const uint8_t* fa, uint64_t n, int K) {
   return count_records<Key, ENC_MAIN>(c, rec, K, 2 * K, key_mask<Key>(2 * K));
 }
 
-// L-mer frequencies of the whole input into freq (device, LMER_BINS u64),
-// with the record rule of Sliding_window_l (a record needs L bytes).  Packs the
-// input into rec.
-int lmer_frequency_impl(pk_ctx* c, const uint8_t* fa, uint64_t n, Records* rec, ull** freq_out) {
+// L-mer frequencies (device, LMER_BINS u64) from the packed input and the
+// L-mers' ends W.
+int lmer_frequency_impl(pk_ctx* c, const Records& rec, const ull* W, ull** freq_out) {
   hipStream_t st = c->stream;
-  rec->n = n;
-  PK_TRY(pack_buffers(c, n, true, &rec->pk));
-  PK_TRY(windows_main(c, fa, n, LMER_L, rec));
   ull* freq;
   PK_TRY(need(c, B_LFREQ, LMER_BINS, &freq));
   PK_TRY(fill_u64(c, freq, 0, LMER_BINS));
-  if (rec->N) {
-    const uint64_t nb = (n + NL_PER_BLOCK - 1) / NL_PER_BLOCK;
+  const uint64_t nb = (rec.n + NL_PER_BLOCK - 1) / NL_PER_BLOCK;
+  if (nb) {
     const int np = (int)std::min<uint64_t>(nb, (uint64_t)c->ncu);
     uint32_t* part;
     PK_TRY(need(c, B_LPART, (uint64_t)np * (LMER_BINS / 2), &part));
-    hipLaunchKernelGGL(k_lmer_count, dim3((unsigned)np), dim3(LM_NT), 0, st, rec->pk.E, rec->pk.RX,
-                       reinterpret_cast<const uint16_t*>(rec->pk.W), (ull)nb, part, freq);
+    hipLaunchKernelGGL(k_lmer_count, dim3((unsigned)np), dim3(LM_NT), 0, st, rec.pk.E, rec.pk.RX,
+                       reinterpret_cast<const uint16_t*>(W), (ull)nb, part, freq);
     PK_HIP(c, hipGetLastError());
     hipLaunchKernelGGL(k_lmer_sum, dim3(LMER_BINS / 128), dim3(1024), 0, st, part, np, freq);
     PK_HIP(c, hipGetLastError());
@@ -5006,14 +5022,12 @@ int rank_share_impl(pk_ctx* c, const uint8_t* fa, uint64_t n, int K, int P, int 
   c->key_bits = 2 * K;
   PK_HIP(c, hipEventRecord(c->ev[0], c->stream));
   Records rec;
-  ull* freq = nullptr;
-  if (by_key) {
-    rec.n = n;
-    PK_TRY(pack_buffers(c, n, true, &rec.pk));
-  } else {
-    PK_TRY(lmer_frequency_impl(c, fa, n, &rec, &freq));
-  }
-  PK_TRY(windows_main(c, fa, n, K, &rec, !by_key));
+  ull *freq = nullptr, *W2 = nullptr;
+  rec.n = n;
+  PK_TRY(pack_buffers(c, n, true, &rec.pk));
+  if (!by_key) PK_TRY(need(c, B_LW, (n + NL_PER_BLOCK - 1) / NL_PER_BLOCK * (NL_PER_BLOCK / 64), &W2));
+  PK_TRY(windows_main(c, fa, n, K, &rec, W2));
+  if (!by_key && rec.N) PK_TRY(lmer_frequency_impl(c, rec, W2, &freq));
   if (rec.N) PK_TRY(own_windows(c, K, freq, P, rank, &rec));
   return count_records<Key, ENC_MAIN>(c, rec, K, 2 * K, key_mask<Key>(2 * K));
 }
@@ -5699,7 +5713,10 @@ int pk_lmer_frequency(pk_ctx* c, const char* fasta, uint64_t nbytes, int fasta_o
   PK_TRY(fasta_to_device(c, fasta, nbytes, fasta_on_device, &fa));
   ull* freq;
   Records rec;
-  PK_TRY(lmer_frequency_impl(c, fa, nbytes, &rec, &freq));
+  rec.n = nbytes;
+  PK_TRY(pack_buffers(c, nbytes, true, &rec.pk));
+  PK_TRY(windows_main(c, fa, nbytes, LMER_L, &rec));
+  PK_TRY(lmer_frequency_impl(c, rec, rec.pk.W, &freq));
   return d2h(c, freq_host, freq, LMER_BINS * 8);
 }
 
