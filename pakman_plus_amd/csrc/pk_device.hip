@@ -843,15 +843,16 @@ __global__ void k_fmt_lines(const uint8_t* in, uint64_t n, const ull* nl, uint64
 }
 
 // The copy, by output: a block writes FC_BYTES of it, a thread 16 bytes at a
-// time, aligned.  A chunk's line is found among the starts of the block's
-// lines, which lie in LDS (FC_LINES of them; a block of more, shorter lines
-// searches the list in memory).  Sixteen bytes are one unaligned load, one for
-// each line they hold, shifted into place.  Bound by memory latency (0.21 GB
-// of FASTQ, 0.11 GB written: 176 us; by input bytes, with a store of 16 bytes
-// at any address, it took 371).
+// time, aligned.  The fields of the block's lines lie in LDS (FC_LINES of them;
+// lines beyond come from memory), so that a chunk waits for memory only for
+// its bytes: one unaligned load for each line it holds, shifted into place.
+// Bound by issue: a wave goes through as many lines as its chunk of the most
+// (0.21 GB of FASTQ, 0.11 GB written: 134 us; with the fields read per chunk
+// 176; by input bytes, with a store of 16 bytes at any address, 371; blocks of
+// 32 or 64 KiB and of 512 or 1024 threads within 5 %).
 constexpr int FC_NT = 256;
 constexpr uint32_t FC_BYTES = 16384;
-constexpr uint32_t FC_LINES = 2048;
+constexpr uint32_t FC_LINES = 1024;
 
 __device__ __forceinline__ u128 load16(const uint8_t* in, uint64_t n, uint64_t a) {
   u128 v = 0;
@@ -870,58 +871,64 @@ __global__ __launch_bounds__(FC_NT) void k_fmt_copy(const uint8_t* __restrict__ 
                                                     const uint32_t* __restrict__ llen,
                                                     const uint32_t* __restrict__ olen,
                                                     const ull* __restrict__ ooff, ull L, uint8_t* __restrict__ out) {
-  __shared__ uint32_t rel[FC_LINES];  // starts of the lines after the first, in the block's bytes
+  // line i of the block: its output starts at rel[i] (the first one's before)
+  __shared__ uint32_t rel[FC_LINES], len[FC_LINES], ol[FC_LINES];
+  __shared__ ull src[FC_LINES];
   const ull total = ooff[L];
   const ull o0 = (ull)blockIdx.x * FC_BYTES;
   if (o0 >= total) return;
   const uint32_t m = total - o0 < FC_BYTES ? (uint32_t)(total - o0) : FC_BYTES;
   // the last line that starts at or before the block's first byte
   const ull j0 = uniform(block_upper<FC_NT>(ooff, L, o0) - 1);
-  const uint32_t nl = L - j0 - 1 < FC_LINES ? (uint32_t)(L - j0 - 1) : FC_LINES;
+  const uint32_t q0 = (uint32_t)uniform(o0 - ooff[j0]);  // place in it
+  const uint32_t nl = L - j0 < FC_LINES ? (uint32_t)(L - j0) : FC_LINES;
   for (uint32_t i = threadIdx.x; i < nl; i += FC_NT) {
-    const ull d = ooff[j0 + 1 + i] - o0;
+    const ull d = i ? ooff[j0 + i] - o0 : 0;
     rel[i] = d < FC_BYTES ? (uint32_t)d : FC_BYTES;
+    len[i] = llen[j0 + i];
+    ol[i] = olen[j0 + i];
+    src[i] = lstart[j0 + i];
   }
   __syncthreads();
   const bool fits = nl < FC_LINES || rel[FC_LINES - 1] >= m;
   for (uint32_t b = threadIdx.x * 16; b < m; b += FC_NT * 16) {
-    ull j;
+    ull i;  // the line of the chunk's first byte, from j0
+    uint32_t q;
     if (fits) {
-      uint32_t lo = 0, hi = nl;  // lines after the first that start at or before b
+      uint32_t lo = 1, hi = nl;  // lines after the first that start at or before b
       while (lo < hi) {
         const uint32_t mid = (lo + hi) >> 1;
         if (rel[mid] <= b) lo = mid + 1; else hi = mid;
       }
-      j = j0 + lo;
+      i = lo - 1;
+      q = i ? b - rel[i] : q0 + b;
     } else {
       ull lo = j0, hi = L;
       while (hi - lo > 1) {
         const ull mid = (lo + hi) >> 1;
         if (ooff[mid] <= o0 + b) lo = mid; else hi = mid;
       }
-      j = lo;
+      i = lo - j0;
+      q = (uint32_t)(o0 + b - ooff[lo]);
     }
     const uint32_t cnt = m - b < 16 ? m - b : 16;
-    uint32_t q = (uint32_t)(o0 + b - ooff[j]);  // place in the line's output
     u128 v = 0;
-    for (uint32_t p = 0; p < cnt;) {
-      const uint32_t len = llen[j], ol = olen[j];
-      if (q < len) {
-        const uint32_t t = len - q < cnt - p ? len - q : cnt - p;
-        u128 x = load16(in, n, lstart[j] + q);
-        if (FMT == FMT_FASTQ && q == 0 && (j & 3) == 0) x = (x & ~(u128)0xFF) | '>';
+    // (FASTQ: the lines after a read's have no output)
+    for (uint32_t p = 0; p < cnt && j0 + i < L; i += FMT == FMT_FASTQ && ((j0 + i) & 3) == 1 ? 3 : 1) {
+      const bool in_lds = i < (ull)FC_LINES;
+      const uint32_t n0 = in_lds ? len[i] : llen[j0 + i], n1 = in_lds ? ol[i] : olen[j0 + i];
+      if (q < n0 && n1) {
+        const uint32_t t = n0 - q < cnt - p ? n0 - q : cnt - p;
+        u128 x = load16(in, n, (in_lds ? src[i] : lstart[j0 + i]) + q);
+        if (FMT == FMT_FASTQ && q == 0 && ((j0 + i) & 3) == 0) x = (x & ~(u128)0xFF) | '>';
         if (t < 16) x &= ((u128)1 << (8 * t)) - 1;
         v |= x << (8 * p);
         p += t;
         q += t;
       }
-      for (; p < cnt && q < ol; q++, p++) v |= (u128)'\n' << (8 * p);
-      if (p < cnt) {
-        j++;  // (a line without output adds nothing)
-        q = 0;
-        if (j >= L) break;
-        while (j + 1 < L && olen[j] == 0) j++;
-      }
+      // (a line without output adds nothing)
+      for (; p < cnt && q < n1; q++, p++) v |= (u128)'\n' << (8 * p);
+      q = 0;
     }
     if (cnt == 16) {
       *reinterpret_cast<uint4*>(out + o0 + b) =
