@@ -44,6 +44,14 @@ struct Job {
 
 inline uint64_t align256(uint64_t x) { return (x + 255) & ~255ull; }
 
+// A result block's size: up to an eighth more than asked for, so that blocks of
+// a few sizes serve jobs of many.
+inline uint64_t block_bytes(uint64_t x) {
+  uint64_t g = 256;
+  while (g * 16 <= x) g *= 2;
+  return (x + g - 1) & ~(g - 1);
+}
+
 // Working-set estimate of a job: FASTA copy (host input), line index and read
 // table, two instance arrays and the per-instance counts, the table.  The
 // instance count is bounded by the byte count.
@@ -75,6 +83,16 @@ struct pk_server {
   bool stop = false;
   std::string err;
   std::vector<pk_tune_entry> tune;  // ascending max_bytes
+  // Result blocks of released jobs, oldest first, kept for later results: at
+  // 2000 jobs/s the device maps and unmaps 170 GB/s of them otherwise, and an
+  // unmap stopped every slot for 0.05 to 1.6 s (p99 2.9 s against 0.1 s).  At
+  // most an eighth of the budget; given back when a job needs the room.
+  struct Block {
+    void* p;
+    uint64_t bytes;
+  };
+  std::deque<Block> spare;
+  uint64_t spare_bytes = 0;
   std::chrono::steady_clock::time_point t0 = std::chrono::steady_clock::now();
 
   double now() const {
@@ -84,6 +102,59 @@ struct pk_server {
     if (queue.empty()) return false;
     if (running == 0) return true;
     return running_est + resident + queue.front()->res.est_bytes <= budget;
+  }
+  // Takes the oldest spare blocks out until at most `keep` bytes are left; the
+  // caller frees them without mu, which every slot needs.
+  std::vector<Block> drop_spare(uint64_t keep) {
+    std::vector<Block> out;
+    while (!spare.empty() && spare_bytes > keep) {
+      out.push_back(spare.front());
+      spare_bytes -= spare.front().bytes;
+      spare.pop_front();
+    }
+    return out;
+  }
+  void free_blocks(const std::vector<Block>& v) {
+    for (const Block& b : v) {
+      if (pools) (void)hipFreeAsync(b.p, free_stream);
+      else (void)hipFree(b.p);
+    }
+  }
+  // All spare blocks back to the device; false when there were none.
+  bool free_spare() {
+    std::vector<Block> v;
+    {
+      std::lock_guard<std::mutex> lk(mu);
+      v = drop_spare(0);
+    }
+    free_blocks(v);
+    if (!v.empty()) (void)hipStreamSynchronize(free_stream);
+    return !v.empty();
+  }
+  // A block of *bytes or a little more (*bytes is then its size): the smallest
+  // spare one that fits, else a new one.  Every use of a spare block ended
+  // before its job was done.
+  hipError_t take_block(uint64_t* bytes, hipStream_t st, void** out) {
+    {
+      std::lock_guard<std::mutex> lk(mu);
+      auto best = spare.end();
+      for (auto it = spare.begin(); it != spare.end(); ++it)
+        if (it->bytes >= *bytes && it->bytes <= *bytes + *bytes / 4 && (best == spare.end() || it->bytes < best->bytes))
+          best = it;
+      if (best != spare.end()) {
+        *out = best->p;
+        *bytes = best->bytes;
+        spare_bytes -= best->bytes;
+        spare.erase(best);
+        return hipSuccess;
+      }
+    }
+    for (;;) {
+      const hipError_t e = pools ? hipMallocAsync(out, *bytes, st) : hipMalloc(out, *bytes);
+      if (e == hipSuccess) return e;
+      (void)hipGetLastError();
+      if (!free_spare()) return e;
+    }
   }
   // err is written under mu (callers hold it, or use fail_unlocked)
   int fail(int code, const std::string& m) {
@@ -119,6 +190,8 @@ void pk_server::run(int slot, Job* j) {
   pk_ctx_set_tuning(c, &tu);
   pk_table t{};
   int rc = pk_count(c, j->spec.fasta, j->spec.nbytes, j->spec.k, j->spec.fasta_on_device, &t);
+  if (rc == PK_ENOMEM && free_spare())
+    rc = pk_count(c, j->spec.fasta, j->spec.nbytes, j->spec.k, j->spec.fasta_on_device, &t);
   if (rc) {
     set_err(rc);
     return;
@@ -150,6 +223,7 @@ void pk_server::run(int slot, Job* j) {
   const uint64_t o1 = 0, o2 = align256(o1 + t.n * w), o3 = align256(o2 + t.n * 4),
                  o4 = align256(o3 + kt.n * w), o5 = align256(o4 + kt.n * 4),
                  end = align256(o5 + mt.n * sizeof(pk_mnode));
+  uint64_t held = block_bytes(end ? end : 256);
   hipStream_t st = (hipStream_t)pk_ctx_stream(c);
   // the job's kernels finish before its result block is allocated
   hipError_t e = hipStreamSynchronize(st);
@@ -159,9 +233,8 @@ void pk_server::run(int slot, Job* j) {
     return;
   }
   void* mem = nullptr;
-  e = pools ? hipMallocAsync(&mem, end ? end : 256, st) : hipMalloc(&mem, end ? end : 256);
+  e = take_block(&held, st, &mem);
   if (e != hipSuccess) {
-    (void)hipGetLastError();
     r.status = PK_ENOMEM;
     std::snprintf(r.message, sizeof(r.message), "result allocation failed: %s", hipGetErrorString(e));
     return;
@@ -181,7 +254,7 @@ void pk_server::run(int slot, Job* j) {
     std::snprintf(r.message, sizeof(r.message), "result copy failed: %s", hipGetErrorString(e));
   }
   j->mem = mem;
-  j->mem_bytes = end;
+  j->mem_bytes = held;
   r.table = pk_table{t.n, t.words, t.k, (const uint64_t*)(m + o1), (const int32_t*)(m + o2)};
   r.kept = pk_table{kt.n, t.words, t.k, (const uint64_t*)(m + o3), (const int32_t*)(m + o4)};
   r.nodes = pk_mn_table{mt.n, t.k, (const pk_mnode*)(m + o5)};
@@ -206,6 +279,7 @@ void pk_server::worker(int slot) {
   const uint64_t slot_keep = budget / (uint64_t)(n_slots > 0 ? n_slots : 1);
   for (;;) {
     Job* j;
+    std::vector<Block> drop;
     {
       std::unique_lock<std::mutex> lk(mu);
       cv_q.wait(lk, [&] { return stop || admissible(); });
@@ -215,8 +289,11 @@ void pk_server::worker(int slot) {
       j->state = 1;
       running++;
       running_est += j->res.est_bytes;
+      const uint64_t used = running_est + resident;
+      drop = drop_spare(used < budget ? budget - used : 0);
       j->res.t_start = now();
     }
+    free_blocks(drop);
     run_guarded(slot, j);
     // a slot that grew past its share gives its buffers back
     if (pk_ctx_device_bytes(ctx[slot]) > slot_keep) (void)pk_ctx_release_buffers(ctx[slot]);
@@ -313,6 +390,7 @@ void pk_server_destroy(pk_server* s) {
     }
     delete kv.second;
   }
+  s->free_blocks(s->drop_spare(0));
   (void)hipStreamSynchronize(s->free_stream);
   (void)hipStreamDestroy(s->free_stream);
   for (auto* c : s->ctx) pk_ctx_destroy(c);
@@ -459,6 +537,7 @@ int pk_server_set_tuning(pk_server* s, const pk_tune_entry* entries, int n) {
 int pk_server_release(pk_server* s, uint64_t ticket) {
   if (!s) return PK_EINVAL;
   Job* j;
+  std::vector<pk_server::Block> drop;
   {
     std::unique_lock<std::mutex> lk(s->mu);
     auto it = s->jobs.find(ticket);
@@ -475,11 +554,16 @@ int pk_server_release(pk_server* s, uint64_t ticket) {
     j = it->second;
     s->jobs.erase(it);
     s->resident -= j->mem_bytes;
+    if (j->mem) {
+      s->spare.push_back(pk_server::Block{j->mem, j->mem_bytes});
+      s->spare_bytes += j->mem_bytes;
+      const uint64_t used = s->running_est + s->resident;
+      drop = s->drop_spare(std::min(s->budget / 8, used < s->budget ? s->budget - used : 0));
+    }
   }
-  if (j->mem) {
+  if (!drop.empty()) {
     (void)hipSetDevice(s->device);
-    if (s->pools) (void)hipFreeAsync(j->mem, s->free_stream);
-    else (void)hipFree(j->mem);
+    s->free_blocks(drop);
   }
   delete j;
   s->cv_q.notify_all();

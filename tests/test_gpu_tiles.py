@@ -265,3 +265,33 @@ def test_rewrite_by_output(ctx, oracle_mod, size, end):
                     ctx.normalize(data, fmt)
                 continue
             assert ctx.normalize(data, fmt) == want, (fmt, cut)
+
+
+def test_served_results_in_reused_blocks(ctx):
+    """Result blocks of released jobs serve later jobs: sizes that fit a spare
+    block, nearly fit and do not, two slots, results downloaded while others'
+    blocks change hands."""
+    from pakman_plus_amd import api
+    rng = np.random.default_rng(11)
+    sets = []
+    for reads in (400, 430, 380, 2_000, 60, 405):
+        one = b"".join(b">r\n" + _bases(rng, 90, b"ACGT") + b"\n" for _ in range(reads))
+        sets.append(one * 3)
+    want = []
+    for fa in sets:
+        ctx.count(fa, 31)
+        want.append(ctx.table_host())
+    srv = api.Server(0, n_slots=2)
+    try:
+        for rnd in range(4):
+            order = rng.permutation(len(sets))
+            _p(f"case: served round {rnd} order {order.tolist()}")
+            tickets = [srv.submit(fasta=sets[int(i)], k=31, t=2) for i in order]
+            for i, tk in zip(order, tickets):
+                r = srv.wait(tk)
+                got = srv.download(r)
+                keys, counts = want[int(i)]
+                assert np.array_equal(got["keys"], keys) and np.array_equal(got["counts"], counts)
+                srv.release(tk)
+    finally:
+        srv.close()
