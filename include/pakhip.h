@@ -129,7 +129,7 @@ uint64_t pk_ctx_device_bytes(const pk_ctx* ctx);
  *                  rank shares as few as keep their runs at 32 keys)
  *   bucket_factor  instances per final bucket as a multiple of the LDS hash
  *                  table's key capacity, i.e. the inverse hash load target
- *                  (built-in: at most 2.1 for one-word keys, 2.2 for two)
+ *                  (built-in: at most 2.6)
  *   ms_scatter     0..2, no effect (chose between two former scatter kernels)
  *   ms_fold        0..2, no effect (switched a former histogram fold off)
  */

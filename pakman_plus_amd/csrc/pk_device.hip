@@ -2373,7 +2373,11 @@ __global__ __launch_bounds__(256) void k_bits_count(const ull* W, uint32_t* cnt)
 
 // Blocks of 512 threads, as many waves per CU as the keys' registers allow.
 // Batches of a whole bucket: a second batch costs a second run map and its
-// barriers (k = 63, 1.5e8 keys: 2.46 ms with batches of 2048 against 1.41).
+// barriers (k = 63, 1.5e8 keys: 2.46 ms with batches of 2048 against 1.41; k =
+// 32, 2.5e8 keys of 3900 a bucket: 1.30 with 4096, 1.17 with 5120).  Buckets up
+// to a batch: fewer of them for the same keys (7.6e7 keys: 0.32 ms with 2300 a
+// bucket, 0.26 with 4600), and two partition levels instead of three more often
+// (2.9e9 two-word keys: 88.7 -> 82.4 ms).
 template <class Key>
 struct HashCfg;
 template <>
@@ -2383,18 +2387,18 @@ struct HashCfg<uint64_t> {
   static constexpr int T = 2560;      // table slots (12 bytes each)
   static constexpr int LIMIT = 1920;  // distinct keys per task (load 0.75)
   static constexpr int SUB = 11;      // sub-bin bits of the ordering
-  static constexpr int HB = 8;        // keys per thread and batch
-  static constexpr float FILL = 2.1f;  // built-in instances per bucket: FILL * LIMIT at most, one batch
+  static constexpr int HB = 10;       // keys per thread and batch
+  static constexpr float FILL = 2.6f;  // built-in instances per bucket: FILL * LIMIT at most, one batch
 };
 template <>
 struct HashCfg<u128> {
   static constexpr int NT = 512;
-  static constexpr int WAVES = 6;  // three blocks: at 64 VGPRs the keys spill (1.41 -> 1.77 ms, 1.5e8 keys)
+  static constexpr int WAVES = 8;
   static constexpr int T = 1536;   // 20 bytes each
   static constexpr int LIMIT = 1152;
   static constexpr int SUB = 10;
-  static constexpr int HB = 5;
-  static constexpr float FILL = 2.2f;
+  static constexpr int HB = 6;
+  static constexpr float FILL = 2.6f;
 };
 
 // a 32-bit hash scaled to T slots
@@ -2919,25 +2923,28 @@ __device__ __forceinline__ int count_task(HashShared<Key>& L, const Key* S, Key*
         *reinterpret_cast<int32_t*>(Co + p * 4u) = (int32_t)oc[i];
       }
       out += nd;
+      if (!MULTI) break;
       __syncthreads();
     }
     // too many distinct keys: once more with one more split bit; splitting
     // does not help a fingerprint collision
-    if (fail != 1) break;
+    if (!MULTI || fail != 1) break;
   }
   *out_n = out;
   return fail;
 }
 
-// What bounds it: issue.  Per one-word key (2.5e8 keys, 7.7e7 distinct) 115 VALU
-// and 20 LDS lane instructions; inserts overlap with the loads of other
-// blocks, the ordering of the distinct keys is half the kernel (timing
-// copies: loads alone 0.49 of 1.5 ms, with inserts 0.57).  Sub-bins of about
-// one key, vector clears, a DPP scan and one packed register for (bin, index)
-// took it from 1.51 to 1.34 ms; tables of 256 or 1024 threads and of 2048 to
-// 6144 slots were within 10 % of each other.  Two-word keys (1.5e8): 2.83 ms
-// with 28-byte slots in 1024-slot tables that overflow at 0.4 distinct keys
-// per key, 1.41 ms now.
+// What bounds it: VALU and LDS are each busy half of the time, and barriers
+// between the phases hold the rest.  Of 1.35 ms for 2.5e8 one-word keys, 7.7e7
+// distinct (timing copies): loads and map 0.69, inserts 0.23, ordering 0.27,
+// writes 0.16.  Sub-bins, vector clears, a DPP scan and one packed register for
+// (bin, index) took it from 1.51 to 1.34 ms; without the pass loops around the
+// single pass nothing is hoisted out of them and no register spills (the spills
+// moved 2.3 of 5.3 GB), which with larger batches gives 1.17.  Two-word keys
+// (1.5e8): 2.83 ms with 28-byte slots, 1.42 at 6 waves per SIMD, 1.17 at the 8
+// that fit without spills.  256 or 1024 threads and 2048 to 6144 slots were
+// within 10 % of each other; resident blocks that load the next bucket's keys
+// early, or a map built by all waves, were slower.
 //
 // One block per bucket of `in`: tu[b] = the bucket's distinct keys, bstart[b]
 // = where they are.  Buckets the table is too small for go to the retry list
