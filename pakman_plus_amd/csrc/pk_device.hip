@@ -3836,6 +3836,9 @@ struct pk_ctx {
   uint64_t held = 0;
   std::string err;
   DevBuf buf[B_COUNT];
+  // buffers whose contents no work to come will read: given back when a
+  // budget (or the device) has no room for another one
+  bool idle[B_COUNT] = {};
   // 0-19: stage boundaries; 20 + 2 L, 21 + 2 L: around k_split of further
   // partition level L for the first MS_TIMED_LEVELS levels
   hipEvent_t ev[20 + 2 * MS_TIMED_LEVELS] = {};
@@ -3903,9 +3906,32 @@ struct pk_ctx {
 
 namespace {
 
+// Frees idle buffers until `bytes` more fit the budget (all of them without
+// one); false when there were none.
+bool reclaim(pk_ctx* c, uint64_t bytes) {
+  bool any = false;
+  for (int i = 0; i < B_COUNT; i++) {
+    if (!c->idle[i] || !c->buf[i].p) continue;
+    if (any && c->budget && c->held + bytes <= c->budget) break;
+    if (!any) (void)hipStreamSynchronize(c->stream);
+    any = true;
+    (void)(c->stream_alloc ? hipFreeAsync(c->buf[i].p, c->stream) : hipFree(c->buf[i].p));
+    c->held -= c->buf[i].cap;
+    c->buf[i] = DevBuf{};
+  }
+  return any;
+}
+
+// A new count begins: the last results are void, and every buffer but its
+// input is idle until the count asks for it.
+void begin_buffers(pk_ctx* c) {
+  for (int i = 0; i < B_COUNT; i++) c->idle[i] = i != B_FASTA && i != B_NORM;
+}
+
 template <class T>
 int need(pk_ctx* c, int id, uint64_t count, T** out) {
   DevBuf& b = c->buf[id];
+  c->idle[id] = false;
   const uint64_t bytes = count * sizeof(T) + 256;
   if (c->arena_mode) {
     if (c->arena_fixed[id]) {
@@ -3937,10 +3963,16 @@ int need(pk_ctx* c, int id, uint64_t count, T** out) {
       b.p = nullptr;
       b.cap = 0;
     }
-    if (c->budget && c->held + bytes > c->budget)
-      return c->fail(PK_ENOMEM, "device budget exceeded");
+    if (c->budget && c->held + bytes > c->budget) {
+      (void)reclaim(c, bytes);
+      if (c->held + bytes > c->budget) return c->fail(PK_ENOMEM, "device budget exceeded");
+    }
     void* p = nullptr;
     hipError_t e = c->stream_alloc ? hipMallocAsync(&p, bytes, c->stream) : hipMalloc(&p, bytes);
+    if (e != hipSuccess && reclaim(c, bytes)) {
+      (void)hipGetLastError();
+      e = c->stream_alloc ? hipMallocAsync(&p, bytes, c->stream) : hipMalloc(&p, bytes);
+    }
     if (e != hipSuccess) {
       (void)hipGetLastError();
       return c->fail(PK_ENOMEM, std::string("hipMalloc failed: ") + hipGetErrorString(e));
@@ -4691,6 +4723,11 @@ int count_partitioned(pk_ctx* c, Key* S, Key* S2, int32_t* C, Part p, int btot, 
     PK_TRY(d2h(c, &U, uoff + nleaves, 8));
   }
   c->U = U;
+  // what is left to do reads the buckets' results and their places only
+  for (int id : {B_BOFF, B_TP, B_HIST1, B_OFF1, B_BOFF2, B_TP2, B_HIST2, B_OFF2, B_RETRY, B_OVF, B_WOFF, B_OWNOFF})
+    c->idle[id] = true;
+  for (int id : {B_S, B_S2, B_TMP})
+    if (c->buf[id].p != static_cast<const void*>(Res)) c->idle[id] = true;
   PK_TRY(need(c, B_TK, U, &TK));
   PK_TRY(need(c, B_TC, U, &TC));
   PK_HIP(c, hipEventRecord(c->ev[10], st));
@@ -4807,6 +4844,8 @@ int count_records(pk_ctx* c, const Records& rec, int K, int KB, Key mask) {
   // the packed input has been read: its scratch is free for what follows
   // in stream order
   c->arena_lim = c->arena_cap;
+  c->idle[B_PACK] = c->idle[B_OWNW] = c->idle[B_LW] = c->idle[B_WCNT] = true;
+  c->idle[B_RSTART] = c->idle[B_RLEN] = c->idle[B_KC] = c->idle[B_KOFS] = c->idle[B_NL] = true;
   PK_TRY(need(c, B_S2, N, &S2));
   PK_TRY(need(c, B_C, N, &C));
   p.B = 1ull << d1;
@@ -4913,6 +4952,7 @@ int windows_count_impl(pk_ctx* c, const uint8_t* fa, const ull* rstart, const ui
 template <class Key>
 int count_impl(pk_ctx* c, const uint8_t* fa, uint64_t n, int K) {
   c->have_table = c->have_kept = c->have_nodes = false;
+  begin_buffers(c);
   c->timing = pk_timing{};
   c->pend_count = c->pend_split = c->pend_cutoff = c->pend_mn = c->pend_norm = false;
   c->key_bits = 2 * K;
@@ -5031,6 +5071,7 @@ int own_windows(pk_ctx* c, int K, const ull* freq, int P, int rank, Records* rec
 template <class Key>
 int rank_share_impl(pk_ctx* c, const uint8_t* fa, uint64_t n, int K, int P, int rank, bool by_key) {
   c->have_table = c->have_kept = c->have_nodes = false;
+  begin_buffers(c);
   c->timing = pk_timing{};
   c->pend_count = c->pend_split = c->pend_cutoff = c->pend_mn = c->pend_norm = false;
   c->key_bits = 2 * K;
@@ -5050,6 +5091,7 @@ template <class Key>
 int builder_count_impl(pk_ctx* c, const uint8_t* fa, uint64_t n, int klen, uint64_t read_len,
                        BldSyms sy) {
   c->have_table = c->have_kept = c->have_nodes = false;
+  begin_buffers(c);
   c->timing = pk_timing{};
   c->pend_count = c->pend_split = c->pend_cutoff = c->pend_mn = c->pend_norm = false;
   c->key_bits = (int)sizeof(Key) * 8;
@@ -5773,6 +5815,7 @@ int pk_builder_count_windows(pk_ctx* c, const char* fasta, uint64_t nbytes, int 
   c->timing = pk_timing{};
   c->pend_count = c->pend_split = c->pend_cutoff = c->pend_mn = c->pend_norm = false;
   c->have_table = c->have_kept = c->have_nodes = false;
+  begin_buffers(c);
   const BldSyms sy{(uint8_t)delimiter, (uint8_t)skip_symbol};
   PK_HIP(c, hipSetDevice(c->device));
   const uint8_t* fa;

@@ -295,3 +295,46 @@ def test_served_results_in_reused_blocks(ctx):
                 srv.release(tk)
     finally:
         srv.close()
+
+
+@pytest.mark.parametrize("k", [21, 32, 55])
+def test_budget_gives_idle_buffers_back(k):
+    """Budgets below what a count holds without one: the same results, from
+    buffers given back and asked for again, or PK_ENOMEM; two counts, cutoff
+    and nodes per budget, and a count of the other kind between."""
+    from pakman_plus_amd import api
+    rng = np.random.default_rng(k)
+    genome = _bases(rng, 30_000, b"ACGT")
+    fa = b"".join(b">r\n" + genome[i:i + 100] + b"\n" for i in rng.integers(0, 29_900, 9_000))
+    free = api.Context(0)
+    free.count(fa, k)
+    want = free.table_host()
+    free.cutoff_threshold(2)
+    free.macro_nodes()
+    kept, nodes, held = free.kept_host(), free.nodes_host(), free.device_bytes
+    free.close()
+    done = 0
+    for share in (1.0, 0.9, 0.8, 0.7, 0.6, 0.45):
+        _p(f"case: budget k={k} share={share}")
+        c = api.Context(0, int(held * share))
+        try:
+            for _ in range(2):
+                c.count(fa, k)
+                got = c.table_host()
+                assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])
+                c.cutoff_threshold(2)
+                c.macro_nodes()
+                got = c.kept_host()
+                assert np.array_equal(got[0], kept[0]) and np.array_equal(got[1], kept[1])
+                assert np.array_equal(c.nodes_host(), nodes)
+                assert c.device_bytes <= held * share
+                try:  # needs more than the main path's count
+                    c.builder_count(fa, k, read_len=90, kmer_bits=64 if k <= 32 else 128)
+                except api.PakHipError as e:
+                    assert e.code == api.PK_ENOMEM
+            done += 1
+        except api.PakHipError as e:
+            assert e.code == api.PK_ENOMEM
+        finally:
+            c.close()
+    assert done >= 2
