@@ -338,3 +338,25 @@ def test_budget_gives_idle_buffers_back(k):
         finally:
             c.close()
     assert done >= 2
+
+
+def test_lmer_frequency_budgets():
+    """L-mer frequencies with room for every block's table, for a few, and
+    without room for the packed input (the read table's walk)."""
+    from pakman_plus_amd import api
+    import rank_util as RU
+    rng = np.random.default_rng(2)
+    fa = b"".join(b">r\n" + _bases(rng, 100, b"ACGTN") + b"\n" for _ in range(20_000))
+    want = RU.lmer_freq(fa)
+    done = 0
+    for budget in (0, 40 << 20, 8 << 20, 4_200_000, 3_600_000, 3_300_000, 2_500_000):
+        _p(f"case: L-mers budget={budget}")
+        c = api.Context(0, budget)
+        try:
+            assert np.array_equal(c.lmer_frequency(fa), want)
+            done += 1
+        except api.PakHipError as e:
+            assert e.code == api.PK_ENOMEM
+        finally:
+            c.close()
+    assert done >= 4
