@@ -2204,8 +2204,10 @@ __global__ __launch_bounds__(OWN_NT) void k_own(const uint32_t* __restrict__ E, 
       pre[i] = (uint32_t)rk[l] << 16 | (((ob[l >> 5] >> (l & 31u)) & 1u) | (uint32_t)((i + 2) << 1));
       suf[i] = pre[i];
     }
-    // (no window reaches past a line's end: the ends before one do not count)
-    const uint32_t nl = (rx >> 16 | (__shfl_down(rx, 1, 64) & 0x10000u)) >> 1;
+    // (no window reaches past a line's end, so that the ends before one need not
+    // be followed; the last lane, which does not see the next word, keeps its)
+    const uint32_t rn = __shfl_down(rx, 1, 64);
+    const uint32_t nl = (rx >> 16 | ((tid & 63) == 63 ? 0u : rn & 0x10000u)) >> 1;
     dirty = dirty >> 16 & ~nl;
 #pragma unroll
     for (int i = 14; i >= 0; i--)

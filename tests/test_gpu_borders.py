@@ -1,0 +1,85 @@
+"""Inputs that put the thing a kernel treats specially right at the border of
+a wave, a block, a tile or a batch, bit-exact against the oracle or a
+restatement."""
+from __future__ import annotations
+
+import sys
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _p(*a):
+    print(*a, flush=True)
+    sys.stdout.flush()
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    from pakman_plus_amd import api
+    c = api.Context(0)
+    yield c
+    c.close()
+
+
+def _bases(rng, n, alpha=b"ACGT"):
+    return bytes(rng.choice(np.frombuffer(alpha, dtype=np.uint8), n))
+
+
+def _shares_match(ctx, fa, k, P):
+    """Every rank's share against the window-by-window restatement."""
+    import rank_util as RU
+    freq = RU.lmer_freq(fa)
+    walk = RU.owner_walk(fa, k, P, freq)
+    for r in range(P):
+        ctx.count_rank_share(fa, k, P, r)
+        keys, counts = ctx.table_host()
+        assert RU.table_counter(keys, counts) == RU.share_counter(walk, r), r
+
+
+@pytest.mark.parametrize("k", [9, 15, 31, 64])
+@pytest.mark.parametrize("tile", [0, 1])
+@pytest.mark.parametrize("ends", ["header", "sequence"])
+def test_share_line_end_in_a_waves_last_word(ctx, k, tile, ends):
+    """The owner rule takes 16-byte words, 64 a wave and 508 a tile (its first
+    wave starts four words before the tile): a line end at the first byte of a
+    wave's last word, and of the words on either side of it, and right behind
+    that word a byte whose third code bit is set, after a base whose low code
+    bit is clear, so that the L-mer that ends there is another one when it is
+    read back from the k-mer.  The line end is a header's, or a read's with an
+    empty header after it."""
+    rng = np.random.default_rng(1000 * k + 10 * tile + len(ends))
+    for word in [508 * tile + 64 * wave + lane - 4 for wave in (0, 1, 7) for lane in (62, 63, 64)]:
+        at = 16 * word
+        for trial in range(8):
+            _p(f"case: share line end k={k} tile={tile} {ends} word={word} trial={trial}")
+            if ends == "header":
+                last, first = b">" + b"h" * 9 + b"\n", _bases(rng, 14)
+            else:
+                last, first = b">\n" + _bases(rng, 30) + b"\n", b">\n" + _bases(rng, 12)
+            fill = b"\n" + _bases(rng, 80) + b"\n"
+            fa = b">" + b"f" * (at + 1 - len(last) - len(fill) - 1) + fill + last
+            assert len(fa) == at + 1
+            fa += first + b"AN" + _bases(rng, 130) + b"\n"
+            assert fa[at] == 10 and fa[at + 15:at + 17] == b"AN"
+            _shares_match(ctx, fa, k, 3)
+
+
+@pytest.mark.parametrize("k", [9, 31, 64])
+def test_share_of_reads_at_every_alignment(ctx, k):
+    """As many records of 131 bytes as a tile has bytes (8128), each with bytes
+    outside A, C, G and T among its first bases: every place of a line end in a
+    tile occurs."""
+    rng = np.random.default_rng(k)
+    reads = []
+    for i in range(8128):
+        r = bytearray(_bases(rng, 128))
+        for p in rng.integers(17, 60, 2):
+            r[p] = b"NnX"[p % 3]
+        r[14:16] = b"AN"
+        reads.append(b">\n" + bytes(r) + b"\n")
+    assert len(reads[0]) == 131
+    _p(f"case: share at every alignment k={k}")
+    _shares_match(ctx, b"".join(reads), k, 2)
