@@ -2767,8 +2767,9 @@ __device__ __forceinline__ int count_task(HashShared<Key>& L, const Key* S, Key*
       Key kb[HB];
       int ksl[HB];  // u128: the slot each key of the batch landed in, or -1 - its place in the queue
       bool clash = false;
-      // over as read after the last batch's final barrier (nothing writes it
-      // between that read and the next barrier): all threads leave together
+      // over as read between two barriers of the last batch (the first wave
+      // writes it while it makes the next batch's map): all threads leave
+      // together
       int ov = 0, m = 0;
       for (ull b = 0; b < n && !ov; b += m) {
         m = load_batch<Key, RUNS, !MULTI, HB>(L, Sb, in, rb, b, kb);
@@ -2830,6 +2831,7 @@ __device__ __forceinline__ int count_task(HashShared<Key>& L, const Key* S, Key*
               }
             }
           }
+          if (b + m < n) __syncthreads();
         } else {
 #pragma unroll
           for (int j = 0; j < HB; j++) {

@@ -83,3 +83,29 @@ def test_share_of_reads_at_every_alignment(ctx, k):
     assert len(reads[0]) == 131
     _p(f"case: share at every alignment k={k}")
     _shares_match(ctx, b"".join(reads), k, 2)
+
+
+@pytest.mark.parametrize("k", [24, 32, 33, 40, 64])
+def test_bucket_whose_later_batch_has_too_many_runs(ctx, oracle_mod, k):
+    """Buckets of several batches: the first keys come from a few tiles, the last
+    ones from 900 tiles with two keys each, more runs than a batch's map holds,
+    which the first wave finds while the others end the batch before."""
+    rng = np.random.default_rng(k)
+    genome = _bases(rng, 8_000)
+
+    def cut(n):
+        a = int(rng.integers(0, len(genome) - n))
+        return genome[a:a + n]
+
+    fa = b"".join(b">a\n" + cut(k + 99) + b"\n" for _ in range(500))
+    fa += b"".join(b">" + b"h" * (16_384 - k - 18) + b"\n" + cut(k + 15) + b"\n" for _ in range(900))
+    try:
+        ctx.set_tuning(l1_bits=10, bucket_factor=10.0)
+        _p(f"case: late runs k={k}")
+        ctx.count(fa, k)
+        keys, counts = ctx.table_host()
+    finally:
+        ctx.set_tuning()
+    want_k, want_c = oracle_mod.count(fa, k)
+    assert np.array_equal(keys.reshape(-1), np.asarray(want_k).reshape(-1))
+    assert np.array_equal(counts, want_c)
