@@ -984,7 +984,11 @@ __global__ __launch_bounds__(256) void k_bld_bits(const uint8_t* fa, uint64_t n,
     // the header's delimiter lies right before the read
     uint64_t e2 = e + 1;
     while (e2 < m && ev[e2] < rb) e2++;
-    if (e2 < m && ev[e2] < rb + rl) stat[1] = 1;
+    if (e2 < m && ev[e2] < rb + rl) {
+      // (no ends: reads that all run to the input's end would set n^2 of them)
+      stat[1] = 1;
+      continue;
+    }
     const ull a = rb + (uint64_t)klen - 1, b = rb + rl;  // ends [a, b)
     for (ull w = a >> 6; w * 64 < b; w++) {
       ull bits = ~0ull;

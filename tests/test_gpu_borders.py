@@ -4,6 +4,7 @@ restatement."""
 from __future__ import annotations
 
 import sys
+import time
 
 import numpy as np
 import pytest
@@ -109,3 +110,31 @@ def test_bucket_whose_later_batch_has_too_many_runs(ctx, oracle_mod, k):
     want_k, want_c = oracle_mod.count(fa, k)
     assert np.array_equal(keys.reshape(-1), np.asarray(want_k).reshape(-1))
     assert np.array_equal(counts, want_c)
+
+
+@pytest.mark.parametrize("klen,bits", [(32, 64), (64, 128)])
+def test_builder_reads_to_the_end_of_the_input(klen, bits):
+    """A million records with a read length beyond the input: their reads run to
+    its end, 4e13 windows, which no budget has room for; refused as soon as their
+    number is known, and the context counts on."""
+    from pakman_plus_amd import api
+    rng = np.random.default_rng(klen)
+    rows = np.full((1_000_000, 74), 10, dtype=np.uint8)
+    rows[:, 0] = ord(">")
+    rows[:, 2:73] = rng.choice(np.frombuffer(b"ACGT", dtype=np.uint8), (rows.shape[0], 71))
+    fa = rows.tobytes()
+    c = api.Context(0, 8 << 30)
+    try:
+        c.builder_count(fa, klen, read_len=71, kmer_bits=bits)
+        want = c.table_host()
+        _p(f"case: reads to the end klen={klen}")
+        t = time.perf_counter()
+        with pytest.raises(api.PakHipError) as e:
+            c.builder_count(fa, klen, read_len=0xFFFFFFF0, kmer_bits=bits)
+        assert e.value.code == api.PK_ENOMEM
+        assert time.perf_counter() - t < 5.0
+        assert c.builder_count(fa, klen, read_len=71, kmer_bits=bits) == rows.shape[0]
+        got = c.table_host()
+        assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])
+    finally:
+        c.close()
