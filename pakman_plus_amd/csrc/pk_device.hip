@@ -3138,12 +3138,16 @@ __global__ void k_copy_tasks(Key* S, const Key* T, const ull* tstart, const ull*
   for (uint64_t i = off + threadIdx.x; i < n && i < off + PT_PER; i += blockDim.x) S[s + i] = T[s + i];
 }
 
-// The runs of the listed buckets gathered at their virtual places (one block
-// per bucket; oversize buckets only).
+// The runs of the listed buckets gathered at their virtual places: gridDim.x
+// blocks per bucket (blockIdx.y), each every gridDim.x-th run.  Bound by the
+// reads of the runs (3.6e7 builder words of 11 bases and more, 8 oversize buckets
+// of 1300 runs: the whole split 3.4 ms, with one block per bucket 13.5).
+constexpr unsigned GATHER_BLOCKS = 256;
+
 template <class Key>
 __global__ void k_gather_buckets(const Key* S, Runs in, const ull* buckets, Key* out) {
-  const RunBucket rb = run_bucket(in, buckets[blockIdx.x]);
-  for (ull t = 0; t < rb.nt; t++) {
+  const RunBucket rb = run_bucket(in, buckets[blockIdx.y]);
+  for (ull t = blockIdx.x; t < rb.nt; t += gridDim.x) {
     const ull e = rb.e0 + t, v = in.V[e], c = in.V[e + 1] - v;
     const Key* src = S + rb.base + tile_place(in, t) + (in.M[e] >> 16);
     for (ull i = threadIdx.x; i < c; i += blockDim.x) out[v + i] = src[i];
@@ -4732,9 +4736,12 @@ int count_partitioned(pk_ctx* c, Key* S, Key* S2, int32_t* C, Part p, int btot, 
       ull* od;
       PK_TRY(need(c, B_PT0, oi.size(), &od));
       PK_HIP(c, hipMemcpyAsync(od, oi.data(), oi.size() * 8, hipMemcpyHostToDevice, st));
-      hipLaunchKernelGGL(HIP_KERNEL_NAME(k_gather_buckets<Key>), dim3((unsigned)oi.size()), dim3(256), 0, st, S, in,
-                         od, tmp);
-      PK_HIP(c, hipGetLastError());
+      for (size_t q = 0; q < oi.size(); q += 32768) {
+        const unsigned nq = (unsigned)std::min<size_t>(32768, oi.size() - q);
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_gather_buckets<Key>), dim3(GATHER_BLOCKS, nq), dim3(256), 0, st, S, in,
+                           od + q, tmp);
+        PK_HIP(c, hipGetLastError());
+      }
       PK_HIP(c, hipStreamSynchronize(st));  // od's buffer is used again below
       std::swap(S, tmp);
     }
