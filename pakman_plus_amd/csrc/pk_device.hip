@@ -2458,7 +2458,7 @@ template <int T>
 __device__ __forceinline__ uint32_t next_slot(uint32_t slot) {
   return slot + 1 == (uint32_t)T ? 0u : slot + 1;
 }
-// tasks with more instances than this are split without trying
+// instances of a task that one block goes through more than once
 constexpr uint64_t TASK_MAX_INSTANCES = 1u << 18;
 // linear-probe bound of an insert: a table too full to place a key within
 // it sends the task to the next pass split (the host sizes buckets for a
@@ -2763,7 +2763,10 @@ __device__ __forceinline__ int load_batch(HashShared<Key>& L, const Key* Sb, con
 // 1 when the table is too small for the distinct keys, 2 on a u128
 // fingerprint collision, 3 when a batch has too many runs.  With MULTI a task with too many distinct keys is
 // processed in 2^s passes, pass p taking the keys whose next s bits equal p
-// (s = 1, 2, ... up to MAX_PASS_BITS).
+// (s = 1, 2, ... up to MAX_PASS_BITS).  A task of more instances than
+// TASK_MAX_INSTANCES takes all keys at once first, which costs a batch or two
+// where they are distinct, and then as many passes as leave that number to each
+// (1.4e7 equal keys of one bucket: 190 ms in 16 passes, 32 in one).
 template <class Key, bool RUNS, bool MULTI>
 __device__ __forceinline__ int count_task(HashShared<Key>& L, const Key* S, Key* R, int32_t* C, const Runs& in,
                                           const RunBucket& rb, bool top, int K, int fixed, ull* out_n) {
@@ -2783,8 +2786,8 @@ __device__ __forceinline__ int count_task(HashShared<Key>& L, const Key* S, Key*
   int s = 0, fail = 0;
   // a first try with all keys is pointless when there are too many of them
   if (!MULTI && (n > (ull)TASK_MAX_INSTANCES || rb.nt > WAVE_MAP_RUNS)) return 1;
-  while (MULTI && s < max_s && (n >> s) > (ull)TASK_MAX_INSTANCES) s++;
   for (; s <= max_s; s++) {
+    while (MULTI && s > 0 && s < max_s && (n >> s) > (ull)TASK_MAX_INSTANCES) s++;
     out = 0;
     fail = 0;
     for (int pass = 0; pass < (MULTI ? 1 << s : 1) && !fail; pass++) {

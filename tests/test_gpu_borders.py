@@ -193,3 +193,24 @@ def test_split_of_buckets_with_many_runs(ctx, oracle_mod):
             assert np.array_equal(keys, np.asarray(want_k).reshape(-1)) and np.array_equal(counts, want_c)
     assert np.all(keys[1:] > keys[:-1]) and int(counts.sum()) == 90 * reads
     assert t["split_ms"] < 8.0
+
+
+@pytest.mark.parametrize("k", [32, 64])
+def test_bucket_of_equal_keys(ctx, oracle_mod, k):
+    """Most k-mers of the input equal, the others in the same bucket and beside
+    it: one block counts them, in one pass (1e7 of k = 32: 23 ms; in sixteen passes
+    137)."""
+    rng = np.random.default_rng(k)
+    tail = b"".join(b">t\n" + b"A" * (k // 2) + _bases(rng, 2 * k) + b"\n" for _ in range(50))
+    read = b">r\n" + b"A" * 150 + b"\n"
+    n = 10_000_000 // (151 - k)
+    _p(f"case: equal keys k={k}")
+    for _ in range(2):
+        ctx.count(read * n + tail, k)
+    keys, counts = ctx.table_host()
+    want_k, want_c = oracle_mod.count(read + tail, k)
+    want_c = np.array(want_c)
+    want_c[0] += (n - 1) * (151 - k)  # A is 0: the first key
+    assert np.array_equal(keys.reshape(-1), np.asarray(want_k).reshape(-1))
+    assert np.array_equal(counts, want_c)
+    assert ctx.timing()["sort_ms"] < 60.0
