@@ -2412,7 +2412,7 @@ __global__ __launch_bounds__(256) void k_bits_count(const ull* W, uint32_t* cnt)
 
 // ---------------------------------------------------------------------------
 // Per-bucket count: LDS hash table of the bucket's distinct keys (64-bit CAS,
-// linear probing; duplicates cost one atomic add), then a counting sort of
+// double hashing; duplicates cost one atomic add), then a counting sort of
 // the distinct keys by a 12-bit sub-digit into LDS, a per-sub-bin insertion
 // sort (sub-bins hold ~1-2 distinct keys) and a coalesced write of the
 // bucket's (key, count) pairs.  This is the reference's sort + run-length +
@@ -2454,16 +2454,24 @@ template <int T>
 __device__ __forceinline__ uint32_t slot_of(uint32_t h) {
   return __umulhi(h, (uint32_t)T);
 }
+// Probes step by an odd number from the hash's low bits, so that keys that
+// meet in a slot part ways (steps of one run into each other: 6.2e7 keys in
+// tables 0.9 full 0.73 ms, with steps of one 2.6).  A step divisible by T's odd
+// factor is back after T / 3 or T / 5 = 512 probes.
 template <int T>
-__device__ __forceinline__ uint32_t next_slot(uint32_t slot) {
-  return slot + 1 == (uint32_t)T ? 0u : slot + 1;
+__device__ __forceinline__ uint32_t next_slot(uint32_t slot, uint32_t step) {
+  const uint32_t s = slot + step;
+  return s < (uint32_t)T ? s : s - (uint32_t)T;
 }
+__device__ __forceinline__ uint32_t probe_step(uint32_t h) { return (h & 255u) | 1u; }
 // instances of a task that one block goes through more than once
 constexpr uint64_t TASK_MAX_INSTANCES = 1u << 18;
-// linear-probe bound of an insert: a table too full to place a key within
-// it sends the task to the next pass split (the host sizes buckets for a
-// load of about 0.75, where probes average a few slots)
-constexpr int HASH_PROBES = 256;
+// probe bound of an insert: a table too full to place a key within it sends the
+// task to more passes.  48 places all keys of a table 0.8 full; a table that
+// cannot hold its keys costs up to twice one that can (six times with steps of
+// one and a bound of 256: 1.3e8 keys, 0.72 of them distinct, 3.1 ms; now 0.9).
+// The bound of a pass that is one of several is longer: it may be the last.
+constexpr int HASH_PROBES = 48, HASH_PROBES_MULTI = 128;
 // a probe chain longer than STOP_AFTER slots re-reads the task's overflow
 // flag every 8 probes: once one thread has found the table full, the others
 // stop probing it (short chains, the usual case, never read it)
@@ -2483,15 +2491,15 @@ struct HashTable<uint64_t> {
     for (int i = tid; i < T / 2; i += nt) reinterpret_cast<ulonglong2*>(hk)[i] = make_ulonglong2(empty, empty);
     for (int i = tid; i < T / 4; i += nt) reinterpret_cast<uint4*>(hc)[i] = make_uint4(0u, 0u, 0u, 0u);
   }
-  // returns false when no free slot is found within HASH_PROBES probes, or
-  // when a long chain finds the table already reported full (*stop)
+  // returns false when no free slot is found within PROBES probes, or when a
+  // long chain finds the table already reported full (*stop)
   // (a read before the CAS, as for u128 keys, was slower here: a new key
   // then waits on two LDS round trips)
   // one 32-bit product: the kernel is bound by issue, and a 64-bit one is
   // three quarter-rate instructions
-  __device__ __forceinline__ static uint32_t home(uint64_t k) {
+  __device__ __forceinline__ static uint32_t hash(uint64_t k) {
     const uint32_t lo = (uint32_t)k, hi = (uint32_t)(k >> 32);
-    return slot_of<T>((lo ^ __builtin_amdgcn_alignbit(hi, hi, 13)) * 0x9E3779B1u);
+    return (lo ^ __builtin_amdgcn_alignbit(hi, hi, 13)) * 0x9E3779B1u;
   }
   __device__ __forceinline__ bool try_slot(uint32_t slot, uint64_t k) {
     const ull prev = atomicCAS(&hk[slot], empty, (ull)k);
@@ -2501,16 +2509,19 @@ struct HashTable<uint64_t> {
     }
     return false;
   }
+  template <int PROBES>
   __device__ __forceinline__ bool insert(uint64_t k, const volatile int* stop) {
-    uint32_t slot = home(k);
+    const uint32_t h = hash(k), step = probe_step(h);
+    uint32_t slot = slot_of<T>(h);
     for (int probe = 0; probe < STOP_AFTER; probe++) {
       if (try_slot(slot, k)) return true;
-      slot = next_slot<T>(slot);
+      slot = next_slot<T>(slot, step);
     }
-    for (int probe = STOP_AFTER; probe < HASH_PROBES; probe++) {
+#pragma unroll 1
+    for (int probe = STOP_AFTER; probe < PROBES; probe++) {
       if ((probe & 7) == 0 && *stop) return false;
       if (try_slot(slot, k)) return true;
-      slot = next_slot<T>(slot);
+      slot = next_slot<T>(slot, step);
     }
     return false;
   }
@@ -2543,11 +2554,9 @@ struct HashTable<u128> {
     for (int i = tid; i < T / 2; i += nt) reinterpret_cast<ulonglong2*>(hf)[i] = make_ulonglong2(EMPTY, EMPTY);
     for (int i = tid; i < T / 4; i += nt) reinterpret_cast<uint4*>(hc)[i] = make_uint4(0u, 0u, 0u, 0u);
   }
-  // home slot: one more 32-bit product; probes step to the next slot
-  __device__ __forceinline__ static uint32_t home(ull f) {
-    return slot_of<T>(((uint32_t)f ^ (uint32_t)(f >> 32)) * 0x9E3779B1u);
-  }
-  __device__ __forceinline__ static uint32_t next(uint32_t slot) { return next_slot<T>(slot); }
+  // one more 32-bit product
+  __device__ __forceinline__ static uint32_t hash(ull f) { return ((uint32_t)f ^ (uint32_t)(f >> 32)) * 0x9E3779B1u; }
+  __device__ __forceinline__ static uint32_t home(ull f) { return slot_of<T>(hash(f)); }
   // a slot changes only once, from EMPTY to its fingerprint: a plain read
   // finds a repeated key or steps over another one without an atomic, and
   // only an empty slot is claimed by CAS (k = 64 bacterial: 2.73 -> 2.56 ms)
@@ -2571,16 +2580,19 @@ struct HashTable<u128> {
   }
   // the rest, for a key whose home slot holds another fingerprint: the slot
   // that counts k, or -1 (table full, or reported full by another thread)
+  template <int PROBES>
   __device__ __forceinline__ int insert_after_home(u128 k, ull f, const volatile int* stop) {
-    uint32_t slot = next(home(f));
+    const uint32_t h = hash(f), step = probe_step(h);
+    uint32_t slot = next_slot<T>(slot_of<T>(h), step);
     for (int probe = 1; probe < STOP_AFTER; probe++) {
       if (try_slot(slot, f, k)) return (int)slot;
-      slot = next(slot);
+      slot = next_slot<T>(slot, step);
     }
-    for (int probe = STOP_AFTER; probe < HASH_PROBES; probe++) {
+#pragma unroll 1
+    for (int probe = STOP_AFTER; probe < PROBES; probe++) {
       if ((probe & 7) == 0 && *stop) return -1;
       if (try_slot(slot, f, k)) return (int)slot;
-      slot = next(slot);
+      slot = next_slot<T>(slot, step);
     }
     return -1;
   }
@@ -2631,12 +2643,16 @@ constexpr int MAX_PASS_BITS = 4;
 constexpr int RUN_CAP = 512;
 constexpr int HASH_QUEUE = 1024;
 
-template <class Key>
+constexpr int map_words(int batch) { return batch / 32 * 2 + RUN_CAP; }
+
+template <class Key, bool MULTI>
 struct HashShared {
   HashLds<Key> lds;
   // sub-bin starts of the ordering (and the end of the last); a batch's run map
-  // before
+  // before, which several passes over one batch keep apart
   alignas(16) uint32_t hs[(1 << HashCfg<Key>::SUB) + 4];
+  alignas(8) uint32_t keep[MULTI ? map_words(HashCfg<Key>::NT * HashCfg<Key>::HB) : 2];
+  __device__ __forceinline__ uint32_t* map() { return MULTI ? keep : hs; }
   uint32_t nw[HashCfg<Key>::NT / 64 + 1];
   int over;
   // u128: keys of the batch queued for their probe chains (place in the batch,
@@ -2714,12 +2730,11 @@ __device__ __forceinline__ bool wave_map(uint2* mw, int nwords, uint32_t* off, c
 // WAVE_MAP_RUNS runs): the map by the first wave, which sets over to 3 when the
 // runs do not fit (kb then holds other keys of the parent).
 template <class Key, bool RUNS, bool LIGHT, int HB>
-__device__ __forceinline__ int load_batch(HashShared<Key>& L, const Key* Sb, const Runs& in, const RunBucket& rb,
+__device__ __forceinline__ int load_batch(HashShared<Key, !LIGHT>& L, const Key* Sb, const Runs& in, const RunBucket& rb,
                                           ull b, Key (&kb)[HB]) {
   constexpr int BS_NT = HashCfg<Key>::NT;
   constexpr int BATCH = BS_NT * HB;
-  static_assert(BATCH % 32 == 0 && BATCH / 32 * sizeof(uint2) + RUN_CAP * 4 <= sizeof(L.hs),
-                "the run map fits the sub-bins");
+  static_assert(BATCH % 32 == 0 && map_words(BATCH) * 4 <= sizeof(L.hs), "the run map fits the sub-bins");
   if constexpr (!RUNS) {
 #pragma unroll
     for (int j = 0; j < HB; j++) {
@@ -2729,8 +2744,8 @@ __device__ __forceinline__ int load_batch(HashShared<Key>& L, const Key* Sb, con
     return rb.n - b < (ull)BATCH ? (int)(rb.n - b) : BATCH;
   } else {
     int m = rb.n - b < (ull)BATCH ? (int)(rb.n - b) : BATCH;
-    uint2* mw = reinterpret_cast<uint2*>(L.hs);
-    uint32_t* off = L.hs + BATCH / 32 * 2;
+    uint2* mw = reinterpret_cast<uint2*>(L.map());
+    uint32_t* off = L.map() + BATCH / 32 * 2;
     if constexpr (LIGHT) {
       if (threadIdx.x < 64 && !wave_map(mw, (m + 31) >> 5, off, in, rb, (uint32_t)b, m)) L.over = 3;
       __syncthreads();
@@ -2739,7 +2754,7 @@ __device__ __forceinline__ int load_batch(HashShared<Key>& L, const Key* Sb, con
       const ull f = rb.e0 + (rb.nt > BS_NT ? block_upper<BS_NT>(in.V + rb.e0, rb.nt, vb) - 1 : 0);
       auto src = [&](ull e) { return tile_place(in, e - rb.e0) + (in.M[e] >> 16); };
       for (;;) {
-        __syncthreads();  // hs may still be read
+        __syncthreads();  // the last map may still be read
         const int np = map_pieces<BS_NT>(mw, L.nw, RUN_CAP, in.V, f, end, vb, m, src,
                                          [&](uint32_t r, ull d, ull) { off[r] = (uint32_t)d; });
         if (np <= RUN_CAP) break;
@@ -2761,20 +2776,26 @@ __device__ __forceinline__ int load_batch(HashShared<Key>& L, const Key* Sb, con
 // 1; top = the first of them).  Writes the task's unique (key, count) pairs
 // in ascending order to R / C at rb.v0 and their number to *out_n, returns 0;
 // 1 when the table is too small for the distinct keys, 2 on a u128
-// fingerprint collision, 3 when a batch has too many runs.  With MULTI a task with too many distinct keys is
+// fingerprint collision, 3 when a batch has too many runs, 4 when the task is
+// left to MULTI untried.  With MULTI a task with too many distinct keys is
 // processed in 2^s passes, pass p taking the keys whose next s bits equal p
 // (s = 1, 2, ... up to MAX_PASS_BITS).  A task of more instances than
 // TASK_MAX_INSTANCES takes all keys at once first, which costs a batch or two
 // where they are distinct, and then as many passes as leave that number to each
-// (1.4e7 equal keys of one bucket: 190 ms in 16 passes, 32 in one).
+// (1.4e7 equal keys of one bucket: 190 ms in 16 passes, 32 in one).  full: a
+// table has been too small for it already, so that it starts with two passes or,
+// if its keys fit one batch, with as many as leave a table 0.85 full if all are
+// distinct; such a task's keys stay in registers over its passes.
 template <class Key, bool RUNS, bool MULTI>
-__device__ __forceinline__ int count_task(HashShared<Key>& L, const Key* S, Key* R, int32_t* C, const Runs& in,
-                                          const RunBucket& rb, bool top, int K, int fixed, ull* out_n) {
+__device__ __forceinline__ int count_task(HashShared<Key, MULTI>& L, const Key* S, Key* R, int32_t* C, const Runs& in,
+                                          const RunBucket& rb, bool top, int K, int fixed, bool full, ull* out_n) {
   constexpr int BS_NT = HashCfg<Key>::NT;
   constexpr int T = HashCfg<Key>::T;
   constexpr int PER = T / BS_NT;  // table slots per thread
   constexpr int HB = HashCfg<Key>::HB;
+  constexpr int PROBES = MULTI ? HASH_PROBES_MULTI : HASH_PROBES;
   uint32_t* hs = L.hs;
+  const uint32_t* map = L.map();
   const ull start = rb.v0, n = rb.n;
   const int rem = 2 * K - fixed;
   // EMPTY for u64 tables: a key whose top bit differs from the task's (all
@@ -2785,7 +2806,15 @@ __device__ __forceinline__ int count_task(HashShared<Key>& L, const Key* S, Key*
   ull out = 0;
   int s = 0, fail = 0;
   // a first try with all keys is pointless when there are too many of them
-  if (!MULTI && (n > (ull)TASK_MAX_INSTANCES || rb.nt > WAVE_MAP_RUNS)) return 1;
+  if (!MULTI && (n > (ull)TASK_MAX_INSTANCES || rb.nt > WAVE_MAP_RUNS)) return 4;
+  if (MULTI && full && max_s) {
+    s = 1;
+    while (n <= (ull)(BS_NT * HB) && s < max_s && (n >> s) > (ull)(T * 17 / 20)) s++;
+  }
+  // keys are loaded HB at a time into registers so that the global-load
+  // latency is paid once per batch, not once per insert
+  Key kb[HB];
+  int m = 0;
   for (; s <= max_s; s++) {
     while (MULTI && s > 0 && s < max_s && (n >> s) > (ull)TASK_MAX_INSTANCES) s++;
     out = 0;
@@ -2797,17 +2826,15 @@ __device__ __forceinline__ int count_task(HashShared<Key>& L, const Key* S, Key*
       // (the first batch's map is built before the barrier that ends the
       // clearing)
       if (!RUNS || MULTI) __syncthreads();
-      // keys are loaded HB at a time into registers so that the global-load
-      // latency is paid once per batch, not once per insert
-      Key kb[HB];
       int ksl[HB];  // u128: the slot each key of the batch landed in, or -1 - its place in the queue
       bool clash = false;
       // over as read between two barriers of the last batch (the first wave
       // writes it while it makes the next batch's map): all threads leave
       // together
-      int ov = 0, m = 0;
+      int ov = 0;
       for (ull b = 0; b < n && !ov; b += m) {
-        m = load_batch<Key, RUNS, !MULTI, HB>(L, Sb, in, rb, b, kb);
+        // (one batch: the keys are still there)
+        if (!MULTI || (ull)m != n) m = load_batch<Key, RUNS, !MULTI, HB>(L, Sb, in, rb, b, kb);
         if constexpr (sizeof(Key) == 16) {
           // A wave runs each probe step as long as its slowest lane needs
           // it, so a batch goes in two phases: every key tries its home slot
@@ -2833,7 +2860,7 @@ __device__ __forceinline__ int count_task(HashShared<Key>& L, const Key* S, Key*
                     L.hq[q] = (uint16_t)i;
                     ksl[j] = -1 - q;
                   } else {
-                    ksl[j] = ht.insert_after_home(kb[j], f, &L.over);
+                    ksl[j] = ht.template insert_after_home<PROBES>(kb[j], f, &L.over);
                     if (ksl[j] < 0) L.over = 1;
                   }
                 }
@@ -2846,9 +2873,9 @@ __device__ __forceinline__ int count_task(HashShared<Key>& L, const Key* S, Key*
             const int i = L.hq[q];
             ull o = b + (ull)i;
             if constexpr (RUNS)
-              o = (ull)(hs[BS_NT * HB / 32 * 2 + map_piece(reinterpret_cast<const uint2*>(hs), i)] + (uint32_t)i);
+              o = (ull)(map[BS_NT * HB / 32 * 2 + map_piece(reinterpret_cast<const uint2*>(map), i)] + (uint32_t)i);
             const u128 k = Sb[o];
-            const int sl = ht.insert_after_home(k, HashTable<u128>::fp(k), &L.over);
+            const int sl = ht.template insert_after_home<PROBES>(k, HashTable<u128>::fp(k), &L.over);
             if (sl < 0) L.over = 1;
             L.hq[q] = (uint16_t)sl;
           }
@@ -2871,7 +2898,7 @@ __device__ __forceinline__ int count_task(HashShared<Key>& L, const Key* S, Key*
 #pragma unroll
           for (int j = 0; j < HB; j++) {
             const int i = (int)threadIdx.x + j * BS_NT;
-            if (i < m && mine(kb[j]) && !ht.insert(kb[j], &L.over)) L.over = 1;
+            if (i < m && mine(kb[j]) && !ht.template insert<PROBES>(kb[j], &L.over)) L.over = 1;
           }
           if (b + m < n) {
             __syncthreads();
@@ -3000,50 +3027,72 @@ __device__ __forceinline__ int count_task(HashShared<Key>& L, const Key* S, Key*
 // early, or a map built by all waves, were slower.
 //
 // One block per bucket of `in`: tu[b] = the bucket's distinct keys, bstart[b]
-// = where they are.  Buckets the table is too small for go to the retry list
-// (a single pass needs fewer registers).
+// = where they are.  Buckets the table is too small for are left to the retry
+// (a single pass needs fewer registers): tu = RETRY_FULL, or RETRY_UNTRIED.
+constexpr long long RETRY_FULL = -2, RETRY_UNTRIED = -3;
+
 template <class Key, bool RUNS>
 __global__ __launch_bounds__(HashCfg<Key>::NT, HashCfg<Key>::WAVES) void k_bucket_hash(const Key* S, Key* R, int32_t* C,
                                                                             Runs in, int K, int fixed, long long* tu,
-                                                                            ull* bstart, ull* retry_count,
-                                                                            ull* retry_list) {
-  __shared__ HashShared<Key> L;
+                                                                            ull* bstart) {
+  __shared__ HashShared<Key, false> L;
   const ull task = blockIdx.x;
   const RunBucket rb = uniform(run_bucket(in, task));
   ull out = 0;
   int fail = 0;
   if (rb.n) {
-    fail = 1;
+    fail = 4;
     // (runs are reached by 32-bit offsets from the parent's first tile)
     if (!RUNS || in.boff[(task >> in.db) + 1] - rb.base < (1ull << 32))
-      fail = count_task<Key, RUNS, false>(L, S, R, C, in, rb, (bool)((task >> (fixed - 1)) & 1), K, fixed, &out);
+      fail = count_task<Key, RUNS, false>(L, S, R, C, in, rb, (bool)((task >> (fixed - 1)) & 1), K, fixed, false,
+                                          &out);
   }
   if (threadIdx.x == 0) {
     bstart[task] = rb.v0;
-    tu[task] = (long long)out;
-    if (fail) retry_list[atomicAdd(retry_count, 1ull)] = task;
+    tu[task] = fail == 0 ? (long long)out : fail == 1 ? RETRY_FULL : RETRY_UNTRIED;
   }
 }
 
-// The buckets of the retry list in several passes; what still fails goes to
-// ovf_list with tu = -1 for the host-driven split.
+// The buckets left to it in several passes, every gridDim.x-th of the B buckets
+// to a block (a list of them by atomics on one counter took 50 ns a bucket); what
+// still fails goes to ovf_list with tu = -1 for the host-driven split.  Bound by
+// latency: two blocks per CU, 112 to 128 VGPRs with a batch's keys in registers.
+// Bucket count of distinct-rich input, first try and this (before the tiled
+// partition; loading the keys for every pass, the first of them the one that had
+// failed already; now): 1.3e8 keys of 32 bases, 0.72 distinct, 3.3 / 8.7 / 2.8 ms;
+// 6.9e7, all distinct, 2.7 / 5.6 / 1.8; 1.1e8 of 64 bases, 0.95 distinct, 6.5 /
+// 12.4 / 4.6; 8.7e7, all distinct, 4.5 / 11.7 / 3.8.
 template <class Key, bool RUNS>
-__global__ __launch_bounds__(HashCfg<Key>::NT) void k_bucket_retry(const Key* S, Key* R, int32_t* C, Runs in, int K, int fixed,
-                                                        long long* tu, const ull* retry_count, const ull* retry_list,
-                                                        ull* ovf_count, ull* ovf_list) {
-  __shared__ HashShared<Key> L;
-  const ull nt = *retry_count;
-  for (ull q = blockIdx.x; q < nt; q += gridDim.x) {
-    const ull task = uniform(retry_list[q]);
-    const RunBucket rb = uniform(run_bucket(in, task));
-    ull out = 0;
-    int fail = 1;
-    if (!RUNS || in.boff[(task >> in.db) + 1] - rb.base < (1ull << 32))
-      fail = count_task<Key, RUNS, true>(L, S, R, C, in, rb, (bool)((task >> (fixed - 1)) & 1), K, fixed, &out);
-    if (threadIdx.x == 0) {
-      tu[task] = fail ? -1 : (long long)out;
-      if (fail) ovf_list[atomicAdd(ovf_count, 1ull)] = task;
+__global__ __launch_bounds__(HashCfg<Key>::NT, 4) void k_bucket_retry(const Key* S, Key* R, int32_t* C, Runs in, ull B,
+                                                                   int K, int fixed, long long* tu, ull* ovf_count,
+                                                                   ull* ovf_list) {
+  constexpr int NT = HashCfg<Key>::NT;
+  __shared__ HashShared<Key, true> L;
+  __shared__ uint32_t left[NT];  // place among the block's buckets << 1 | full
+  __shared__ uint32_t nleft;
+  for (ull c0 = 0; c0 * gridDim.x + blockIdx.x < B; c0 += NT) {
+    if (threadIdx.x == 0) nleft = 0;
+    __syncthreads();
+    const ull t = (c0 + threadIdx.x) * gridDim.x + blockIdx.x;
+    const long long u = t < B ? tu[t] : 0;
+    if (u < -1) left[atomicAdd(&nleft, 1u)] = threadIdx.x << 1 | (u == RETRY_FULL ? 1u : 0u);
+    __syncthreads();
+    const uint32_t nq = nleft;
+    for (uint32_t q = 0; q < nq; q++) {
+      const uint32_t e = __builtin_amdgcn_readfirstlane(left[q]);
+      const ull task = (c0 + (e >> 1)) * gridDim.x + blockIdx.x;
+      const RunBucket rb = uniform(run_bucket(in, task));
+      ull out = 0;
+      int fail = 1;
+      if (!RUNS || in.boff[(task >> in.db) + 1] - rb.base < (1ull << 32))
+        fail = count_task<Key, RUNS, true>(L, S, R, C, in, rb, (bool)((task >> (fixed - 1)) & 1), K, fixed, e & 1u,
+                                           &out);
+      if (threadIdx.x == 0) {
+        tu[task] = fail ? -1 : (long long)out;
+        if (fail) ovf_list[atomicAdd(ovf_count, 1ull)] = task;
+      }
     }
+    __syncthreads();
   }
 }
 
@@ -3051,7 +3100,7 @@ __global__ __launch_bounds__(HashCfg<Key>::NT) void k_bucket_retry(const Key* S,
 template <class Key>
 __global__ __launch_bounds__(HashCfg<Key>::NT) void k_task_hash(const Key* S, Key* R, int32_t* C, const ull* tstart,
                                                      const ull* tcount, int K, int fixed, long long* tu) {
-  __shared__ HashShared<Key> L;
+  __shared__ HashShared<Key, true> L;
   const ull task = blockIdx.x;
   RunBucket rb{};
   rb.v0 = tstart[task];
@@ -3060,7 +3109,7 @@ __global__ __launch_bounds__(HashCfg<Key>::NT) void k_task_hash(const Key* S, Ke
   int fail = 0;
   if (rb.n) {
     const bool top = (bool)((uint32_t)(S[rb.v0] >> (2 * K - 1)) & 1u);
-    fail = count_task<Key, false, true>(L, S, R, C, Runs{}, rb, top, K, fixed, &out);
+    fail = count_task<Key, false, true>(L, S, R, C, Runs{}, rb, top, K, fixed, false, &out);
   }
   if (threadIdx.x == 0) tu[task] = fail ? -1 : (long long)out;
 }
@@ -3880,7 +3929,7 @@ enum BufId {
   B_FASTA, B_BLK, B_BLKOFF, B_NL, B_RSTART, B_RLEN, B_KC, B_KOFS, B_SMALL, B_BCNT, B_BOFF, B_BCUR,
   B_S, B_C, B_TU, B_UOFF, B_TK, B_TC, B_HIST, B_KBS, B_KBOFF, B_KK, B_KC2, B_MNPLAN,
   B_MNNT, B_MNNG, B_MNNOFF, B_MNFLAG, B_NODES, B_TMP, B_OVF, B_PT0, B_PT1, B_PT2, B_PT3, B_PT4,
-  B_PT5, B_PT6, B_BLKGT, B_S2, B_BCNT2, B_BOFF2, B_BCUR2, B_TP, B_TP2, B_HIST1, B_OFF1, B_HIST2, B_OFF2, B_PACK, B_RETRY, B_WCNT, B_WOFF, B_CUTBH, B_LFREQ, B_LPART, B_LBIG, B_LRANK, B_LW, B_OWNW, B_OWNCNT, B_OWNOFF, B_WORDER, B_WIRE, B_NORM, B_NORMNL, B_NORMLEN, B_NORMOFF, B_NORMLS, B_NORMLL, B_SCAN0, B_SCAN1 = B_SCAN0 + 8, B_COUNT = B_SCAN0 + 16
+  B_PT5, B_PT6, B_BLKGT, B_S2, B_BCNT2, B_BOFF2, B_BCUR2, B_TP, B_TP2, B_HIST1, B_OFF1, B_HIST2, B_OFF2, B_PACK, B_WCNT, B_WOFF, B_CUTBH, B_LFREQ, B_LPART, B_LBIG, B_LRANK, B_LW, B_OWNW, B_OWNCNT, B_OWNOFF, B_WORDER, B_WIRE, B_NORM, B_NORMNL, B_NORMLEN, B_NORMOFF, B_NORMLS, B_NORMLL, B_SCAN0, B_SCAN1 = B_SCAN0 + 8, B_COUNT = B_SCAN0 + 16
 };
 
 }  // namespace
@@ -4420,8 +4469,8 @@ int windows_main(pk_ctx* c, const uint8_t* fa, uint64_t n, int K, Records* rec, 
   hipStream_t st = c->stream;
   ull* small;
   PK_TRY(need(c, B_SMALL, 16, &small));
-  // small[2] = first format error, [3] = a line may be too long, [4], [5] =
-  // overflow and retry counts, [6] .. [9] = k_lines' facts, [10] = first '>',
+  // small[2] = first format error, [3] = a line may be too long, [4] = overflow
+  // count, [6] .. [9] = k_lines' facts, [10] = first '>',
   // [11] = records of the L-mers
   const uint64_t nb = (n + NL_PER_BLOCK - 1) / NL_PER_BLOCK;
   if (!nb) {
@@ -4490,7 +4539,7 @@ int records_main(pk_ctx* c, const uint8_t* fa, uint64_t n, int K, Records* rec) 
   ull* small;
   PK_TRY(need(c, B_SMALL, 16, &small));
   // small[0] = first '>', [1] = first unprocessed, [2] = first format error,
-  // [3] = first over-long read, [4], [5] = overflow and retry counts
+  // [3] = first over-long read, [4] = overflow count
   PK_TRY(fill_u64(c, small, ~0ull, 4));
   PK_TRY(fill_u64(c, small + 4, 0, 2));
   if (n >> NL_FLAG_SHIFT) return c->fail(PK_EINVAL, "input larger than 2^62 bytes");
@@ -4640,7 +4689,7 @@ int level_bits(int left) {
 // Further partition levels, the per-bucket count and the dense table.  S
 // holds the N keys (KB key bits) as p says; levels follow until btot bits are
 // fixed.  S2 is the other instance array, C the per-instance counts;
-// small[4] and small[5] (the overflow and retry counts) start at zero.
+// small[4] (the overflow count) starts at zero.
 template <class Key>
 int count_partitioned(pk_ctx* c, Key* S, Key* S2, int32_t* C, Part p, int btot, int KB, uint64_t N) {
   Key* TK;
@@ -4682,25 +4731,24 @@ int count_partitioned(pk_ctx* c, Key* S, Key* S2, int32_t* C, Part p, int btot, 
   PK_HIP(c, hipEventRecord(c->ev[5], st));
   // 4. per-bucket count
   long long* tu;
-  ull *ovl, *uoff, *bstart, *retry;
+  ull *ovl, *uoff, *bstart;
   PK_TRY(need(c, B_BCNT, B, &bstart));
   PK_TRY(need(c, B_TU, B, &tu));
-  PK_TRY(need(c, B_RETRY, B, &retry));
   PK_TRY(need(c, B_OVF, B + 1, &ovl));
   PK_TRY(need(c, B_UOFF, B + 1, &uoff));
   const unsigned rgrid = (unsigned)std::min<uint64_t>(B, 4ull * (uint64_t)c->ncu);
   if (in.M) {
     hipLaunchKernelGGL(HIP_KERNEL_NAME(k_bucket_hash<Key, true>), dim3((unsigned)B), dim3(HashCfg<Key>::NT), 0, st, S, Res, C,
-                       in, KB / 2, btot, tu, bstart, small + 5, retry);
+                       in, KB / 2, btot, tu, bstart);
     PK_HIP(c, hipGetLastError());
     hipLaunchKernelGGL(HIP_KERNEL_NAME(k_bucket_retry<Key, true>), dim3(rgrid), dim3(HashCfg<Key>::NT), 0, st, S, Res, C, in,
-                       KB / 2, btot, tu, small + 5, retry, small + 4, ovl);
+                       (ull)B, KB / 2, btot, tu, small + 4, ovl);
   } else {
     hipLaunchKernelGGL(HIP_KERNEL_NAME(k_bucket_hash<Key, false>), dim3((unsigned)B), dim3(HashCfg<Key>::NT), 0, st, S, Res, C,
-                       in, KB / 2, btot, tu, bstart, small + 5, retry);
+                       in, KB / 2, btot, tu, bstart);
     PK_HIP(c, hipGetLastError());
     hipLaunchKernelGGL(HIP_KERNEL_NAME(k_bucket_retry<Key, false>), dim3(rgrid), dim3(HashCfg<Key>::NT), 0, st, S, Res, C, in,
-                       KB / 2, btot, tu, small + 5, retry, small + 4, ovl);
+                       (ull)B, KB / 2, btot, tu, small + 4, ovl);
   }
   PK_HIP(c, hipGetLastError());
   PK_HIP(c, hipEventRecord(c->ev[7], st));
@@ -4784,7 +4832,7 @@ int count_partitioned(pk_ctx* c, Key* S, Key* S2, int32_t* C, Part p, int btot, 
   }
   c->U = U;
   // what is left to do reads the buckets' results and their places only
-  for (int id : {B_BOFF, B_TP, B_HIST1, B_OFF1, B_BOFF2, B_TP2, B_HIST2, B_OFF2, B_RETRY, B_OVF, B_WOFF, B_OWNOFF})
+  for (int id : {B_BOFF, B_TP, B_HIST1, B_OFF1, B_BOFF2, B_TP2, B_HIST2, B_OFF2, B_OVF, B_WOFF, B_OWNOFF})
     c->idle[id] = true;
   for (int id : {B_S, B_S2, B_TMP})
     if (c->buf[id].p != static_cast<const void*>(Res)) c->idle[id] = true;

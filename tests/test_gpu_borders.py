@@ -214,3 +214,52 @@ def test_bucket_of_equal_keys(ctx, oracle_mod, k):
     assert np.array_equal(keys.reshape(-1), np.asarray(want_k).reshape(-1))
     assert np.array_equal(counts, want_c)
     assert ctx.timing()["sort_ms"] < 60.0
+
+
+@pytest.mark.parametrize("k", [32, 40])
+def test_retry_of_few_buckets_among_a_million(ctx, oracle_mod, k):
+    """2^20 buckets, nearly all of one or two keys, and a few with more distinct
+    keys than a table holds, up to the very last one: each is found and counted
+    in several passes, with more and with fewer keys than a batch."""
+    rng = np.random.default_rng(k)
+    acgt = np.frombuffer(b"ACGT", dtype=np.uint8)
+    some = rng.choice(acgt, (1_200_000, k))
+    groups = [some]
+    for prefix, n in ((b"A" * 10, 3_000), (b"ACGTACGTAC", 7_000), (b"T" * 10, 4_000), (b"G" * 9 + b"T", 2_700),
+                      (b"G" * 10, 30_000)):
+        g = rng.choice(acgt, (n, k))
+        g[:, :10] = np.frombuffer(prefix, dtype=np.uint8)
+        groups.append(g)
+    reads = np.concatenate(groups)
+    rows = np.full((reads.shape[0], k + 4), 10, dtype=np.uint8)
+    rows[:, :3] = np.frombuffer(b">r\n", dtype=np.uint8)
+    rows[:, 3:-1] = reads[rng.permutation(reads.shape[0])]
+    fa = rows.tobytes()
+    try:
+        ctx.set_tuning(bucket_factor=1.2 / (1920 if k <= 32 else 1152))  # one instance a bucket
+        _p(f"case: retry among a million buckets k={k}")
+        ctx.count(fa, k)
+        assert ctx.timing()["bucket_bits"] == 20
+        keys, counts = ctx.table_host()
+    finally:
+        ctx.set_tuning()
+    want_k, want_c = oracle_mod.count(fa, k)
+    assert np.array_equal(keys.reshape(-1), np.asarray(want_k).reshape(-1))
+    assert np.array_equal(counts, want_c)
+
+
+def test_time_of_distinct_keys(ctx):
+    """6.9e7 k-mers, all distinct: every bucket's first table is too small.  The
+    bucket count takes 1.8 ms (5.6 with the pass that had failed repeated and the
+    keys loaded again for each pass)."""
+    rng = np.random.default_rng(3)
+    rows = np.full((1_000_000, 104), 10, dtype=np.uint8)
+    rows[:, :3] = np.frombuffer(b">r\n", dtype=np.uint8)
+    rows[:, 3:103] = rng.choice(np.frombuffer(b"ACGT", dtype=np.uint8), (rows.shape[0], 100))
+    fa = rows.tobytes()
+    _p("case: time of distinct keys")
+    for _ in range(3):
+        n = ctx.count(fa, 32).n
+    keys, counts = ctx.table_host()
+    assert np.all(keys[1:, 0] > keys[:-1, 0]) and n > 68_900_000 and int(counts.sum()) == 69_000_000
+    assert ctx.timing()["sort_ms"] < 3.6
