@@ -188,10 +188,15 @@ void pk_server::run(int slot, Job* j) {
       }
   }
   pk_ctx_set_tuning(c, &tu);
+  // a step short of memory once more without the spare blocks
+  auto step = [&](auto&& f) {
+    int rc = f();
+    if (rc == PK_ENOMEM && free_spare()) rc = f();
+    return rc;
+  };
   pk_table t{};
-  int rc = pk_count(c, j->spec.fasta, j->spec.nbytes, j->spec.k, j->spec.fasta_on_device, &t);
-  if (rc == PK_ENOMEM && free_spare())
-    rc = pk_count(c, j->spec.fasta, j->spec.nbytes, j->spec.k, j->spec.fasta_on_device, &t);
+  const int rc = step(
+      [&] { return pk_count(c, j->spec.fasta, j->spec.nbytes, j->spec.k, j->spec.fasta_on_device, &t); });
   if (rc) {
     set_err(rc);
     return;
@@ -209,11 +214,11 @@ void pk_server::run(int slot, Job* j) {
     j->hist.assign((size_t)tt, 0);
     uint64_t nk = 0;
     int mb = 0;
-    crc = pk_cutoff(c, j->spec.t, j->hist.data(), &mb, &nk);
+    crc = step([&] { return pk_cutoff(c, j->spec.t, j->hist.data(), &mb, &nk); });
     r.min_bucket = mb;
     if (crc == PK_OK) {
       pk_kept_table(c, &kt);
-      if (j->spec.want_nodes) crc = pk_macro_nodes(c, &mt);
+      if (j->spec.want_nodes) crc = step([&] { return pk_macro_nodes(c, &mt); });
     }
     if (crc) set_err(crc);
     if (crc && crc != PK_EEMPTY) return;
