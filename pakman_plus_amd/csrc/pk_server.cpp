@@ -19,6 +19,7 @@
 #include <cstdio>
 #include <cstring>
 #include <deque>
+#include <list>
 #include <mutex>
 #include <new>
 #include <numeric>
@@ -31,6 +32,15 @@
 
 namespace {
 
+// A result block.  Blocks change hands as nodes of lists, which allocates
+// nothing: a job's node is made when it takes its block, where a failed host
+// allocation is the job's.
+struct Block {
+  void* p = nullptr;
+  uint64_t bytes = 0;
+};
+using Blocks = std::list<Block>;
+
 struct Job {
   pk_job spec{};
   uint64_t ticket = 0;
@@ -38,8 +48,8 @@ struct Job {
   int readers = 0;  // pk_server_download calls copying the results now
   pk_job_result res{};
   std::vector<uint64_t> hist;
-  void* mem = nullptr;
-  uint64_t mem_bytes = 0;
+  Blocks mem;  // at most one
+  uint64_t mem_bytes() const { return mem.empty() ? 0 : mem.front().bytes; }
 };
 
 inline uint64_t align256(uint64_t x) { return (x + 255) & ~255ull; }
@@ -87,11 +97,7 @@ struct pk_server {
   // 2000 jobs/s the device maps and unmaps 170 GB/s of them otherwise, and an
   // unmap stopped every slot for 0.05 to 1.6 s (p99 2.9 s against 0.1 s).  At
   // most an eighth of the budget; given back when a job needs the room.
-  struct Block {
-    void* p;
-    uint64_t bytes;
-  };
-  std::deque<Block> spare;
+  Blocks spare;
   uint64_t spare_bytes = 0;
   std::chrono::steady_clock::time_point t0 = std::chrono::steady_clock::now();
 
@@ -105,16 +111,15 @@ struct pk_server {
   }
   // Takes the oldest spare blocks out until at most `keep` bytes are left; the
   // caller frees them without mu, which every slot needs.
-  std::vector<Block> drop_spare(uint64_t keep) {
-    std::vector<Block> out;
+  Blocks drop_spare(uint64_t keep) {
+    Blocks out;
     while (!spare.empty() && spare_bytes > keep) {
-      out.push_back(spare.front());
       spare_bytes -= spare.front().bytes;
-      spare.pop_front();
+      out.splice(out.end(), spare, spare.begin());
     }
     return out;
   }
-  void free_blocks(const std::vector<Block>& v) {
+  void free_blocks(const Blocks& v) {
     for (const Block& b : v) {
       if (pools) (void)hipFreeAsync(b.p, free_stream);
       else (void)hipFree(b.p);
@@ -122,7 +127,7 @@ struct pk_server {
   }
   // All spare blocks back to the device; false when there were none.
   bool free_spare() {
-    std::vector<Block> v;
+    Blocks v;
     {
       std::lock_guard<std::mutex> lk(mu);
       v = drop_spare(0);
@@ -131,27 +136,30 @@ struct pk_server {
     if (!v.empty()) (void)hipStreamSynchronize(free_stream);
     return !v.empty();
   }
-  // A block of *bytes or a little more (*bytes is then its size): the smallest
-  // spare one that fits, else a new one.  Every use of a spare block ended
-  // before its job was done.
-  hipError_t take_block(uint64_t* bytes, hipStream_t st, void** out) {
+  // A block of `bytes` or a little more, appended to out: the smallest spare one
+  // that fits, else a new one.  Every use of a spare block ended before its job
+  // was done.
+  hipError_t take_block(uint64_t bytes, hipStream_t st, Blocks& out) {
     {
       std::lock_guard<std::mutex> lk(mu);
       auto best = spare.end();
       for (auto it = spare.begin(); it != spare.end(); ++it)
-        if (it->bytes >= *bytes && it->bytes <= *bytes + *bytes / 4 && (best == spare.end() || it->bytes < best->bytes))
+        if (it->bytes >= bytes && it->bytes <= bytes + bytes / 4 && (best == spare.end() || it->bytes < best->bytes))
           best = it;
       if (best != spare.end()) {
-        *out = best->p;
-        *bytes = best->bytes;
         spare_bytes -= best->bytes;
-        spare.erase(best);
+        out.splice(out.end(), spare, best);
         return hipSuccess;
       }
     }
+    Blocks one(1);
     for (;;) {
-      const hipError_t e = pools ? hipMallocAsync(out, *bytes, st) : hipMalloc(out, *bytes);
-      if (e == hipSuccess) return e;
+      const hipError_t e = pools ? hipMallocAsync(&one.front().p, bytes, st) : hipMalloc(&one.front().p, bytes);
+      if (e == hipSuccess) {
+        one.front().bytes = bytes;
+        out.splice(out.end(), one);
+        return e;
+      }
       (void)hipGetLastError();
       if (!free_spare()) return e;
     }
@@ -228,7 +236,6 @@ void pk_server::run(int slot, Job* j) {
   const uint64_t o1 = 0, o2 = align256(o1 + t.n * w), o3 = align256(o2 + t.n * 4),
                  o4 = align256(o3 + kt.n * w), o5 = align256(o4 + kt.n * 4),
                  end = align256(o5 + mt.n * sizeof(pk_mnode));
-  uint64_t held = block_bytes(end ? end : 256);
   hipStream_t st = (hipStream_t)pk_ctx_stream(c);
   // the job's kernels finish before its result block is allocated
   hipError_t e = hipStreamSynchronize(st);
@@ -237,14 +244,13 @@ void pk_server::run(int slot, Job* j) {
     std::snprintf(r.message, sizeof(r.message), "job failed: %s", hipGetErrorString(e));
     return;
   }
-  void* mem = nullptr;
-  e = take_block(&held, st, &mem);
+  e = take_block(block_bytes(end ? end : 256), st, j->mem);
   if (e != hipSuccess) {
     r.status = PK_ENOMEM;
     std::snprintf(r.message, sizeof(r.message), "result allocation failed: %s", hipGetErrorString(e));
     return;
   }
-  char* m = (char*)mem;
+  char* m = (char*)j->mem.front().p;
   auto cp = [&](uint64_t off, const void* src, uint64_t bytes) {
     if (bytes && e == hipSuccess) e = hipMemcpyAsync(m + off, src, bytes, hipMemcpyDeviceToDevice, st);
   };
@@ -258,8 +264,6 @@ void pk_server::run(int slot, Job* j) {
     r.status = PK_EHIP;
     std::snprintf(r.message, sizeof(r.message), "result copy failed: %s", hipGetErrorString(e));
   }
-  j->mem = mem;
-  j->mem_bytes = held;
   r.table = pk_table{t.n, t.words, t.k, (const uint64_t*)(m + o1), (const int32_t*)(m + o2)};
   r.kept = pk_table{kt.n, t.words, t.k, (const uint64_t*)(m + o3), (const int32_t*)(m + o4)};
   r.nodes = pk_mn_table{mt.n, t.k, (const pk_mnode*)(m + o5)};
@@ -284,7 +288,7 @@ void pk_server::worker(int slot) {
   const uint64_t slot_keep = budget / (uint64_t)(n_slots > 0 ? n_slots : 1);
   for (;;) {
     Job* j;
-    std::vector<Block> drop;
+    Blocks drop;
     {
       std::unique_lock<std::mutex> lk(mu);
       cv_q.wait(lk, [&] { return stop || admissible(); });
@@ -306,7 +310,7 @@ void pk_server::worker(int slot) {
       std::lock_guard<std::mutex> lk(mu);
       running--;
       running_est -= j->res.est_bytes;
-      resident += j->mem_bytes;
+      resident += j->mem_bytes();
       j->res.t_end = now();
       j->state = 2;
     }
@@ -389,10 +393,7 @@ void pk_server_destroy(pk_server* s) {
   for (auto& t : s->workers) t.join();
   (void)hipSetDevice(s->device);
   for (auto& kv : s->jobs) {
-    if (kv.second->mem) {
-      if (s->pools) (void)hipFreeAsync(kv.second->mem, s->free_stream);
-      else (void)hipFree(kv.second->mem);
-    }
+    s->free_blocks(kv.second->mem);
     delete kv.second;
   }
   s->free_blocks(s->drop_spare(0));
@@ -542,7 +543,7 @@ int pk_server_set_tuning(pk_server* s, const pk_tune_entry* entries, int n) {
 int pk_server_release(pk_server* s, uint64_t ticket) {
   if (!s) return PK_EINVAL;
   Job* j;
-  std::vector<pk_server::Block> drop;
+  Blocks drop;
   {
     std::unique_lock<std::mutex> lk(s->mu);
     auto it = s->jobs.find(ticket);
@@ -558,10 +559,10 @@ int pk_server_release(pk_server* s, uint64_t ticket) {
     if (it == s->jobs.end()) return s->fail(PK_EINVAL, "unknown ticket");
     j = it->second;
     s->jobs.erase(it);
-    s->resident -= j->mem_bytes;
-    if (j->mem) {
-      s->spare.push_back(pk_server::Block{j->mem, j->mem_bytes});
-      s->spare_bytes += j->mem_bytes;
+    s->resident -= j->mem_bytes();
+    if (!j->mem.empty()) {
+      s->spare_bytes += j->mem_bytes();
+      s->spare.splice(s->spare.end(), j->mem);
       const uint64_t used = s->running_est + s->resident;
       drop = s->drop_spare(std::min(s->budget / 8, used < s->budget ? s->budget - used : 0));
     }

@@ -181,14 +181,23 @@ int main(int argc, char** argv) {
     if (run_job(s, second, 21, 1, &b)) return fail("second job refused");
     if (pk_server_release(s, b)) return fail("release");
   } else if (which == "release") {
-    // no host memory: the block is kept or given back, and nothing is thrown
+    // the second block is kept and the first, beyond what is kept, given back,
+    // without a host allocation and without an exception
+    if (run_job(s, first, -1, 0, &b)) return fail("second job");
+    if (pk_server_release(s, a)) return fail("release");
+    const uint64_t used = dev_used;
     no_host_memory = true;
-    const int rc = pk_server_release(s, a);
+    int rc = -200;
+    try {
+      rc = pk_server_release(s, b);
+    } catch (...) {
+    }
     no_host_memory = false;
     if (rc) return fail("release without host memory");
     pk_job_result r{};
-    if (pk_server_poll(s, a, &r) != PK_EINVAL) return fail("still known");
-    if (run_job(s, first, -1, 0, &b)) return fail("second job");
+    if (pk_server_poll(s, b, &r) != PK_EINVAL) return fail("still known");
+    if (dev_used >= used) return fail("nothing given back");
+    if (run_job(s, first, -1, 0, &a)) return fail("third job");
   } else {
     return fail("unknown case");
   }

@@ -27,3 +27,10 @@ def test_later_steps_get_the_kept_blocks(server_bin, case):
     back, as a count does."""
     r = subprocess.run([server_bin, case], capture_output=True, text=True, timeout=60)
     assert (r.returncode, r.stdout.strip()) == (0, "ok"), r.stdout + r.stderr
+
+
+def test_release_without_host_memory(server_bin):
+    """A release that can allocate nothing on the host neither throws through the
+    C entry nor loses the result block."""
+    r = subprocess.run([server_bin, "release"], capture_output=True, text=True, timeout=60)
+    assert (r.returncode, r.stdout.strip()) == (0, "ok"), r.stdout + r.stderr
