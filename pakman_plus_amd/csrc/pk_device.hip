@@ -459,11 +459,8 @@ constexpr int ENC_BUILDER = 1;
 
 __device__ __forceinline__ bool base_is_acgt(uint32_t c) { return c == 'A' || c == 'C' || c == 'G' || c == 'T'; }
 
-template <int ENC>
-__device__ __forceinline__ uint32_t base_code(uint32_t c) {
-  if (ENC == ENC_MAIN) return (c >> 1) & 7u;
-  return base_is_acgt(c) ? (c >> 1) & 3u : 0u;
-}
+// char_to_el
+__device__ __forceinline__ uint32_t base_code(uint32_t c) { return (c >> 1) & 7u; }
 
 // ---------------------------------------------------------------------------
 // Packed input.  The counting path reads the input's bytes once and works on
@@ -1222,7 +1219,7 @@ static_assert(sizeof(pk_timing::ms_level_form) / sizeof(int32_t) == MS_TIMED_LEV
 // long for the buffer is walked from global memory, alone in its chunk).
 // Records are in file order, so a chunk's bytes are one contiguous range.
 // The buffer holds the base code of every byte, not the byte: bits 0-1 of the
-// code in plane A (32 bytes per word) and, on the main path, bit 2 in plane B
+// code in plane A (32 bytes per word) and bit 2 in plane B
 // (32 bytes per word), 3/8 of the raw size.  Its size (sb bytes, in dynamic
 // LDS) is chosen per input so that NT typical records fit.
 constexpr int L1_SB_MIN = 8192, L1_SB_MAX = 98304;  // staged bytes per chunk
@@ -1235,7 +1232,7 @@ struct ChunkLds {
 
 struct Stage {
   ull* A;       // code bits 0-1 of byte 32 w + i at bits 2i, 2i+1 of A[w]
-  uint32_t* B;  // code bit 2 of byte 32 w + i at bit i of B[w] (main path)
+  uint32_t* B;  // code bit 2 of byte 32 w + i at bit i of B[w]
   int sb;       // capacity in bytes (a multiple of 32)
 };
 
@@ -1246,7 +1243,7 @@ __host__ __device__ constexpr uint32_t l1_lds_bytes(int sb, int nd, int dig_byte
 }
 
 // Sets up the chunk starting at read c0 (< r1) and stages its codes.
-template <int ENC, int NT>
+template <int NT>
 __device__ __forceinline__ void stage_chunk(ChunkLds& C, Stage sg, const uint8_t* fa, uint64_t n,
                                             const ull* rstart, const uint32_t* rlen, uint64_t c0,
                                             uint64_t r1) {
@@ -1274,13 +1271,13 @@ __device__ __forceinline__ void stage_chunk(ChunkLds& C, Stage sg, const uint8_t
         const ull w = load_word8(fa, n, first + 32 * i + 8 * h);
 #pragma unroll
         for (int k = 0; k < 8; k++) {
-          const uint32_t el = base_code<ENC>((uint32_t)(w >> (8 * k)) & 0xFFu);
+          const uint32_t el = base_code((uint32_t)(w >> (8 * k)) & 0xFFu);
           a |= (ull)(el & 3u) << (16 * h + 2 * k);
           b |= (el >> 2) << (8 * h + k);
         }
       }
       sg.A[i] = a;
-      if (ENC == ENC_MAIN) sg.B[i] = b;
+      sg.B[i] = b;
     }
   }
   __syncthreads();
@@ -1291,7 +1288,7 @@ __device__ __forceinline__ void stage_chunk(ChunkLds& C, Stage sg, const uint8_t
 // km rolls unmasked (bits above the key shift out of the word, and the
 // key's own bits are the same either way): the mask is applied to the keys
 // handed out, once per k-mer instead of once per base.
-template <class Key, int ENC, class Emit>
+template <class Key, class Emit>
 __device__ __forceinline__ int walk_read(const ChunkLds& C, Stage sg, const uint8_t* fa, ull s, uint32_t len,
                                          uint32_t& i,
                                          Key& km, int K, Key mask, int Q,
@@ -1307,11 +1304,11 @@ __device__ __forceinline__ int walk_read(const ChunkLds& C, Stage sg, const uint
       const uint32_t sh = (uint32_t)(off & 31);
       const uint32_t cnt = len - i < 32u ? len - i : 32u;
       ull a = sg.A[w] >> (2 * sh);
-      uint32_t b = ENC == ENC_MAIN ? sg.B[w] >> sh : 0u;
+      uint32_t b = sg.B[w] >> sh;
       if (sh + cnt > 32u) {
         // the piece runs into the next word, which holds bases of this read
         a |= sg.A[w + 1] << (64 - 2 * sh);
-        if (ENC == ENC_MAIN) b |= sg.B[w + 1] << (32 - sh);
+        b |= sg.B[w + 1] << (32 - sh);
       }
       for (uint32_t t = 0; t < cnt && q < Q; t++) {
         const uint32_t el = ((uint32_t)a & 3u) | ((b & 1u) << 2);
@@ -1325,7 +1322,7 @@ __device__ __forceinline__ int walk_read(const ChunkLds& C, Stage sg, const uint
     return q;
   }
   while (q < Q && i < len) {
-    const uint32_t el = base_code<ENC>(fa[s + i]);
+    const uint32_t el = base_code(fa[s + i]);
     km = (km << 2) | (Key)el;
     i++;
     if (i >= (uint32_t)K) emit(q++, km & mask);
@@ -1336,7 +1333,7 @@ __device__ __forceinline__ int walk_read(const ChunkLds& C, Stage sg, const uint
 // Level-1 histogram of the walk: digit = bits [KB - d1, KB) of each key.  Block b's count of digit d goes to H[d * nblk + b] (digit-major),
 // so an exclusive scan of H gives every block the output base of each of its
 // digit runs.
-template <class Key, int ENC>
+template <class Key>
 __global__ __launch_bounds__(L1_NT) void k_l1_hist(const uint8_t* fa, uint64_t n, const ull* rstart,
                                                    const uint32_t* rlen, uint64_t R, int K, int KB,
                                                    Key mask, int d1, int rpb, int sb, uint32_t* H) {
@@ -1351,13 +1348,13 @@ __global__ __launch_bounds__(L1_NT) void k_l1_hist(const uint8_t* fa, uint64_t n
   const uint64_t r1 = r0 + rpb < R ? r0 + rpb : R;
   const int bpos = KB - d1;
   for (uint64_t c0 = r0; c0 < r1;) {
-    stage_chunk<ENC, L1_NT>(C, sg, fa, n, rstart, rlen, c0, r1);
+    stage_chunk<L1_NT>(C, sg, fa, n, rstart, rlen, c0, r1);
     const int m = C.m;
     if ((int)threadIdx.x < m) {
       const uint64_t r = c0 + threadIdx.x;
       uint32_t i = 0;
       Key km = 0;
-      walk_read<Key, ENC>(C, sg, fa, rstart[r], rlen[r], i, km, K, mask, 0x7fffffff,
+      walk_read<Key>(C, sg, fa, rstart[r], rlen[r], i, km, K, mask, 0x7fffffff,
                                [&](int, Key x) { atomicAdd(&h[key_digit<Key>(x, bpos, d1)], 1u); });
     }
     c0 += m;
@@ -1371,7 +1368,7 @@ __global__ __launch_bounds__(L1_NT) void k_l1_hist(const uint8_t* fa, uint64_t n
 // the block's LDS cursor (the return value of one 64-bit atomic) and is
 // stored at once.  The order of keys inside a bucket is arbitrary, which the
 // bucket count does not depend on.
-template <class Key, int ENC>
+template <class Key>
 __global__ __launch_bounds__(L1_NT) void k_l1_scatter(const uint8_t* fa, uint64_t n, const ull* rstart,
                                                       const uint32_t* rlen, uint64_t R, int K, int KB, Key mask,
                                                       int d1, int rpb, int sb, const ull* O,
@@ -1388,13 +1385,13 @@ __global__ __launch_bounds__(L1_NT) void k_l1_scatter(const uint8_t* fa, uint64_
   const int bpos = KB - d1;
   // stage_chunk's barriers order the set-up above before the first walk
   for (uint64_t c0 = r0; c0 < r1;) {
-    stage_chunk<ENC, L1_NT>(C, sg, fa, n, rstart, rlen, c0, r1);
+    stage_chunk<L1_NT>(C, sg, fa, n, rstart, rlen, c0, r1);
     const int m = C.m;
     if ((int)threadIdx.x < m) {
       const uint64_t r = c0 + threadIdx.x;
       uint32_t i = 0;
       Key km = 0;
-      walk_read<Key, ENC>(C, sg, fa, rstart[r], rlen[r], i, km, K, mask, 0x7fffffff,
+      walk_read<Key>(C, sg, fa, rstart[r], rlen[r], i, km, K, mask, 0x7fffffff,
                                [&](int, Key x) {
                                  const uint32_t d = key_digit<Key>(x, bpos, d1);
                                  S1[atomicAdd(&cur[d], 1ull)] = x;
@@ -2099,7 +2096,7 @@ __global__ void k_lmer_walk(const uint8_t* fa, const ull* rstart, const uint32_t
     const uint32_t len = rlen[r];
     uint32_t lm = 0;
     for (uint32_t i = 0; i < len; i++) {
-      lm = ((lm << 2) | base_code<ENC_MAIN>(fa[s + i])) & (LMER_BINS - 1);
+      lm = ((lm << 2) | base_code(fa[s + i])) & (LMER_BINS - 1);
       if (i >= (uint32_t)(LMER_L - 1)) atomicAdd(&freq[lm], 1ull);
     }
   }
@@ -2841,7 +2838,7 @@ __device__ __forceinline__ int count_task(HashShared<Key, MULTI>& L, const Key* 
           // (one probe, the common case), and the keys whose home slot holds
           // another fingerprint queue up and are then probed by all lanes
           // together, so a long chain holds up one queue round instead of
-          // each of the eight keys of its lane.
+          // each of its lane's keys.
           if (threadIdx.x == 0) L.qn = 0;
           __syncthreads();
 #pragma unroll
@@ -3926,10 +3923,10 @@ struct DevBuf {
 };
 
 enum BufId {
-  B_FASTA, B_BLK, B_BLKOFF, B_NL, B_RSTART, B_RLEN, B_KC, B_KOFS, B_SMALL, B_BCNT, B_BOFF, B_BCUR,
+  B_FASTA, B_BLK, B_BLKOFF, B_NL, B_RSTART, B_RLEN, B_KC, B_KOFS, B_SMALL, B_BCNT, B_BOFF,
   B_S, B_C, B_TU, B_UOFF, B_TK, B_TC, B_HIST, B_KBS, B_KBOFF, B_KK, B_KC2, B_MNPLAN,
   B_MNNT, B_MNNG, B_MNNOFF, B_MNFLAG, B_NODES, B_TMP, B_OVF, B_PT0, B_PT1, B_PT2, B_PT3, B_PT4,
-  B_PT5, B_PT6, B_BLKGT, B_S2, B_BCNT2, B_BOFF2, B_BCUR2, B_TP, B_TP2, B_HIST1, B_OFF1, B_HIST2, B_OFF2, B_PACK, B_WCNT, B_WOFF, B_CUTBH, B_LFREQ, B_LPART, B_LBIG, B_LRANK, B_LW, B_OWNW, B_OWNCNT, B_OWNOFF, B_WORDER, B_WIRE, B_NORM, B_NORMNL, B_NORMLEN, B_NORMOFF, B_NORMLS, B_NORMLL, B_SCAN0, B_SCAN1 = B_SCAN0 + 8, B_COUNT = B_SCAN0 + 16
+  B_PT5, B_PT6, B_BLKGT, B_S2, B_BOFF2, B_TP, B_TP2, B_HIST1, B_OFF1, B_HIST2, B_OFF2, B_PACK, B_WCNT, B_WOFF, B_CUTBH, B_LFREQ, B_LPART, B_LBIG, B_LRANK, B_LW, B_OWNW, B_OWNCNT, B_OWNOFF, B_WORDER, B_WIRE, B_NORM, B_NORMNL, B_NORMLEN, B_NORMOFF, B_NORMLS, B_NORMLL, B_SCAN0, B_SCAN1 = B_SCAN0 + 8, B_COUNT = B_SCAN0 + 16
 };
 
 }  // namespace
@@ -4166,8 +4163,9 @@ int d2h(pk_ctx* c, void* dst, const void* src, size_t bytes) {
 }
 
 // Bucket bits: at least 1 (the hash table's EMPTY value flips the top key
-// bit), and enough that a bucket holds about 3 tables of instances (a bucket
-// with more distinct keys than a table holds takes extra passes).
+// bit), and enough that a bucket holds at most `factor` times cap_keys
+// instances (a bucket with more distinct keys than a table holds takes extra
+// passes).
 int choose_bits(uint64_t N, int K, int cap_keys, float factor) {
   int b = 1;
   const uint64_t target = (uint64_t)((double)cap_keys * factor);
@@ -5005,7 +5003,7 @@ int count_walk(pk_ctx* c, const uint8_t* fa, uint64_t n, const Records& rec, int
   PK_TRY(need(c, B_C, N, &C));
   c->have_hist = true;
   PK_HIP(c, hipEventRecord(c->ev[2], st));
-  hipLaunchKernelGGL(HIP_KERNEL_NAME(k_l1_hist<Key, ENC_MAIN>), dim3((unsigned)nblk), dim3(L1_NT),
+  hipLaunchKernelGGL(HIP_KERNEL_NAME(k_l1_hist<Key>), dim3((unsigned)nblk), dim3(L1_NT),
                      l1_lds_bytes(sb, (int)B1, 4), st, fa, n, rec.rstart, rec.rlen, R, K, KB, mask, d1, rpb, sb, H);
   PK_HIP(c, hipGetLastError());
   PK_HIP(c, hipEventRecord(c->ev[3], st));
@@ -5014,7 +5012,7 @@ int count_walk(pk_ctx* c, const uint8_t* fa, uint64_t n, const Records& rec, int
                      boff);
   PK_HIP(c, hipGetLastError());
   PK_HIP(c, hipEventRecord(c->ev[4], st));
-  hipLaunchKernelGGL(HIP_KERNEL_NAME(k_l1_scatter<Key, ENC_MAIN>), dim3((unsigned)nblk), dim3(L1_NT),
+  hipLaunchKernelGGL(HIP_KERNEL_NAME(k_l1_scatter<Key>), dim3((unsigned)nblk), dim3(L1_NT),
                      l1_lds_bytes(sb, (int)B1, 8), st, fa, n, rec.rstart, rec.rlen, R, K, KB, mask, d1, rpb, sb, O,
                      nblk, S);
   PK_HIP(c, hipGetLastError());

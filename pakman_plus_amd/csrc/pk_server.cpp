@@ -62,8 +62,8 @@ inline uint64_t block_bytes(uint64_t x) {
   return (x + g - 1) & ~(g - 1);
 }
 
-// Working-set estimate of a job: FASTA copy (host input), line index and read
-// table, two instance arrays and the per-instance counts, the table.  The
+// Working-set estimate of a job: FASTA copy (host input), packed input and run
+// tables, two instance arrays and the per-instance counts, the table.  The
 // instance count is bounded by the byte count.
 uint64_t estimate_bytes(const pk_job& j) {
   const uint64_t W = j.k <= 32 ? 8 : 16;
