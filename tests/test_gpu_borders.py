@@ -263,3 +263,30 @@ def test_time_of_distinct_keys(ctx):
     keys, counts = ctx.table_host()
     assert np.all(keys[1:, 0] > keys[:-1, 0]) and n > 68_900_000 and int(counts.sum()) == 69_000_000
     assert ctx.timing()["sort_ms"] < 3.6
+
+
+@pytest.mark.parametrize("k", [32, 50])
+@pytest.mark.parametrize("l1_bits,further", [(10, 0), (7, 1), (5, 1), (3, 2), (2, 2)])
+def test_partition_levels(ctx, oracle_mod, k, l1_bits, further):
+    """One, two and three partition levels over the same reads, ragged tiles and
+    empty digits among them."""
+    rng = np.random.default_rng(9)
+    genome = _bases(rng, 60_000)
+    fa = b"".join(b">r%d\n" % i + genome[a:a + 60 + i % 90] + b"\n"
+                  for i, a in enumerate(rng.integers(0, 59_800, 12_000).tolist()))
+    bits = 10 if further == 0 else 14
+    n = sum(max(60 + i % 90 - k + 1, 0) for i in range(12_000))
+    cap = 1920 if k <= 32 else 1152
+    try:
+        # a factor that gives a bucket its share of n at that many bits
+        ctx.set_tuning(l1_bits=l1_bits, bucket_factor=1.01 * (n >> bits) / cap)
+        _p(f"case: levels k={k} l1_bits={l1_bits}")
+        ctx.count(fa, k)
+        t = ctx.timing()
+        assert (t["bucket_bits"], t["ms_levels"]) == (bits, further)
+        keys, counts = ctx.table_host()
+    finally:
+        ctx.set_tuning()
+    want_k, want_c = oracle_mod.count(fa, k)
+    assert np.array_equal(keys.reshape(-1), np.asarray(want_k).reshape(-1))
+    assert np.array_equal(counts, want_c)
