@@ -1827,7 +1827,8 @@ __global__ __launch_bounds__(SP_NT, 4) void k_split(const Key* __restrict__ Sin,
 // instead of the key, so one round covers the tile, and bytes that end no
 // k-mer cost only the first two passes.  Bound by VALU: with whole keys
 // exchanged through LDS in rounds it issued 115 lane instructions per one-word
-// key and took 783 us for 1.27e8 keys, now 474.
+// key and took 783 us for 2.5e8 keys, now 498.  (WPT = 2 at eight waves spills one
+// vector register.)
 constexpr int SM_NT = 1024;
 
 template <class Key, int WPT>
@@ -2419,7 +2420,8 @@ __global__ __launch_bounds__(256) void k_bits_count(const ull* W, uint32_t* cnt)
 // Blocks of 512 threads, as many waves per CU as the keys' registers allow.
 // Batches of a whole bucket: a second batch costs a second run map and its
 // barriers (k = 63, 1.5e8 keys: 2.46 ms with batches of 2048 against 1.41; k =
-// 32, 2.5e8 keys of 3900 a bucket: 1.30 with 4096, 1.17 with 5120).  Buckets up
+// 32, 2.5e8 keys of 3900 a bucket: 1.30 with 4096, 1.17 with 5120, both before
+// double hashing).  Buckets up
 // to a batch: fewer of them for the same keys (7.6e7 keys: 0.32 ms with 2300 a
 // bucket, 0.26 with 4600), and two partition levels instead of three more often
 // (2.9e9 two-word keys: 88.7 -> 82.4 ms).
@@ -3016,12 +3018,15 @@ __device__ __forceinline__ int count_task(HashShared<Key, MULTI>& L, const Key* 
 // distinct (timing copies): loads and map 0.69, inserts 0.23, ordering 0.27,
 // writes 0.16.  Sub-bins, vector clears, a DPP scan and one packed register for
 // (bin, index) took it from 1.51 to 1.34 ms; without the pass loops around the
-// single pass nothing is hoisted out of them and no register spills (the spills
-// moved 2.3 of 5.3 GB), which with larger batches gives 1.17.  Two-word keys
-// (1.5e8): 2.83 ms with 28-byte slots, 1.42 at 6 waves per SIMD, 1.17 at the 8
-// that fit without spills.  256 or 1024 threads and 2048 to 6144 slots were
-// within 10 % of each other; resident blocks that load the next bucket's keys
-// early, or a map built by all waves, were slower.
+// single pass no vector register spills (that moved 2.3 of 5.3 GB), which with
+// larger batches gave 1.14, and probes by double hashing 1.00.  84 scalar registers
+// are kept in vector lanes (66 for two-word keys): masks of the first eight
+// probes, which are unrolled; without that there are 5, and it is slower (1.3e8
+// keys, 0.72 distinct: 3.4 against 2.8 ms with the retry).  Two-word keys (1.5e8):
+// 2.83 ms with 28-byte slots, 1.42 at 6 waves per SIMD, 1.14 at the 8 that fit,
+// now 1.05.  256 or 1024 threads and 2048 to 6144 slots were within 10 % of each
+// other; resident blocks that load the next bucket's keys early, or a map built by
+// all waves, were slower.
 //
 // One block per bucket of `in`: tu[b] = the bucket's distinct keys, bstart[b]
 // = where they are.  Buckets the table is too small for are left to the retry
@@ -3051,8 +3056,11 @@ __global__ __launch_bounds__(HashCfg<Key>::NT, HashCfg<Key>::WAVES) void k_bucke
 }
 
 // The buckets left to it in several passes, every gridDim.x-th of the B buckets
-// to a block (a list of them by atomics on one counter took 50 ns a bucket); what
-// still fails goes to ovf_list with tu = -1 for the host-driven split.  Bound by
+// to a block (a list of them by atomics on one counter took 50 ns a bucket; eight
+// neighbours to a block read their counts in whole lines, 20 us less for 2^20
+// buckets, but the heavy buckets are neighbours: 8.8 ms against 1.3 for 2.1e7
+// builder words); what still fails goes to ovf_list with tu = -1 for the
+// host-driven split.  Bound by
 // latency: two blocks per CU, 112 to 128 VGPRs with a batch's keys in registers.
 // Bucket count of distinct-rich input, first try and this (before the tiled
 // partition; loading the keys for every pass, the first of them the one that had
